@@ -72,81 +72,75 @@ VKZG_DEV G1J g1j_from_affine(const G1A &a) {
     return r;
 }
 
+// dbl-2009-l with its additions folded into the products: W = 2 X Y^2,
+// X3 = E^2 - 4W, Y3 = E (2W - X3) - 8 Y^4, Z3 = 2 Y Z (E = 3 X^2).
 VKZG_DEV_CALL G1J g1j_dbl(const G1J &p) {
     if (fp_is_zero(p.z)) return p;
-    const Fp A = fp_sqr(p.x);
+    const Fp E = fp_triple(fp_sqr(p.x));
     const Fp B = fp_sqr(p.y);
     const Fp C = fp_sqr(B);
-    Fp t = fp_add(p.x, B);
-    t = fp_sqr(t);
-    t = fp_sub(t, A);
-    t = fp_sub(t, C);
-    const Fp D = fp_dbl(t);
-    const Fp E = fp_add(fp_dbl(A), A);
-    const Fp F = fp_sqr(E);
+    const Fp W = fp_mul(fp_dbl_raw(p.x), B);
     G1J r;
-    r.x = fp_sub(F, fp_dbl(D));
-    const Fp C8 = fp_dbl(fp_dbl(fp_dbl(C)));
-    r.y = fp_sub(fp_mul(E, fp_sub(D, r.x)), C8);
-    r.z = fp_dbl(fp_mul(p.y, p.z));
+    r.x = fp_sqr_fold(E, W, -4);
+    r.y = fp_mul_fold(E, fp_dbl_sub(W, r.x), C, -8);
+    r.z = fp_mul(fp_dbl_raw(p.y), p.z);
     return r;
 }
 
 VKZG_DEV_COLD G1J g1j_dbl_cold(const G1J &p);
 
-// add-2007-bl
+// add-2007-bl without its factors of two: H = U2 - U1, R = S2 - S1, V = U1 H^2,
+// X3 = R^2 - H^3 - 2V, Y3 = R (V - X3) - S1 H^3, Z3 = Z1 Z2 H.
 VKZG_DEV_CALL G1J g1j_add(const G1J &a, const G1J &b) {
     if (fp_is_zero(a.z)) return b;
     if (fp_is_zero(b.z)) return a;
     const Fp Z1Z1 = fp_sqr(a.z);
     const Fp Z2Z2 = fp_sqr(b.z);
     const Fp U1 = fp_mul(a.x, Z2Z2);
-    const Fp U2 = fp_mul(b.x, Z1Z1);
     const Fp S1 = fp_mul(a.y, fp_mul(b.z, Z2Z2));
-    const Fp S2 = fp_mul(b.y, fp_mul(a.z, Z1Z1));
-    if (fp_eq(U1, U2)) {
-        if (fp_eq(S1, S2)) return g1j_dbl_cold(a);
+    const Fp H = fp_mul_fold(b.x, Z1Z1, U1, -1);
+    const Fp R = fp_mul_fold(b.y, fp_mul(a.z, Z1Z1), S1, -1);
+    const Fp HH = fp_sqr(H);
+    if (fp_is_zero(HH)) {
+        if (fp_is_zero_mod(R)) return g1j_dbl_cold(a);
         return g1j_identity();
     }
-    const Fp H = fp_sub(U2, U1);
-    const Fp I = fp_sqr(fp_dbl(H));
-    const Fp J = fp_mul(H, I);
-    const Fp K = fp_dbl(fp_sub(S2, S1));
-    const Fp V = fp_mul(U1, I);
+    const Fp HHH = fp_mul(H, HH);
+    const Fp V = fp_mul(U1, HH);
     G1J r;
-    r.x = fp_sub(fp_sub(fp_sqr(K), J), fp_dbl(V));
-    r.y = fp_sub(fp_mul(K, fp_sub(V, r.x)), fp_dbl(fp_mul(S1, J)));
-    Fp z = fp_sqr(fp_add(a.z, b.z));
-    z = fp_sub(fp_sub(z, Z1Z1), Z2Z2);
-    r.z = fp_mul(z, H);
+    r.x = fp_sqr_fold2(R, HHH, -1, V, -2);
+    r.y = fp_mul_sum(R, fp_sub(V, r.x), S1, fp_neg(HHH));
+    r.z = fp_mul(fp_mul(a.z, b.z), H);
     return r;
 }
 
 VKZG_DEV_COLD G1J g1j_dbl_cold(const G1J &p) { return g1j_dbl(p); }
 
-// madd-2007-bl (b affine, may be the identity)
+// The same with b affine and not the identity, a not the identity: H and R
+// given, H not 0 mod p.
+VKZG_DEV G1J g1j_madd_tail(const G1J &a, const Fp &H, const Fp &HH, const Fp &R) {
+    const Fp HHH = fp_mul(H, HH);
+    const Fp V = fp_mul(a.x, HH);
+    G1J r;
+    r.x = fp_sqr_fold2(R, HHH, -1, V, -2);
+    r.y = fp_mul_sum(R, fp_sub(V, r.x), a.y, fp_neg(HHH));
+    r.z = fp_mul(a.z, H);
+    return r;
+}
+
+// madd (b affine, may be the identity)
 VKZG_DEV_CALL G1J g1j_madd(const G1J &a, const G1A &b) {
     if (g1a_is_identity(b)) return a;
     if (fp_is_zero(a.z)) return g1j_from_affine(b);
     const Fp Z1Z1 = fp_sqr(a.z);
-    const Fp U2 = fp_mul(b.x, Z1Z1);
-    const Fp S2 = fp_mul(b.y, fp_mul(a.z, Z1Z1));
-    if (fp_eq(a.x, U2)) {
-        if (fp_eq(a.y, S2)) return g1j_dbl_cold(a);
+    const Fp H = fp_mul_fold(b.x, Z1Z1, a.x, -1);
+    const Fp R = fp_mul_fold(b.y, fp_mul(a.z, Z1Z1), a.y, -1);
+    const Fp HH = fp_sqr(H);
+    if (fp_is_zero(HH)) {
+        if (fp_is_zero_mod(R)) return g1j_dbl_cold(a);
         return g1j_identity();
     }
-    const Fp H = fp_sub(U2, a.x);
-    const Fp HH = fp_sqr(H);
-    const Fp I = fp_dbl(fp_dbl(HH));
-    const Fp J = fp_mul(H, I);
-    const Fp K = fp_dbl(fp_sub(S2, a.y));
-    const Fp V = fp_mul(a.x, I);
-    G1J r;
-    r.x = fp_sub(fp_sub(fp_sqr(K), J), fp_dbl(V));
-    r.y = fp_sub(fp_mul(K, fp_sub(V, r.x)), fp_dbl(fp_mul(a.y, J)));
-    Fp z = fp_sqr(fp_add(a.z, H));
-    r.z = fp_sub(fp_sub(z, Z1Z1), HH);
-    return r;
+    return g1j_madd_tail(a, H, HH, R);
 }
 
 // Jacobian + affine for hot loops (see g1x_madd_fast for the contract).
@@ -154,20 +148,11 @@ VKZG_DEV G1J g1j_madd_fast(const G1J &a, const G1A &b, bool &exc) {
     if (g1a_is_identity(b)) return a;
     if (fp_is_zero(a.z)) return g1j_from_affine(b);
     const Fp Z1Z1 = fp_sqr(a.z);
-    const Fp U2 = fp_mul(b.x, Z1Z1);
-    const Fp S2 = fp_mul(b.y, fp_mul(a.z, Z1Z1));
-    const Fp H = fp_sub(U2, a.x);
-    exc |= fp_is_zero(H);
+    const Fp H = fp_mul_fold(b.x, Z1Z1, a.x, -1);
+    const Fp R = fp_mul_fold(b.y, fp_mul(a.z, Z1Z1), a.y, -1);
     const Fp HH = fp_sqr(H);
-    const Fp I = fp_dbl(fp_dbl(HH));
-    const Fp J = fp_mul(H, I);
-    const Fp K = fp_dbl(fp_sub(S2, a.y));
-    const Fp V = fp_mul(a.x, I);
-    G1J r;
-    r.x = fp_sub(fp_sub(fp_sqr(K), J), fp_dbl(V));
-    r.y = fp_sub(fp_mul(K, fp_sub(V, r.x)), fp_dbl(fp_mul(a.y, J)));
-    r.z = fp_sub(fp_sub(fp_sqr(fp_add(a.z, H)), Z1Z1), HH);
-    return r;
+    exc |= fp_is_zero(HH);
+    return g1j_madd_tail(a, H, HH, R);
 }
 
 VKZG_DEV G1J g1j_neg(const G1J &p) {
@@ -218,40 +203,44 @@ VKZG_DEV_CALL G1J g1j_from_xyzz(const G1X &p) {
     return r;
 }
 
-// dbl-2008-s-1
+// dbl-2008-s-1 in halves: V = 4 Y^2 and W = 8 Y^3 enter their products as
+// twice V2 = 2 Y^2 and W2 = 4 Y^3, so every operand stays within its class.
+// The identity (ZZ = ZZZ = 0) doubles to ZZ3 = ZZZ3 = 0, the identity again,
+// so no input has to stay live for a select; doubling has no exceptional case.
+VKZG_DEV G1X g1x_dbl_core(const G1X &p) {
+    const Fp V2 = fp_mul(fp_dbl_raw(p.y), p.y);
+    const Fp V = fp_dbl_raw(V2);
+    const Fp W2 = fp_mul(V, p.y);
+    const Fp S = fp_mul(V, p.x);
+    G1X r;
+    r.zz = fp_mul(V, p.zz);
+    r.zzz = fp_mul(fp_dbl_raw(W2), p.zzz);
+    const Fp M = fp_triple(fp_sqr(p.x));
+    r.x = fp_sqr_fold(M, S, -2);
+    r.y = fp_mul_sum(M, fp_sub(S, r.x), fp_dbl(W2), fp_neg(p.y));
+    return r;
+}
 VKZG_DEV_CALL G1X g1x_dbl(const G1X &p) {
     if (fp_is_zero(p.zz)) return p;
-    const Fp U = fp_dbl(p.y);
-    const Fp V = fp_sqr(U);
-    const Fp W = fp_mul(U, V);
-    const Fp S = fp_mul(p.x, V);
-    const Fp X2 = fp_sqr(p.x);
-    const Fp M = fp_add(fp_dbl(X2), X2);
-    G1X r;
-    r.x = fp_sub(fp_sqr(M), fp_dbl(S));
-    r.y = fp_sub(fp_mul(M, fp_sub(S, r.x)), fp_mul(W, p.y));
-    r.zz = fp_mul(V, p.zz);
-    r.zzz = fp_mul(W, p.zzz);
-    return r;
+    return g1x_dbl_core(p);
 }
 
 VKZG_DEV_COLD G1X g1x_dbl_cold(const G1X &p) { return g1x_dbl(p); }
 
-// g1x_dbl without the identity test: the identity (ZZ = ZZZ = 0) doubles to
-// ZZ3 = ZZZ3 = 0, the identity again, so no input has to stay live for a
-// select.  Never flags: doubling has no exceptional case.
-VKZG_DEV G1X g1x_dbl_core(const G1X &p) {
-    const Fp U = fp_dbl(p.y);
-    const Fp V = fp_sqr(U);
-    const Fp W = fp_mul(U, V);
+// The rest of an XYZZ addition once P = U2 - U1, PP = P^2 and R = S2 - S1
+// are there: (X1, Y1) are the first point's scaled coordinates (U1, S1; with
+// an affine second point its own X and Y), zz and zzz the product of both
+// points' ZZ and of both ZZZ.  X3 = R^2 - PPP - 2Q is folded into the square
+// and Y3 = R (Q - X3) - Y1 PPP takes one reduction for its two products.
+VKZG_DEV G1X g1x_add_tail(const Fp &X1, const Fp &Y1, const Fp &zz, const Fp &zzz, const Fp &P, const Fp &PP,
+                          const Fp &R) {
+    const Fp PPP = fp_mul(P, PP);
+    const Fp Q = fp_mul(X1, PP);
     G1X r;
-    r.zz = fp_mul(V, p.zz);
-    r.zzz = fp_mul(W, p.zzz);
-    const Fp S = fp_mul(p.x, V);
-    const Fp X2 = fp_sqr(p.x);
-    const Fp M = fp_add(fp_dbl(X2), X2);
-    r.x = fp_sub(fp_sqr(M), fp_dbl(S));
-    r.y = fp_mul_sum(M, fp_sub_lazy(S, r.x), p.y, fp_neg_lazy(W));
+    r.zz = fp_mul(zz, PP);
+    r.zzz = fp_mul(zzz, PPP);
+    r.x = fp_sqr_fold2(R, PPP, -1, Q, -2);
+    r.y = fp_mul_sum(R, fp_sub(Q, r.x), Y1, fp_neg(PPP));
     return r;
 }
 
@@ -259,23 +248,14 @@ VKZG_DEV G1X g1x_dbl_core(const G1X &p) {
 VKZG_DEV_CALL G1X g1x_madd(const G1X &a, const G1A &b) {
     if (g1a_is_identity(b)) return a;
     if (fp_is_zero(a.zz)) return g1x_from_affine(b);
-    const Fp U2 = fp_mul(b.x, a.zz);
-    const Fp S2 = fp_mul(b.y, a.zzz);
-    const Fp P = fp_sub(U2, a.x);
-    const Fp R = fp_sub(S2, a.y);
-    if (fp_is_zero(P)) {
-        if (fp_is_zero(R)) return g1x_dbl_cold(g1x_from_affine(b));
+    const Fp P = fp_mul_fold(b.x, a.zz, a.x, -1);
+    const Fp R = fp_mul_fold(b.y, a.zzz, a.y, -1);
+    const Fp PP = fp_sqr(P);
+    if (fp_is_zero(PP)) {
+        if (fp_is_zero_mod(R)) return g1x_dbl_cold(g1x_from_affine(b));
         return g1x_identity();
     }
-    const Fp PP = fp_sqr(P);
-    const Fp PPP = fp_mul(P, PP);
-    const Fp Q = fp_mul(a.x, PP);
-    G1X r;
-    r.x = fp_sub(fp_sub(fp_sqr(R), PPP), fp_dbl(Q));
-    r.y = fp_sub(fp_mul(R, fp_sub(Q, r.x)), fp_mul(a.y, PPP));
-    r.zz = fp_mul(a.zz, PP);
-    r.zzz = fp_mul(a.zzz, PPP);
-    return r;
+    return g1x_add_tail(a.x, a.y, a.zz, a.zzz, P, PP, R);
 }
 
 // Hot-loop variants.  When the inputs are equal or opposite (the doubling /
@@ -283,36 +263,25 @@ VKZG_DEV_CALL G1X g1x_madd(const G1X &a, const G1A &b) {
 // return an unspecified point; callers then recompute that result with the
 // checked forms above outside their loops.  Keeping the rare path out of the
 // loop body is what keeps the accumulator in VGPRs (a call inside the loop
-// that takes the point by address pins it to scratch memory).  P, R and
-// Q - X3 only feed products, so they are lazy (fp_sub_lazy), and P == 0 is
-// detected on PP = P^2.
+// that takes the point by address pins it to scratch memory).  P == 0 is
+// detected on PP = P^2, whose residue 0 is the zero limbs.
 
 // Accumulator step a + (+-b) for an accumulator that is never the identity
 // (callers start it from their first point).  b is an affine point in
 // normalised limbs, negated when `neg`; `exc` is also set when b is the
 // identity (all-zero limbs: no point of the prime-order group has y = 0).
 VKZG_DEV G1X g1x_madd_acc(const G1X &a, const G1A &b, bool neg, bool &exc) {
-    exc |= limbs_zero<kFpLimbs>(b.y.v);
-    const Fp by = fp_neg_lazy_if(b.y, neg);
-    const Fp U2 = fp_mul(b.x, a.zz);
-    const Fp S2 = fp_mul(by, a.zzz);
-    const Fp P = fp_sub_lazy(U2, a.x);
-    const Fp R = fp_sub_lazy(S2, a.y);
+    exc |= fp_is_zero(b.y);
+    const Fp P = fp_mul_fold(b.x, a.zz, a.x, -1);
+    const Fp R = fp_mul_fold(fp_cond_neg(b.y, neg), a.zzz, a.y, -1);
     const Fp PP = fp_sqr(P);
     exc |= fp_is_zero(PP);
-    const Fp PPP = fp_mul(P, PP);
-    const Fp Q = fp_mul(a.x, PP);
-    G1X r;
-    r.x = fp_sub(fp_sub(fp_sqr(R), PPP), fp_dbl(Q));
-    r.y = fp_mul_sum(R, fp_sub_lazy(Q, r.x), a.y, fp_neg_lazy(PPP));
-    r.zz = fp_mul(a.zz, PP);
-    r.zzz = fp_mul(a.zzz, PPP);
-    return r;
+    return g1x_add_tail(a.x, a.y, a.zz, a.zzz, P, PP, R);
 }
 
 // The first point of an accumulator: (+-b) in XYZZ; flags the identity.
 VKZG_DEV G1X g1x_start(const G1A &b, bool neg, bool &exc) {
-    exc |= limbs_zero<kFpLimbs>(b.y.v);
+    exc |= fp_is_zero(b.y);
     G1X r;
     r.x = b.x;
     r.y = fp_cond_neg(b.y, neg);
@@ -335,23 +304,14 @@ VKZG_DEV G1X g1x_madd_fast(const G1X &a, const G1A &b, bool &exc) {
 // register budget where two other points are live.
 VKZG_DEV G1X g1x_add_core(const G1X &a, const G1X &b, bool &exc) {
     const Fp U1 = fp_mul(a.x, b.zz);
-    const Fp U2 = fp_mul(b.x, a.zz);
+    const Fp P = fp_mul_fold(b.x, a.zz, U1, -1);
     const Fp ZZ12 = fp_mul(a.zz, b.zz);
     const Fp S1 = fp_mul(a.y, b.zzz);
-    const Fp S2 = fp_mul(b.y, a.zzz);
+    const Fp R = fp_mul_fold(b.y, a.zzz, S1, -1);
     const Fp ZZZ12 = fp_mul(a.zzz, b.zzz);
-    const Fp P = fp_sub_lazy(U2, U1);
-    const Fp R = fp_sub_lazy(S2, S1);
     const Fp PP = fp_sqr(P);
     exc |= fp_is_zero(PP);
-    const Fp PPP = fp_mul(P, PP);
-    const Fp Q = fp_mul(U1, PP);
-    G1X r;
-    r.zz = fp_mul(ZZ12, PP);
-    r.zzz = fp_mul(ZZZ12, PPP);
-    r.x = fp_sub(fp_sub(fp_sqr(R), PPP), fp_dbl(Q));
-    r.y = fp_mul_sum(R, fp_sub_lazy(Q, r.x), S1, fp_neg_lazy(PPP));
-    return r;
+    return g1x_add_tail(U1, S1, ZZ12, ZZZ12, P, PP, R);
 }
 
 // a + b for hot loops (see g1x_madd_acc for the `exc` contract); either may
@@ -371,92 +331,87 @@ VKZG_DEV_CALL G1X g1x_add(const G1X &a, const G1X &b) {
     if (fp_is_zero(a.zz)) return b;
     if (fp_is_zero(b.zz)) return a;
     const Fp U1 = fp_mul(a.x, b.zz);
-    const Fp U2 = fp_mul(b.x, a.zz);
+    const Fp P = fp_mul_fold(b.x, a.zz, U1, -1);
     const Fp S1 = fp_mul(a.y, b.zzz);
-    const Fp S2 = fp_mul(b.y, a.zzz);
-    const Fp P = fp_sub(U2, U1);
-    const Fp R = fp_sub(S2, S1);
-    if (fp_is_zero(P)) {
-        if (fp_is_zero(R)) return g1x_dbl_cold(a);
+    const Fp R = fp_mul_fold(b.y, a.zzz, S1, -1);
+    const Fp PP = fp_sqr(P);
+    if (fp_is_zero(PP)) {
+        if (fp_is_zero_mod(R)) return g1x_dbl_cold(a);
         return g1x_identity();
     }
-    const Fp PP = fp_sqr(P);
-    const Fp PPP = fp_mul(P, PP);
-    const Fp Q = fp_mul(U1, PP);
-    G1X r;
-    r.x = fp_sub(fp_sub(fp_sqr(R), PPP), fp_dbl(Q));
-    r.y = fp_sub(fp_mul(R, fp_sub(Q, r.x)), fp_mul(S1, PPP));
-    r.zz = fp_mul(fp_mul(a.zz, b.zz), PP);
-    r.zzz = fp_mul(fp_mul(a.zzz, b.zzz), PPP);
-    return r;
+    return g1x_add_tail(U1, S1, fp_mul(a.zz, b.zz), fp_mul(a.zzz, b.zzz), P, PP, R);
 }
 
 // The four lanes of a quad hold the same point(s) and share one operation:
 // its products are split into dependent rounds of at most four, and DPP quad
-// broadcasts give every lane each round's products.  Same formulas and
-// operand order as g1x_dbl (3 rounds instead of 9 products) and g1x_add_fast
-// (4 rounds instead of 14); sums that only feed products stay lazy.
+// broadcasts give every lane each round's products.  The same formulas as
+// g1x_dbl (3 rounds instead of 9 products) and g1x_add_fast (4 rounds instead
+// of 14).
 VKZG_DEV G1X g1x_dbl_quad(const G1X &p, uint32_t q) {
     if (fp_is_zero(p.zz)) return p;  // uniform in the quad
-    const Fp U = fp_add_lazy(p.y, p.y);  // U and M feed products only
-    const Fp r1 = fp_sqr((q & 1u) ? p.x : U);
-    const Fp V = fp_quad_bcast<0>(r1), X2 = fp_quad_bcast<1>(r1);
-    const Fp M = fp_triple_lazy(X2);
-    const Fp r2 = fp_mul(q == 0 ? U : (q == 1 ? p.x : (q == 2 ? M : V)), q == 2 ? M : (q == 3 ? p.zz : V));
-    const Fp W = fp_quad_bcast<0>(r2), S = fp_quad_bcast<1>(r2);
+    const bool odd = (q & 1u) != 0;
+    const Fp r1 = fp_mul(fp_select(odd, p.x, fp_dbl_raw(p.y)), fp_select(odd, p.x, p.y));
+    const Fp V = fp_dbl_raw(fp_quad_bcast<0>(r1));  // 4 Y^2
+    const Fp M = fp_triple(fp_quad_bcast<1>(r1));   // 3 X^2
+    const Fp r2 = fp_mul(fp_select(q == 2, M, V), q == 0 ? p.y : (q == 1 ? p.x : (q == 2 ? M : p.zz)));
+    const Fp W = fp_dbl_raw(fp_quad_bcast<0>(r2)), S = fp_quad_bcast<1>(r2);  // 8 Y^3, 4 X Y^2
     G1X r;
-    r.x = fp_sub(fp_quad_bcast<2>(r2), fp_dbl(S));  // M^2 - 2S
-    r.zz = fp_quad_bcast<3>(r2);                    // V ZZ
-    const Fp r3 = fp_mul(q == 0 ? M : W, q == 0 ? fp_sub_lazy(S, r.x) : (q == 1 ? p.y : p.zzz));
+    r.x = fp_neg(fp_dbl_sub(S, fp_quad_bcast<2>(r2)));  // M^2 - 2S
+    r.zz = fp_quad_bcast<3>(r2);                        // V ZZ
+    const Fp r3 = fp_mul(q == 0 ? fp_sub_raw(S, r.x) : W, q == 0 ? M : (q == 1 ? p.y : p.zzz));
     r.y = fp_sub(fp_quad_bcast<0>(r3), fp_quad_bcast<1>(r3));  // M (S - X3) - W Y
     r.zzz = fp_quad_bcast<2>(r3);                               // W ZZZ
     return r;
 }
 
+// Rounds: {U1, U2, S1, S2}, {PP, RR, ZZ1 ZZ2, ZZZ1 ZZZ2}, {PPP, Q, ZZ3, -X3},
+// {R (Q - X3), S1 PPP, ZZZ3}.  With PPP + 2Q = (U1 + U2) PP the fourth lane of
+// the third round makes -X3 = (U1 + U2) PP - R^2 itself.
 VKZG_DEV G1X g1x_add_quad(const G1X &a, const G1X &b, uint32_t q, bool &exc) {
     if (fp_is_zero(a.zz)) return b;  // uniform in the quad
     if (fp_is_zero(b.zz)) return a;
     const Fp r1 = fp_mul(q == 0 ? a.x : (q == 1 ? b.x : (q == 2 ? a.y : b.y)),
                          q == 0 ? b.zz : (q == 1 ? a.zz : (q == 2 ? b.zzz : a.zzz)));
-    const Fp U1 = fp_quad_bcast<0>(r1), S1 = fp_quad_bcast<2>(r1);
-    const Fp P = fp_sub_lazy(fp_quad_bcast<1>(r1), U1);  // U2 - U1
-    const Fp R = fp_sub_lazy(fp_quad_bcast<3>(r1), S1);  // S2 - S1
+    const Fp U1 = fp_quad_bcast<0>(r1), U2 = fp_quad_bcast<1>(r1);
+    const Fp S1 = fp_quad_bcast<2>(r1), S2 = fp_quad_bcast<3>(r1);
+    const Fp P = fp_sub(U2, U1), R = fp_sub(S2, S1);
     const Fp r2 = fp_mul(q == 0 ? P : (q == 1 ? R : (q == 2 ? a.zz : a.zzz)),
                          q == 0 ? P : (q == 1 ? R : (q == 2 ? b.zz : b.zzz)));
     const Fp PP = fp_quad_bcast<0>(r2), RR = fp_quad_bcast<1>(r2);
     const Fp ZZab = fp_quad_bcast<2>(r2), ZZZab = fp_quad_bcast<3>(r2);
     exc |= fp_is_zero(PP);
-    const Fp r3 = fp_mul(q == 0 ? P : (q == 1 ? U1 : ZZab), PP);
-    const Fp PPP = fp_quad_bcast<0>(r3), Q = fp_quad_bcast<1>(r3);
+    const Fp r3 = fp_mul_fold_v(q == 0 ? P : (q == 1 ? U1 : (q == 2 ? ZZab : fp_add_raw(U1, U2))), PP, RR,
+                              q == 3 ? -1 : 0);
+    const Fp PPP = fp_quad_bcast<0>(r3), Q = fp_quad_bcast<1>(r3), nX = fp_quad_bcast<3>(r3);
     G1X r;
     r.zz = fp_quad_bcast<2>(r3);
-    r.x = fp_sub(fp_sub(RR, PPP), fp_dbl(Q));
-    const Fp r4 = fp_mul(q == 0 ? R : (q == 1 ? S1 : ZZZab), q == 0 ? fp_sub_lazy(Q, r.x) : PPP);
+    r.x = fp_neg(nX);
+    const Fp r4 = fp_mul(q == 0 ? fp_add_raw(Q, nX) : PPP, q == 0 ? R : (q == 1 ? S1 : ZZZab));
     r.y = fp_sub(fp_quad_bcast<0>(r4), fp_quad_bcast<1>(r4));
     r.zzz = fp_quad_bcast<2>(r4);
     return r;
 }
 
 // g1x_madd_acc shared by the four lanes of a quad that all hold a, b and
-// neg: its products in four dependent rounds -- {U2, S2}, {P^2, R^2},
-// {P PP, X1 PP, ZZ1 PP}, {R (Q - X3), Y1 PPP, ZZZ1 PPP} -- instead of ten
-// products in a row; same operands and lazy sums, so the same field elements.
+// neg: its products in four dependent rounds -- {P = U2 - X1, R = S2 - Y1,
+// U2 + X1}, {P^2, R^2}, {P PP, X1 PP, ZZ1 PP, -X3 = (U2 + X1) PP - R^2},
+// {R (Q - X3), Y1 PPP, ZZZ1 PPP} -- instead of ten products in a row.
 VKZG_DEV G1X g1x_madd_acc_quad(const G1X &a, const G1A &b, bool neg, uint32_t q, bool &exc) {
-    exc |= limbs_zero<kFpLimbs>(b.y.v);
+    exc |= fp_is_zero(b.y);
     const bool odd = (q & 1u) != 0;
-    const Fp by = fp_neg_lazy_if(b.y, neg);
-    const Fp r1 = fp_mul(fp_select(odd, by, b.x), fp_select(odd, a.zzz, a.zz));
-    const Fp P = fp_sub_lazy(fp_quad_bcast<0>(r1), a.x);  // U2 - X1
-    const Fp R = fp_sub_lazy(fp_quad_bcast<1>(r1), a.y);  // S2 - Y1
+    const Fp by = fp_cond_neg(b.y, neg);
+    const Fp r1 = fp_mul_fold_v(fp_select(odd, by, b.x), fp_select(odd, a.zzz, a.zz), fp_select(odd, a.y, a.x),
+                              q == 2 ? 1 : -1);
+    const Fp P = fp_quad_bcast<0>(r1), R = fp_quad_bcast<1>(r1), V = fp_quad_bcast<2>(r1);
     const Fp r2 = fp_sqr(fp_select(odd, R, P));
     const Fp PP = fp_quad_bcast<0>(r2), RR = fp_quad_bcast<1>(r2);
     exc |= fp_is_zero(PP);
-    const Fp r3 = fp_mul(q == 0 ? P : (q == 1 ? a.x : a.zz), PP);
-    const Fp PPP = fp_quad_bcast<0>(r3), Q = fp_quad_bcast<1>(r3);
+    const Fp r3 = fp_mul_fold_v(q == 0 ? P : (q == 1 ? a.x : (q == 2 ? a.zz : V)), PP, RR, q == 3 ? -1 : 0);
+    const Fp PPP = fp_quad_bcast<0>(r3), Q = fp_quad_bcast<1>(r3), nX = fp_quad_bcast<3>(r3);
     G1X r;
     r.zz = fp_quad_bcast<2>(r3);
-    r.x = fp_sub(fp_sub(RR, PPP), fp_dbl(Q));
-    const Fp r4 = fp_mul(q == 0 ? R : (q == 1 ? a.y : a.zzz), q == 0 ? fp_sub_lazy(Q, r.x) : PPP);
+    r.x = fp_neg(nX);
+    const Fp r4 = fp_mul(q == 0 ? fp_add_raw(Q, nX) : PPP, q == 0 ? R : (q == 1 ? a.y : a.zzz));
     r.y = fp_sub(fp_quad_bcast<0>(r4), fp_quad_bcast<1>(r4));  // R (Q - X3) - Y1 PPP
     r.zzz = fp_quad_bcast<2>(r4);
     return r;
@@ -480,8 +435,8 @@ VKZG_DEV_CALL void g1a_compress_words(uint32_t *w, const G1A &p) {
         for (int i = 1; i < 12; i++) w[i] = 0;
         return;
     }
-    const Fp x = fp_to_canonical(p.x);
-    const Fp y = fp_to_canonical(p.y);
+    const FpU x = fp_to_canonical(p.x);
+    const FpU y = fp_to_canonical(p.y);
     uint32_t xw[12];
     fp_to_words(xw, x);
 #pragma unroll
@@ -514,7 +469,7 @@ VKZG_DEV bool g1a_decompress(G1A &out, const uint32_t *src) {
 #pragma unroll
     for (int k = 0; k < 12; k++) xw[k] = w[11 - k];
     xw[11] &= 0x1fffffffu;
-    const Fp x = fp_from_words(xw);
+    const FpU x = fp_from_words(xw);
     if (!fp_limbs_lt_p(x)) ok = false;
     const Fp xm = fp_from_canonical(x);
     const Fp rhs = fp_add(fp_mul(fp_sqr(xm), xm), fp_const(cfp::FOUR_M));

@@ -6,7 +6,7 @@
 // 96-bit column accumulator; r's top limb has a clear top bit, so one
 // conditional subtraction finishes.
 //
-// Fp: 14 x 28-bit limbs, radix 2^392, values in [0, 2p) (see the Fp section).
+// Fp: 13 signed limbs of 30 bits, radix 2^390 (field_fp.h).
 //
 // Semantics follow the reference's field library (src/shaders/field.glsl.inc
 // :69-297): the same field elements in Montgomery form; byte encodings are
@@ -18,17 +18,12 @@
 #include <cstdint>
 
 #include "constants.h"
-#include "inverse.h"
-
-#define VKZG_DEV __device__ __forceinline__
+#include "field_fp.h"
 
 namespace vkzg_amd {
 
 struct Fr {
     uint32_t v[8];
-};
-struct Fp {
-    uint32_t v[14];  // 28-bit limbs, see below
 };
 
 // ------------------------------------------------------------ limb helpers
@@ -418,391 +413,7 @@ VKZG_DEV void fr_to_be_words(uint32_t *w, const Fr &a) {
     for (int i = 0; i < 8; i++) w[7 - i] = __builtin_bswap32(a.v[i]);
 }
 
-// ------------------------------------------------------------------ Fp
-//
-// Fp in registers: 14 limbs of 28 bits (one per 32-bit word), Montgomery
-// form with radix R = 2^392, value kept in [0, 2p) ("almost reduced") with
-// every limb below 2^28.
-//  - Limb products are below 2^56, so one Montgomery column (at most 28
-//    products plus the incoming carry) fits a single 64-bit accumulator: each
-//    product is one v_mad_u64_u32 and no carry is propagated inside a column.
-//  - 4p < R, so the Montgomery product of two values below 2p is below 2p
-//    and needs no final subtraction.
-//  - add/sub bring their result back to [0, 2p) with one conditional
-//    correction by 2p; comparisons and encodings reduce to [0, p) first
-//    (fp_canonical).
-
-constexpr int kFpLimbs = 14;
-constexpr uint32_t kFpMask = (1u << 28) - 1u;
-
-VKZG_DEV Fp fp_zero() {
-    Fp r;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) r.v[i] = 0;
-    return r;
-}
-VKZG_DEV Fp fp_const(const uint32_t (&c)[kFpLimbs]) {
-    Fp r;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) r.v[i] = c[i];
-    return r;
-}
-VKZG_DEV Fp fp_one() { return fp_const(cfp::ONE); }
-
-// acc += x * y: the compiler emits one v_mad_u64_u32 (no carry-out needed,
-// the accumulator cannot overflow).
-VKZG_DEV void fp_mac(uint64_t &acc, uint32_t x, uint32_t y) { acc += (uint64_t)x * y; }
-
-// Montgomery multiplication by finely integrated product scanning: column k
-// of a*b and of m*p share the accumulator, m_k = low 28 bits * N0 clears the
-// low limb of columns k < 14, and the accumulator shifts down 28 bits per
-// column.  Inputs below 2p give a result below 2p (no final subtraction).
-VKZG_DEV Fp fp_mul(const Fp &a, const Fp &b) {
-    uint32_t m[kFpLimbs];
-    uint64_t acc = 0;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) {
-#pragma unroll
-        for (int j = 0; j < i; j++) {
-            fp_mac(acc, a.v[j], b.v[i - j]);
-            fp_mac(acc, m[j], cfp::P[i - j]);
-        }
-        fp_mac(acc, a.v[i], b.v[0]);
-        m[i] = ((uint32_t)acc * cfp::N0) & kFpMask;
-        fp_mac(acc, m[i], cfp::P[0]);
-        acc >>= 28;
-    }
-    Fp r;
-#pragma unroll
-    for (int i = kFpLimbs; i < 2 * kFpLimbs; i++) {
-#pragma unroll
-        for (int j = i - kFpLimbs + 1; j < kFpLimbs; j++) {
-            fp_mac(acc, a.v[j], b.v[i - j]);
-            fp_mac(acc, m[j], cfp::P[i - j]);
-        }
-        r.v[i - kFpLimbs] = (uint32_t)acc & kFpMask;
-        acc >>= 28;
-    }
-    return r;
-}
-// a^2: the off-diagonal products of a column are summed once and doubled
-// (one v_lshl_add_u64), 105 limb products instead of 196.
-VKZG_DEV Fp fp_sqr(const Fp &a) {
-    uint32_t m[kFpLimbs];
-    uint64_t acc = 0;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) {
-        uint64_t t = 0;
-#pragma unroll
-        for (int j = 0; 2 * j < i; j++) fp_mac(t, a.v[j], a.v[i - j]);
-        acc += t << 1;
-        if ((i & 1) == 0) fp_mac(acc, a.v[i / 2], a.v[i / 2]);
-#pragma unroll
-        for (int j = 0; j < i; j++) fp_mac(acc, m[j], cfp::P[i - j]);
-        m[i] = ((uint32_t)acc * cfp::N0) & kFpMask;
-        fp_mac(acc, m[i], cfp::P[0]);
-        acc >>= 28;
-    }
-    Fp r;
-#pragma unroll
-    for (int i = kFpLimbs; i < 2 * kFpLimbs; i++) {
-        uint64_t t = 0;
-#pragma unroll
-        for (int j = i - kFpLimbs + 1; 2 * j < i; j++) fp_mac(t, a.v[j], a.v[i - j]);
-        acc += t << 1;
-        if ((i & 1) == 0) fp_mac(acc, a.v[i / 2], a.v[i / 2]);
-#pragma unroll
-        for (int j = i - kFpLimbs + 1; j < kFpLimbs; j++) fp_mac(acc, m[j], cfp::P[i - j]);
-        r.v[i - kFpLimbs] = (uint32_t)acc & kFpMask;
-        acc >>= 28;
-    }
-    return r;
-}
-
-// Lazy forms, valid only as inputs of fp_mul / fp_sqr: limbs below 3 * 2^28
-// and values below 6p.  A Montgomery column of two such inputs stays below
-// 14 * 9 * 2^56 + 14 * 2^56 + carry < 2^63.2, and 36p < R keeps the product
-// below 2p.  P4S is 4p with every limb but the top one in [2^28 - 1, 2^29),
-// so subtracting a normalised value below 2p leaves no negative limb.
-VKZG_DEV Fp fp_sub_lazy(const Fp &a, const Fp &b) {
-    Fp r;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) r.v[i] = a.v[i] + cfp::P4S[i] - b.v[i];
-    return r;
-}
-// a + b and 3a limb by limb, for normalised inputs below 2p: limbs below
-// 3 * 2^28 and values below 6p, the lazy form above.
-VKZG_DEV Fp fp_add_lazy(const Fp &a, const Fp &b) {
-    Fp r;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) r.v[i] = a.v[i] + b.v[i];
-    return r;
-}
-VKZG_DEV Fp fp_triple_lazy(const Fp &a) {
-    Fp r;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) r.v[i] = 3 * a.v[i];
-    return r;
-}
-VKZG_DEV Fp fp_neg_lazy_if(const Fp &a, bool neg) {
-    Fp r;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) r.v[i] = neg ? cfp::P4S[i] - a.v[i] : a.v[i];
-    return r;
-}
-// 4p - a limb by limb for a normalised a < 2p: limbs below 2^29, value in
-// (2p, 4p], congruent to -a.
-VKZG_DEV Fp fp_neg_lazy(const Fp &a) {
-    Fp r;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) r.v[i] = cfp::P4S[i] - a.v[i];
-    return r;
-}
-
-// a*b + c*d with one Montgomery reduction: the two products and m*p share
-// fp_mul's column accumulators, so the second product costs its 196 limb
-// products and no reduction of its own.  Contract: a and b lazy (limbs below
-// 3 * 2^28, values below 6p), c normalised (limbs below 2^28, value below
-// 2p), d limbs below 2^29 and value below 4p.  A column then stays below
-// 14 * (9 + 2 + 1) * 2^56 + carry < 2^63.4, and a*b + c*d < 44p^2 keeps the
-// result below p + 44p^2/R < 2p.
-VKZG_DEV Fp fp_mul_sum(const Fp &a, const Fp &b, const Fp &c, const Fp &d) {
-    uint32_t m[kFpLimbs];
-    uint64_t acc = 0;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) {
-#pragma unroll
-        for (int j = 0; j < i; j++) {
-            fp_mac(acc, a.v[j], b.v[i - j]);
-            fp_mac(acc, c.v[j], d.v[i - j]);
-            fp_mac(acc, m[j], cfp::P[i - j]);
-        }
-        fp_mac(acc, a.v[i], b.v[0]);
-        fp_mac(acc, c.v[i], d.v[0]);
-        m[i] = ((uint32_t)acc * cfp::N0) & kFpMask;
-        fp_mac(acc, m[i], cfp::P[0]);
-        acc >>= 28;
-    }
-    Fp r;
-#pragma unroll
-    for (int i = kFpLimbs; i < 2 * kFpLimbs; i++) {
-#pragma unroll
-        for (int j = i - kFpLimbs + 1; j < kFpLimbs; j++) {
-            fp_mac(acc, a.v[j], b.v[i - j]);
-            fp_mac(acc, c.v[j], d.v[i - j]);
-            fp_mac(acc, m[j], cfp::P[i - j]);
-        }
-        r.v[i - kFpLimbs] = (uint32_t)acc & kFpMask;
-        acc >>= 28;
-    }
-    return r;
-}
-
-// a + b in [0, 2p): s = a + b and t = s - 2p with their own signed carry
-// chains; t when non-negative.
-VKZG_DEV Fp fp_add(const Fp &a, const Fp &b) {
-    Fp s, t;
-    int32_t cs = 0, ct = 0;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) {
-        const int32_t x = (int32_t)(a.v[i] + b.v[i]) + cs;
-        s.v[i] = (uint32_t)x & kFpMask;
-        cs = x >> 28;
-        const int32_t y = (int32_t)s.v[i] - (int32_t)cfp::P2[i] + ct;
-        t.v[i] = (uint32_t)y & kFpMask;
-        ct = y >> 28;
-    }
-    Fp r;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) r.v[i] = ct < 0 ? s.v[i] : t.v[i];
-    return r;
-}
-VKZG_DEV Fp fp_dbl(const Fp &a) { return fp_add(a, a); }
-
-// a - b in [0, 2p): d = a - b (two's complement over 392 bits) and d + 2p;
-// the latter when d is negative.
-VKZG_DEV Fp fp_sub(const Fp &a, const Fp &b) {
-    Fp d, e;
-    int32_t cd = 0, ce = 0;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) {
-        const int32_t x = (int32_t)a.v[i] - (int32_t)b.v[i] + cd;
-        d.v[i] = (uint32_t)x & kFpMask;
-        cd = x >> 28;
-        const int32_t y = (int32_t)d.v[i] + (int32_t)cfp::P2[i] + ce;
-        e.v[i] = (uint32_t)y & kFpMask;
-        ce = y >> 28;
-    }
-    Fp r;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) r.v[i] = cd < 0 ? e.v[i] : d.v[i];
-    return r;
-}
-VKZG_DEV Fp fp_neg(const Fp &a) { return fp_sub(fp_zero(), a); }
-
-// [0, 2p) -> [0, p)
-VKZG_DEV Fp fp_canonical(const Fp &a) {
-    Fp t;
-    int32_t c = 0;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) {
-        const int32_t y = (int32_t)a.v[i] - (int32_t)cfp::P[i] + c;
-        t.v[i] = (uint32_t)y & kFpMask;
-        c = y >> 28;
-    }
-    Fp r;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) r.v[i] = c < 0 ? a.v[i] : t.v[i];
-    return r;
-}
-// For a value in [0, 2p): zero iff its limbs are those of 0 or of p.
-VKZG_DEV bool fp_is_zero(const Fp &a) {
-    uint32_t z = 0, zp = 0;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) {
-        z |= a.v[i];
-        zp |= a.v[i] ^ cfp::P[i];
-    }
-    return z == 0 || zp == 0;
-}
-VKZG_DEV bool fp_eq(const Fp &a, const Fp &b) {
-    return limbs_eq<kFpLimbs>(fp_canonical(a).v, fp_canonical(b).v);
-}
-// c ? a : b limb by limb (v_cndmask), so a lane-varying choice between two
-// register values never goes through an address.
-VKZG_DEV Fp fp_select(bool c, const Fp &a, const Fp &b) {
-    Fp r;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) r.v[i] = c ? a.v[i] : b.v[i];
-    return r;
-}
-VKZG_DEV Fp fp_cond_neg(const Fp &a, bool neg) {
-    const Fp n = fp_neg(a);
-    Fp r;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) r.v[i] = neg ? n.v[i] : a.v[i];
-    return r;
-}
-
-// Montgomery -> canonical integer in [0, p).
-VKZG_DEV Fp fp_to_canonical(const Fp &a) {
-    Fp one = fp_zero();
-    one.v[0] = 1;
-    return fp_canonical(fp_mul(a, one));
-}
-// Integer below p (28-bit limbs) -> Montgomery form.
-VKZG_DEV Fp fp_from_canonical(const Fp &a) { return fp_mul(a, fp_const(cfp::R2)); }
-
-// 12 little-endian 32-bit words (a value below 2^384) <-> 28-bit limbs.
-VKZG_DEV Fp fp_from_words(const uint32_t (&w)[12]) {
-    Fp r;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) {
-        const int bit = 28 * i, wi = bit >> 5, sh = bit & 31;
-        uint32_t x = w[wi] >> sh;
-        if (sh > 4 && wi + 1 < 12) x |= w[wi + 1] << (32 - sh);
-        r.v[i] = x & kFpMask;
-    }
-    return r;
-}
-VKZG_DEV void fp_to_words(uint32_t (&w)[12], const Fp &a) {
-#pragma unroll
-    for (int k = 0; k < 12; k++) {
-        const int bit = 32 * k, li = bit / 28, sh = bit % 28;
-        uint32_t x = a.v[li] >> sh;
-        if (li + 1 < kFpLimbs) x |= a.v[li + 1] << (28 - sh);
-        if (sh > 24 && li + 2 < kFpLimbs) x |= a.v[li + 2] << (56 - sh);
-        w[k] = x;
-    }
-}
-// a < p for a value in 28-bit limbs
-VKZG_DEV bool fp_limbs_lt_p(const Fp &a) {
-    int32_t c = 0;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) c = ((int32_t)a.v[i] - (int32_t)cfp::P[i] + c) >> 28;
-    return c < 0;
-}
-
-template <int NE>
-VKZG_DEV Fp fp_pow_const(const Fp &a, const uint32_t (&e)[NE]) {
-    Fp acc = fp_one();
-#pragma unroll 1
-    for (int i = NE - 1; i >= 0; i--) {
-        const uint32_t limb = e[i];
-#pragma unroll 1
-        for (int b = 31; b >= 0; b--) {
-            acc = fp_sqr(acc);
-            if ((limb >> b) & 1u) acc = fp_mul(acc, a);
-        }
-    }
-    return acc;
-}
-VKZG_DEV Fp fp_inv_fermat(const Fp &a) { return fp_pow_const<12>(a, cfp::P_MINUS_2); }
-
-// a^e for a constant exponent by a sliding window of 4 bits over the odd
-// powers a, a^3, ..., a^15: the same squarings as fp_pow_const and about a
-// fifth of its multiplications.
-template <int NE>
-VKZG_DEV Fp fp_pow_const_window(const Fp &a, const uint32_t (&e)[NE]) {
-    Fp odd[8];
-    odd[0] = a;
-    const Fp a2 = fp_sqr(a);
-#pragma unroll
-    for (int k = 1; k < 8; k++) odd[k] = fp_mul(odd[k - 1], a2);
-    Fp acc = fp_one();
-    int i = NE * 32 - 1;
-    while (i >= 0 && !((e[i / 32] >> (i % 32)) & 1u)) i--;
-    bool started = false;
-#pragma unroll 1
-    while (i >= 0) {
-        if (!((e[i / 32] >> (i % 32)) & 1u)) {
-            acc = fp_sqr(acc);
-            i--;
-            continue;
-        }
-        // longest window of at most 4 bits ending in a set bit
-        int j = i - 3 < 0 ? 0 : i - 3;
-        while (!((e[j / 32] >> (j % 32)) & 1u)) j++;
-        uint32_t w = 0;
-        for (int k = i; k >= j; k--) w = (w << 1) | ((e[k / 32] >> (k % 32)) & 1u);
-        if (started) {
-            for (int k = i; k >= j; k--) acc = fp_sqr(acc);
-            acc = fp_mul(acc, odd[w >> 1]);
-        } else {
-            acc = odd[w >> 1];
-            started = true;
-        }
-        i = j - 1;
-    }
-    return acc;
-}
-
-// Inverse of a Montgomery value xR (0 -> 0): the binary GCD of inverse.h gives
-// the plain inverse (xR)^-1 as a signed value in (-31p, 31p); adding 32p makes
-// it non-negative and a Montgomery product by R^3 turns it into x^-1 R.
-VKZG_DEV Fp fp_inv(const Fp &a) {
-    if (fp_is_zero(a)) return fp_zero();
-    int32_t v[kFpLimbs];
-    if (!bgcd::inverse(v, a.v)) return fp_inv_fermat(a);
-    Fp t;
-    int64_t c = 0;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) {
-        c += (int64_t)v[i] + cfp::P32[i];
-        t.v[i] = (uint32_t)c & kFpMask;
-        c >>= 28;
-    }
-    return fp_mul(t, fp_const(cfp::R3_M));
-}
-
-// canonical value > (p-1)/2 (the sign flag of the compressed encoding)
-VKZG_DEV bool fp_is_lex_largest(const Fp &canonical) {
-    // (p-1)/2 < x  <=>  HALF - x < 0
-    int32_t c = 0;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) c = ((int32_t)cfp::HALF[i] - (int32_t)canonical.v[i] + c) >> 28;
-    return c < 0;
-}
+// ------------------------------------------------------ Fp across lanes
 
 // The value lane k of this lane's quad holds (DPP quad_perm [k,k,k,k]), word
 // by word; the quad's four lanes must all be active.
@@ -811,7 +422,7 @@ VKZG_DEV Fp fp_quad_bcast(const Fp &v) {
     Fp r;
 #pragma unroll
     for (int i = 0; i < kFpLimbs; i++)
-        r.v[i] = (uint32_t)__builtin_amdgcn_mov_dpp((int)v.v[i], K * 0x55, 0xf, 0xf, false);
+        r.v[i] = __builtin_amdgcn_mov_dpp(v.v[i], K * 0x55, 0xf, 0xf, false);
     return r;
 }
 
@@ -822,32 +433,8 @@ VKZG_DEV Fp fp_pair_bcast(const Fp &v) {
     Fp r;
 #pragma unroll
     for (int i = 0; i < kFpLimbs; i++)
-        r.v[i] = (uint32_t)__builtin_amdgcn_mov_dpp((int)v.v[i], K ? 0xF5 : 0xA0, 0xf, 0xf, false);
+        r.v[i] = __builtin_amdgcn_mov_dpp(v.v[i], K ? 0xF5 : 0xA0, 0xf, 0xf, false);
     return r;
-}
-
-// Reference Montgomery product (operand scanning, plain C++) for the test
-// hooks: same radix and limbs, fully reduced.
-VKZG_DEV Fp fp_mul_reference(const Fp &a, const Fp &b) {
-    uint64_t t[kFpLimbs + 2];
-#pragma unroll
-    for (int j = 0; j < kFpLimbs + 2; j++) t[j] = 0;
-    for (int i = 0; i < kFpLimbs; i++) {
-        for (int j = 0; j < kFpLimbs; j++) t[j] += (uint64_t)a.v[j] * b.v[i];
-        const uint32_t m = ((uint32_t)t[0] * cfp::N0) & kFpMask;
-        for (int j = 0; j < kFpLimbs; j++) t[j] += (uint64_t)m * cfp::P[j];
-        // t[0] is now divisible by 2^28: shift the whole array one limb down
-        uint64_t carry = t[0] >> 28;
-        for (int j = 1; j <= kFpLimbs; j++) {
-            const uint64_t v = t[j] + carry;
-            t[j - 1] = v & kFpMask;
-            carry = v >> 28;
-        }
-        t[kFpLimbs] = carry;
-    }
-    Fp r;
-    for (int j = 0; j < kFpLimbs; j++) r.v[j] = (uint32_t)t[j];
-    return fp_canonical(r);
 }
 
 }  // namespace vkzg_amd

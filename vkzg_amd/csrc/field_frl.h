@@ -75,6 +75,9 @@ VKZG_DEV FrL frl_const(const uint32_t (&c)[9]) {
     return r;
 }
 
+// acc += x * y, one v_mad_u64_u32 (the accumulator cannot overflow).
+VKZG_DEV void frl_mac(uint64_t &acc, uint32_t x, uint32_t y) { acc += (uint64_t)x * y; }
+
 VKZG_DEV FrL frl_mul(const FrL &a, const FrL &b) {
     uint32_t m[9];
     uint64_t acc = 0;
@@ -82,10 +85,10 @@ VKZG_DEV FrL frl_mul(const FrL &a, const FrL &b) {
     for (int i = 0; i < 9; i++) {
 #pragma unroll
         for (int j = 0; j < i; j++) {
-            fp_mac(acc, a.v[j], b.v[i - j]);
-            fp_mac(acc, m[j], cfrl::P[i - j]);
+            frl_mac(acc, a.v[j], b.v[i - j]);
+            frl_mac(acc, m[j], cfrl::P[i - j]);
         }
-        fp_mac(acc, a.v[i], b.v[0]);
+        frl_mac(acc, a.v[i], b.v[0]);
         m[i] = (0u - (uint32_t)acc) & cfrl::kMask;  // P[0] = 1
         acc += m[i];
         acc >>= 29;
@@ -95,8 +98,8 @@ VKZG_DEV FrL frl_mul(const FrL &a, const FrL &b) {
     for (int i = 9; i < 18; i++) {
 #pragma unroll
         for (int j = i - 8; j < 9; j++) {
-            fp_mac(acc, a.v[j], b.v[i - j]);
-            fp_mac(acc, m[j], cfrl::P[i - j]);
+            frl_mac(acc, a.v[j], b.v[i - j]);
+            frl_mac(acc, m[j], cfrl::P[i - j]);
         }
         r.v[i - 9] = (uint32_t)acc & cfrl::kMask;
         acc >>= 29;

@@ -7,8 +7,9 @@ integers, so the header is reproducible:  python3 gen_constants.py > constants.h
 
 P = 0x1A0111EA397FE69A4B1BA7B6434BACD764774B84F38512BF6730D2A0F6B0F6241EABFFFEB153FFFFB9FEFFFFFFFFAAAB
 R = 0x73EDA753299D7D483339D80809A1D80553BDA402FFFE5BFEFFFFFFFF00000001
-FP_LIMBS, FP_BITS = 14, 28  # Fp in registers: 14 limbs of 28 bits
-RP = 1 << (FP_LIMBS * FP_BITS)  # Montgomery radix for Fp, 2^392
+FP_LIMBS, FP_BITS = 13, 30  # Fp in registers: 13 signed limbs of 30 bits
+RP = 1 << (FP_LIMBS * FP_BITS)  # Montgomery radix for Fp, 2^390
+GCD_LIMBS, GCD_BITS = 14, 28  # Fp inside the binary-GCD inversion
 RR = 1 << 256  # Montgomery radix for Fr
 # Endomorphism constants of BLS12-381 G1: beta is a cube root of unity in Fp,
 # lambda the matching cube root of unity in Fr with phi(x, y) = (beta*x, y) = lambda*P.
@@ -42,46 +43,53 @@ def arr(name, x, n):
     return "constexpr uint32_t %s[%d] = {%s};" % (name, n, body)
 
 
-def arr28(name, x):
-    assert 0 <= x < 1 << (FP_LIMBS * FP_BITS)
-    body = ", ".join("0x%07xu" % ((x >> (FP_BITS * i)) & ((1 << FP_BITS) - 1)) for i in range(FP_LIMBS))
-    return "constexpr uint32_t %s[%d] = {%s};" % (name, FP_LIMBS, body)
+def arr30(name, x):
+    """x in balanced limbs: 30-bit digits in [-2^29, 2^29), the top one what remains."""
+    assert 0 <= x < 1 << (FP_LIMBS * FP_BITS - 2)
+    d = []
+    for _ in range(FP_LIMBS - 1):
+        v = x & ((1 << FP_BITS) - 1)
+        if v >> (FP_BITS - 1):
+            v -= 1 << FP_BITS
+        d.append(v)
+        x = (x - v) >> FP_BITS
+    d.append(x)
+    return "constexpr int32_t %s[%d] = {%s};" % (name, FP_LIMBS, ", ".join("%d" % v for v in d))
+
+
+def arr_digits(name, x, n, bits):
+    """x in n unsigned digits of that many bits."""
+    assert 0 <= x < 1 << (n * bits)
+    body = ", ".join("0x%xu" % ((x >> (bits * i)) & ((1 << bits) - 1)) for i in range(n))
+    return "constexpr uint32_t %s[%d] = {%s};" % (name, n, body)
 
 
 def main():
     out = []
     out.append("// Generated by gen_constants.py -- BLS12-381 field constants, little-endian limbs:")
-    out.append("// Fp values in 28-bit limbs (14 of them, Montgomery radix 2^392), Fp exponents")
-    out.append("// and all Fr values in 32-bit limbs.")
+    out.append("// Fp values in balanced 30-bit limbs (13 of them, Montgomery radix 2^390), Fp")
+    out.append("// exponents and all Fr values in 32-bit limbs.")
     out.append("#pragma once")
     out.append("#include <cstdint>")
     out.append("namespace vkzg_amd {")
     out.append("namespace cfp {")
-    assert 4 * P < RP  # Montgomery products of values below 2p stay below 2p
-    out.append(arr28("P", P))
-    out.append(arr28("P2", 2 * P))
-    out.append("constexpr uint32_t N0 = 0x%07xu;  // -p^-1 mod 2^28" % ((-pow(P, -1, 1 << FP_BITS)) % (1 << FP_BITS)))
-    out.append(arr28("ONE", RP % P))
-    out.append(arr28("R2", RP * RP % P))
-    out.append(arr28("HALF", (P - 1) // 2))
-    out.append(arr28("FOUR_M", 4 * RP % P))
-    out.append(arr28("BETA_M", BETA * RP % P))
-    # 4p with every limb but the top raised into [2^28 - 1, 2^29) by
-    # borrowing from the limb above: 4p - b then has no negative limb for any
-    # b < 2p in normalised 28-bit limbs.
-    for name, mult in (("P4S", 4),):
-        v = mult * P
-        n = [(v >> (FP_BITS * i)) & ((1 << FP_BITS) - 1) for i in range(FP_LIMBS)]
-        c = [n[0] + (1 << FP_BITS)] + [n[i] + (1 << FP_BITS) - 1 for i in range(1, FP_LIMBS - 1)] + [n[-1] - 1]
-        assert sum(x << (FP_BITS * i) for i, x in enumerate(c)) == v
-        assert all((1 << FP_BITS) - 1 <= x < 1 << (FP_BITS + 1) for x in c[:-1])
-        assert c[-1] >= ((2 * P - 1) >> (FP_BITS * (FP_LIMBS - 1)))  # top limb of any b < 2p
-        out.append("constexpr uint32_t %s[%d] = {%s};" % (name, FP_LIMBS, ", ".join("0x%08xu" % x for x in c)))
-    out.append(arr28("R3_M", RP ** 3 % P))  # Montgomery form of R^2: turns a plain inverse of xR into x^-1 R
-    out.append(arr28("P32", 32 * P))       # added to the signed binary-GCD result to make it non-negative
+    out.append(arr30("P", P))
+    out.append("constexpr uint32_t N0 = 0x%xu;  // -p^-1 mod 2^32" % ((-pow(P, -1, 1 << 32)) % (1 << 32)))
+    out.append(arr30("ONE", RP % P))
+    out.append(arr30("R2", RP * RP % P))
+    out.append(arr30("FOUR_M", 4 * RP % P))
+    out.append(arr30("BETA_M", BETA * RP % P))
+    out.append(arr30("R3_M", RP ** 3 % P))  # Montgomery form of R^2: turns a plain inverse of xR into x^-1 R
     # 2^384 mod p as a plain value: a Montgomery product of x R by it gives
     # x 2^384 mod p, the reference's 12 x 32-bit Montgomery form (tables file v1)
-    out.append(arr28("REF_R", (1 << 384) % P))
+    out.append(arr30("REF_R", (1 << 384) % P))
+    out.append("// p and (p - 1) / 2 in unsigned 30-bit digits")
+    out.append(arr_digits("PU", P, FP_LIMBS, FP_BITS))
+    out.append(arr_digits("HALFU", (P - 1) // 2, FP_LIMBS, FP_BITS))
+    out.append("// p, -p^-1 mod 2^28 and 32p in the 28-bit limbs of the binary-GCD inversion")
+    out.append(arr_digits("GCD_P", P, GCD_LIMBS, GCD_BITS))
+    out.append("constexpr uint32_t GCD_N0 = 0x%07xu;" % ((-pow(P, -1, 1 << GCD_BITS)) % (1 << GCD_BITS)))
+    out.append(arr_digits("GCD_P32", 32 * P, GCD_LIMBS, GCD_BITS))  # makes the signed GCD result non-negative
     out.append("// exponents, 32-bit words")
     out.append(arr("P_MINUS_2", P - 2, 12))
     out.append(arr("SQRT_EXP", (P + 1) // 4, 12))
@@ -95,9 +103,9 @@ def main():
         g1 = f2pow((1, 1), m * (P - 1) // 6)
         g2 = f2pow((1, 1), m * (P * P - 1) // 6)
         assert g2[1] == 0
-        out.append(arr28("FROB1_%d_C0" % m, g1[0] * RP % P))
-        out.append(arr28("FROB1_%d_C1" % m, g1[1] * RP % P))
-        out.append(arr28("FROB2_%d" % m, g2[0] * RP % P))
+        out.append(arr30("FROB1_%d_C0" % m, g1[0] * RP % P))
+        out.append(arr30("FROB1_%d_C1" % m, g1[1] * RP % P))
+        out.append(arr30("FROB2_%d" % m, g2[0] * RP % P))
     out.append("}  // namespace cfp")
     out.append("namespace cfr {")
     out.append(arr("P", R, 8))

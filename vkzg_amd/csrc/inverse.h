@@ -71,11 +71,11 @@ VKZG_HD void negate(uint32_t (&r)[kLimbs]) {
 VKZG_HD void lin_shift_mod(int32_t (&r)[kLimbs], const int32_t (&u)[kLimbs], const int32_t (&v)[kLimbs],
                            int32_t f, int32_t g) {
     int64_t c = (int64_t)u[0] * f + (int64_t)v[0] * g;
-    const uint32_t q = ((uint32_t)c * cfp::N0) & kMask;
-    c += (int64_t)q * cfp::P[0];
+    const uint32_t q = ((uint32_t)c * cfp::GCD_N0) & kMask;
+    c += (int64_t)q * cfp::GCD_P[0];
     c >>= 28;
     for (int i = 1; i < kLimbs; i++) {
-        c += (int64_t)u[i] * f + (int64_t)v[i] * g + (int64_t)q * cfp::P[i];
+        c += (int64_t)u[i] * f + (int64_t)v[i] * g + (int64_t)q * cfp::GCD_P[i];
         r[i - 1] = (int32_t)((uint32_t)c & kMask);
         c >>= 28;
     }
@@ -105,7 +105,7 @@ VKZG_HD bool inverse(int32_t (&v)[kLimbs], const uint32_t (&y)[kLimbs]) {
     int32_t u[kLimbs];
     for (int i = 0; i < kLimbs; i++) {
         a[i] = y[i];
-        b[i] = cfp::P[i];
+        b[i] = cfp::GCD_P[i];
         u[i] = 0;
         v[i] = 0;
     }

@@ -4,53 +4,49 @@
 namespace vkzg_amd {
 
 namespace {
-// g1j_dbl (dbl-2009-l) shared by the two lanes of a pair, which both hold p.
-// Its seven products fall into four dependent rounds of at most two -- {X^2,
-// Y^2}, {B^2, (X+B)^2}, {E^2} (computed by both lanes) and {E(D - X3), YZ} --
-// and DPP exchanges hand each round's results to both lanes: a doubling waits
-// on three squarings and one product instead of five and two.  The formulas
-// and operand order are g1j_dbl's; the sums that only feed products (X + B,
-// E = 3A, D - X3) stay lazy, so coordinates are the same field elements (the
-// proofs, canonical, are unchanged).
+// g1j_dbl (curve.h) shared by the two lanes of a pair, which both hold p.
+// Its products fall into four dependent rounds of at most two -- {X^2, Y^2},
+// {W = 2X B, B^2}, {X3 = E^2 - 4W} (computed by both lanes) and
+// {E (2W - X3) - 8 B^2, 2Y Z} -- and DPP exchanges hand each round's results
+// to both lanes: a doubling waits on two products and two squarings instead
+// of four and three.  The sums are folded into the products (field_fp.h), so
+// what is left between the rounds is one carry pass each for E = 3 X^2 and
+// 2W - X3.
 VKZG_DEV G1J g1j_dbl_pair(const G1J &p, uint32_t q) {
     if (fp_is_zero(p.z)) return p;  // uniform in the pair
-    const Fp r1 = fp_sqr(fp_select(q != 0, p.y, p.x));
-    const Fp A = fp_pair_bcast<0>(r1), B = fp_pair_bcast<1>(r1);
-    const Fp r2 = fp_sqr(fp_select(q != 0, fp_add_lazy(p.x, B), B));
-    const Fp C = fp_pair_bcast<0>(r2), T = fp_pair_bcast<1>(r2);
-    const Fp E = fp_triple_lazy(A);  // feeds products only
-    const Fp F = fp_sqr(E);
-    const Fp D = fp_dbl(fp_sub(fp_sub(T, A), C));
+    const bool odd = q != 0;
+    const Fp r1 = fp_sqr(fp_select(odd, p.y, p.x));
+    const Fp E = fp_triple(fp_pair_bcast<0>(r1)), B = fp_pair_bcast<1>(r1);
+    const Fp r2 = fp_mul(fp_select(odd, B, fp_dbl_raw(p.x)), B);
+    const Fp W = fp_pair_bcast<0>(r2);
     G1J r;
-    r.x = fp_sub(F, fp_dbl(D));
-    const Fp C8 = fp_dbl(fp_dbl(fp_dbl(C)));
-    const Fp r4 = fp_mul(fp_select(q != 0, p.y, E), fp_select(q != 0, p.z, fp_sub_lazy(D, r.x)));
-    r.y = fp_sub(fp_pair_bcast<0>(r4), C8);
-    r.z = fp_dbl(fp_pair_bcast<1>(r4));
+    r.x = fp_sqr_fold(E, W, -4);
+    // lane 0 multiplies E by 2W - X3 and folds -8 B^2 in, lane 1 2Y by Z
+    const Fp r4 = fp_mul_fold_v(fp_select(odd, fp_dbl_raw(p.y), E), fp_select(odd, p.z, fp_dbl_sub(W, r.x)),
+                              fp_pair_bcast<1>(r2), odd ? 0 : -8);
+    r.y = fp_pair_bcast<0>(r4);
+    r.z = fp_pair_bcast<1>(r4);
     return r;
 }
 
-// The same doubling on the four lanes of a quad: E^2 needs only A, so it
-// joins round two on a third lane, and a doubling waits on two squarings and
-// one product -- {X^2, Y^2}, {B^2, (X+B)^2, E^2}, {E(D - X3), YZ} -- at twice
-// the lanes per chain.  Operands and lazy sums are g1j_dbl_pair's, so the
-// results are the same field elements.  For batches whose pair ladder leaves
-// SIMDs idle: there the chain's length, not the issue rate, sets the time.
+// The same doubling on the four lanes of a quad: E^2 needs only X^2, so it
+// joins round two on a third lane, and a doubling waits on one squaring and
+// two products -- {X^2, Y^2}, {2X B, B^2, E^2}, {E (4XB - X3) - 8 B^2, 2Y Z} --
+// at twice the lanes per chain.  For batches whose pair ladder leaves SIMDs
+// idle: there the chain's length, not the issue rate, sets the time.
 VKZG_DEV G1J g1j_dbl_quad(const G1J &p, uint32_t q) {
     if (fp_is_zero(p.z)) return p;  // uniform in the quad
     const bool odd = (q & 1u) != 0;
     const Fp r1 = fp_sqr(fp_select(odd, p.y, p.x));
-    const Fp A = fp_quad_bcast<0>(r1), B = fp_quad_bcast<1>(r1);
-    const Fp E = fp_triple_lazy(A);  // feeds products only
-    const Fp r2 = fp_sqr(fp_select(q == 2, E, fp_select(q == 0, B, fp_add_lazy(p.x, B))));
-    const Fp C = fp_quad_bcast<0>(r2), T = fp_quad_bcast<1>(r2), F = fp_quad_bcast<2>(r2);
-    const Fp D = fp_dbl(fp_sub(fp_sub(T, A), C));
+    const Fp E = fp_triple(fp_quad_bcast<0>(r1)), B = fp_quad_bcast<1>(r1);
+    const Fp r2 = fp_mul(fp_select(q == 2, E, fp_select(odd, B, fp_dbl_raw(p.x))), fp_select(q == 2, E, B));
+    const Fp S = fp_dbl(fp_quad_bcast<0>(r2));  // 4 X Y^2
     G1J r;
-    r.x = fp_sub(F, fp_dbl(D));
-    const Fp C8 = fp_dbl(fp_dbl(fp_dbl(C)));
-    const Fp r4 = fp_mul(fp_select(odd, p.y, E), fp_select(odd, p.z, fp_sub_lazy(D, r.x)));
-    r.y = fp_sub(fp_quad_bcast<0>(r4), C8);
-    r.z = fp_dbl(fp_quad_bcast<1>(r4));
+    r.x = fp_neg(fp_dbl_sub(S, fp_quad_bcast<2>(r2)));  // E^2 - 2S
+    const Fp r3 = fp_mul_fold_v(fp_select(odd, fp_dbl_raw(p.y), fp_sub_raw(S, r.x)), fp_select(odd, p.z, E),
+                              fp_quad_bcast<1>(r2), odd ? 0 : -8);
+    r.y = fp_quad_bcast<0>(r3);
+    r.z = fp_quad_bcast<1>(r3);
     return r;
 }
 

@@ -20,7 +20,7 @@ hipError_t launch_g2_lines(Fp2 *lines, const G2A *qs, uint32_t nq, uint32_t *err
 hipError_t launch_pairing_check(uint32_t *status, Fp *out12, Fp *L, const Fp2 *lines1, const Fp2 *lines2,
                                 const G1A *p1, const G1A *p2, bool neg2, hipStream_t s);
 
-// Montgomery -> canonical integers (28-bit limbs), in place.
+// Montgomery -> canonical integers (unsigned 30-bit digits), in place.
 hipError_t launch_fp_canonical(Fp *a, uint32_t n, hipStream_t s);
 
 }  // namespace vkzg_amd

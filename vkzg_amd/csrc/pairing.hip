@@ -91,7 +91,7 @@ __global__ void __launch_bounds__(64) k_g2_decompress(G2A *out, uint32_t *inf, c
         x0w[k] = w[23 - k];
     }
     x1w[11] &= 0x1fffffffu;
-    const Fp x1 = fp_from_words(x1w), x0 = fp_from_words(x0w);
+    const FpU x1 = fp_from_words(x1w), x0 = fp_from_words(x0w);
     if (!fp_limbs_lt_p(x1) || !fp_limbs_lt_p(x0)) bad = true;
     r.x = {fp_from_canonical(x0), fp_from_canonical(x1)};
     const Fp four = fp_const(cfp::FOUR_M);
@@ -130,8 +130,8 @@ __global__ void __launch_bounds__(64) k_g2_lines(Fp2 *lines, const G2A *qs, uint
             s++;
             const Fp2 x3 = fp2_sub(fp2_sub(fp2_sqr(lam), T.x), T.x);
             const Fp2 y3 = fp2_sub(fp2_mul(lam, fp2_sub(T.x, x3)), T.y);
-            T.x = x3;
-            T.y = y3;
+            T.x = fp2_reduce(x3);  // x3 and y3 add the last x and y
+            T.y = fp2_reduce(y3);
         }
         if ((kZAbs >> i) & 1u) {
             const Fp2 num = fp2_sub(Q.y, T.y);
@@ -143,8 +143,8 @@ __global__ void __launch_bounds__(64) k_g2_lines(Fp2 *lines, const G2A *qs, uint
             s++;
             const Fp2 x3 = fp2_sub(fp2_sub(fp2_sqr(lam), T.x), Q.x);
             const Fp2 y3 = fp2_sub(fp2_mul(lam, fp2_sub(T.x, x3)), T.y);
-            T.x = x3;
-            T.y = y3;
+            T.x = fp2_reduce(x3);  // x3 and y3 add the last x and y
+            T.y = fp2_reduce(y3);
         }
     }
     if (bad) atomicOr(err, 2u);
@@ -186,14 +186,9 @@ __device__ void fp12_copy(Fp *dst, const Fp *src) {
     if (threadIdx.x < 12) dst[threadIdx.x] = src[threadIdx.x];
     __syncthreads();
 }
-// Fp12 products leave coefficients below 12p (tower.h); the helpers that
-// negate or add them reduce to [0, 2p) first.
 __device__ void fp12_conj_inplace(Fp *a) {
     const uint32_t t = threadIdx.x;
-    if (t < 12) {
-        const Fp v = fp_reduce16(a[t]);
-        a[t] = ((t >> 1) & 1u) ? fp_neg(v) : v;
-    }
+    if (t < 12 && ((t >> 1) & 1u)) a[t] = fp_neg(a[t]);
     __syncthreads();
 }
 // dst = src^|z| (dst != src)
@@ -208,7 +203,7 @@ __device__ void fp12_pow_zabs(Fp *dst, const Fp *src) {
 __device__ void fp12_frob1(Fp *dst, const Fp *src) {
     const uint32_t t = threadIdx.x;
     if (t < 6) {
-        const Fp2 a = {fp_reduce16(src[2 * t]), fp_reduce16(src[2 * t + 1])};
+        const Fp2 a = {src[2 * t], src[2 * t + 1]};
         const Fp2 r = fp2_mul(fp2_conj(a), frob1_const(t));
         dst[2 * t] = r.c0;
         dst[2 * t + 1] = r.c1;
@@ -226,7 +221,7 @@ __device__ void fp12_frob2(Fp *dst, const Fp *src) {
 // the result (12 Fp, Montgomery).
 __global__ void __launch_bounds__(kPairThreads) k_pair_final(uint32_t *status, Fp *out12, const Fp *L) {
     __shared__ Fp f[12], g[12], h[12], A[12], B[12], C[12], D[12];
-    __shared__ Fp Ls[kPairSteps * 12];  // the step products, staged in LDS (45 KiB)
+    __shared__ Fp Ls[kPairSteps * 12];  // the step products, staged in LDS (42 KiB)
     __shared__ uint32_t ok;
     const uint32_t t = threadIdx.x;
     for (uint32_t i = t; i < kPairSteps * 12; i += blockDim.x) Ls[i] = L[i];
@@ -287,7 +282,6 @@ __global__ void __launch_bounds__(kPairThreads) k_pair_final(uint32_t *status, F
     fp12_mul_lds(g, f, f);
     fp12_mul_lds(g, g, f);  // F^3
     fp12_mul_lds(A, A, g);
-    fp12_reduce(A);
     if (t == 0) ok = 1;
     __syncthreads();
     if (t < 12) {
@@ -301,7 +295,7 @@ __global__ void __launch_bounds__(kPairThreads) k_pair_final(uint32_t *status, F
 
 __global__ void k_fp_canonical(Fp *a, uint32_t n) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) a[i] = fp_to_canonical(a[i]);
+    if (i < n) a[i] = fp_from_digits(fp_to_canonical(a[i]));
 }
 
 }  // namespace

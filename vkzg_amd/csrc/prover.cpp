@@ -20,9 +20,9 @@ extern "C" const uint8_t vkzg_amd_mainnet_g1_end[];
 
 using namespace vkzg_amd;
 
-// Fp is 14 x 28-bit limbs in 32-bit words (56 bytes) in memory as in registers.
-static_assert(sizeof(Fr) == 32 && sizeof(Fp) == 56, "field layout");
-static_assert(sizeof(G1A) == 112 && sizeof(G1J) == 168 && sizeof(G1X) == 224 && sizeof(G1AT) == 128,
+// Fp is 13 x 30-bit limbs in 32-bit words (52 bytes) in memory as in registers.
+static_assert(sizeof(Fr) == 32 && sizeof(Fp) == 52, "field layout");
+static_assert(sizeof(G1A) == 104 && sizeof(G1J) == 156 && sizeof(G1X) == 208 && sizeof(G1AT) == 128,
               "point layout");
 
 namespace vkzg_amd {

@@ -6,10 +6,15 @@ namespace vkzg_amd {
 namespace {
 // One output's reduction recomputed with the checked point operations.
 __device__ __attribute__((noinline)) void reduce_slow(G1X *out, const G1X *B) {
+    // run += B[k], then sum += run, through one copy of the addition: with two,
+    // the function is longer than a branch reaches.
     G1X run = g1x_identity(), sum = g1x_identity();
-    for (int k = (int)kBuckets - 1; k >= 0; k--) {
-        run = g1x_add(run, B[k]);
-        sum = g1x_add(sum, run);
+#pragma unroll 1
+    for (int i = 2 * (int)kBuckets - 1; i >= 0; i--) {
+        const bool first = (i & 1) != 0;
+        const G1X r = g1x_add(first ? run : sum, first ? B[i >> 1] : run);
+        if (first) run = r;
+        else sum = r;
     }
     *out = sum;
 }
@@ -18,7 +23,7 @@ __device__ __attribute__((noinline)) void reduce_slow(G1X *out, const G1X *B) {
 // k * 256 + t), so the running sum waits there while the bucket sum is
 // updated: three live points would not fit 256 VGPRs without spilling.
 struct G1XStash {
-    uint32_t *w;  // this thread's word 0
+    int32_t *w;  // this thread's word 0
     VKZG_DEV void put(const G1X &p) const {
 #pragma unroll
         for (int i = 0; i < kFpLimbs; i++) {
@@ -94,7 +99,7 @@ __global__ void __launch_bounds__(256, 2)
     constexpr uint32_t ranges = LANES / Q;
     constexpr uint32_t per = kBuckets / ranges;
     constexpr uint32_t teams = 64 / LANES;
-    __shared__ uint32_t stash_words[4 * kFpLimbs * 256];
+    __shared__ int32_t stash_words[4 * kFpLimbs * 256];
     const uint32_t wave_base = __builtin_amdgcn_readfirstlane(threadIdx.x) & ~63u;
     const uint32_t nitems = (nout + teams - 1) / teams;
     // Lane-dependent values are rederived per item from lane_here(), so none

@@ -77,9 +77,9 @@ __global__ void k_debug_fp_mul(uint32_t *out, const uint32_t *a, const uint32_t 
     }
     const Fp xm = fp_from_canonical(fp_from_words(aw)), ym = fp_from_canonical(fp_from_words(bw));
     const Fp prod = fp_mul(xm, ym);
-    const Fp r = fp_to_canonical(prod);
+    const FpU r = fp_to_canonical(prod);
     // the scheduled product must equal the plain operand-scanning one modulo p
-    const bool agree = limbs_eq<kFpLimbs>(fp_canonical(prod).v, fp_mul_reference(xm, ym).v);
+    const bool agree = fpu_eq(fp_canonical(prod), fp_mul_reference(xm, ym));
     uint32_t rw[12];
     fp_to_words(rw, r);
 #pragma unroll
@@ -127,8 +127,8 @@ __global__ void k_debug_fr_mul(uint32_t *out, const uint32_t *a, const uint32_t 
 __global__ void k_debug_fp_mul_chain(Fp *out, uint32_t n) {
     const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
     Fp a = fp_one(), b = fp_const(cfp::BETA_M);
-    a.v[0] += gid & 0xffffu;
-    b.v[1] ^= threadIdx.x & 7u;
+    a.v[0] += (int32_t)(gid & 0xffffu);
+    b.v[1] ^= (int32_t)(threadIdx.x & 7u);
 #pragma unroll 1
     for (uint32_t i = 0; i < n; i++) a = fp_mul(a, b);
     out[gid & 1023u] = a;

@@ -33,19 +33,20 @@ VKZG_DEV Fp2 fp2_one() { return {fp_one(), fp_zero()}; }
 VKZG_DEV Fp2 fp2_add(const Fp2 &a, const Fp2 &b) { return {fp_add(a.c0, b.c0), fp_add(a.c1, b.c1)}; }
 VKZG_DEV Fp2 fp2_sub(const Fp2 &a, const Fp2 &b) { return {fp_sub(a.c0, b.c0), fp_sub(a.c1, b.c1)}; }
 VKZG_DEV Fp2 fp2_neg(const Fp2 &a) { return {fp_neg(a.c0), fp_neg(a.c1)}; }
+VKZG_DEV Fp2 fp2_reduce(const Fp2 &a) { return {fp_reduce(a.c0), fp_reduce(a.c1)}; }
 VKZG_DEV Fp2 fp2_conj(const Fp2 &a) { return {a.c0, fp_neg(a.c1)}; }
-VKZG_DEV bool fp2_is_zero(const Fp2 &a) { return fp_is_zero(a.c0) && fp_is_zero(a.c1); }
+VKZG_DEV bool fp2_is_zero(const Fp2 &a) { return fp_is_zero_mod(a.c0) && fp_is_zero_mod(a.c1); }
 VKZG_DEV bool fp2_eq(const Fp2 &a, const Fp2 &b) { return fp_eq(a.c0, b.c0) && fp_eq(a.c1, b.c1); }
 // Karatsuba: (a0 + a1 u)(b0 + b1 u) = a0 b0 - a1 b1 + ((a0 + a1)(b0 + b1) - a0 b0 - a1 b1) u
 VKZG_DEV Fp2 fp2_mul(const Fp2 &a, const Fp2 &b) {
     const Fp t0 = fp_mul(a.c0, b.c0);
     const Fp t1 = fp_mul(a.c1, b.c1);
-    const Fp t2 = fp_mul(fp_add(a.c0, a.c1), fp_add(b.c0, b.c1));
-    return {fp_sub(t0, t1), fp_sub(fp_sub(t2, t0), t1)};
+    const Fp t2 = fp_mul_fold(fp_add_raw(a.c0, a.c1), fp_add(b.c0, b.c1), t0, -1);
+    return {fp_sub(t0, t1), fp_sub(t2, t1)};
 }
 // (a0 + a1 u)^2 = (a0 + a1)(a0 - a1) + 2 a0 a1 u
 VKZG_DEV Fp2 fp2_sqr(const Fp2 &a) {
-    return {fp_mul(fp_add(a.c0, a.c1), fp_sub(a.c0, a.c1)), fp_dbl(fp_mul(a.c0, a.c1))};
+    return {fp_mul(fp_add_raw(a.c0, a.c1), fp_sub(a.c0, a.c1)), fp_mul(fp_dbl_raw(a.c0), a.c1)};
 }
 VKZG_DEV Fp2 fp2_mul_fp(const Fp2 &a, const Fp &s) { return {fp_mul(a.c0, s), fp_mul(a.c1, s)}; }
 // a * xi = (a0 - a1) + (a0 + a1) u
@@ -95,8 +96,8 @@ VKZG_DEV bool fp2_sqrt(Fp2 &out, const Fp2 &a) {
 // Sign of the compressed G2 encoding: y is "larger" when y.c1 > (p-1)/2, or
 // y.c1 == 0 and y.c0 > (p-1)/2 (the ZCash serialisation of BLS12-381).
 VKZG_DEV bool fp2_is_lex_largest(const Fp2 &y) {
-    const Fp c1 = fp_to_canonical(y.c1);
-    if (!limbs_zero<kFpLimbs>(c1.v)) return fp_is_lex_largest(c1);
+    const FpU c1 = fp_to_canonical(y.c1);
+    if (!fpu_is_zero(c1)) return fp_is_lex_largest(c1);
     return fp_is_lex_largest(fp_to_canonical(y.c0));
 }
 
@@ -105,91 +106,57 @@ VKZG_DEV bool fp2_is_lex_largest(const Fp2 &y) {
 VKZG_DEV Fp fp_shfl_xor(const Fp &v, int mask) {
     Fp r;
 #pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) r.v[i] = (uint32_t)__shfl_xor((int)v.v[i], mask);
+    for (int i = 0; i < kFpLimbs; i++) r.v[i] = __shfl_xor(v.v[i], mask);
     return r;
 }
 
 constexpr uint32_t kFp12Threads = 192;  // lanes an Fp12 product uses (blockDim.x >= this)
 
-// Limb-wise sum without carries (limbs of values below 2p stay below 2^31
-// for up to 8 terms).
-VKZG_DEV Fp fp_add_raw(const Fp &a, const Fp &b) {
-    Fp r;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) r.v[i] = a.v[i] + b.v[i];
-    return r;
-}
-// Carries of a raw sum propagated: 28-bit limbs, same value.
-VKZG_DEV Fp fp_normalize(const Fp &a) {
-    Fp r;
-    uint32_t c = 0;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs - 1; i++) {
-        const uint32_t x = a.v[i] + c;
-        r.v[i] = x & kFpMask;
-        c = x >> 28;
-    }
-    r.v[kFpLimbs - 1] = a.v[kFpLimbs - 1] + c;
-    return r;
-}
-// A normalised value below 16p -> [0, 2p) (conditional subtractions of 8p, 4p, 2p).
-VKZG_DEV Fp fp_reduce16(const Fp &a) {
-    Fp r = a;
-#pragma unroll
-    for (int k = 3; k >= 1; k--) {
-        Fp t;
-        int32_t c = 0;
-#pragma unroll
-        for (int i = 0; i < kFpLimbs; i++) {
-            // subtract (2^k p) limb by limb: 2^k * P[i] fits 31 bits
-            const int64_t y = (int64_t)r.v[i] - ((int64_t)cfp::P[i] << k) + c;
-            t.v[i] = (uint32_t)y & kFpMask;
-            c = (int32_t)(y >> 28);
-        }
-        if (c >= 0) r = t;
-    }
-    return r;
-}
-
 // dst = a * b for Fp12 values held in LDS (12 Fp each).  Every thread of the
 // block calls it (it contains barriers); blockDim.x >= 192.  dst may alias a
 // or b.  Lane t works on output power M = t / 32 and on term m1 = (t % 32) / 4
 // (terms 6 and 7 of a group are empty): the quad's four lanes multiply
-// a_{m1} and b_{m2}, m2 = M - m1 mod 6, component by component, DPP quad
+// a_{m1} (times xi when m1 + m2 >= 6: (x + y u) xi = (x - y) + (x + y) u, an
+// N2 operand) and b_{m2}, m2 = M - m1 mod 6, component by component, DPP quad
 // broadcasts give every lane the four products, lane 0 of the quad forms the
-// real and lane 1 the imaginary part of a_{m1} b_{m2} (times xi when
-// m1 + m2 >= 6: (x + y u) xi = (x - y) + (x + y) u), and an xor tree over the
-// group's eight quads adds the six terms without carries, normalised once.
-// The result is below 12p in 28-bit limbs: a valid Montgomery input (any
-// input below 45p gives a product below 2p), but callers that add, negate or
-// compare it reduce it first (fp12_reduce).  Operands and result stay in
-// LDS; the partial sums never leave registers.
+// real and lane 1 the imaginary part of the term, and an xor tree over the
+// group's eight quads adds the six terms.  A term's limbs are below 2^30 and
+// the sum of two just fits 32 bits, so the tree takes one carry pass after its
+// first level and one at its end.  The result is 12 products of magnitude
+// c p: operands of up to 9.3p give c <= 2 * 9.3 * 9.3 / 630 + 1/2 < 0.775 and so
+// a result below 9.3p again, a valid operand of the next product.
+// Operands and result stay in LDS; the partial sums never leave registers.
 __device__ __forceinline__ void fp12_mul_lds(Fp *dst, const Fp *a, const Fp *b) {
     const uint32_t t = threadIdx.x;
     const uint32_t M = (t / 32) % 6, m1 = (t % 32) / 4, q = t & 3u;
     const bool term = t < kFp12Threads && m1 < 6;
     const uint32_t m1c = term ? m1 : 0;
     const uint32_t m2 = (M + 6 - m1c) % 6;
-    const Fp x_in = a[2 * m1c + (q >> 1)];
+    const bool wrap = m1c > M;
+    const uint32_t e = q >> 1;
+    const Fp x_in = a[2 * m1c + e], x_other = a[2 * m1c + (e ^ 1u)];
     const Fp y_in = b[2 * m2 + (q & 1u)];
     __syncthreads();  // dst may alias a or b
-    const Fp prod = fp_mul(x_in, y_in);
+    // wrapped: real part a0 - a1, imaginary part a1 + a0
+    const int32_t k = wrap ? (e ? 1 : -1) : 0;
+    Fp xs;
+#pragma unroll
+    for (int i = 0; i < kFpLimbs; i++) xs.v[i] = x_in.v[i] + k * x_other.v[i];
+    const Fp prod = fp_mul(xs, y_in);
     const Fp p00 = fp_quad_bcast<0>(prod), p01 = fp_quad_bcast<1>(prod);
     const Fp p10 = fp_quad_bcast<2>(prod), p11 = fp_quad_bcast<3>(prod);
-    const Fp x = fp_sub(p00, p11), y = fp_add(p01, p10);
-    const bool wrap = m1c > M;
-    Fp v = (q == 0) ? (wrap ? fp_sub(x, y) : x) : (wrap ? fp_add(x, y) : y);
+    Fp v = fp_select(q == 0, fp_sub_raw(p00, p11), fp_add_raw(p01, p10));
     if (!term || q > 1) v = fp_zero();
-    v = fp_add_raw(v, fp_shfl_xor(v, 4));
+    v = fp_norm_wide(fp_add_raw(v, fp_shfl_xor(v, 4)));
     v = fp_add_raw(v, fp_shfl_xor(v, 8));
     v = fp_add_raw(v, fp_shfl_xor(v, 16));
-    if (t < kFp12Threads && (t % 32) < 2) dst[2 * M + (t % 32)] = fp_normalize(v);
+    if (t < kFp12Threads && (t % 32) < 2) dst[2 * M + (t % 32)] = fp_norm_wide(v);
     __syncthreads();
 }
 
-// The 12 coefficients of an Fp12 product (below 12p) brought to [0, 2p).
+// The coefficients of an Fp12 product brought below p in magnitude.
 __device__ __forceinline__ void fp12_reduce(Fp *a) {
-    if (threadIdx.x < 12) a[threadIdx.x] = fp_reduce16(a[threadIdx.x]);
+    if (threadIdx.x < 12) a[threadIdx.x] = fp_reduce(a[threadIdx.x]);
     __syncthreads();
 }
 

@@ -310,13 +310,13 @@ vkzg_result locked(vkzg_prover *p, Body body) {
 // Device -> 48-byte big-endian canonical encodings of n Fp values.
 void fp_to_be(uint8_t *out, const Fp *vals, size_t n) {
     for (size_t i = 0; i < n; i++) {
-        // vals are canonical integers in 28-bit limbs
-        uint8_t le[56] = {0};
+        // vals are canonical integers in unsigned 30-bit digits
+        uint8_t le[kFpLimbs * kFpBits / 8 + 1] = {0};
         uint64_t acc = 0;
         int bits = 0, o = 0;
-        for (int l = 0; l < 14; l++) {
+        for (int l = 0; l < kFpLimbs; l++) {
             acc |= (uint64_t)vals[i].v[l] << bits;
-            bits += 28;
+            bits += kFpBits;
             while (bits >= 8) {
                 le[o++] = (uint8_t)acc;
                 acc >>= 8;
