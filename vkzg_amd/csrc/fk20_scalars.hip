@@ -4,8 +4,8 @@
 //                    columns -> NTT_128 -> phase-A scalars (1-8 blocks per
 //                    blob, each with the whole polynomial resident in LDS)
 //   k_phase_a        u[j] = sum_i scal[j][i] * xext[j][i]: fixed-base windowed
-//                    MSM against the resident multiples table, 8 lanes per tile
-//   k_sum_groups     the window-group partials of each MSM summed
+//                    MSM against the resident multiples table, a lane per share
+//   k_sum_groups     the shares of each MSM summed
 //   k_ladder         2^(8d) times the split-circulant folds of u
 //   k_phase_b        phase-B buckets, one lane per (blob, output, bucket)
 //   k_bucket_reduce  sum_k k * B[k-1] per output
@@ -21,6 +21,39 @@ constexpr int kScalarWaves = kScalarThreads / 64;
 constexpr int kPolyPitch = 4096;                 // LDS pitch of the polynomial (SoA limbs)
 constexpr int kColPitch = kScalarWaves * 128;    // LDS pitch of the per-wave circulant columns
 
+// The form phase A reads: sign (bit 255) and magnitude (below 2^254) plus the
+// plan's digit bias.
+VKZG_DEV Fr biased_magnitude(const Fr &canonical, const Fr &bias) {
+    const Fr m = fr_signed_magnitude(canonical);
+    Fr r;
+    uint32_t c = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const uint64_t x = (uint64_t)m.v[i] + bias.v[i] + c;
+        r.v[i] = (uint32_t)x;
+        c = (uint32_t)(x >> 32);
+    }
+    return r;
+}
+
+// sum over the windows below the top one of (2^(width - 1) - 1) 2^bit: added
+// to a magnitude below 2^254 it stays below 2^255, and each of those windows'
+// bits then are its signed digit plus 2^(width - 1) - 1.
+Fr scalar_bias(const WindowPlan &plan) {
+    Fr r{};
+    for (uint32_t w = 0; w + 1 < plan.W; w++) {
+        const uint64_t v = (plan.H() << plan.wide(w)) - 1;
+        const uint32_t li = plan.bit(w) >> 5;
+        uint64_t c = v << (plan.bit(w) & 31u);
+        for (uint32_t i = li; i < 8 && c; i++) {
+            c += r.v[i];
+            r.v[i] = (uint32_t)c;
+            c >>= 32;
+        }
+    }
+    return r;
+}
+
 // `parts` blocks per blob (1, 2, 4 or 8), 8 waves each (2 per SIMD).  LDS:
 // 8 x 4096 words of polynomial + 8 x 1024 words of circulant columns =
 // 160 KiB, all of a CU.  Every part parses the blob and runs the inverse
@@ -31,7 +64,7 @@ constexpr int kColPitch = kScalarWaves * 128;    // LDS pitch of the per-wave ci
 __global__ void __launch_bounds__(kScalarThreads)
     k_fk20_scalars(Fr *scal, const uint8_t *blobs, uint64_t blob_stride, uint32_t *err,
                    const Fr *roots, const Fr *roots_inv, uint32_t *queue, Fr *coeffs,
-                   uint32_t splits, uint32_t parts) {
+                   uint32_t splits, uint32_t parts, Fr bias) {
     __shared__ uint32_t poly[8 * kPolyPitch];
     __shared__ uint32_t cols[8 * kColPitch];
     const uint32_t blob = blockIdx.x / parts, part = blockIdx.x % parts;
@@ -130,11 +163,11 @@ __global__ void __launch_bounds__(kScalarThreads)
         for (int h = 0; h < 2; h++) {
             const int j = lane + 64 * h;
             const Fr v = lds_load_fr(col, kColPitch, j);
-            out[j * 64 + i] = fr_signed_magnitude(fr_to_canonical(v));
+            out[j * 64 + i] = biased_magnitude(fr_to_canonical(v), bias);
 #pragma unroll
             for (uint32_t m = 1; m < kMaxLadSplits; m++)
                 if (m < splits)
-                    out[(size_t)m * 8192 + j * 64 + i] = fr_signed_magnitude(fr_to_canonical(fr_mul(v, mult[m])));
+                    out[(size_t)m * 8192 + j * 64 + i] = biased_magnitude(fr_to_canonical(fr_mul(v, mult[m])), bias);
         }
         __syncthreads();
     }
@@ -144,12 +177,12 @@ __global__ void __launch_bounds__(kScalarThreads)
 
 hipError_t launch_fk20_scalars(Fr *scal, const uint8_t *blobs, uint64_t blob_stride, uint32_t *err,
                                const Fr *roots, const Fr *roots_inv, uint32_t *queue, Fr *coeffs,
-                               uint32_t splits, uint32_t nblobs, hipStream_t s) {
+                               uint32_t splits, uint32_t nblobs, WindowPlan plan, hipStream_t s) {
     // blocks of a blob: up to 8 while the batch fills fewer than 256 blocks
     uint32_t parts = 1;
     while (parts < 8 && nblobs * parts * 2 <= 256) parts *= 2;
     hipLaunchKernelGGL(k_fk20_scalars, dim3(nblobs * parts), dim3(kScalarThreads), 0, s, scal, blobs,
-                       blob_stride, err, roots, roots_inv, queue, coeffs, splits, parts);
+                       blob_stride, err, roots, roots_inv, queue, coeffs, splits, parts, scalar_bias(plan));
     return hipGetLastError();
 }
 

@@ -13,8 +13,10 @@
 //                             d * 2^bit(w) * xext[j][i], d <= 2^(width(w)-1),
 //                             one 128-byte line per entry
 //   Fr scal[B][128][64]       phase-A scalars, CANONICAL (not Montgomery), as
-//                             sign (bit 255) and magnitude (< 2^254)
-//   G1X u[B][128][G]          phase-A partial sums, one per window group g < G
+//                             sign (bit 255) and magnitude (< 2^254) plus
+//                             the window plan's digit bias (scalar_digit)
+//   G1X u[B][128][P]          phase-A partial sums, one per share (a run of an
+//                             MSM's terms and a group of its windows)
 //   G1J lad[B][16][128]       2^(8d) * f[j], d < kLadPos, for the folds f of u:
 //                             Fc (j < 32), Fn (32 <= j < 64), F- (j >= 64);
 //                             normalised into G1A lad_aff with the same
@@ -104,18 +106,26 @@ hipError_t launch_phase_b_scalars(Fr *out, const Fr *roots, hipStream_t s);
 // sign and magnitude).
 hipError_t launch_fk20_scalars(Fr *scal, const uint8_t *blobs, uint64_t blob_stride, uint32_t *err,
                                const Fr *roots, const Fr *roots_inv, uint32_t *queue, Fr *coeffs,
-                               uint32_t splits, uint32_t nblobs, hipStream_t s);
-// Persistent: `grid` blocks drain (msm, window group) tiles from queue[0].
-// force_checked != 0 (a test switch) sends every tile down the checked
+                               uint32_t splits, uint32_t nblobs, WindowPlan plan, hipStream_t s);
+// Persistent: `grid` blocks drain the (64 MSMs, share) items from queue[0];
+// an MSM has parts * groups shares (parts divides 64): part[msm][share].
+// force_checked != 0 (a test switch) sends every share down the checked
 // recompute, as if the fast additions had met a doubling or cancellation; the
 // same holds for launch_phase_b and launch_bucket_reduce.
-hipError_t launch_phase_a(G1X *part, const Fr *scal, const G1AT *table, WindowPlan plan,
-                          uint32_t nmsm, uint32_t groups, uint32_t grid, uint32_t *queue,
+hipError_t launch_phase_a(G1X *part, const Fr *scal, const G1AT *table, WindowPlan plan, uint32_t nblobs,
+                          uint32_t splits, uint32_t parts, uint32_t groups, uint32_t grid, uint32_t *queue,
                           uint32_t force_checked, hipStream_t s);
-// usum[msm] = sum over g < groups of part[msm * groups + g] (groups <= 24,
-// nmsm a multiple of 32).
-// quad: four lanes share each addition (force_checked: the checked recompute).
-hipError_t launch_sum_groups(G1X *usum, const G1X *part, uint32_t groups, uint32_t nmsm, bool quad,
+// The launch shape of the sum of `shares` partials for each of nmsm MSMs:
+// `sums` partial sums per MSM on `quad` (4 or 1) lanes each, and its estimated
+// time.
+struct SumShape {
+    uint32_t quad, sums;
+    double us;
+};
+SumShape sum_shape(uint64_t nmsm, uint32_t shares, uint32_t cus);
+// usum[msm] = sum over k < shares of part[msm * shares + k] (nmsm a multiple
+// of 32); force_checked: quads take their checked recompute.
+hipError_t launch_sum_groups(G1X *usum, const G1X *part, uint32_t shares, uint32_t nmsm, uint32_t cus,
                              uint32_t force_checked, hipStream_t s);
 // u: one sum per MSM, [nblobs][splits][128].
 hipError_t launch_ladder(G1J *lad, const G1X *u, uint32_t splits, uint32_t nblobs, uint32_t lanes,

@@ -1,4 +1,6 @@
 // FK20 phase B inputs: doubling ladders of the split-circulant folds of u.
+#include <algorithm>
+
 #include "proof_common.h"
 
 namespace vkzg_amd {
@@ -98,47 +100,48 @@ __global__ __launch_bounds__(256) void k_ladder(G1J *lad, const G1X *u, uint32_t
     }
 }
 
-// The window-group partials of phase A summed per MSM:
-// usum[msm] = sum_g part[msm * G + g].  Eight partial sums per MSM: sum t
-// adds partials t, t + 8 and t + 16, then a three-level tree.  Q = 1: a lane
-// per sum, with the checked additions; Q = 4 (small batches, where this
-// chain of additions is the kernel's time): a quad per sum sharing each
-// addition (g1x_add_quad, four rounds of products instead of fourteen), any
-// flagged doubling or cancellation redone checked by the quad's lane 0.
-// With G > 1 the ladder reads these sums, so its prologue (a dependent chain
-// per group of lanes) adds no partials of its own.  nmsm is a multiple of
-// 128, so the grid holds whole MSMs and no lane leaves before the shuffles.
+// The shares of phase A summed per MSM: usum[msm] = sum_k part[msm * shares + k].
+// SUMS partial sums per MSM, sum t adding shares t, t + SUMS, ..., then a tree
+// of log2(SUMS) levels.  Q = 4 (while SIMDs are idle and this chain of
+// additions is the kernel's time): a quad per sum shares each addition
+// (g1x_add_quad, four rounds of products instead of fourteen); any flagged
+// doubling or cancellation is redone checked by the MSM's first lane.  Q = 1:
+// a lane per sum, with the checked additions.  sum_shape picks both.  The
+// ladder reads these sums, so its prologue (a dependent chain per group of
+// lanes) adds no partials of its own.  nmsm is a multiple of 128, so the grid
+// holds whole MSMs and no lane leaves before the shuffles.
 VKZG_DEV_COLD void sum_groups_checked(G1X *out, const G1X *part, uint32_t groups) {
     G1X acc = g1x_identity();
     for (uint32_t g = 0; g < groups; g++) acc = g1x_add(acc, part[g]);
     *out = acc;
 }
 
-template <uint32_t Q>
-__global__ __launch_bounds__(256) void k_sum_groups(G1X *usum, const G1X *part, uint32_t groups, uint32_t nmsm,
+template <uint32_t Q, uint32_t SUMS>
+__global__ __launch_bounds__(256) void k_sum_groups(G1X *usum, const G1X *part, uint32_t shares, uint32_t nmsm,
                                                     uint32_t force_checked) {
     const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t msm = tid / (8 * Q), t = (tid / Q) % 8, qd = tid % Q;
+    const uint32_t msm = tid / (SUMS * Q), t = (tid / Q) % SUMS, qd = tid % Q;
     if (msm >= nmsm) return;
-    G1X acc = g1x_identity();
+    const G1X *p = part + (size_t)msm * shares;
+    G1X acc = t < shares ? p[t] : g1x_identity();
     if constexpr (Q == 4) {
         bool exc = force_checked != 0;
 #pragma unroll 1
-        for (uint32_t g = t; g < groups; g += 8) acc = g1x_add_quad(acc, part[(size_t)msm * groups + g], qd, exc);
+        for (uint32_t k = t + SUMS; k < shares; k += SUMS) acc = g1x_add_quad(acc, p[k], qd, exc);
 #pragma unroll 1
-        for (uint32_t m = 1; m < 8; m <<= 1) acc = g1x_add_quad(acc, g1x_shfl_xor(acc, m * Q), qd, exc);
-        // a flag anywhere in the MSM's 32 lanes: lane 0 redoes the sum
-        const uint64_t flagged = __ballot(exc);
-        const uint32_t sub = (threadIdx.x & 63u) / 32u;
-        if (((flagged >> (32u * sub)) & 0xffffffffull) != 0) {
-            if (t == 0 && qd == 0) sum_groups_checked(&usum[msm], part + (size_t)msm * groups, groups);
+        for (uint32_t m = 1; m < SUMS; m <<= 1) acc = g1x_add_quad(acc, g1x_shfl_xor(acc, m * Q), qd, exc);
+        // a flag anywhere in the MSM's lanes
+        constexpr uint32_t kLanes = SUMS * Q;
+        const uint64_t mask = kLanes == 64 ? ~0ull : (1ull << kLanes) - 1;
+        if ((__ballot(exc) >> ((threadIdx.x & 63u) / kLanes * kLanes) & mask) != 0) {
+            if (t == 0 && qd == 0) sum_groups_checked(&usum[msm], p, shares);
             return;
         }
     } else {
 #pragma unroll 1
-        for (uint32_t g = t; g < groups; g += 8) acc = g1x_add(acc, part[(size_t)msm * groups + g]);
+        for (uint32_t k = t + SUMS; k < shares; k += SUMS) acc = g1x_add(acc, p[k]);
 #pragma unroll 1
-        for (uint32_t m = 1; m < 8; m <<= 1) acc = g1x_add(acc, g1x_shfl_xor(acc, m));
+        for (uint32_t m = 1; m < SUMS; m <<= 1) acc = g1x_add(acc, g1x_shfl_xor(acc, m));
     }
     if (t == 0 && qd == 0) usum[msm] = acc;
 }
@@ -207,15 +210,43 @@ hipError_t launch_ladder(G1J *lad, const G1X *u, uint32_t splits, uint32_t nblob
     return hipGetLastError();
 }
 
-hipError_t launch_sum_groups(G1X *usum, const G1X *part, uint32_t groups, uint32_t nmsm, bool quad,
+// An addition of the chain takes 7.5 us on a quad and 14 us on a lane with a
+// wave per SIMD (measured at 1 to 21 blobs), and in proportion above.  Quads
+// do four times the work, so they win while the lanes are few: 16 of them per
+// MSM at 1 blob, 8 or 4 at tens of blobs, a lane or two per MSM at 256.
+SumShape sum_shape(uint64_t nmsm, uint32_t shares, uint32_t cus) {
+    const double simd_lanes = (double)cus * 4 * 64;
+    SumShape best{1, 1, 0.0};
+    bool have = false;
+    for (uint32_t q : {4u, 1u})
+        for (uint32_t sums = q == 4 ? 16 : 8; sums >= (q == 4 ? 4u : 1u); sums /= 2) {
+            uint32_t adds = (shares + sums - 1) / sums - 1;
+            for (uint32_t m = 1; m < sums; m <<= 1) adds++;
+            const double us = adds * (q == 4 ? 7.5 : 14.0) * std::max(1.0, nmsm * sums * q / simd_lanes);
+            if (!have || us < best.us) best = SumShape{q, sums, us};
+            have = true;
+        }
+    if (shares <= 1) best.us = 0.0;
+    return best;
+}
+
+hipError_t launch_sum_groups(G1X *usum, const G1X *part, uint32_t shares, uint32_t nmsm, uint32_t cus,
                              uint32_t force_checked, hipStream_t s) {
-    if (nmsm % 32 != 0 || groups > 24) return hipErrorInvalidValue;
-    if (quad)
-        hipLaunchKernelGGL(k_sum_groups<4>, dim3(blocks_for(nmsm * 32ull, 256)), dim3(256), 0, s, usum, part,
-                           groups, nmsm, force_checked);
-    else
-        hipLaunchKernelGGL(k_sum_groups<1>, dim3(blocks_for(nmsm * 8ull, 256)), dim3(256), 0, s, usum, part,
-                           groups, nmsm, force_checked);
+    if (nmsm % 32 != 0) return hipErrorInvalidValue;
+    auto run = [&](auto kernel, uint32_t lanes) {
+        hipLaunchKernelGGL(kernel, dim3(blocks_for((uint64_t)nmsm * lanes, 256)), dim3(256), 0, s, usum, part, shares,
+                           nmsm, force_checked);
+    };
+    const SumShape f = sum_shape(nmsm, shares, cus);
+    switch (f.quad * 100 + f.sums) {
+        case 416: run(k_sum_groups<4, 16>, 64); break;
+        case 408: run(k_sum_groups<4, 8>, 32); break;
+        case 404: run(k_sum_groups<4, 4>, 16); break;
+        case 108: run(k_sum_groups<1, 8>, 8); break;
+        case 104: run(k_sum_groups<1, 4>, 4); break;
+        case 102: run(k_sum_groups<1, 2>, 2); break;
+        default: run(k_sum_groups<1, 1>, 1); break;
+    }
     return hipGetLastError();
 }
 

@@ -4,107 +4,149 @@
 namespace vkzg_amd {
 
 namespace {
-// The `width` bits of s from bit `off` (bits above 255 read as zero).
-VKZG_DEV uint32_t window_bits(const Fr &s, uint32_t off, uint32_t width) {
-    const uint32_t li = off >> 5;
-    const uint32_t sh = off & 31u;
-    uint32_t lo = li < 8 ? s.v[li] >> sh : 0u;
-    if (sh && li + 1 < 8) lo |= s.v[li + 1] << (32u - sh);
-    return lo & ((1u << width) - 1u);
+// Phase-A scalars come as sign (bit 255) and magnitude plus scalar_bias
+// (k_fk20_scalars): with the bias of (half - 1) 2^bit(w) in every window below
+// the top one, the window's bits are its signed digit plus half - 1, so no
+// carry comes up from the windows below.  The digit of window w from the
+// window's bits: its magnitude, and in neg its sign times the scalar's.
+VKZG_DEV uint32_t window_digit(uint32_t raw, const WindowPlan &plan, uint32_t w, bool sneg, bool &neg) {
+    const int32_t d = (int32_t)raw - (w + 1 < plan.W ? (int32_t)((plan.H() << plan.wide(w)) - 1u) : 0);
+    neg = (d < 0) != sneg;
+    return (uint32_t)(d < 0 ? -d : d);
 }
 
-// A phase-A scalar's magnitude (bit 255 cleared) and its sign.
-VKZG_DEV Fr scalar_magnitude(const Fr &s, bool &neg) {
-    Fr m = s;
-    neg = (s.v[7] >> 31) != 0;
-    m.v[7] &= 0x7fffffffu;
-    return m;
-}
+// A scalar whose low bits are the bits of the window at hand.  Windows are
+// uniform in a wave, so stepping to the next one is eight funnel shifts.
+struct ScalarBits {
+    Fr v;
+    bool neg;
+    VKZG_DEV void load(const Fr &s) {
+        v = s;
+        neg = (s.v[7] >> 31) != 0;
+        v.v[7] &= 0x7fffffffu;
+    }
+    VKZG_DEV void skip(uint32_t bits) {
+#pragma unroll 1
+        for (; bits >= 32; bits -= 32) {
+#pragma unroll
+            for (int i = 0; i < 7; i++) v.v[i] = v.v[i + 1];
+            v.v[7] = 0;
+        }
+#pragma unroll
+        for (int i = 0; i < 7; i++) v.v[i] = __builtin_amdgcn_alignbit(v.v[i + 1], v.v[i], bits);
+        v.v[7] >>= bits;
+    }
+    VKZG_DEV uint32_t low(uint32_t width) const { return v.v[0] & ((1u << width) - 1u); }
+};
 
-constexpr int kMsmLanes = 8;  // lanes per tile (64 terms / 8 = 8 each)
-constexpr int kTilesPerItem = 256 / kMsmLanes;  // tiles one 256-thread block takes per queue item
-
-// Windows [w0, w1) of the 64 terms of one MSM, recomputed with the checked
+// Windows [w0, w1) of `terms` terms of one MSM, recomputed with the checked
 // point operations: reached only when the fast path flagged a doubling or
-// cancellation case in this tile.
-__device__ __attribute__((noinline)) void phase_a_slow(G1X *out, const Fr *scal, const G1AT *tab_j,
-                                                       WindowPlan plan, uint32_t w0, uint32_t w1) {
+// cancellation case in this lane's share.
+__device__ __attribute__((noinline)) void phase_a_slow(G1X *out, const Fr *scal, const G1AT *tab, WindowPlan plan,
+                                                       uint32_t terms, uint32_t w0, uint32_t w1) {
     G1X acc = g1x_identity();
-    for (uint32_t i = 0; i < 64; i++) {
-        bool sneg;
-        const Fr s = scalar_magnitude(scal[i], sneg);
-        const G1AT *tab = tab_j + (size_t)i * plan.entries();
-        uint32_t carry = 0;
-        for (uint32_t w = 0; w < w1; w++) {
-            const uint32_t Hw = plan.H() << plan.wide(w);
-            const uint32_t raw = window_bits(s, plan.bit(w), plan.c + plan.wide(w)) + carry;
-            carry = raw > Hw ? 1u : 0u;
-            const uint32_t mag = carry ? (2u * Hw - raw) : raw;
-            if (w >= w0 && mag)
-                acc = g1x_madd(acc, g1a_neg_if(tab[plan.entry(w) + (mag - 1)].p, (carry != 0) != sneg));
+#pragma unroll 1
+    for (uint32_t i = 0; i < terms; i++) {
+        ScalarBits s;
+        s.load(scal[i]);
+        s.skip(plan.bit(w0));
+        const G1AT *row = tab + (size_t)i * plan.entries();
+#pragma unroll 1
+        for (uint32_t w = w0; w < w1; w++) {
+            const uint32_t width = plan.c + plan.wide(w);
+            bool neg;
+            const uint32_t mag = window_digit(s.low(width), plan, w, s.neg, neg);
+            s.skip(width);
+            if (mag) acc = g1x_madd(acc, g1a_neg_if(row[plan.entry(w) + (mag - 1)].p, neg));
         }
     }
     *out = acc;
 }
 
-// Persistent phase A.  The work is a queue of tiles (msm, g): windows
-// [g W / G, (g+1) W / G) of MSM msm = (blob * splits + m) * 128 + j, where
-//   u[msm] = sum_{i<64} scal[msm][i] * xext[j][i]
-// with the scalar as sign and magnitude (k_fk20_scalars) and the magnitude in
-// signed digits v in [-(2^(b-1)-1), 2^(b-1)] of each window's width b (the
-// recoding of k_phase_a_sort.comp:31-40 with the plan's windows), each digit's
-// sign flipped for a negative scalar, and
-// table[j][i][entry(w) + |v| - 1] = |v| * 2^bit(w) * xext[j][i].  Tile (msm, g) writes its
-// partial sum to part[msm * G + g]; k_sum_groups adds the G partials.  Tiles
-// are numbered group-major (tile = g * nmsm + msm): nmsm is a multiple of 128,
-// so the 8 tiles of a wave share g and run the same windows -- mixed groups
-// in one wave would make it step through the union of their windows.  A
-// block takes 32 consecutive tiles per queue item (8 lanes per tile, 8 terms
-// per lane) from the counter q[0] until the queue is drained; every block
-// exits after one failed take, so the grid always drains.  q[0] is cleared by
-// the kernel that runs before this one.
+// Persistent phase A.  MSM m = (blob * splits + seg) * 128 + j is
+//   u[m] = sum_{i<64} scal[m][i] * xext[j][i]
+// with the scalar in signed digits v in [-(2^(b-1)-1), 2^(b-1)] of each window's
+// width b (the recoding of k_phase_a_sort.comp:31-40 with the plan's windows),
+// each digit's sign flipped for a negative scalar, and
+// table[j][i][entry(w) + |v| - 1] = |v| * 2^bit(w) * xext[j][i].  Its terms are
+// cut into `parts` runs of 64 / parts and its windows into `groups` groups, and
+// one lane adds up one (run, group) share: part[m * parts * groups + share].
+// k_sum_groups adds an MSM's shares.
+//
+// A wave's 64 lanes are 64 MSMs of one share, in the order (j, seg, blob) with
+// the blob fastest: they run the same windows of the same terms, and from 64
+// blobs on also against the same base, so that their random 128-byte lines
+// lie in one megabyte of the table.  A wave over 8 bases and 8 runs of terms,
+// with a lane tree over the runs, gathered from 64 such places at once and
+// spent three additions per lane on the tree: 256 blobs 5.16 -> 4.91 ms, 64
+// blobs 1.37 -> 1.25 ms, and with the shares fitted to the batch 21 blobs 1.20
+// -> 0.42 ms, 9 blobs 0.38 -> 0.22 ms, 1 blob 0.19 -> 0.11 ms (the sums over more
+// shares cost 0.05 to 0.07 ms of that at 1 to 64 blobs).  What bounds it at 256
+// blobs is the multiply-adds: against a table cut to a few lines it takes 4.4
+// ms, and the kernels after it get 7% faster too, so the gathers cost power
+// more than time.
+//
+// The gathers come from a table far larger than any cache, and two waves per
+// SIMD do not hide such a load behind each other's additions.  The lane runs
+// one flat loop over its (term, window) pairs in two stages: the digit and the
+// load of the next point are issued before the addition of the current one,
+// and a term's scalar is loaded while the term before it is added (1 blob
+// 0.228 -> 0.192 ms, 21 blobs 1.32 -> 1.20 ms).
+//
+// A wave takes items (share, 64 MSMs) from the counter q[0], cleared by the
+// kernel that runs before, until the queue is drained, and leaves after one
+// failed take; nmsm is a multiple of 128, so items are whole waves.
 __global__ void __launch_bounds__(256, 2)
-    k_phase_a(G1X *part, const Fr *scal, const G1AT *table, WindowPlan plan, uint32_t nmsm,
-              uint32_t groups, uint32_t *q, uint32_t force_checked) {
-    __shared__ uint32_t item_sh;
-    const uint32_t t = threadIdx.x % kMsmLanes;
-    const uint32_t W = plan.W, H = plan.H(), narrow = plan.W - plan.k;
-    const uint32_t ntiles = nmsm * groups;
-    const uint32_t nitems = (ntiles + kTilesPerItem - 1) / kTilesPerItem;
+    k_phase_a(G1X *part, const Fr *scal, const G1AT *table, WindowPlan plan, uint32_t nblobs, uint32_t splits,
+              uint32_t parts, uint32_t groups, uint32_t *q, uint32_t force_checked) {
+    const uint32_t lane = threadIdx.x % 64;
+    const uint32_t per_share = nblobs * splits * 2;  // items of 64 MSMs
+    const uint32_t shares = parts * groups, nitems = per_share * shares;
+    const uint32_t terms = 64 / parts;
 #pragma unroll 1
     for (;;) {
-        if (threadIdx.x == 0) item_sh = atomicAdd(q, 1u);
-        __syncthreads();
-        const uint32_t item = item_sh;
-        __syncthreads();
+        uint32_t item = 0;
+        if (lane == 0) item = atomicAdd(q, 1u);
+        item = __builtin_amdgcn_readfirstlane(item);
         if (item >= nitems) break;
-        const uint32_t tile = item * kTilesPerItem + threadIdx.x / kMsmLanes;
-        const bool live = tile < ntiles;
-        const uint32_t g = live ? tile / nmsm : 0u;
-        const uint32_t msm = live ? tile % nmsm : 0u;
-        const uint32_t j = msm % 128;
-        const uint32_t w0 = g * W / groups, w1 = (g + 1) * W / groups;
+        const uint32_t share = item / per_share;
+        const uint32_t run = share / groups, g = share % groups;
+        const uint32_t idx = (item % per_share) * 64 + lane;
+        const uint32_t blob = idx % nblobs, js = idx / nblobs;
+        const uint32_t j = js / splits, msm = (blob * splits + js % splits) * 128 + j;
+        const uint32_t w0 = g * plan.W / groups, w1 = (g + 1) * plan.W / groups;
+        const Fr *sc = scal + (size_t)msm * 64 + run * terms;
+        const G1AT *tab = table + (size_t)(j * 64 + run * terms) * plan.entries();
         G1X acc = g1x_identity();
         bool exc = force_checked != 0, started = false;
-        if (live) {
+        if (w0 < w1) {  // (more groups than windows leave some empty)
+            const uint32_t first = plan.bit(w0);
+            uint32_t k = 0, w = w0;
+            ScalarBits s;
+            s.load(sc[0]);
+            s.skip(first);
+            Fr ahead = sc[terms > 1 ? 1 : 0];
+            bool neg_next;
+            uint32_t mag_next = window_digit(s.low(plan.c + plan.wide(w)), plan, w, s.neg, neg_next);
+            G1A next = tab[plan.entry(w) + (mag_next ? mag_next - 1 : 0u)].p;
 #pragma unroll 1
-            for (uint32_t qq = 0; qq < 64 / kMsmLanes; qq++) {
-                const uint32_t i = t * (64 / kMsmLanes) + qq;
-                bool sneg;
-                const Fr s = scalar_magnitude(scal[(size_t)msm * 64 + i], sneg);
-                const G1AT *tab = table + (size_t)(j * 64 + i) * plan.entries();
-                uint32_t carry = 0;
-#pragma unroll 1
-                for (uint32_t w = 0; w < w1; w++) {
-                    // windows at or above `narrow` are one bit wider
-                    const uint32_t wide = w >= narrow ? 1u : 0u, below = w > narrow ? w - narrow : 0u;
-                    const uint32_t Hw = H << wide;
-                    const uint32_t raw = window_bits(s, w * plan.c + below, plan.c + wide) + carry;
-                    carry = raw > Hw ? 1u : 0u;
-                    const bool neg = (carry != 0) != sneg;
-                    const uint32_t mag = carry ? (2u * Hw - raw) : raw;
-                    if (w < w0 || mag == 0) continue;
-                    const G1A pt = tab[(w + below) * H + (mag - 1)].p;
+            for (;;) {
+                const G1A pt = next;
+                const bool neg = neg_next, skip = mag_next == 0;
+                s.skip(plan.c + plan.wide(w));
+                if (++w == w1) {
+                    w = w0;
+                    k++;
+                    s.load(ahead);
+                    s.skip(first);
+                    if (k + 1 < terms) ahead = sc[k + 1];
+                }
+                const bool more = k < terms;
+                if (more) {
+                    mag_next = window_digit(s.low(plan.c + plan.wide(w)), plan, w, s.neg, neg_next);
+                    next = tab[(size_t)k * plan.entries() + plan.entry(w) + (mag_next ? mag_next - 1 : 0u)].p;
+                }
+                if (!skip) {
                     if (started) {
                         acc = g1x_madd_acc(acc, pt, neg, exc);
                     } else {
@@ -112,34 +154,26 @@ __global__ void __launch_bounds__(256, 2)
                         started = true;
                     }
                 }
+                if (!more) break;
             }
         }
-        // Sum the 8 lanes' partial results of this tile.
-#pragma unroll 1
-        for (int m = 1; m < kMsmLanes; m <<= 1) acc = g1x_add_fast(acc, g1x_shfl_xor(acc, m), exc);
-        const uint64_t flagged = __ballot(exc);
-        const uint32_t sub = (threadIdx.x & 63u) / kMsmLanes;
-        const bool redo = ((flagged >> (sub * kMsmLanes)) & ((1ull << kMsmLanes) - 1)) != 0;
-        if (live && t == 0) {
-            G1X *out = &part[(size_t)msm * groups + g];
-            if (redo)
-                phase_a_slow(out, scal + (size_t)msm * 64, table + (size_t)j * 64 * plan.entries(), plan, w0, w1);
-            else
-                *out = acc;
-        }
+        G1X *out = &part[(size_t)msm * shares + share];
+        if (exc) phase_a_slow(out, sc, tab, plan, terms, w0, w1);
+        else *out = acc;
     }
 }
 
 }  // namespace
 
-hipError_t launch_phase_a(G1X *part, const Fr *scal, const G1AT *table, WindowPlan plan,
-                          uint32_t nmsm, uint32_t groups, uint32_t grid, uint32_t *queue,
+hipError_t launch_phase_a(G1X *part, const Fr *scal, const G1AT *table, WindowPlan plan, uint32_t nblobs,
+                          uint32_t splits, uint32_t parts, uint32_t groups, uint32_t grid, uint32_t *queue,
                           uint32_t force_checked, hipStream_t s) {
-    const uint32_t nitems = (nmsm * groups + kTilesPerItem - 1) / kTilesPerItem;
-    if (grid > nitems) grid = nitems;
+    if (parts == 0 || 64 % parts != 0) return hipErrorInvalidValue;
+    const uint32_t blocks = (nblobs * splits * 2 * parts * groups + 3) / 4;  // four waves each
+    if (grid > blocks) grid = blocks;
     if (grid == 0) grid = 1;
-    hipLaunchKernelGGL(k_phase_a, dim3(grid), dim3(256), 0, s, part, scal, table, plan, nmsm, groups,
-                       queue, force_checked);
+    hipLaunchKernelGGL(k_phase_a, dim3(grid), dim3(256), 0, s, part, scal, table, plan, nblobs, splits, parts,
+                       groups, queue, force_checked);
     return hipGetLastError();
 }
 

@@ -362,7 +362,7 @@ void build_tables(vkzg_prover *p, const uint8_t *setup) {
 uint64_t WorkSet::bytes_per_blob() {
     const uint64_t npos = 128ull * kLadPos;
     return kBlobBytes + kProofBytes + 4 * 4 + 128 + kMaxLadSplits * 128 * 64 * sizeof(Fr) +
-           kMaxLadSplits * 128 * (kMaxGroups + 1) * sizeof(G1X) +
+           kSlotsPerBlob * sizeof(G1X) +
            npos * sizeof(G1J) + 2 * npos * sizeof(G1A) + npos * sizeof(Fp) +
            128 * kBuckets * (sizeof(G1X) + 1) + 128 * sizeof(G1X) + 2 * kCellsBytes + 128 +
            2 * 8192 * sizeof(Fr);
@@ -380,7 +380,9 @@ void WorkSet::allocate(uint32_t B) {
     queue_r = arena.dalloc<uint32_t>(B);
     ck(hipMemset(queue_r, 0, (size_t)B * sizeof(uint32_t)));
     scal = arena.dalloc<Fr>((size_t)B * 128 * 64 * kMaxLadSplits);
-    u = arena.dalloc<G1X>((size_t)B * 128 * (kMaxGroups + 1) * kMaxLadSplits);
+    // room for a few blobs' partials at least, so that one blob can be spread too
+    u_slots = (uint64_t)std::max(B, kMinPartialBlobs) * kSlotsPerBlob;
+    u = arena.dalloc<G1X>((size_t)u_slots);
     lad = arena.dalloc<G1J>((size_t)B * 128 * kLadPos);
     lad_aff = arena.dalloc<G1A>((size_t)B * 128 * kLadPos);
     lad_phi = arena.dalloc<G1A>((size_t)B * 128 * kLadPos);
@@ -417,18 +419,16 @@ Tuning tuning_for(const vkzg_prover *p, uint32_t nb) {
     return t;
 }
 
-// Defaults before (or without) autotuning: small batches split each MSM into
-// more window groups and the ladder into segments, so that more lanes work on
-// the few MSMs and chains there are (one wave per SIMD already saturates
-// phase A at 64 blobs); the normalisation chunk is fitted to the chip
-// (norm_chunk 0).
+// Defaults before (or without) autotuning: small batches split the ladder into
+// segments, so that more lanes work on the few chains there are; phase A's
+// shares and the normalisation chunk are fitted to the batch and the chip
+// (groups 0, norm_chunk 0).
 void default_tunings(vkzg_prover *p) {
-    static const uint32_t groups[kTuneClasses] = {10, 10, 4, 1, 1};
     static const uint32_t ladder_splits[kTuneClasses] = {4, 2, 1, 1, 1};
     static const uint32_t reduce_lanes[kTuneClasses] = {64, 64, 32, 16, 4};
     for (int c = 0; c < kTuneClasses; c++) {
         p->tune[c] = Tuning{};
-        p->tune[c].groups = groups[c];
+        p->tune[c].groups = 0;
         p->tune[c].ladder_splits = ladder_splits[c];
         p->tune[c].reduce_lanes = reduce_lanes[c];
         p->tune[c].norm_chunk = 0;
@@ -462,8 +462,42 @@ uint32_t fit_norm_chunk(uint64_t count, uint32_t cus) {
     return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(c, 256));
 }
 
+// Shares an MSM is cut into in phase A: `parts` runs of its terms times
+// `groups` groups of its windows (a lane adds up one run of one group), as far
+// as the partials have room.  The shape with the least estimated time of phase
+// A and of the sum of the shares; groups != 0 fixes the groups.
+//
+// A lane's chain has (64 / parts) ceil(windows / groups) mixed additions.  One
+// takes 7.65 us while its wave has a SIMD to itself and 14.6 us with two waves
+// on it, which is all the kernel has resident, so the waves run in rounds of
+// two per SIMD and the last round counts whole (measured at 1 to 256 blobs).
+// More shares shorten the chain while SIMDs are idle; past that, and wherever
+// they start another round, they only lengthen the sum.
+struct PhaseAShape {
+    uint32_t parts, groups;
+};
+PhaseAShape phase_a_shape(uint64_t nmsm, uint32_t groups, uint32_t windows, uint64_t slots, uint32_t cus) {
+    const uint64_t simds = (uint64_t)cus * 4;
+    PhaseAShape best{1, groups ? groups : 1};
+    double best_us = 0;
+    for (uint32_t parts = 1; parts <= 64; parts *= 2)
+        for (uint32_t g = groups ? groups : 1; g <= (groups ? groups : kMaxGroups); g++) {
+            const uint64_t shares = (uint64_t)parts * g;
+            if (shares > 1 && nmsm * (shares + 1) > slots) continue;
+            const uint64_t waves = nmsm * shares / 64, rest = waves % (2 * simds);
+            const double chain = 64.0 / parts * ((windows + g - 1) / g);
+            const double us = chain * (14.6 * (double)(waves / (2 * simds)) + (rest > simds ? 14.6 : rest ? 7.65 : 0.0)) +
+                              sum_shape(nmsm, (uint32_t)shares, cus).us;
+            if (best_us == 0 || us < best_us) {
+                best = PhaseAShape{parts, g};
+                best_us = us;
+            }
+        }
+    return best;
+}
+
 bool tuning_valid(const Tuning &t) {
-    return t.groups >= 1 && t.groups <= kMaxGroups && t.blocks_per_cu >= 1 && t.blocks_per_cu <= 2 &&
+    return t.groups <= kMaxGroups && t.blocks_per_cu >= 1 && t.blocks_per_cu <= 2 &&
            t.norm_chunk <= 256 && t.splits >= 1 && t.splits <= (uint32_t)kMaxSplits &&
            (t.rec_waves == 1 || t.rec_waves == 2 || t.rec_waves == 4) && (t.rec_radix == 2 || t.rec_radix == 4 || t.rec_radix == 8) &&
            (t.ladder_splits == 1 || t.ladder_splits == 2 || t.ladder_splits == 4) &&
@@ -518,28 +552,32 @@ void proofs_range(vkzg_prover *p, WorkSet &ws, uint32_t off, uint32_t nb, uint8_
     uint32_t *err = ws.err + off;
     uint32_t *queue = ws.queue + off;
     Fr *scal = ws.scal + (size_t)off * 8192 * kMaxLadSplits;
-    // phase-A partials [nb][splits][128][groups], then their sums [nb][splits][128]
-    G1X *u = ws.u + (size_t)off * 128 * (kMaxGroups + 1) * kMaxLadSplits;
-    G1X *usum = u + (size_t)nb * 128 * kMaxGroups * kMaxLadSplits;
+    // phase-A partials [nb][splits][128][shares], then their sums
+    // [nb][splits][128].  A batch in one stream may use the whole buffer, a
+    // sub-batch the slots of its own blobs.
+    const uint64_t nmsm = (uint64_t)nb * 128 * tn.ladder_splits;
+    const uint64_t slots = tn.splits == 1 && off == 0 ? ws.u_slots : (uint64_t)nb * kSlotsPerBlob;
+    const PhaseATable tab = phase_a_table(p, tn.window_bits);
+    const PhaseAShape shape = phase_a_shape(nmsm, tn.groups, tab.W, slots, p->cus);
+    const uint32_t shares = shape.parts * shape.groups;
+    G1X *u = ws.u + (size_t)off * kSlotsPerBlob;
+    G1X *usum = u + (size_t)nmsm * shares;
     const size_t npos = (size_t)128 * kLadPos;  // ladder points per blob
     G1J *lad = ws.lad + off * npos;
     G1A *lad_aff = ws.lad_aff + off * npos, *lad_phi = ws.lad_phi + off * npos;
     Fp *prefix = ws.prefix + off * npos;
     G1X *buckets = ws.buckets + (size_t)off * 128 * kBuckets, *cvals = ws.cvals + (size_t)off * 128;
     ck(launch_fk20_scalars(scal, d_blobs, blob_stride, err, p->roots, p->roots_inv, queue, coeffs,
-                           tn.ladder_splits, nb, s));
+                           tn.ladder_splits, nb, tab.plan(), s));
     clk.mark("fk20_scalars");
-    const PhaseATable tab = phase_a_table(p, tn.window_bits);
-    ck(launch_phase_a(u, scal, tab.table, tab.plan(), nb * 128 * tn.ladder_splits, tn.groups,
+    ck(launch_phase_a(u, scal, tab.table, tab.plan(), nb, tn.ladder_splits, shape.parts, shape.groups,
                       p->cus * tn.blocks_per_cu, queue, tn.force_checked, s));
     clk.mark("phase_a");
-    if (tn.groups > 1) {
-        const uint64_t nsum = (uint64_t)nb * 128 * tn.ladder_splits;  // quads while they fit a wave per SIMD
-        ck(launch_sum_groups(usum, u, tn.groups, (uint32_t)nsum, nsum * 32 <= (uint64_t)p->cus * 4 * 64,
-                             tn.force_checked, s));
+    if (shares > 1) {
+        ck(launch_sum_groups(usum, u, shares, (uint32_t)nmsm, p->cus, tn.force_checked, s));
         clk.mark("sum_groups");
     }
-    ck(launch_ladder(lad, tn.groups > 1 ? usum : u, tn.ladder_splits, nb,
+    ck(launch_ladder(lad, shares > 1 ? usum : u, tn.ladder_splits, nb,
                      ladder_lanes((uint64_t)nb * 128 * tn.ladder_splits, p->cus), s));
     clk.mark("ladder");
     // Small unsplit batches skip the normalisation: phase B's quads add the
@@ -1240,6 +1278,12 @@ vkzg_result vkzg_amd_get_tuning(const vkzg_prover *p, size_t num_blobs, vkzg_amd
         std::lock_guard<std::mutex> lock(p->tune_mu);
         t = p->tune[tune_class((uint32_t)std::min<size_t>(num_blobs, 0xffffffffu))];
     }
+    if (!t.groups) {  // fitted: the groups a batch of this size takes
+        const uint32_t nb = (uint32_t)std::min<size_t>(num_blobs, p->max_batch);
+        t.groups = phase_a_shape((uint64_t)nb * 128 * t.ladder_splits, 0, phase_a_table(p, t.window_bits).W,
+                                 (uint64_t)std::max(p->max_batch, kMinPartialBlobs) * kSlotsPerBlob, p->cus)
+                       .groups;
+    }
     out->phase_a_groups = t.groups;
     out->phase_a_blocks_per_cu = t.blocks_per_cu;
     out->normalize_chunk = t.norm_chunk;
@@ -1264,7 +1308,7 @@ vkzg_result vkzg_amd_set_tuning(vkzg_prover *p, size_t num_blobs, const vkzg_amd
     t.ladder_splits = in->ladder_splits;
     t.reduce_lanes = in->reduce_lanes;
     t.window_bits = in->phase_a_window_bits == p->c ? 0u : in->phase_a_window_bits;
-    if (!tuning_valid(t)) return VKZG_ERR_BADARGS;
+    if (t.groups == 0 || !tuning_valid(t)) return VKZG_ERR_BADARGS;
     std::lock_guard<std::mutex> lock(p->mu);
     if (t.window_bits) {  // only a resident smaller table
         if (!p->extra_tables[t.window_bits - kExtraWindowMin].table) return VKZG_ERR_BADARGS;

@@ -21,11 +21,14 @@ constexpr size_t kProofBytes = (size_t)VKZG_NUM_CELL_PROOFS * VKZG_BYTES_PER_PRO
 constexpr size_t kCellsBytes = (size_t)VKZG_NUM_CELL_PROOFS * VKZG_BYTES_PER_CELL;
 constexpr int kMaxSplits = 4;  // sub-streams one batch may be spread over
 constexpr uint32_t kMaxGroups = 20;  // phase-A window groups per MSM
+// Phase-A partials per blob: every group of every MSM of a split ladder, and their sums.
+constexpr uint64_t kSlotsPerBlob = 128ull * (kMaxGroups + 1) * 4;
+constexpr uint32_t kMinPartialBlobs = 8;
 
 // Launch shape of the proof pipeline for one batch-size class.  Every choice
 // gives bit-identical proofs; only the time differs.
 struct Tuning {
-    uint32_t groups = 1;         // phase-A window groups (tiles) per MSM, 1..kMaxGroups
+    uint32_t groups = 0;         // phase-A window groups per MSM, 1..kMaxGroups (0: fitted to the batch and the chip)
     uint32_t blocks_per_cu = 2;  // persistent phase-A grid = CUs x this, 1..2
     uint32_t norm_chunk = 0;     // points per batched inversion in the normalisation (0: fitted to the chip)
     uint32_t splits = 1;         // sub-streams, 1..kMaxSplits
@@ -124,6 +127,7 @@ struct WorkSet {
     uint32_t *queue_r = nullptr;  // bucket-reduction work counter, likewise
     Fr *scal = nullptr;
     G1X *u = nullptr, *buckets = nullptr, *cvals = nullptr;
+    uint64_t u_slots = 0;  // G1X entries of u
     uint8_t *bucket_flags = nullptr;  // phase-B buckets to recompute with checked operations
     uint8_t *cval_flags = nullptr;    // reduced outputs to recompute likewise
     G1J *lad = nullptr;
