@@ -1,8 +1,9 @@
 // Fp inversion by a binary GCD on 28-bit approximations (the "optimized
 // binary GCD" of T. Pornin, 2020, eprint 2020/972), for values in 14 x 28-bit
 // limbs.  Fermat's p - 2 power needs ~570 dependent multiplications; this
-// runs a fixed 30 outer iterations of ~1,100 integer instructions each, with
-// no data-dependent branches, so every lane of a wave follows the same path.
+// runs outer iterations of ~1,100 integer instructions each until every lane
+// of the wave is done: 19 to 21 for almost every value, at most 30.  Within an
+// iteration there are no data-dependent branches.
 //
 // Invariants (a, b >= 0, u and v signed, all mod p):  a = u*y,  b = v*y.
 // Start a = y, b = p, u = 1, v = 0.  Each outer iteration
@@ -16,7 +17,7 @@
 //  - and u <- (u f0 + v g0) / 2^28 mod p, v likewise, the division by 2^28
 //    done Montgomery-style (add q p with q = -w p^-1 mod 2^28).
 // 28 outer iterations reach a = 0, b = gcd = 1 for every y (2 * 381 - 1 binary
-// steps suffice); two more are harmless.  Then v = y^-1 mod p, held as a
+// steps suffice), and one after a = 0 would leave v as it is.  Then v = y^-1 mod p, held as a
 // signed value of magnitude below 31p (u and v grow by less than p per
 // iteration and are never reduced).
 //
@@ -159,12 +160,16 @@ VKZG_HD bool inverse(int32_t (&v)[kLimbs], const uint32_t (&y)[kLimbs]) {
         int32_t nu[kLimbs], nv[kLimbs];
         lin_shift_mod(nu, u, v, f0, g0);
         lin_shift_mod(nv, u, v, f1, g1);
+        uint32_t left = 0;
         for (int i = 0; i < kLimbs; i++) {
             a[i] = na[i];
             b[i] = nb[i];
             u[i] = nu[i];
             v[i] = nv[i];
+            left |= na[i];
         }
+        // a = 0: what is left would only multiply v by 2^28 and divide it again
+        if (left == 0) break;
     }
     uint32_t bad = b[0] ^ 1u;
     for (int i = 0; i < kLimbs; i++) bad |= a[i] | (i ? b[i] : 0u);
