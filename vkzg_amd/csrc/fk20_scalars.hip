@@ -21,39 +21,6 @@ constexpr int kScalarWaves = kScalarThreads / 64;
 constexpr int kPolyPitch = 4096;                 // LDS pitch of the polynomial (SoA limbs)
 constexpr int kColPitch = kScalarWaves * 128;    // LDS pitch of the per-wave circulant columns
 
-// The form phase A reads: sign (bit 255) and magnitude (below 2^254) plus the
-// plan's digit bias.
-VKZG_DEV Fr biased_magnitude(const Fr &canonical, const Fr &bias) {
-    const Fr m = fr_signed_magnitude(canonical);
-    Fr r;
-    uint32_t c = 0;
-#pragma unroll
-    for (int i = 0; i < 8; i++) {
-        const uint64_t x = (uint64_t)m.v[i] + bias.v[i] + c;
-        r.v[i] = (uint32_t)x;
-        c = (uint32_t)(x >> 32);
-    }
-    return r;
-}
-
-// sum over the windows below the top one of (2^(width - 1) - 1) 2^bit: added
-// to a magnitude below 2^254 it stays below 2^255, and each of those windows'
-// bits then are its signed digit plus 2^(width - 1) - 1.
-Fr scalar_bias(const WindowPlan &plan) {
-    Fr r{};
-    for (uint32_t w = 0; w + 1 < plan.W; w++) {
-        const uint64_t v = (plan.H() << plan.wide(w)) - 1;
-        const uint32_t li = plan.bit(w) >> 5;
-        uint64_t c = v << (plan.bit(w) & 31u);
-        for (uint32_t i = li; i < 8 && c; i++) {
-            c += r.v[i];
-            r.v[i] = (uint32_t)c;
-            c >>= 32;
-        }
-    }
-    return r;
-}
-
 // `parts` blocks per blob (1, 2, 4 or 8), 8 waves each (2 per SIMD).  LDS:
 // 8 x 4096 words of polynomial + 8 x 1024 words of circulant columns =
 // 160 KiB, all of a CU.  Every part parses the blob and runs the inverse

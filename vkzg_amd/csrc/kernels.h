@@ -88,10 +88,10 @@ hipError_t launch_decompress(G1A *out, const uint8_t *in, uint32_t n, uint32_t *
 hipError_t launch_xext_fft(G1J *out, const G1A *srs, const Fr *roots, hipStream_t s);
 hipError_t launch_jac_to_affine(G1A *out, const G1J *in, Fp *prefix, uint64_t count, uint32_t chunk,
                                 hipStream_t s);
-hipError_t launch_table_chains(G1J *out, const G1A *xext, WindowPlan plan, hipStream_t s);
+hipError_t launch_table_chains(G1J *out, const G1A *bases, uint32_t n, WindowPlan plan, hipStream_t s);
 // The reference's v1 position table (8192 x 32 entries of 24 words) from pw = 2^(8d) xext.
 hipError_t launch_v1_positions(uint32_t *out, const G1A *pw, hipStream_t s);
-hipError_t launch_table_multiples(G1AT *table, const G1A *pw, WindowPlan plan,
+hipError_t launch_table_multiples(G1AT *table, const G1A *pw, uint32_t n, WindowPlan plan,
                                   uint64_t thread_begin, uint32_t thread_count, G1J *scratch,
                                   Fp *prefix, hipStream_t s);
 hipError_t launch_phase_b_scalars(Fr *out, const Fr *roots, hipStream_t s);
@@ -107,13 +107,14 @@ hipError_t launch_phase_b_scalars(Fr *out, const Fr *roots, hipStream_t s);
 hipError_t launch_fk20_scalars(Fr *scal, const uint8_t *blobs, uint64_t blob_stride, uint32_t *err,
                                const Fr *roots, const Fr *roots_inv, uint32_t *queue, Fr *coeffs,
                                uint32_t splits, uint32_t nblobs, WindowPlan plan, hipStream_t s);
+// nblobs * splits * nj MSMs of 64 terms (nj, a multiple of 64: bases of a blob).
 // Persistent: `grid` blocks drain the (64 MSMs, share) items from queue[0];
 // an MSM has parts * groups shares (parts divides 64): part[msm][share].
 // force_checked != 0 (a test switch) sends every share down the checked
 // recompute, as if the fast additions had met a doubling or cancellation; the
 // same holds for launch_phase_b and launch_bucket_reduce.
-hipError_t launch_phase_a(G1X *part, const Fr *scal, const G1AT *table, WindowPlan plan, uint32_t nblobs,
-                          uint32_t splits, uint32_t parts, uint32_t groups, uint32_t grid, uint32_t *queue,
+hipError_t launch_phase_a(G1X *part, const Fr *scal, const G1AT *table, WindowPlan plan, uint32_t nj,
+                          uint32_t nblobs, uint32_t splits, uint32_t parts, uint32_t groups, uint32_t grid, uint32_t *queue,
                           uint32_t force_checked, hipStream_t s);
 // The launch shape of the sum of `shares` partials for each of nmsm MSMs:
 // `sums` partial sums per MSM on `quad` (4 or 1) lanes each, and its estimated
@@ -123,8 +124,7 @@ struct SumShape {
     double us;
 };
 SumShape sum_shape(uint64_t nmsm, uint32_t shares, uint32_t cus);
-// usum[msm] = sum over k < shares of part[msm * shares + k] (nmsm a multiple
-// of 32); force_checked: quads take their checked recompute.
+// usum[msm] = sum over k < shares of part[msm * shares + k]; force_checked: quads take their checked recompute.
 hipError_t launch_sum_groups(G1X *usum, const G1X *part, uint32_t shares, uint32_t nmsm, uint32_t cus,
                              uint32_t force_checked, hipStream_t s);
 // u: one sum per MSM, [nblobs][splits][128].

@@ -108,8 +108,8 @@ __global__ __launch_bounds__(256) void k_ladder(G1J *lad, const G1X *u, uint32_t
 // doubling or cancellation is redone checked by the MSM's first lane.  Q = 1:
 // a lane per sum, with the checked additions.  sum_shape picks both.  The
 // ladder reads these sums, so its prologue (a dependent chain per group of
-// lanes) adds no partials of its own.  nmsm is a multiple of 128, so the grid
-// holds whole MSMs and no lane leaves before the shuffles.
+// lanes) adds no partials of its own.  An MSM's lanes sit in one wave and leave
+// together, so the shuffles only meet lanes that are there.
 VKZG_DEV_COLD void sum_groups_checked(G1X *out, const G1X *part, uint32_t groups) {
     G1X acc = g1x_identity();
     for (uint32_t g = 0; g < groups; g++) acc = g1x_add(acc, part[g]);
@@ -232,7 +232,6 @@ SumShape sum_shape(uint64_t nmsm, uint32_t shares, uint32_t cus) {
 
 hipError_t launch_sum_groups(G1X *usum, const G1X *part, uint32_t shares, uint32_t nmsm, uint32_t cus,
                              uint32_t force_checked, hipStream_t s) {
-    if (nmsm % 32 != 0) return hipErrorInvalidValue;
     auto run = [&](auto kernel, uint32_t lanes) {
         hipLaunchKernelGGL(kernel, dim3(blocks_for((uint64_t)nmsm * lanes, 256)), dim3(256), 0, s, usum, part, shares,
                            nmsm, force_checked);

@@ -1,6 +1,7 @@
 // Variable-base multi-scalar multiplication on G1 (Pippenger's bucket method
-// with the GLV split), for the sums of batch cell-proof verification and for
-// commitments.  No reference counterpart: the reference only has the FK20
+// with the GLV split), for the sums of batch cell-proof verification (for
+// commitments, over fixed points, phase A's kernel and a multiples table).  No
+// reference counterpart: the reference only has the FK20
 // MSMs with fixed scalars or fixed points (k_phase_a.comp, k_phase_b_split.comp).
 //
 // Several independent sums ("MSMs") run in one launch sequence.  Entry e adds
@@ -12,11 +13,9 @@
 //   scan     bucket offsets (one block; three passes above 16k buckets)
 //   scatter  point references sorted by key               (atomics)
 //   buckets  one lane per bucket sums its points          (XYZZ, checked);
-//            buckets of more than 24 points by a team of 64 lanes (large
-//            launches: 16)
+//            buckets of more than 24 points by a wave
 //   windows  blocks per (msm, window): sum_b (b+1) B_b by running sums over
-//            segments of at most 4 (large launches: 16) buckets, then trees
-//            in LDS
+//            segments of at most 4 buckets, then trees in LDS
 //   combine  four lanes per MSM: Horner over windows (c doublings each),
 //            each doubling and addition shared by the quad, and the
 //            conversion to affine.
@@ -32,15 +31,8 @@ namespace vkzg_amd {
 namespace {
 
 constexpr uint32_t kWinThreads = 128;
-constexpr uint32_t kHotLen = 24; // longer buckets are summed by a team of lanes (k_msm_hot)
-// Launch regimes.  Small sums (verification) are latency-bound: 4 buckets per
-// window thread, and a hot bucket (often hundreds of points: a narrow top
-// window) summed by 64 lanes.  From kBigK buckets on (commitments of many
-// blobs) the launches are throughput-bound: 16 buckets per window thread
-// spread its fixed costs (the offset multiple and the tree), and hot buckets
-// (thousands, of some 30 points) are summed by teams of 16 lanes.
-constexpr uint32_t kBigK = 1u << 18;
-constexpr uint32_t kWinSegSmall = 4, kWinSegBig = 16;
+constexpr uint32_t kHotLen = 24;    // longer buckets are summed by a wave (k_msm_hot)
+constexpr uint32_t kWinSeg = 4;     // buckets per window thread: the sums are latency-bound
 constexpr uint32_t kHotBlocks = 2048;
 constexpr uint32_t kScanOneBlock = 16384;  // larger scans use k_msm_scan_tiles
 constexpr uint32_t kScanTile = 4096;       // buckets per block of k_msm_scan_tiles
@@ -238,34 +230,27 @@ __global__ void __launch_bounds__(64) k_msm_buckets(G1X *buckets, const uint32_t
     buckets[key] = acc;
 }
 
-// Hot buckets, TEAM lanes each (64 / TEAM per block; blocks stride over the
-// list): the team's lanes sum interleaved shares of the bucket's points, then
-// a tree in LDS.  The loop bound is uniform over the block (barriers).
-template <uint32_t TEAM>
+// Hot buckets, one wave each (blocks stride over the list): the lanes sum
+// interleaved shares of the bucket's points, then a tree in LDS.
 __global__ void __launch_bounds__(64) k_msm_hot(G1X *buckets, const uint32_t *off, const uint32_t *list,
                                                 const G1A *pts, const uint32_t *hot, const uint32_t *hot_n) {
-    constexpr uint32_t kTeams = 64 / TEAM;
     __shared__ G1X sh[64];
-    const uint32_t t = threadIdx.x, l = t % TEAM;
+    const uint32_t t = threadIdx.x;
     const uint32_t n = *hot_n;
 #pragma unroll 1
-    for (uint32_t q0 = blockIdx.x * kTeams; q0 < n; q0 += gridDim.x * kTeams) {
-        const uint32_t q = q0 + t / TEAM;
-        uint32_t key = 0;
+    for (uint32_t q = blockIdx.x; q < n; q += gridDim.x) {
+        const uint32_t key = hot[q];
+        const uint32_t lo = off[key], hi = off[key + 1];
         G1X acc = g1x_identity();
-        if (q < n) {
-            key = hot[q];
-            const uint32_t lo = off[key], hi = off[key + 1];
 #pragma unroll 1
-            for (uint32_t i = lo + l; i < hi; i += TEAM) acc = g1x_madd(acc, msm_point(pts, list[i]));
-        }
+        for (uint32_t i = lo + t; i < hi; i += 64) acc = g1x_madd(acc, msm_point(pts, list[i]));
         sh[t] = acc;
         __syncthreads();
-        for (uint32_t stride = TEAM / 2; stride > 0; stride >>= 1) {
-            if (l < stride) sh[t] = g1x_add(sh[t], sh[t + stride]);
+        for (uint32_t stride = 32; stride > 0; stride >>= 1) {
+            if (t < stride) sh[t] = g1x_add(sh[t], sh[t + stride]);
             __syncthreads();
         }
-        if (q < n && l == 0) buckets[key] = sh[t];
+        if (t == 0) buckets[key] = sh[0];
         __syncthreads();
     }
 }
@@ -285,7 +270,7 @@ VKZG_DEV G1X g1x_mul_small(const G1X &p, uint32_t k) {
 // Thread t owns buckets [lo, lo + seg): running sums from the top give
 // R = sum B_b and T = sum (b - lo + 1) B_b, and its share is T + lo R; a
 // tree in LDS adds the shares.  A window's parts (enough of them for at most
-// kWinSegSmall or kWinSegBig buckets per thread) are added by k_msm_parts.
+// kWinSeg buckets per thread) are added by k_msm_parts.
 __global__ void __launch_bounds__(kWinThreads) k_msm_windows(G1X *wpart, const G1X *buckets, uint32_t bk,
                                                              uint32_t parts) {
     __shared__ G1X sh[kWinThreads];
@@ -380,9 +365,7 @@ MsmShape msm_shape(uint32_t ne, uint32_t nmsm) {
     sh.W = (129 + c - 1) / c;
     sh.bk = 1u << (c - 1);
     sh.K = nmsm * sh.W * sh.bk;
-    const bool big = sh.K >= kBigK;
-    const uint32_t seg = big ? kWinSegBig : kWinSegSmall;
-    sh.parts = sh.bk > kWinThreads * seg ? sh.bk / (kWinThreads * seg) : 1;
+    sh.parts = sh.bk > kWinThreads * kWinSeg ? sh.bk / (kWinThreads * kWinSeg) : 1;
     return sh;
 }
 
@@ -436,10 +419,7 @@ hipError_t launch_msm(const MsmShape &sh, void *scratch, const G1A *pts, const u
     hipLaunchKernelGGL(k_msm_buckets, dim3(blocks_for(sh.K, 64)), dim3(64), 0, s, buckets, off, list, pts,
                        sh.K, hot, cnt + sh.K);
     const dim3 hot_grid(sh.K < kHotBlocks ? sh.K : kHotBlocks);
-    if (sh.K >= kBigK)
-        hipLaunchKernelGGL(k_msm_hot<16>, hot_grid, dim3(64), 0, s, buckets, off, list, pts, hot, cnt + sh.K);
-    else
-        hipLaunchKernelGGL(k_msm_hot<64>, hot_grid, dim3(64), 0, s, buckets, off, list, pts, hot, cnt + sh.K);
+    hipLaunchKernelGGL(k_msm_hot, hot_grid, dim3(64), 0, s, buckets, off, list, pts, hot, cnt + sh.K);
     hipLaunchKernelGGL(k_msm_windows, dim3(sh.nmsm * sh.W * sh.parts), dim3(kWinThreads), 0, s, wpart, buckets,
                        sh.bk, sh.parts);
     hipLaunchKernelGGL(k_msm_parts, dim3(sh.nmsm * sh.W), dim3(64), 0, s, wsum, wpart, sh.parts);

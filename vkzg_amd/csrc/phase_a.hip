@@ -63,12 +63,14 @@ __device__ __attribute__((noinline)) void phase_a_slow(G1X *out, const Fr *scal,
     *out = acc;
 }
 
-// Persistent phase A.  MSM m = (blob * splits + seg) * 128 + j is
-//   u[m] = sum_{i<64} scal[m][i] * xext[j][i]
+// Persistent phase A.  MSM m = (blob * splits + seg) * nj + j, j < nj, is
+//   u[m] = sum_{i<64} scal[m][i] * base[j][i]
+// (nj = 128 and the bases x_ext_fft for the proofs; nj = 64 and the setup's
+// 4096 points for commitments)
 // with the scalar in signed digits v in [-(2^(b-1)-1), 2^(b-1)] of each window's
 // width b (the recoding of k_phase_a_sort.comp:31-40 with the plan's windows),
 // each digit's sign flipped for a negative scalar, and
-// table[j][i][entry(w) + |v| - 1] = |v| * 2^bit(w) * xext[j][i].  Its terms are
+// table[j][i][entry(w) + |v| - 1] = |v| * 2^bit(w) * base[j][i].  Its terms are
 // cut into `parts` runs of 64 / parts and its windows into `groups` groups, and
 // one lane adds up one (run, group) share: part[m * parts * groups + share].
 // k_sum_groups adds an MSM's shares.
@@ -95,12 +97,12 @@ __device__ __attribute__((noinline)) void phase_a_slow(G1X *out, const Fr *scal,
 //
 // A wave takes items (share, 64 MSMs) from the counter q[0], cleared by the
 // kernel that runs before, until the queue is drained, and leaves after one
-// failed take; nmsm is a multiple of 128, so items are whole waves.
+// failed take; nj is a multiple of 64, so items are whole waves.
 __global__ void __launch_bounds__(256, 2)
-    k_phase_a(G1X *part, const Fr *scal, const G1AT *table, WindowPlan plan, uint32_t nblobs, uint32_t splits,
-              uint32_t parts, uint32_t groups, uint32_t *q, uint32_t force_checked) {
+    k_phase_a(G1X *part, const Fr *scal, const G1AT *table, WindowPlan plan, uint32_t nj, uint32_t nblobs,
+              uint32_t splits, uint32_t parts, uint32_t groups, uint32_t *q, uint32_t force_checked) {
     const uint32_t lane = threadIdx.x % 64;
-    const uint32_t per_share = nblobs * splits * 2;  // items of 64 MSMs
+    const uint32_t per_share = nblobs * splits * (nj / 64);  // items of 64 MSMs
     const uint32_t shares = parts * groups, nitems = per_share * shares;
     const uint32_t terms = 64 / parts;
 #pragma unroll 1
@@ -113,7 +115,7 @@ __global__ void __launch_bounds__(256, 2)
         const uint32_t run = share / groups, g = share % groups;
         const uint32_t idx = (item % per_share) * 64 + lane;
         const uint32_t blob = idx % nblobs, js = idx / nblobs;
-        const uint32_t j = js / splits, msm = (blob * splits + js % splits) * 128 + j;
+        const uint32_t j = js / splits, msm = (blob * splits + js % splits) * nj + j;
         const uint32_t w0 = g * plan.W / groups, w1 = (g + 1) * plan.W / groups;
         const Fr *sc = scal + (size_t)msm * 64 + run * terms;
         const G1AT *tab = table + (size_t)(j * 64 + run * terms) * plan.entries();
@@ -165,15 +167,15 @@ __global__ void __launch_bounds__(256, 2)
 
 }  // namespace
 
-hipError_t launch_phase_a(G1X *part, const Fr *scal, const G1AT *table, WindowPlan plan, uint32_t nblobs,
-                          uint32_t splits, uint32_t parts, uint32_t groups, uint32_t grid, uint32_t *queue,
+hipError_t launch_phase_a(G1X *part, const Fr *scal, const G1AT *table, WindowPlan plan, uint32_t nj,
+                          uint32_t nblobs, uint32_t splits, uint32_t parts, uint32_t groups, uint32_t grid, uint32_t *queue,
                           uint32_t force_checked, hipStream_t s) {
-    if (parts == 0 || 64 % parts != 0) return hipErrorInvalidValue;
-    const uint32_t blocks = (nblobs * splits * 2 * parts * groups + 3) / 4;  // four waves each
+    if (parts == 0 || 64 % parts != 0 || nj % 64 != 0) return hipErrorInvalidValue;
+    const uint32_t blocks = (nblobs * splits * (nj / 64) * parts * groups + 3) / 4;  // four waves each
     if (grid > blocks) grid = blocks;
     if (grid == 0) grid = 1;
-    hipLaunchKernelGGL(k_phase_a, dim3(grid), dim3(256), 0, s, part, scal, table, plan, nblobs, splits, parts,
-                       groups, queue, force_checked);
+    hipLaunchKernelGGL(k_phase_a, dim3(grid), dim3(256), 0, s, part, scal, table, plan, nj, nblobs, splits,
+                       parts, groups, queue, force_checked);
     return hipGetLastError();
 }
 

@@ -238,34 +238,34 @@ void build_phase_b_items(const Fr *kpm, std::vector<uint32_t> &items, std::vecto
     offsets.push_back(n2);
 }
 
-// Fills t with a freshly built phase-A table of the window plan: the W chains
-// 2^bit(w) xext (affine), then every multiple d * 2^bit(w) xext,
+// Fills t with a freshly built table of the window plan over n bases: the W
+// chains 2^bit(w) base (affine), then every multiple d * 2^bit(w) base,
 // d <= 2^(width(w)-1).
-void build_phase_a_table(vkzg_prover *p, PhaseATable &t, WindowPlan plan) {
+void build_phase_a_table(vkzg_prover *p, PhaseATable &t, WindowPlan plan, const G1A *bases, uint32_t nbases) {
     hipStream_t s = p->stream;
     const uint32_t c = plan.c;
     t.c = c;
     t.W = plan.W;
     t.H = plan.H();
     t.k = plan.k;
-    t.bytes = 8192ull * plan.entries() * sizeof(G1AT);
+    t.bytes = (uint64_t)nbases * plan.entries() * sizeof(G1AT);
     t.table = p->arena.dalloc<G1AT>(t.bytes / sizeof(G1AT));
-    G1J *pwj = p->arena.dalloc<G1J>((size_t)t.W * 8192);
-    Fp *pw_prefix = p->arena.dalloc<Fp>((size_t)t.W * 8192);
-    G1A *pw = p->arena.dalloc<G1A>((size_t)t.W * 8192);
-    ck(launch_table_chains(pwj, p->xext, plan, s));
-    ck(launch_jac_to_affine(pw, pwj, pw_prefix, (uint64_t)t.W * 8192, 16, s));
+    G1J *pwj = p->arena.dalloc<G1J>((size_t)t.W * nbases);
+    Fp *pw_prefix = p->arena.dalloc<Fp>((size_t)t.W * nbases);
+    G1A *pw = p->arena.dalloc<G1A>((size_t)t.W * nbases);
+    ck(launch_table_chains(pwj, bases, nbases, plan, s));
+    ck(launch_jac_to_affine(pw, pwj, pw_prefix, (uint64_t)t.W * nbases, 16, s));
     ck(hipStreamSynchronize(s));
     p->arena.dfree(pwj);
     p->arena.dfree(pw_prefix);
     const uint32_t S = t.H < 64 ? t.H : 64;
-    const uint64_t total_threads = 8192ull * (t.W + t.k) * (t.H / S);  // S entries each
+    const uint64_t total_threads = (uint64_t)nbases * (t.W + t.k) * (t.H / S);  // S entries each
     const uint32_t slice = 1u << 18;
     G1J *scratch = p->arena.dalloc<G1J>((size_t)S * slice);
     Fp *pref = p->arena.dalloc<Fp>((size_t)S * slice);
     for (uint64_t t0 = 0; t0 < total_threads; t0 += slice) {
         const uint32_t n = (uint32_t)std::min<uint64_t>(slice, total_threads - t0);
-        ck(launch_table_multiples(t.table, pw, plan, t0, n, scratch, pref, s));
+        ck(launch_table_multiples(t.table, pw, nbases, plan, t0, n, scratch, pref, s));
     }
     ck(hipStreamSynchronize(s));
     p->arena.dfree(scratch);
@@ -345,7 +345,7 @@ void build_tables(vkzg_prover *p, const uint8_t *setup) {
     size_t free_b = 0, total_b = 0;
     ck(hipMemGetInfo(&free_b, &total_b));
     PhaseATable main_table;
-    build_phase_a_table(p, main_table, choose_window(free_b));
+    build_phase_a_table(p, main_table, choose_window(free_b), p->xext, 8192);
     p->c = main_table.c;
     p->W = main_table.W;
     p->H = main_table.H;
@@ -473,9 +473,6 @@ uint32_t fit_norm_chunk(uint64_t count, uint32_t cus) {
 // two per SIMD and the last round counts whole (measured at 1 to 256 blobs).
 // More shares shorten the chain while SIMDs are idle; past that, and wherever
 // they start another round, they only lengthen the sum.
-struct PhaseAShape {
-    uint32_t parts, groups;
-};
 PhaseAShape phase_a_shape(uint64_t nmsm, uint32_t groups, uint32_t windows, uint64_t slots, uint32_t cus) {
     const uint64_t simds = (uint64_t)cus * 4;
     PhaseAShape best{1, groups ? groups : 1};
@@ -570,7 +567,7 @@ void proofs_range(vkzg_prover *p, WorkSet &ws, uint32_t off, uint32_t nb, uint8_
     ck(launch_fk20_scalars(scal, d_blobs, blob_stride, err, p->roots, p->roots_inv, queue, coeffs,
                            tn.ladder_splits, nb, tab.plan(), s));
     clk.mark("fk20_scalars");
-    ck(launch_phase_a(u, scal, tab.table, tab.plan(), nb, tn.ladder_splits, shape.parts, shape.groups,
+    ck(launch_phase_a(u, scal, tab.table, tab.plan(), 128, nb, tn.ladder_splits, shape.parts, shape.groups,
                       p->cus * tn.blocks_per_cu, queue, tn.force_checked, s));
     clk.mark("phase_a");
     if (shares > 1) {
@@ -843,7 +840,7 @@ void autotune(vkzg_prover *p) {
             size_t free_b = 0, total_b = 0;
             ck(hipMemGetInfo(&free_b, &total_b));
             if (table_bytes_for(w) > free_b / 2) continue;
-            build_phase_a_table(p, slot, window_plan(w, 0));
+            build_phase_a_table(p, slot, window_plan(w, 0), p->xext, 8192);
         }
         windows.push_back(w);
     }
@@ -1333,7 +1330,7 @@ vkzg_result vkzg_amd_load_window_table(vkzg_prover *p, uint32_t window_bits) {
         size_t free_b = 0, total_b = 0;
         ck(hipMemGetInfo(&free_b, &total_b));
         if (table_bytes_for(window_bits) > free_b) return VKZG_ERR_MALLOC;
-        build_phase_a_table(p, slot, window_plan(window_bits, 0));
+        build_phase_a_table(p, slot, window_plan(window_bits, 0), p->xext, 8192);
     } catch (HipFail &) {
         if (slot.table) p->arena.dfree(slot.table);
         slot = PhaseATable{};

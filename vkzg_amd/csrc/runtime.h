@@ -45,8 +45,9 @@ struct Tuning {
     uint32_t force_checked = 0;
 };
 
-// A resident phase-A multiples table of window c: W = ceil(256 / c) windows
-// of H = 2^(c-1) multiples (table[128][64][W][H], one 128-byte line each).
+// A resident multiples table of a window plan, one 128-byte line per multiple:
+// table[128][64][entries] over x_ext_fft for the proofs, table[64][64][entries]
+// over the setup points for commitments.
 struct PhaseATable {
     uint32_t c = 0, W = 0, H = 0, k = 0;  // window plan (c, W, k), H = 2^(c-1)
     uint64_t bytes = 0;
@@ -329,6 +330,20 @@ Tuning tuning_for(const vkzg_prover *p, uint32_t nb);
 
 // The phase-A table a tuning names (window_bits 0: the main one).
 PhaseATable phase_a_table(const vkzg_prover *p, uint32_t window_bits);
+
+// Fills t with a multiples table of `plan` over n affine bases (device memory of
+// the prover's arena).
+void build_phase_a_table(vkzg_prover *p, PhaseATable &t, WindowPlan plan, const G1A *bases, uint32_t n);
+
+// The shares phase A cuts each of nmsm MSMs into (groups != 0: that many window
+// groups), with room for `slots` partials and sums.
+struct PhaseAShape {
+    uint32_t parts, groups;
+};
+PhaseAShape phase_a_shape(uint64_t nmsm, uint32_t groups, uint32_t windows, uint64_t slots, uint32_t cus);
+
+// host (pageable) -> pinned staging -> dev, enqueued on s.
+void stage_upload(int device, uint8_t *dev, uint8_t *pinned, const uint8_t *host, size_t bytes, hipStream_t s);
 
 // Enqueue a pipeline through `cache` when graphs are on and stage timing is
 // off (timing records events between stages), else launch it directly.

@@ -40,14 +40,14 @@ __global__ void __launch_bounds__(256) k_jac_to_affine(G1A *out, const G1J *in, 
     }
 }
 
-// out[w][b] = 2^bit(w) * xext[b] for the 8192 bases.
-__global__ void k_table_chains(G1J *out, const G1A *xext, WindowPlan plan) {
+// out[w][b] = 2^bit(w) * bases[b] for the n bases.
+__global__ void k_table_chains(G1J *out, const G1A *bases, uint32_t n, WindowPlan plan) {
     const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= 8192) return;
-    G1J p = g1j_from_affine(xext[b]);
+    if (b >= n) return;
+    G1J p = g1j_from_affine(bases[b]);
 #pragma unroll 1
     for (uint32_t w = 0; w < plan.W; w++) {
-        out[(size_t)w * 8192 + b] = p;
+        out[(size_t)w * n + b] = p;
 #pragma unroll 1
         for (uint32_t k = 0; k < plan.c + plan.wide(w); k++) p = g1j_dbl(p);
     }
@@ -77,7 +77,7 @@ __device__ __attribute__((noinline)) void table_run_slow(G1J *scratch, Fp *prefi
 // from entry v H + seg S: the multiples d in [d0, d0 + S) of P = pw[w][b] for
 // the window w that owns slot v (d0 = seg S + 1, plus H in a wide window's
 // second slot), a running sum normalised with one inversion per thread.
-__global__ void __launch_bounds__(64) k_table_multiples(G1AT *table, const G1A *pw, WindowPlan plan,
+__global__ void __launch_bounds__(64) k_table_multiples(G1AT *table, const G1A *pw, uint32_t n, WindowPlan plan,
                                   uint64_t thread_begin, uint32_t thread_count, G1J *scratch,
                                   Fp *prefix) {
     const uint32_t lt = blockIdx.x * blockDim.x + threadIdx.x;
@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(64) k_table_multiples(G1AT *table, const G1A *
     const uint32_t b = (uint32_t)(bv / slots);
     const uint32_t w = v < narrow ? v : narrow + (v - narrow) / 2;
     const uint32_t half = v < narrow ? 0u : (v - narrow) % 2;
-    const G1A P = pw[(size_t)w * 8192 + b];
+    const G1A P = pw[(size_t)w * n + b];
     const uint32_t d0 = (half * nseg + seg) * S + 1;
 
     // d0 * P by double-and-add (no addition there meets equal points), then
@@ -150,8 +150,8 @@ hipError_t launch_jac_to_affine(G1A *out, const G1J *in, Fp *prefix, uint64_t co
     return hipGetLastError();
 }
 
-hipError_t launch_table_chains(G1J *out, const G1A *xext, WindowPlan plan, hipStream_t s) {
-    hipLaunchKernelGGL(k_table_chains, dim3(8192 / 64), dim3(64), 0, s, out, xext, plan);
+hipError_t launch_table_chains(G1J *out, const G1A *bases, uint32_t n, WindowPlan plan, hipStream_t s) {
+    hipLaunchKernelGGL(k_table_chains, dim3(blocks_for(n, 64)), dim3(64), 0, s, out, bases, n, plan);
     return hipGetLastError();
 }
 
@@ -182,11 +182,11 @@ hipError_t launch_v1_positions(uint32_t *out, const G1A *pw, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_table_multiples(G1AT *table, const G1A *pw, WindowPlan plan,
+hipError_t launch_table_multiples(G1AT *table, const G1A *pw, uint32_t n, WindowPlan plan,
                                   uint64_t thread_begin, uint32_t thread_count, G1J *scratch,
                                   Fp *prefix, hipStream_t s) {
     hipLaunchKernelGGL(k_table_multiples, dim3(blocks_for(thread_count, 64)), dim3(64), 0, s, table,
-                       pw, plan, thread_begin, thread_count, scratch, prefix);
+                       pw, n, plan, thread_begin, thread_count, scratch, prefix);
     return hipGetLastError();
 }
 

@@ -92,7 +92,7 @@ extern "C" vkzg_result vkzg_amd_write_v1_tables(vkzg_prover *p, const char *path
         uint32_t *words = tmp.dalloc<uint32_t>(positions.size());
         Fr *d_kpm = tmp.dalloc<Fr>(128);
         static_assert(kV1Positions == 32, "2^(8d) positions d < 32: the (8, 0) window plan");
-        ck(launch_table_chains(pwj, p->xext, window_plan(8, 0), s));
+        ck(launch_table_chains(pwj, p->xext, 8192, window_plan(8, 0), s));
         ck(launch_jac_to_affine(pw, pwj, prefix, (uint64_t)kV1Positions * 8192, 16, s));
         ck(launch_v1_positions(words, pw, s));
         ck(launch_phase_b_scalars(d_kpm, p->roots, s));

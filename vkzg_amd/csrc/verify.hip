@@ -170,17 +170,23 @@ __global__ void k_vfy_entries(Fr *sc, uint32_t *pidx, uint8_t *mid, const Fr *rp
     mid[e] = (uint8_t)m;
 }
 
-// Commitment scalars of nb <= 256 blobs: sc[b * 4096 + i] = coefficient i of
-// blob b's polynomial (canonical), pidx = i, mid = b; err[b] = 1 for a blob with a
-// non-canonical element (as k_fk20_scalars, k_blob_to_fr.comp:23-37).
-constexpr int kCommitThreads = 256;
-__global__ void __launch_bounds__(kCommitThreads) k_commit_scalars(Fr *sc, uint32_t *pidx, uint8_t *mid,
-                                                                  uint32_t *err, const uint8_t *blobs,
-                                                                  const Fr *roots_inv) {
+// Commitment scalars of nb blobs: sc[b * 4096 + i] = coefficient i of blob b's
+// polynomial in phase A's form (sign and biased magnitude), MSM j of a blob
+// taking coefficients [64 j, 64 j + 64); err[b] = 1 for a blob with a
+// non-canonical element (as k_fk20_scalars, k_blob_to_fr.comp:23-37).  Clears
+// the work counter of the phase-A launch that follows.
+// One block per blob holds the whole transform in LDS; with 16 waves (four per
+// SIMD) instead of 4 it takes 0.09 instead of 0.14 ms.
+constexpr int kCommitThreads = 1024;
+
+__global__ void __launch_bounds__(kCommitThreads) k_commit_scalars(Fr *sc, uint32_t *queue, uint32_t *err,
+                                                                   const uint8_t *blobs, const Fr *roots_inv,
+                                                                   Fr bias) {
     __shared__ uint32_t poly[8 * 4096];
     const uint32_t blob = blockIdx.x;
     const int tid = threadIdx.x;
     const uint32_t *src = reinterpret_cast<const uint32_t *>(blobs + (size_t)131072 * blob);
+    if (blob == 0 && tid == 0) queue[0] = 0;
     bool bad = false;
 #pragma unroll 1
     for (int i = tid; i < 4096; i += kCommitThreads) {
@@ -196,15 +202,30 @@ __global__ void __launch_bounds__(kCommitThreads) k_commit_scalars(Fr *sc, uint3
     lds_ntt_dit<12>(poly, 4096, 1, roots_inv, tid, kCommitThreads);
     const Fr inv_n = fr_const(cfr::INV_4096_M);
 #pragma unroll 1
-    for (int i = tid; i < 4096; i += kCommitThreads) {
-        const size_t e = (size_t)blob * 4096 + i;
-        sc[e] = fr_to_canonical(fr_mul(lds_load_fr(poly, 4096, i), inv_n));
-        pidx[e] = (uint32_t)i;
-        mid[e] = (uint8_t)blob;  // one MSM per blob: at most 256 blobs per launch
-    }
+    for (int i = tid; i < 4096; i += kCommitThreads)
+        sc[(size_t)blob * 4096 + i] =
+            biased_magnitude(fr_to_canonical(fr_mul(lds_load_fr(poly, 4096, i), inv_n)), bias);
 }
 
-__global__ void k_compress_points(uint8_t *out, const G1A *pts, uint32_t n) {
+// Compressed affine form of n points.
+__global__ void __launch_bounds__(64) k_compress_points(uint8_t *out, const G1X *pts, uint32_t n) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const G1X p = pts[i];
+    G1A a = g1a_identity();
+    if (!g1x_is_identity(p)) {
+        // x = X / ZZ = X ZZZ / (ZZ ZZZ), y = Y / ZZZ = Y ZZ / (ZZ ZZZ): one inversion
+        const Fp inv = fp_inv(fp_mul(p.zz, p.zzz));
+        a.x = fp_mul(fp_mul(p.x, p.zzz), inv);
+        a.y = fp_mul(fp_mul(p.y, p.zz), inv);
+    }
+    uint32_t w[12];
+    g1a_compress_words(w, a);
+    uint32_t *dst = reinterpret_cast<uint32_t *>(out + 48ull * i);
+#pragma unroll
+    for (int k = 0; k < 12; k++) dst[k] = w[k];
+}
+__global__ void k_compress_affine(uint8_t *out, const G1A *pts, uint32_t n) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     uint32_t w[12];
@@ -248,14 +269,18 @@ hipError_t launch_vfy_entries(Fr *sc, uint32_t *pidx, uint8_t *mid, const Fr *rp
                        cgrp_off, cgrp, cell_idx, roots, agg, n, u);
     return hipGetLastError();
 }
-hipError_t launch_commit_scalars(Fr *sc, uint32_t *pidx, uint8_t *mid, uint32_t *err, const uint8_t *blobs,
-                                 uint32_t nb, const Fr *roots_inv, hipStream_t s) {
-    hipLaunchKernelGGL(k_commit_scalars, dim3(nb), dim3(kCommitThreads), 0, s, sc, pidx, mid, err, blobs,
-                       roots_inv);
+hipError_t launch_commit_scalars(Fr *sc, uint32_t *queue, uint32_t *err, const uint8_t *blobs, uint32_t nb,
+                                 const Fr *roots_inv, WindowPlan plan, hipStream_t s) {
+    hipLaunchKernelGGL(k_commit_scalars, dim3(nb), dim3(kCommitThreads), 0, s, sc, queue, err, blobs, roots_inv,
+                       scalar_bias(plan));
     return hipGetLastError();
 }
-hipError_t launch_compress_points(uint8_t *out, const G1A *pts, uint32_t n, hipStream_t s) {
+hipError_t launch_compress_points(uint8_t *out, const G1X *pts, uint32_t n, hipStream_t s) {
     hipLaunchKernelGGL(k_compress_points, dim3(blocks_for(n, 64)), dim3(64), 0, s, out, pts, n);
+    return hipGetLastError();
+}
+hipError_t launch_compress_affine(uint8_t *out, const G1A *pts, uint32_t n, hipStream_t s) {
+    hipLaunchKernelGGL(k_compress_affine, dim3(blocks_for(n, 64)), dim3(64), 0, s, out, pts, n);
     return hipGetLastError();
 }
 
