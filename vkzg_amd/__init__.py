@@ -44,6 +44,28 @@ def _check(rc):
         raise VkzgError(rc)
 
 
+# Results are written by the library straight into the bytes object that is
+# returned: PyBytes_FromStringAndSize(NULL, n) gives one of n uninitialised
+# bytes that nothing else holds yet.  Inputs that are bytes go in by their own
+# address.  A 9.7 MB recovery would otherwise be copied twice and cleared once
+# in Python (about a third of the call).
+_new_bytes = ctypes.pythonapi.PyBytes_FromStringAndSize
+_new_bytes.restype = ctypes.py_object
+_new_bytes.argtypes = [ctypes.c_void_p, ctypes.c_ssize_t]
+_bytes_at = ctypes.pythonapi.PyBytes_AsString
+_bytes_at.restype = ctypes.c_void_p
+_bytes_at.argtypes = [ctypes.py_object]
+
+
+class _Out:
+    """A result of n bytes: .at its address for the library, .value the bytes object."""
+
+    def __init__(self, n):
+        # an empty or one-byte object may be shared: never written to
+        self.value = _new_bytes(None, n) if n > 1 else b""
+        self.at = _bytes_at(self.value)
+
+
 class Prover:
     """One vkzg_prover on the current HIP device."""
 
@@ -96,10 +118,9 @@ class Prover:
         if len(blobs) != blob_count * BYTES_PER_BLOB:
             raise ValueError("blobs.length must be blobCount * %d" % BYTES_PER_BLOB)
         nbytes = blob_count * CELL_PROOFS_PER_BLOB * BYTES_PER_PROOF
-        out = ctypes.create_string_buffer(max(1, nbytes))
-        src = ctypes.create_string_buffer(bytes(blobs), max(1, len(blobs)))
-        _check(load().vkzg_compute_proofs_batch(self._h, out, src, blob_count))
-        return out.raw[:nbytes]
+        out = _Out(nbytes)
+        _check(load().vkzg_compute_proofs_batch(self._h, out.at, bytes(blobs), blob_count))
+        return out.value
 
     def recover_cells_batch(self, cells, cell_present, blob_count):
         per_blob = CELL_PROOFS_PER_BLOB * BYTES_PER_CELL
@@ -107,11 +128,9 @@ class Prover:
             raise ValueError("cells.length must be blobCount * %d" % per_blob)
         if len(cell_present) != blob_count * CELL_PROOFS_PER_BLOB:
             raise ValueError("cellPresent.length must be blobCount * %d" % CELL_PROOFS_PER_BLOB)
-        out = ctypes.create_string_buffer(max(1, len(cells)))
-        c = ctypes.create_string_buffer(bytes(cells), max(1, len(cells)))
-        pm = ctypes.create_string_buffer(bytes(cell_present), max(1, len(cell_present)))
-        _check(load().vkzg_recover_cells_batch(self._h, out, c, pm, blob_count))
-        return out.raw[: len(cells)]
+        out = _Out(len(cells))
+        _check(load().vkzg_recover_cells_batch(self._h, out.at, bytes(cells), bytes(cell_present), blob_count))
+        return out.value
 
     def compute_cells_and_kzg_proofs_batch(self, blobs, blob_count):
         """(cells, proofs) of each blob: the 2x extension and the 128 proofs."""
@@ -119,11 +138,9 @@ class Prover:
             raise ValueError("blobs.length must be blobCount * %d" % BYTES_PER_BLOB)
         ncells = blob_count * CELL_PROOFS_PER_BLOB * BYTES_PER_CELL
         nproofs = blob_count * CELL_PROOFS_PER_BLOB * BYTES_PER_PROOF
-        cells = ctypes.create_string_buffer(max(1, ncells))
-        proofs = ctypes.create_string_buffer(max(1, nproofs))
-        src = ctypes.create_string_buffer(bytes(blobs), max(1, len(blobs)))
-        _check(load().vkzg_amd_compute_cells_and_proofs(self._h, cells, proofs, src, blob_count))
-        return cells.raw[:ncells], proofs.raw[:nproofs]
+        cells, proofs = _Out(ncells), _Out(nproofs)
+        _check(load().vkzg_amd_compute_cells_and_proofs(self._h, cells.at, proofs.at, bytes(blobs), blob_count))
+        return cells.value, proofs.value
 
     def recover_cells_and_kzg_proofs_batch(self, cells, cell_present, blob_count):
         """(all 128 cells, 128 proofs) of each blob from any >= 64 of its cells."""
@@ -133,12 +150,10 @@ class Prover:
         if len(cell_present) != blob_count * CELL_PROOFS_PER_BLOB:
             raise ValueError("cellPresent.length must be blobCount * %d" % CELL_PROOFS_PER_BLOB)
         nproofs = blob_count * CELL_PROOFS_PER_BLOB * BYTES_PER_PROOF
-        out = ctypes.create_string_buffer(max(1, len(cells)))
-        proofs = ctypes.create_string_buffer(max(1, nproofs))
-        c = ctypes.create_string_buffer(bytes(cells), max(1, len(cells)))
-        pm = ctypes.create_string_buffer(bytes(cell_present), max(1, len(cell_present)))
-        _check(load().vkzg_amd_recover_cells_and_proofs(self._h, out, proofs, c, pm, blob_count))
-        return out.raw[:len(cells)], proofs.raw[:nproofs]
+        out, proofs = _Out(len(cells)), _Out(nproofs)
+        _check(load().vkzg_amd_recover_cells_and_proofs(self._h, out.at, proofs.at, bytes(cells), bytes(cell_present),
+                                                        blob_count))
+        return out.value, proofs.value
 
     def load_g2_setup(self, g2_monomial):
         """The 65 compressed G2 setup points [tau^i]G2 (65 x 96 bytes) for verification."""
@@ -182,10 +197,9 @@ class Prover:
         """Commitments (blob_count x 48 bytes) of blob_count blobs."""
         if len(blobs) != blob_count * BYTES_PER_BLOB:
             raise ValueError("blobs.length must be blobCount * %d" % BYTES_PER_BLOB)
-        out = ctypes.create_string_buffer(max(1, 48 * blob_count))
-        src = ctypes.create_string_buffer(bytes(blobs), max(1, len(blobs)))
-        _check(load().vkzg_amd_blob_to_commitments(self._h, out, src, blob_count))
-        return out.raw[: 48 * blob_count]
+        out = _Out(48 * blob_count)
+        _check(load().vkzg_amd_blob_to_commitments(self._h, out.at, bytes(blobs), blob_count))
+        return out.value
 
     def debug_pairing(self, g1_points, g2_points):
         """Device e(P_i, Q_i)^3 for compressed P_i (48 B) and Q_i (96 B): 576 bytes each."""
@@ -259,8 +273,7 @@ class Prover:
                                                      stream))
 
     def recover_cells_device(self, d_out, d_cells, d_present, h_present, blob_count, stream=None):
-        pm = ctypes.create_string_buffer(bytes(h_present), max(1, len(h_present)))
-        _check(load().vkzg_amd_recover_cells_device(self._h, d_out, d_cells, d_present, pm,
+        _check(load().vkzg_amd_recover_cells_device(self._h, d_out, d_cells, d_present, bytes(h_present),
                                                     blob_count, stream))
 
 

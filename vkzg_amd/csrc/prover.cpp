@@ -542,10 +542,14 @@ void enqueue_recovery_into(vkzg_prover *p, Fr *A, Fr *B, uint8_t *d_out, const u
 
 namespace {
 
+// Which steps a pipeline holds: a call that also returns cells runs the first
+// one apart, so that the cells can leave while the rest runs.
+enum ProofSteps { kAllSteps, kScalarsOnly, kAfterScalars };
+
 // One sub-batch: blobs [off, off + nb) of working set ws.
 void proofs_range(vkzg_prover *p, WorkSet &ws, uint32_t off, uint32_t nb, uint8_t *d_proofs,
                   const uint8_t *d_blobs, hipStream_t s, StageClock &clk, const Tuning &tn,
-                  size_t blob_stride = kBlobBytes, Fr *coeffs = nullptr) {
+                  size_t blob_stride = kBlobBytes, Fr *coeffs = nullptr, ProofSteps steps = kAllSteps) {
     uint32_t *err = ws.err + off;
     uint32_t *queue = ws.queue + off;
     Fr *scal = ws.scal + (size_t)off * 8192 * kMaxLadSplits;
@@ -564,9 +568,12 @@ void proofs_range(vkzg_prover *p, WorkSet &ws, uint32_t off, uint32_t nb, uint8_
     G1A *lad_aff = ws.lad_aff + off * npos, *lad_phi = ws.lad_phi + off * npos;
     Fp *prefix = ws.prefix + off * npos;
     G1X *buckets = ws.buckets + (size_t)off * 128 * kBuckets, *cvals = ws.cvals + (size_t)off * 128;
-    ck(launch_fk20_scalars(scal, d_blobs, blob_stride, err, p->roots, p->roots_inv, queue, coeffs,
-                           tn.ladder_splits, nb, tab.plan(), s));
-    clk.mark("fk20_scalars");
+    if (steps != kAfterScalars) {
+        ck(launch_fk20_scalars(scal, d_blobs, blob_stride, err, p->roots, p->roots_inv, queue, coeffs,
+                               tn.ladder_splits, nb, tab.plan(), s));
+        clk.mark("fk20_scalars");
+    }
+    if (steps == kScalarsOnly) return;
     ck(launch_phase_a(u, scal, tab.table, tab.plan(), 128, nb, tn.ladder_splits, shape.parts, shape.groups,
                       p->cus * tn.blocks_per_cu, queue, tn.force_checked, s));
     clk.mark("phase_a");
@@ -686,99 +693,103 @@ void enqueue_recovery(vkzg_prover *p, WorkSet &ws, StreamSet &ss, uint8_t *d_out
     enqueue_maybe_graph(p, *graphs, key, s, clk, body);
 }
 
-// Cells (the 2x extension, as compute_cells_and_kzg_proofs returns them) and
-// proofs of nb blobs read at blob_stride: the proof pipeline also writes the
-// blob coefficients to ws.bufA, and the forward evaluation passes of the
-// recovery turn them into canonical cell bytes.  d_cells may be null.
-void enqueue_cells_and_proofs(vkzg_prover *p, WorkSet &ws, uint8_t *d_cells, uint8_t *d_proofs,
-                              const uint8_t *d_blobs, size_t blob_stride, uint32_t nb, hipStream_t s,
-                              const Tuning &tn, GraphCache *graphs) {
+// Proofs of nb blobs read at d_blobs + b * blob_stride.  With d_cells, their
+// cells too, before the rest of the proofs: cells_ready (an event) is recorded
+// on s behind them.
+void enqueue_cells_and_proofs(vkzg_prover *p, WorkSet &ws, uint8_t *d_cells, hipEvent_t cells_ready,
+                              uint8_t *d_proofs, const uint8_t *d_blobs, size_t blob_stride, uint32_t nb,
+                              hipStream_t s, const Tuning &tn, GraphCache *graphs) {
     StageClock off_clock(p, s, false);
-    auto body = [&](hipStream_t q) {
-        proofs_range(p, ws, 0, nb, d_proofs, d_blobs, q, off_clock, tn, blob_stride,
-                     d_cells ? ws.bufA : nullptr);
-        if (d_cells) {
-            const RecTables t = rec_tables(p);
-            ck(launch_rec_first(ws.bufB, ws.bufA, 1, nullptr, t, nb, tn.rec_radix, tn.rec_waves, q));
-            ck(launch_rec_last(d_cells, ws.bufB, t, nb, tn.rec_radix, tn.rec_waves, q));
-        }
+    const auto run = [&](uint64_t kind, auto body) {
+        if (!graphs) return body(s);
+        const GraphKey key{{kind | ((uint64_t)(uintptr_t)d_cells << 3), nb | ((uint64_t)blob_stride << 32),
+                            tuning_word(tn), (uint64_t)(uintptr_t)d_proofs, (uint64_t)(uintptr_t)d_blobs,
+                            (uint64_t)(uintptr_t)&ws}};
+        enqueue_maybe_graph(p, *graphs, key, s, off_clock, body);
     };
-    if (!graphs) return body(s);
-    const GraphKey key{{3u | ((uint64_t)(uintptr_t)d_cells << 2), nb | ((uint64_t)blob_stride << 32), tuning_word(tn),
-                        (uint64_t)(uintptr_t)d_proofs, (uint64_t)(uintptr_t)d_blobs,
-                        (uint64_t)(uintptr_t)&ws}};
-    enqueue_maybe_graph(p, *graphs, key, s, off_clock, body);
-}
-
-// Host-buffer staging of the synchronous entry points.  A large copy is
-// split over kCopyThreads host threads (one host thread copies pageable
-// memory at about a third of what the PCIe DMA takes); an upload also sends
-// each thread's part by DMA in kCopySlice slices as soon as a slice is
-// staged, so the copy of one slice overlaps the DMA of the previous one.
-// Small copies stay on the calling thread.
-constexpr unsigned kCopyThreads = 4;
-constexpr size_t kCopySlice = (size_t)2 << 20;
-constexpr size_t kThreadedCopyMin = (size_t)4 << 20;
-
-void parallel_copy(uint8_t *dst, const uint8_t *src, size_t bytes) {
-    if (bytes < kThreadedCopyMin) {
-        std::memcpy(dst, src, bytes);
+    if (!d_cells) {
+        run(3, [&](hipStream_t q) {
+            proofs_range(p, ws, 0, nb, d_proofs, d_blobs, q, off_clock, tn, blob_stride);
+        });
         return;
     }
-    const size_t part = (bytes + kCopyThreads - 1) / kCopyThreads;
-    const auto copy_part = [=](size_t off) { std::memcpy(dst + off, src + off, std::min(part, bytes - off)); };
-    std::thread helpers[kCopyThreads - 1];
-    for (unsigned k = 1; k < kCopyThreads; k++) {
-        const size_t off = k * part;
-        if (off >= bytes) break;
-        try {
-            helpers[k - 1] = std::thread(copy_part, off);
-        } catch (const std::system_error &) {
-            copy_part(off);  // no thread to spare: copy it here
-        }
-    }
-    copy_part(0);
-    for (std::thread &t : helpers)
-        if (t.joinable()) t.join();
+    run(4, [&](hipStream_t q) {
+        proofs_range(p, ws, 0, nb, d_proofs, d_blobs, q, off_clock, tn, blob_stride, ws.bufA, kScalarsOnly);
+        const RecTables t = rec_tables(p);
+        ck(launch_rec_first(ws.bufB, ws.bufA, 1, nullptr, t, nb, tn.rec_radix, tn.rec_waves, q));
+        ck(launch_rec_last(d_cells, ws.bufB, t, nb, tn.rec_radix, tn.rec_waves, q));
+    });
+    ck(hipEventRecord(cells_ready, s));
+    run(5, [&](hipStream_t q) {
+        proofs_range(p, ws, 0, nb, d_proofs, d_blobs, q, off_clock, tn, blob_stride, nullptr, kAfterScalars);
+    });
+}
+
+// Host-buffer staging of the synchronous entry points.  One host thread copies
+// pageable memory at a third of what the PCIe DMA takes, so a copy of
+// kPooledCopyMin bytes or more is cut into slices for the prover's copy
+// threads: a slice of an upload goes out by DMA as soon as it is staged, and a
+// slice of a download is copied out as soon as its DMA is done, so both
+// directions overlap their two halves.
+constexpr size_t kPooledCopyMin = (size_t)1 << 20;
+constexpr size_t kMinSlice = (size_t)256 << 10, kMaxSlice = (size_t)2 << 20;
+
+// About sixteen slices, so that the first DMA starts early and the last copy
+// is short, of sizes at which neither side pays for the slicing.
+size_t copy_slice(size_t bytes) {
+    const size_t s = (bytes / 16 + 4095) & ~(size_t)4095;
+    return std::max(kMinSlice, std::min(kMaxSlice, s));
 }
 
 // host (pageable) -> pinned staging -> dev, enqueued on s.
-void stage_upload(int device, uint8_t *dev, uint8_t *pinned, const uint8_t *host, size_t bytes, hipStream_t s) {
-    if (bytes < kThreadedCopyMin) {
+void stage_upload(vkzg_prover *p, uint8_t *dev, uint8_t *pinned, const uint8_t *host, size_t bytes, hipStream_t s) {
+    if (bytes < kPooledCopyMin) {
         std::memcpy(pinned, host, bytes);
         ck(hipMemcpyAsync(dev, pinned, bytes, hipMemcpyHostToDevice, s));
         return;
     }
-    // parts in whole slices, so every slice but the last is full
-    const size_t slices = (bytes + kCopySlice - 1) / kCopySlice;
-    const size_t per = (slices + kCopyThreads - 1) / kCopyThreads;
+    const size_t slice = copy_slice(bytes);
     std::atomic<bool> failed{false};
-    const auto work = [&](size_t first, bool own_thread) {
-        if (own_thread && hipSetDevice(device) != hipSuccess) {
-            failed = true;
-            return;
+    p->copiers.run((bytes + slice - 1) / slice, [&](size_t k) {
+        const size_t off = k * slice, n = std::min(slice, bytes - off);
+        std::memcpy(pinned + off, host + off, n);
+        if (hipMemcpyAsync(dev + off, pinned + off, n, hipMemcpyHostToDevice, s) != hipSuccess) failed = true;
+    });
+    if (failed) throw HipFail{};
+}
+
+// dev -> pinned staging, enqueued on s in slices with an event behind each
+// (small ones whole, with one event).
+void start_download(vkzg_prover *p, uint8_t *pinned, const uint8_t *dev, size_t bytes, hipStream_t s) {
+    const size_t slice = bytes < kPooledCopyMin ? bytes : copy_slice(bytes);
+    size_t k = 0;
+    for (size_t off = 0; off < bytes; off += slice, k++) {
+        if (k == p->download_ev.size()) {
+            hipEvent_t e = nullptr;
+            ck(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+            p->download_ev.push_back(e);
         }
-        for (size_t k = first; k < std::min(slices, first + per); k++) {
-            const size_t off = k * kCopySlice, n = std::min(kCopySlice, bytes - off);
-            std::memcpy(pinned + off, host + off, n);
-            if (hipMemcpyAsync(dev + off, pinned + off, n, hipMemcpyHostToDevice, s) != hipSuccess) {
-                failed = true;
-                return;
-            }
-        }
-    };
-    std::thread helpers[kCopyThreads - 1];
-    for (unsigned t = 1; t < kCopyThreads; t++) {
-        if (t * per >= slices) break;
-        try {
-            helpers[t - 1] = std::thread(work, t * per, true);
-        } catch (const std::system_error &) {
-            work(t * per, false);  // no thread to spare: stage it here
-        }
+        ck(hipMemcpyAsync(pinned + off, dev + off, std::min(slice, bytes - off), hipMemcpyDeviceToHost, s));
+        ck(hipEventRecord(p->download_ev[k], s));
     }
-    work(0, false);
-    for (std::thread &t : helpers)
-        if (t.joinable()) t.join();
+}
+
+// The slices of start_download -> host, each once its DMA is done.
+void finish_download(vkzg_prover *p, uint8_t *host, const uint8_t *pinned, size_t bytes) {
+    const size_t slice = bytes < kPooledCopyMin ? bytes : copy_slice(bytes);
+    std::atomic<bool> failed{false};
+    const auto part = [&](size_t k) {
+        const size_t off = k * slice;
+        if (hipEventSynchronize(p->download_ev[k]) != hipSuccess) failed = true;
+        else std::memcpy(host + off, pinned + off, std::min(slice, bytes - off));
+    };
+    if (bytes < kPooledCopyMin) {
+        part(0);
+    } else {
+        // the copy threads are woken when there is something to copy
+        if (hipEventSynchronize(p->download_ev[0]) != hipSuccess) throw HipFail{};
+        p->copiers.run((bytes + slice - 1) / slice, part);
+    }
     if (failed) throw HipFail{};
 }
 
@@ -985,6 +996,10 @@ vkzg_result create(vkzg_prover **out, const vkzg_options *opts, const uint8_t *s
         p->h_out = p->arena.halloc<uint8_t>(B * kCellsBytes);
         p->h_present = p->arena.halloc<uint8_t>(B * 128);
         p->h_err = p->arena.halloc<uint32_t>(B);
+        p->h_proofs = p->arena.halloc<uint8_t>(B * kProofBytes);
+        p->copiers.set_device(p->device);
+        ck(hipStreamCreateWithFlags(&p->copy_stream, hipStreamNonBlocking));
+        ck(hipEventCreateWithFlags(&p->results_ready, hipEventDisableTiming));
         ck(hipStreamSynchronize(p->stream));
         if (const char *env = std::getenv("VKZG_AMD_AUTOTUNE"))
             if (std::atoi(env) != 0) autotune(p);
@@ -1020,6 +1035,9 @@ vkzg_prover::~vkzg_prover() {
     arena.release();
     for (auto &e : ev)
         if (e) (void)hipEventDestroy(e);
+    for (hipEvent_t e : download_ev) (void)hipEventDestroy(e);
+    if (results_ready) (void)hipEventDestroy(results_ready);
+    if (copy_stream) (void)hipStreamDestroy(copy_stream);
     streams.destroy();
     if (stream) (void)hipStreamDestroy(stream);
     (void)hipSetDevice(cur);
@@ -1079,7 +1097,7 @@ vkzg_result vkzg_compute_proofs_batch(vkzg_prover *p, uint8_t *proofs, const uin
         for (size_t done = 0; done < num_blobs;) {
             const uint32_t nb = (uint32_t)std::min<size_t>(p->max_batch, num_blobs - done);
             hipStream_t s = p->stream;
-            stage_upload(p->device, p->ws.blobs, p->h_in, blobs + done * kBlobBytes, nb * kBlobBytes, s);
+            stage_upload(p, p->ws.blobs, p->h_in, blobs + done * kBlobBytes, nb * kBlobBytes, s);
             StageClock clk(p, s, true);
             const Tuning tn = tuning_for(p, nb);
             p->last_splits = tn.splits;
@@ -1113,7 +1131,7 @@ vkzg_result vkzg_recover_cells_batch(vkzg_prover *p, uint8_t *cells_out, const u
             const uint8_t *pm = cell_present + done * 128;
             if (!chunk_missing_ok(pm, nb)) return VKZG_ERR_BADARGS;
             hipStream_t s = p->stream;
-            stage_upload(p->device, p->ws.cells, p->h_in, cells + done * kCellsBytes, nb * kCellsBytes, s);
+            stage_upload(p, p->ws.cells, p->h_in, cells + done * kCellsBytes, nb * kCellsBytes, s);
             std::memcpy(p->h_present, pm, nb * 128);
             ck(hipMemcpyAsync(p->ws.present, p->h_present, nb * 128, hipMemcpyHostToDevice, s));
             StageClock clk(p, s, true);
@@ -1121,10 +1139,10 @@ vkzg_result vkzg_recover_cells_batch(vkzg_prover *p, uint8_t *cells_out, const u
             p->last_splits = tn.splits;
             enqueue_recovery(p, p->ws, p->streams, p->ws.cells_out, p->ws.cells, p->ws.present, nb,
                              s, clk, tn, &p->graphs);
-            ck(hipMemcpyAsync(p->h_out, p->ws.cells_out, nb * kCellsBytes, hipMemcpyDeviceToHost, s));
+            start_download(p, p->h_out, p->ws.cells_out, nb * kCellsBytes, s);
+            finish_download(p, cells_out + done * kCellsBytes, p->h_out, nb * kCellsBytes);
             ck(hipStreamSynchronize(s));
             clk.finish();
-            parallel_copy(cells_out + done * kCellsBytes, p->h_out, nb * kCellsBytes);
             done += nb;
         }
     } catch (HipFail &) {
@@ -1144,22 +1162,33 @@ vkzg_result vkzg_amd_compute_cells_and_proofs(vkzg_prover *p, uint8_t *cells, ui
         for (size_t done = 0; done < num_blobs;) {
             const uint32_t nb = (uint32_t)std::min<size_t>(p->max_batch, num_blobs - done);
             hipStream_t s = p->stream;
-            stage_upload(p->device, p->ws.blobs, p->h_in, blobs + done * kBlobBytes, nb * kBlobBytes, s);
+            stage_upload(p, p->ws.blobs, p->h_in, blobs + done * kBlobBytes, nb * kBlobBytes, s);
             const Tuning tn = tuning_for(p, nb);
             Tuning one = tn;
             one.splits = 1;
-            enqueue_cells_and_proofs(p, p->ws, cells ? p->ws.cells_out : nullptr, p->ws.proofs,
+            enqueue_cells_and_proofs(p, p->ws, cells ? p->ws.cells_out : nullptr, p->results_ready, p->ws.proofs,
                                      p->ws.blobs, kBlobBytes, nb, s, one, &p->graphs);
-            ck(hipMemcpyAsync(p->h_err, p->ws.err, nb * 4, hipMemcpyDeviceToHost, s));
-            if (cells)
-                ck(hipMemcpyAsync(p->h_out, p->ws.cells_out, nb * kCellsBytes, hipMemcpyDeviceToHost, s));
-            if (proofs)  // h_in's blobs were consumed by the copy above, in stream order
-                ck(hipMemcpyAsync(p->h_in, p->ws.proofs, nb * kProofBytes, hipMemcpyDeviceToHost, s));
+            if (cells) {
+                // The error flags and the cells go out on the copy stream
+                // while the proofs are computed.
+                hipStream_t c = p->copy_stream;
+                ck(hipStreamWaitEvent(c, p->results_ready, 0));
+                ck(hipMemcpyAsync(p->h_err, p->ws.err, nb * 4, hipMemcpyDeviceToHost, c));
+                start_download(p, p->h_out, p->ws.cells_out, nb * kCellsBytes, c);
+                // behind the flags: the first slice
+                if (hipEventSynchronize(p->download_ev[0]) != hipSuccess) throw HipFail{};
+            } else {
+                ck(hipMemcpyAsync(p->h_err, p->ws.err, nb * 4, hipMemcpyDeviceToHost, s));
+            }
+            if (proofs) ck(hipMemcpyAsync(p->h_proofs, p->ws.proofs, nb * kProofBytes, hipMemcpyDeviceToHost, s));
+            if (!cells) ck(hipStreamSynchronize(s));
+            bool bad = false;
+            for (uint32_t b = 0; b < nb; b++) bad |= p->h_err[b] != 0;
+            if (cells && !bad) finish_download(p, cells + done * kCellsBytes, p->h_out, nb * kCellsBytes);
+            if (cells) ck(hipStreamSynchronize(p->copy_stream));
             ck(hipStreamSynchronize(s));
-            for (uint32_t b = 0; b < nb; b++)
-                if (p->h_err[b]) return VKZG_ERR_INVALID_BLOB;
-            if (cells) parallel_copy(cells + done * kCellsBytes, p->h_out, nb * kCellsBytes);
-            if (proofs) std::memcpy(proofs + done * kProofBytes, p->h_in, nb * kProofBytes);
+            if (bad) return VKZG_ERR_INVALID_BLOB;
+            if (proofs) std::memcpy(proofs + done * kProofBytes, p->h_proofs, nb * kProofBytes);
             done += nb;
         }
     } catch (HipFail &) {
@@ -1182,7 +1211,7 @@ vkzg_result vkzg_amd_recover_cells_and_proofs(vkzg_prover *p, uint8_t *cells_out
             const uint8_t *pm = cell_present + done * 128;
             if (!chunk_missing_ok(pm, nb)) return VKZG_ERR_BADARGS;
             hipStream_t s = p->stream;
-            stage_upload(p->device, p->ws.cells, p->h_in, cells + done * kCellsBytes, nb * kCellsBytes, s);
+            stage_upload(p, p->ws.cells, p->h_in, cells + done * kCellsBytes, nb * kCellsBytes, s);
             std::memcpy(p->h_present, pm, nb * 128);
             ck(hipMemcpyAsync(p->ws.present, p->h_present, nb * 128, hipMemcpyHostToDevice, s));
             const Tuning tn = tuning_for(p, nb);
@@ -1191,15 +1220,20 @@ vkzg_result vkzg_amd_recover_cells_and_proofs(vkzg_prover *p, uint8_t *cells_out
             StageClock clk(p, s, false);
             enqueue_recovery(p, p->ws, p->streams, p->ws.cells_out, p->ws.cells, p->ws.present, nb, s,
                              clk, one, &p->graphs);
+            // The cells go out on the copy stream while the proofs are computed
+            // (both only read them).
+            ck(hipEventRecord(p->results_ready, s));
+            ck(hipStreamWaitEvent(p->copy_stream, p->results_ready, 0));
+            start_download(p, p->h_out, p->ws.cells_out, nb * kCellsBytes, p->copy_stream);
             // The first 64 recovered cells of a blob are the blob itself (cell c
             // holds p(w^brev13(64c+t)) and brev13(i) = 2 brev12(i) for i < 4096).
-            enqueue_cells_and_proofs(p, p->ws, nullptr, p->ws.proofs, p->ws.cells_out, kCellsBytes, nb,
+            enqueue_cells_and_proofs(p, p->ws, nullptr, nullptr, p->ws.proofs, p->ws.cells_out, kCellsBytes, nb,
                                      s, one, &p->graphs);
-            ck(hipMemcpyAsync(p->h_out, p->ws.cells_out, nb * kCellsBytes, hipMemcpyDeviceToHost, s));
-            ck(hipMemcpyAsync(p->h_in, p->ws.proofs, nb * kProofBytes, hipMemcpyDeviceToHost, s));
+            ck(hipMemcpyAsync(p->h_proofs, p->ws.proofs, nb * kProofBytes, hipMemcpyDeviceToHost, s));
+            finish_download(p, cells_out + done * kCellsBytes, p->h_out, nb * kCellsBytes);
+            ck(hipStreamSynchronize(p->copy_stream));
             ck(hipStreamSynchronize(s));
-            parallel_copy(cells_out + done * kCellsBytes, p->h_out, nb * kCellsBytes);
-            std::memcpy(proofs_out + done * kProofBytes, p->h_in, nb * kProofBytes);
+            std::memcpy(proofs_out + done * kProofBytes, p->h_proofs, nb * kProofBytes);
             done += nb;
         }
     } catch (HipFail &) {

@@ -5,9 +5,13 @@
 #include <hip/hip_runtime.h>
 
 #include <atomic>
+#include <condition_variable>
 #include <cstdint>
+#include <functional>
 #include <mutex>
 #include <string>
+#include <system_error>
+#include <thread>
 #include <vector>
 
 #include "../../include/vkzg.h"
@@ -231,6 +235,84 @@ struct GraphCache {
     }
 };
 
+// A prover's copy threads: run(n, f) calls f(0) .. f(n - 1), spread over them
+// and the calling thread, and returns when all are done.  Started at the first
+// use (large host-buffer calls only), joined with the prover; where no thread
+// can be started the caller does it all.  One run at a time: the prover's mutex
+// is held.
+class CopyThreads {
+   public:
+    ~CopyThreads() {
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            stop_ = true;
+        }
+        wake_.notify_all();
+        for (std::thread &t : threads_) t.join();
+    }
+    void run(size_t n, const std::function<void(size_t)> &f) {
+        if (!started_) start();
+        {
+            std::lock_guard<std::mutex> lock(mu_);
+            job_ = &f;
+            count_ = n;
+            next_ = 0;
+            busy_ = threads_.size();
+            generation_++;
+        }
+        wake_.notify_all();
+        take(f, n);
+        std::unique_lock<std::mutex> lock(mu_);
+        done_.wait(lock, [this] { return busy_ == 0; });
+        job_ = nullptr;
+    }
+    void set_device(int device) { device_ = device; }
+
+   private:
+    static constexpr unsigned kThreads = 5;
+    void start() {
+        started_ = true;
+        for (unsigned k = 0; k < kThreads; k++) {
+            try {
+                threads_.emplace_back([this] { loop(); });
+            } catch (const std::system_error &) {
+                break;  // fewer threads, or none
+            }
+        }
+    }
+    void take(const std::function<void(size_t)> &f, size_t n) {
+        for (size_t k; (k = next_.fetch_add(1)) < n;) f(k);
+    }
+    void loop() {
+        (void)hipSetDevice(device_);
+        uint64_t seen = 0;
+        for (;;) {
+            const std::function<void(size_t)> *f;
+            size_t n;
+            {
+                std::unique_lock<std::mutex> lock(mu_);
+                wake_.wait(lock, [&] { return stop_ || generation_ != seen; });
+                if (stop_) return;
+                seen = generation_;
+                f = job_;
+                n = count_;
+            }
+            take(*f, n);
+            std::lock_guard<std::mutex> lock(mu_);
+            if (--busy_ == 0) done_.notify_one();
+        }
+    }
+    std::mutex mu_;
+    std::condition_variable wake_, done_;
+    std::vector<std::thread> threads_;
+    const std::function<void(size_t)> *job_ = nullptr;
+    size_t count_ = 0, busy_ = 0;
+    std::atomic<size_t> next_{0};
+    uint64_t generation_ = 0;
+    bool started_ = false, stop_ = false;
+    int device_ = 0;
+};
+
 // Verification state (verify.cpp): G2 setup lines and per-call buffers.
 struct VerifyState;
 void destroy_verify_state(VerifyState *v);
@@ -279,8 +361,14 @@ struct vkzg_prover {
 
     // Working set of the synchronous entry points and its pinned staging.
     vkzg_amd::WorkSet ws;
-    uint8_t *h_in = nullptr, *h_out = nullptr, *h_present = nullptr;
+    uint8_t *h_in = nullptr, *h_out = nullptr, *h_present = nullptr, *h_proofs = nullptr;
     uint32_t *h_err = nullptr;
+    // Host-buffer copies: their threads, the stream that takes cells out while
+    // proofs are computed, an event per slice of a download.
+    vkzg_amd::CopyThreads copiers;
+    hipStream_t copy_stream = nullptr;
+    hipEvent_t results_ready = nullptr;
+    std::vector<hipEvent_t> download_ev;
 
     // Batch verification and commitments (created on first use).
     vkzg_amd::VerifyState *vfy = nullptr;
@@ -343,7 +431,7 @@ struct PhaseAShape {
 PhaseAShape phase_a_shape(uint64_t nmsm, uint32_t groups, uint32_t windows, uint64_t slots, uint32_t cus);
 
 // host (pageable) -> pinned staging -> dev, enqueued on s.
-void stage_upload(int device, uint8_t *dev, uint8_t *pinned, const uint8_t *host, size_t bytes, hipStream_t s);
+void stage_upload(vkzg_prover *p, uint8_t *dev, uint8_t *pinned, const uint8_t *host, size_t bytes, hipStream_t s);
 
 // Enqueue a pipeline through `cache` when graphs are on and stage timing is
 // off (timing records events between stages), else launch it directly.

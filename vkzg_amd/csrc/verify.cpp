@@ -311,11 +311,10 @@ vkzg_result locked(vkzg_prover *p, Body body) {
 // The multiples table commitments are summed from, made at a prover's first
 // commitment call: a commitment is 4096 fixed bases against 4096 scalars, so
 // with W windows it takes 4096 W mixed additions and no buckets, sorting or
-// doublings (64 blobs: 1.25 ms on the device, where the bucket method they
-// replace took 4.9).  W
-// is the smallest of 25 and up (8 GB at 25, 22 ms to build) whose table fits an
-// eighth of the free memory; more windows halve the table and add a few
-// percent each (measured on 25: 64 blobs 0.90 ms for the additions).
+// doublings (64 blobs: 1.25 ms on the device, 0.9 of them the additions, where
+// the bucket method they replace took 4.9).  W is the smallest of 25 and up
+// whose table fits an eighth of the free memory: 7.5 GiB at 25 (the first call
+// takes 30 ms), half as much with each step of a few windows more.
 void build_commit_table(vkzg_prover *p, PhaseATable &t) {
     size_t free_b = 0, total = 0;
     ck(hipMemGetInfo(&free_b, &total));
@@ -456,7 +455,7 @@ vkzg_result vkzg_amd_blob_to_commitments(vkzg_prover *p, uint8_t *commitments, c
             const size_t o_out = l.take(sizeof(G1X) * nb);
             v.ensure(l.size, host_bytes);
             uint8_t *H = v.host, *D = static_cast<uint8_t *>(v.dev);
-            stage_upload(p->device, D + o_blobs, H + o_blobs, blobs + done * kBlobBytes, kBlobBytes * nb, s);
+            stage_upload(p, D + o_blobs, H + o_blobs, blobs + done * kBlobBytes, kBlobBytes * nb, s);
             Fr *sc = reinterpret_cast<Fr *>(D + o_sc);
             uint32_t *queue = reinterpret_cast<uint32_t *>(D + o_queue);
             G1X *part = reinterpret_cast<G1X *>(D + o_part), *out = reinterpret_cast<G1X *>(D + o_out);
