@@ -20,6 +20,28 @@ Z_ABS = 0xD201000000010000  # |z|, z = -0xd201000000010000 is the BLS parameter
 LAMBDA = Z_ABS * Z_ABS - 1  # z^2 - 1: phi(P) = [LAMBDA]P on G1, r = LAMBDA^2 + LAMBDA + 1
 
 
+# The model 3 Y^2 Z = 2 X^3 - Z^3 of proj_quad.h: SIGMA^2 = -12, NU^3 = 3 SIGMA / 2
+SIGMA = pow(-12, (P + 1) // 4, P)
+
+
+def cbrt(a):
+    """A cube root of a cube mod P, from the 3-part of P - 1 and a non-cube."""
+    s, t = 0, P - 1
+    while t % 3 == 0:
+        s, t = s + 1, t // 3
+    g = next(g for g in range(2, 100) if pow(g, (P - 1) // 3, P) != 1)
+    c = pow(g, t, P)  # of order 3^s
+    x = pow(a, pow(3, -1, t), P)  # x^3 = a e with e of order dividing 3^(s-1)
+    for k in range(3 ** (s - 1)):
+        y = x * pow(c, k, P) % P
+        if pow(y, 3, P) == a % P:
+            return y
+    raise ValueError("not a cube")
+
+
+NU = cbrt(3 * SIGMA * pow(2, -1, P))
+
+
 def f2mul(a, b):
     return ((a[0] * b[0] - a[1] * b[1]) % P, (a[0] * b[1] + a[1] * b[0]) % P)
 
@@ -79,6 +101,12 @@ def main():
     out.append(arr30("R2", RP * RP % P))
     out.append(arr30("FOUR_M", 4 * RP % P))
     out.append(arr30("BETA_M", BETA * RP % P))
+    assert SIGMA * SIGMA % P == P - 12 and 2 * pow(NU, 3, P) % P == 3 * SIGMA % P
+    out.append(arr30("SIGMA_M", SIGMA * RP % P))
+    out.append(arr30("INV_SIGMA_M", pow(SIGMA, -1, P) * RP % P))
+    out.append(arr30("NU_M", NU * RP % P))
+    out.append(arr30("SIGMA_OVER_NU_M", SIGMA * pow(NU, -1, P) * RP % P))
+    out.append(arr30("NU_BETA2_M", NU * BETA * BETA * RP % P))
     out.append(arr30("R3_M", RP ** 3 % P))  # Montgomery form of R^2: turns a plain inverse of xR into x^-1 R
     # 2^384 mod p as a plain value: a Montgomery product of x R by it gives
     # x 2^384 mod p, the reference's 12 x 32-bit Montgomery form (tables file v1)

@@ -129,7 +129,10 @@ hipError_t launch_sum_groups(G1X *usum, const G1X *part, uint32_t shares, uint32
                              uint32_t force_checked, hipStream_t s);
 // u: one sum per MSM, [nblobs][splits][128].
 hipError_t launch_ladder(G1J *lad, const G1X *u, uint32_t splits, uint32_t nblobs, uint32_t lanes,
-                         hipStream_t s);
+                         uint32_t force_checked, hipStream_t s);
+// lad -> affine; lanes: what launch_ladder was given (its chains' coordinates).
+hipError_t launch_ladder_to_affine(G1A *out, const G1J *lad, Fp *prefix, uint64_t count, uint32_t chunk,
+                                   uint32_t lanes, hipStream_t s);
 // Also clears the work counters of the phase-B and bucket-reduction launches
 // that follow (queue_b[0], queue_r[0]).
 // The ladder points in XYZZ form and their endomorphism images (small

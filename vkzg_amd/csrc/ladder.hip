@@ -1,6 +1,7 @@
 // FK20 phase B inputs: doubling ladders of the split-circulant folds of u.
 #include <algorithm>
 
+#include "proj_quad.h"
 #include "proof_common.h"
 
 namespace vkzg_amd {
@@ -31,27 +32,6 @@ VKZG_DEV G1J g1j_dbl_pair(const G1J &p, uint32_t q) {
     return r;
 }
 
-// The same doubling on the four lanes of a quad: E^2 needs only X^2, so it
-// joins round two on a third lane, and a doubling waits on one squaring and
-// two products -- {X^2, Y^2}, {2X B, B^2, E^2}, {E (4XB - X3) - 8 B^2, 2Y Z} --
-// at twice the lanes per chain.  For batches whose pair ladder leaves SIMDs
-// idle: there the chain's length, not the issue rate, sets the time.
-VKZG_DEV G1J g1j_dbl_quad(const G1J &p, uint32_t q) {
-    if (fp_is_zero(p.z)) return p;  // uniform in the quad
-    const bool odd = (q & 1u) != 0;
-    const Fp r1 = fp_sqr(fp_select(odd, p.y, p.x));
-    const Fp E = fp_triple(fp_quad_bcast<0>(r1)), B = fp_quad_bcast<1>(r1);
-    const Fp r2 = fp_mul(fp_select(q == 2, E, fp_select(odd, B, fp_dbl_raw(p.x))), fp_select(q == 2, E, B));
-    const Fp S = fp_dbl(fp_quad_bcast<0>(r2));  // 4 X Y^2
-    G1J r;
-    r.x = fp_neg(fp_dbl_sub(S, fp_quad_bcast<2>(r2)));  // E^2 - 2S
-    const Fp r3 = fp_mul_fold_v(fp_select(odd, fp_dbl_raw(p.y), fp_sub_raw(S, r.x)), fp_select(odd, p.z, E),
-                              fp_quad_bcast<1>(r2), odd ? 0 : -8);
-    r.y = fp_quad_bcast<0>(r3);
-    r.z = fp_quad_bcast<1>(r3);
-    return r;
-}
-
 // The phase-B points are linear in u, and so are the doublings, so the
 // split-circulant folds (k_fold_ladder.comp) are taken before the ladder:
 //   F+[i] = u[i] + u[i+64], F-[i] = u[i] - u[i+64] (i < 64),
@@ -61,10 +41,27 @@ VKZG_DEV G1J g1j_dbl_quad(const G1J &p, uint32_t q) {
 // With `splits` = M segments, pair (blob, m, j) starts from the same folds of
 // phase A's 2^(kDigitBits start_m) u (u[(blob*M + m)*128 + k], phase A's MSMs with
 // their window groups summed), start_m = lad_start(M, m), and writes
-// positions [start_m, start_{m+1}).  LANES (2 or 4) lanes share a chain
-// (g1j_dbl_pair or g1j_dbl_quad) and exit together.
+// positions [start_m, start_{m+1}).  LANES (2 or 4) lanes share a chain and exit
+// together.  While four-lane chains leave SIMDs idle or fill them with one wave
+// (ladder_lanes), the chain's length sets the time: quads double in homogeneous
+// coordinates (proj_quad.h, without nu) in two rounds of products, and share
+// the additions of the folds (flagged ones are redone checked).  Beyond that
+// the issue rate does, and pairs double in Jacobian coordinates, whose squares
+// make a doubling the cheaper one in instructions (3 squares and 4 products in
+// place of 8 products).  Positions hold the chain's own coordinates: (X, Y, Z)
+// with x = sigma X / Z, y = sigma Y / Z from quads, Jacobian from pairs.
+template <typename Add>
+VKZG_DEV G1X ladder_fold(const G1X *u, uint32_t j, Add add) {
+    if (j >= 64) return add(u[j - 64], g1x_neg(u[j]));
+    const uint32_t i = j & 31u;
+    const G1X lo = add(u[i], u[i + 64]);
+    const G1X hi = add(u[i + 32], u[i + 96]);
+    return add(lo, j < 32 ? hi : g1x_neg(hi));
+}
+
 template <int LANES>
-__global__ __launch_bounds__(256) void k_ladder(G1J *lad, const G1X *u, uint32_t splits, uint32_t nblobs) {
+__global__ __launch_bounds__(256) void k_ladder(G1J *lad, const G1X *u, uint32_t splits, uint32_t nblobs,
+                                                uint32_t force_checked) {
     // A long dependent chain: give these waves issue priority over the
     // throughput kernels of another sub-batch sharing the SIMD.
     __builtin_amdgcn_s_setprio(3);
@@ -72,31 +69,39 @@ __global__ __launch_bounds__(256) void k_ladder(G1J *lad, const G1X *u, uint32_t
     const uint32_t g = tid / LANES, q = tid % LANES;
     if (g >= nblobs * 128 * splits) return;
     const uint32_t j = g % 128, m = (g / 128) % splits, blob = g / (128 * splits);
-    const size_t base = (size_t)(blob * splits + m) * 128;
-    G1X f;
-    if (j < 64) {
-        const uint32_t i = j & 31u;
-        const G1X lo = g1x_add(u[base + i], u[base + i + 64]);
-        const G1X hi = g1x_add(u[base + i + 32], u[base + i + 96]);
-        f = g1x_add(lo, j < 32 ? hi : g1x_neg(hi));
-    } else {
-        const uint32_t i = j - 64;
-        f = g1x_add(u[base + i], g1x_neg(u[base + i + 64]));
-    }
-    G1J p = g1j_from_xyzz(f);
+    const G1X *ub = u + (size_t)(blob * splits + m) * 128;
     const uint32_t d0 = lad_start(splits, m), d1 = m + 1 == splits ? kLadPos : lad_start(splits, m + 1);
     G1J *dst = lad + (size_t)blob * kLadPos * 128 + j;
+    if constexpr (LANES == 4) {
+        bool exc = force_checked != 0;
+        G1X f = ladder_fold(ub, j, [&](const G1X &a, const G1X &b) { return g1x_add_quad(a, b, q, exc); });
+        // uniform in the quad
+        if (exc) f = ladder_fold(ub, j, [](const G1X &a, const G1X &b) { return g1x_add(a, b); });
+        G1PQ p = g1pq_from_xyzz<false>(f, q);
 #pragma unroll 1
-    for (uint32_t d = d0; d < d1; d++) {
-        if (q == 0) {
-            dst[d * 128].x = p.x;
-            dst[d * 128].z = p.z;
-        } else {
-            dst[d * 128].y = p.y;
+        for (uint32_t d = d0; d < d1; d++) {
+            const Fp y = g1pq_y(p);
+            if (q == 0) dst[d * 128].y = y;
+            else if (q == 2) dst[d * 128].x = p.r;
+            else if (q == 3) dst[d * 128].z = p.r;
+            if (d + 1 == d1) break;
+#pragma unroll 1
+            for (uint32_t k = 0; k < kDigitBits; k++) p = g1pq_dbl(p, q);
         }
-        if (d + 1 == d1) break;
+    } else {
+        G1J p = g1j_from_xyzz(ladder_fold(ub, j, [](const G1X &a, const G1X &b) { return g1x_add(a, b); }));
 #pragma unroll 1
-        for (uint32_t k = 0; k < kDigitBits; k++) p = LANES == 4 ? g1j_dbl_quad(p, q) : g1j_dbl_pair(p, q);
+        for (uint32_t d = d0; d < d1; d++) {
+            if (q == 0) {
+                dst[d * 128].x = p.x;
+                dst[d * 128].z = p.z;
+            } else {
+                dst[d * 128].y = p.y;
+            }
+            if (d + 1 == d1) break;
+#pragma unroll 1
+            for (uint32_t k = 0; k < kDigitBits; k++) p = g1j_dbl_pair(p, q);
+        }
     }
 }
 
@@ -160,41 +165,53 @@ __global__ void k_glv_phi(G1A *phi, const G1A *pts, uint64_t count, uint32_t *qu
     phi[k] = q;
 }
 
-// Small batches: the ladder points in XYZZ form for phase B's quad
-// additions instead of normalised ones -- ZZ = Z^2, ZZZ = Z^3 keep X and Y
-// (Z = 0 gives the XYZZ identity) -- and their images under the
-// endomorphism, (beta X, Y, ZZ, ZZZ).  Two products per point, no inversion.
-// Clears the phase-B and bucket-reduction work counters, as k_glv_phi does.
-__global__ void k_ladder_xyzz(G1X *pts, G1X *phi, const G1J *lad, uint64_t count, uint32_t *queue_b,
-                              uint32_t *queue_r) {
-    const uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k == 0) {
+// Small batches: the ladder points (of quads) in XYZZ form for phase B's quad
+// additions instead of normalised ones, and their images under the
+// endomorphism.  With z = Z / sigma, (X z, Y z^2, z^2, z^3) and (beta X z, ...):
+// no inversion, and a quad per point, whose lanes share the seven products in
+// three rounds, {z}, {z^2, X z}, {z^3, beta X z, Y z^2}.  Clears the phase-B and
+// bucket-reduction work counters, as k_glv_phi does.
+__global__ void __launch_bounds__(256) k_ladder_xyzz(G1X *pts, G1X *phi, const G1J *lad, uint64_t count,
+                                                     uint32_t *queue_b, uint32_t *queue_r) {
+    const uint64_t tid = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (tid == 0) {
         queue_b[0] = 0u;
         queue_r[0] = 0u;
     }
+    const uint64_t k = tid >> 2;
+    const uint32_t q = (uint32_t)tid & 3u;
     if (k >= count) return;
     const G1J p = lad[k];
-    G1X r;
-    r.x = p.x;
-    r.y = p.y;
-    r.zz = fp_sqr(p.z);
-    r.zzz = fp_mul(r.zz, p.z);
-    pts[k] = r;
-    r.x = fp_mul(p.x, fp_const(cfp::BETA_M));
-    phi[k] = r;
+    const Fp z = fp_mul(p.z, fp_const(cfp::INV_SIGMA_M));
+    const Fp r2 = fp_mul(fp_select(q == 1, p.x, z), z);
+    const Fp zz = fp_quad_bcast<0>(r2), x = fp_quad_bcast<1>(r2);
+    const Fp r3 = fp_mul(q == 0 ? z : (q == 1 ? x : p.y), fp_select(q == 1, fp_const(cfp::BETA_M), zz));
+    if (q == 0) {
+        pts[k].zz = zz;
+        pts[k].zzz = r3;
+    } else if (q == 1) {
+        pts[k].x = x;
+        phi[k].x = r3;
+    } else if (q == 2) {
+        pts[k].y = r3;
+        phi[k].y = r3;
+    } else {
+        phi[k].zz = zz;
+    }
+    if (q == 0) phi[k].zzz = r3;
 }
 
 }  // namespace
 
 hipError_t launch_ladder_xyzz(G1X *pts, G1X *phi, const G1J *lad, uint64_t count, uint32_t *queue_b,
                               uint32_t *queue_r, hipStream_t s) {
-    hipLaunchKernelGGL(k_ladder_xyzz, dim3(blocks_for(count, 256)), dim3(256), 0, s, pts, phi, lad, count,
+    hipLaunchKernelGGL(k_ladder_xyzz, dim3(blocks_for(count * 4, 256)), dim3(256), 0, s, pts, phi, lad, count,
                        queue_b, queue_r);
     return hipGetLastError();
 }
 
 hipError_t launch_ladder(G1J *lad, const G1X *u, uint32_t splits, uint32_t nblobs, uint32_t lanes,
-                         hipStream_t s) {
+                         uint32_t force_checked, hipStream_t s) {
     // Workgroups of four waves: the dispatcher spreads a workgroup's waves over
     // a CU's four SIMDs, where one-wave workgroups doubled up on some SIMDs
     // while others idled (1.6 ms instead of 0.9 ms for 256 blobs; each wave's
@@ -202,9 +219,11 @@ hipError_t launch_ladder(G1J *lad, const G1X *u, uint32_t splits, uint32_t nblob
     // of LANES lanes fill each 256-thread block.
     const uint64_t threads = nblobs * 128ull * splits * lanes;
     if (lanes == 4)
-        hipLaunchKernelGGL(k_ladder<4>, dim3(blocks_for(threads, 256)), dim3(256), 0, s, lad, u, splits, nblobs);
+        hipLaunchKernelGGL(k_ladder<4>, dim3(blocks_for(threads, 256)), dim3(256), 0, s, lad, u, splits, nblobs,
+                           force_checked);
     else if (lanes == 2)
-        hipLaunchKernelGGL(k_ladder<2>, dim3(blocks_for(threads, 256)), dim3(256), 0, s, lad, u, splits, nblobs);
+        hipLaunchKernelGGL(k_ladder<2>, dim3(blocks_for(threads, 256)), dim3(256), 0, s, lad, u, splits, nblobs,
+                           force_checked);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();

@@ -435,11 +435,6 @@ void default_tunings(vkzg_prover *p) {
     }
 }
 
-// Points per lane of the normalisation for norm_chunk 0: the smallest chunk
-// whose lanes fit in one wave per SIMD.  Each lane's work is one inversion
-// plus 7 products per point, issued at one wave per SIMD; a second wave on a
-// SIMD doubles the stage, so 557,056 points (256 blobs) take chunks of 9 on
-// 1024 SIMDs, not 8.
 // Lanes per ladder chain: four while four-lane chains still fit one wave per
 // SIMD (the chain's length sets the time there), two above that (the issue
 // rate does).
@@ -456,6 +451,11 @@ bool phase_b_quad(uint32_t nb, uint32_t cus) {
     return (uint64_t)nb * 128 * kBuckets * 4 <= (uint64_t)cus * 4 * 64 * kPhaseBQuadWaves;
 }
 
+// Points per lane of the normalisation for norm_chunk 0: the smallest chunk
+// whose lanes fit in one wave per SIMD.  Each lane's work is one inversion
+// plus 6 or 7 products per point, issued at one wave per SIMD; a second wave on a
+// SIMD doubles the stage, so 524,288 points (256 blobs) take chunks of 8 on
+// 1024 SIMDs, not 7.
 uint32_t fit_norm_chunk(uint64_t count, uint32_t cus) {
     const uint64_t lanes = (uint64_t)cus * 4 * 64;
     const uint64_t c = (count + lanes - 1) / lanes;
@@ -581,14 +581,17 @@ void proofs_range(vkzg_prover *p, WorkSet &ws, uint32_t off, uint32_t nb, uint8_
         ck(launch_sum_groups(usum, u, shares, (uint32_t)nmsm, p->cus, tn.force_checked, s));
         clk.mark("sum_groups");
     }
-    ck(launch_ladder(lad, shares > 1 ? usum : u, tn.ladder_splits, nb,
-                     ladder_lanes((uint64_t)nb * 128 * tn.ladder_splits, p->cus), s));
+    const uint32_t lanes = ladder_lanes((uint64_t)nb * 128 * tn.ladder_splits, p->cus);
+    ck(launch_ladder(lad, shares > 1 ? usum : u, tn.ladder_splits, nb, lanes, tn.force_checked, s));
     clk.mark("ladder");
     // Small unsplit batches skip the normalisation: phase B's quads add the
     // ladder points in XYZZ form, which take twice the bytes of affine ones
     // and sit in the affine buffers' memory (so 2 nb <= the workset's blobs).
     const bool quad_b = phase_b_quad(nb, p->cus);
     static_assert(sizeof(G1X) <= 2 * sizeof(G1A), "XYZZ ladder points must fit the affine buffers");
+    // The conversion takes the quad ladder's coordinates; phase_b_quad's line
+    // (nb * 32 <= CUs) lies within ladder_lanes' for quads at any segment count.
+    static_assert(kBuckets / kPhaseBQuadWaves >= kMaxLadSplits, "quads in phase B imply a quad ladder");
     const bool xyzz = quad_b && tn.splits == 1 && off == 0 && 2 * nb <= ws.cap;
     if (xyzz) {
         G1X *lx = reinterpret_cast<G1X *>(ws.lad_aff), *lpx = reinterpret_cast<G1X *>(ws.lad_phi);
@@ -598,7 +601,7 @@ void proofs_range(vkzg_prover *p, WorkSet &ws, uint32_t off, uint32_t nb, uint8_
                           p->kb_offsets, nb, p->cus * 2, true, true, ws.queue_b + off, tn.force_checked, s));
     } else {
         const uint32_t chunk = tn.norm_chunk ? tn.norm_chunk : fit_norm_chunk((uint64_t)nb * npos, p->cus);
-        ck(launch_jac_to_affine(lad_aff, lad, prefix, (uint64_t)nb * npos, chunk, s));
+        ck(launch_ladder_to_affine(lad_aff, lad, prefix, (uint64_t)nb * npos, chunk, lanes, s));
         ck(launch_glv_phi(lad_phi, lad_aff, (uint64_t)nb * npos, ws.queue_b + off, ws.queue_r + off, s));
         clk.mark("normalize");
         ck(launch_phase_b(buckets, ws.bucket_flags + (size_t)off * 128 * kBuckets, lad_aff, lad_phi,

@@ -5,15 +5,19 @@ namespace vkzg_amd {
 
 namespace {
 
-// Batched Jacobian -> affine (Montgomery's trick, k_normalize.comp:29-56).
-// Thread t converts the points t, t+T, t+2T, ... (T = thread count) so that
+// Batched conversion to affine (Montgomery's trick, k_normalize.comp:29-56) of
+// Jacobian points or (HOMOG) of the quad ladder's homogeneous ones, x = sigma
+// X / Z and y = sigma Y / Z (sigma goes in with the one inversion).  Thread t
+// converts the points t, t+T, t+2T, ... (T = thread count) so that
 // neighbouring lanes touch neighbouring points.
-__global__ void __launch_bounds__(256) k_jac_to_affine(G1A *out, const G1J *in, Fp *prefix, uint64_t count, uint32_t chunk,
-                                uint64_t nthreads) {
+template <bool HOMOG>
+__global__ void __launch_bounds__(256) k_to_affine(G1A *out, const G1J *in, Fp *prefix, uint64_t count, uint32_t chunk,
+                                                   uint64_t nthreads) {
     __builtin_amdgcn_s_setprio(3);  // dependent inversion chain: issue first
     const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nthreads) return;
-    Fp acc = fp_one();
+    // prefix[k]: the product of the Zs before k, times sigma if HOMOG
+    Fp acc = HOMOG ? fp_const(cfp::SIGMA_M) : fp_one();
     uint32_t m = 0;
 #pragma unroll 1
     for (uint64_t k = t; m < chunk && k < count; k += nthreads, m++) {
@@ -22,6 +26,7 @@ __global__ void __launch_bounds__(256) k_jac_to_affine(G1A *out, const G1J *in, 
         if (!fp_is_zero(z)) acc = fp_mul(acc, z);
     }
     Fp inv = fp_inv(acc);
+    if (HOMOG) inv = fp_mul(inv, fp_const(cfp::SIGMA_M));
 #pragma unroll 1
     while (m-- > 0) {
         const uint64_t k = t + (uint64_t)m * nthreads;
@@ -30,12 +35,17 @@ __global__ void __launch_bounds__(256) k_jac_to_affine(G1A *out, const G1J *in, 
             out[k] = g1a_identity();
             continue;
         }
-        const Fp zi = fp_mul(inv, prefix[k]);
+        const Fp zi = fp_mul(inv, prefix[k]);  // 1 / Z or sigma / Z
         inv = fp_mul(inv, p.z);
-        const Fp zi2 = fp_sqr(zi);
         G1A r;
-        r.x = fp_mul(p.x, zi2);
-        r.y = fp_mul(p.y, fp_mul(zi2, zi));
+        if (HOMOG) {
+            r.x = fp_mul(p.x, zi);
+            r.y = fp_mul(p.y, zi);
+        } else {
+            const Fp zi2 = fp_sqr(zi);
+            r.x = fp_mul(p.x, zi2);
+            r.y = fp_mul(p.y, fp_mul(zi2, zi));
+        }
         out[k] = r;
     }
 }
@@ -140,14 +150,27 @@ __global__ void __launch_bounds__(64) k_table_multiples(G1AT *table, const G1A *
 
 }  // namespace
 
-hipError_t launch_jac_to_affine(G1A *out, const G1J *in, Fp *prefix, uint64_t count, uint32_t chunk,
-                                hipStream_t s) {
+namespace {
+template <bool HOMOG>
+hipError_t launch_to_affine(G1A *out, const G1J *in, Fp *prefix, uint64_t count, uint32_t chunk, hipStream_t s) {
     const uint64_t nthreads = (count + chunk - 1) / chunk;
     // four-wave workgroups: spread over a CU's SIMDs (one-wave workgroups
     // can stack on some SIMDs while others idle)
-    hipLaunchKernelGGL(k_jac_to_affine, dim3(blocks_for(nthreads, 256)), dim3(256), 0, s, out, in,
-                       prefix, count, chunk, nthreads);
+    hipLaunchKernelGGL(k_to_affine<HOMOG>, dim3(blocks_for(nthreads, 256)), dim3(256), 0, s, out, in, prefix, count,
+                       chunk, nthreads);
     return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_jac_to_affine(G1A *out, const G1J *in, Fp *prefix, uint64_t count, uint32_t chunk,
+                                hipStream_t s) {
+    return launch_to_affine<false>(out, in, prefix, count, chunk, s);
+}
+
+hipError_t launch_ladder_to_affine(G1A *out, const G1J *lad, Fp *prefix, uint64_t count, uint32_t chunk,
+                                   uint32_t lanes, hipStream_t s) {
+    return lanes == 4 ? launch_to_affine<true>(out, lad, prefix, count, chunk, s)
+                      : launch_to_affine<false>(out, lad, prefix, count, chunk, s);
 }
 
 hipError_t launch_table_chains(G1J *out, const G1A *bases, uint32_t n, WindowPlan plan, hipStream_t s) {
