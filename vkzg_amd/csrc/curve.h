@@ -353,12 +353,12 @@ VKZG_DEV G1X g1x_dbl_quad(const G1X &p, uint32_t q) {
     const Fp r1 = fp_mul(fp_select(odd, p.x, fp_dbl_raw(p.y)), fp_select(odd, p.x, p.y));
     const Fp V = fp_dbl_raw(fp_quad_bcast<0>(r1));  // 4 Y^2
     const Fp M = fp_triple(fp_quad_bcast<1>(r1));   // 3 X^2
-    const Fp r2 = fp_mul(fp_select(q == 2, M, V), q == 0 ? p.y : (q == 1 ? p.x : (q == 2 ? M : p.zz)));
+    const Fp r2 = fp_mul(fp_select(q == 2, M, V), fp_select4(q, p.y, p.x, M, p.zz));
     const Fp W = fp_dbl_raw(fp_quad_bcast<0>(r2)), S = fp_quad_bcast<1>(r2);  // 8 Y^3, 4 X Y^2
     G1X r;
     r.x = fp_neg(fp_dbl_sub(S, fp_quad_bcast<2>(r2)));  // M^2 - 2S
     r.zz = fp_quad_bcast<3>(r2);                        // V ZZ
-    const Fp r3 = fp_mul(q == 0 ? fp_sub_raw(S, r.x) : W, q == 0 ? M : (q == 1 ? p.y : p.zzz));
+    const Fp r3 = fp_mul(fp_select(q == 0, fp_sub_raw(S, r.x), W), fp_select4(q, M, p.y, p.zzz, p.zzz));
     r.y = fp_sub(fp_quad_bcast<0>(r3), fp_quad_bcast<1>(r3));  // M (S - X3) - W Y
     r.zzz = fp_quad_bcast<2>(r3);                               // W ZZZ
     return r;
@@ -370,23 +370,20 @@ VKZG_DEV G1X g1x_dbl_quad(const G1X &p, uint32_t q) {
 VKZG_DEV G1X g1x_add_quad(const G1X &a, const G1X &b, uint32_t q, bool &exc) {
     if (fp_is_zero(a.zz)) return b;  // uniform in the quad
     if (fp_is_zero(b.zz)) return a;
-    const Fp r1 = fp_mul(q == 0 ? a.x : (q == 1 ? b.x : (q == 2 ? a.y : b.y)),
-                         q == 0 ? b.zz : (q == 1 ? a.zz : (q == 2 ? b.zzz : a.zzz)));
+    const Fp r1 = fp_mul(fp_select4(q, a.x, b.x, a.y, b.y), fp_select4(q, b.zz, a.zz, b.zzz, a.zzz));
     const Fp U1 = fp_quad_bcast<0>(r1), U2 = fp_quad_bcast<1>(r1);
     const Fp S1 = fp_quad_bcast<2>(r1), S2 = fp_quad_bcast<3>(r1);
     const Fp P = fp_sub(U2, U1), R = fp_sub(S2, S1);
-    const Fp r2 = fp_mul(q == 0 ? P : (q == 1 ? R : (q == 2 ? a.zz : a.zzz)),
-                         q == 0 ? P : (q == 1 ? R : (q == 2 ? b.zz : b.zzz)));
+    const Fp r2 = fp_mul(fp_select4(q, P, R, a.zz, a.zzz), fp_select4(q, P, R, b.zz, b.zzz));
     const Fp PP = fp_quad_bcast<0>(r2), RR = fp_quad_bcast<1>(r2);
     const Fp ZZab = fp_quad_bcast<2>(r2), ZZZab = fp_quad_bcast<3>(r2);
     exc |= fp_is_zero(PP);
-    const Fp r3 = fp_mul_fold_v(q == 0 ? P : (q == 1 ? U1 : (q == 2 ? ZZab : fp_add_raw(U1, U2))), PP, RR,
-                              q == 3 ? -1 : 0);
+    const Fp r3 = fp_mul_fold_v(fp_select4(q, P, U1, ZZab, fp_add_raw(U1, U2)), PP, RR, q == 3 ? -1 : 0);
     const Fp PPP = fp_quad_bcast<0>(r3), Q = fp_quad_bcast<1>(r3), nX = fp_quad_bcast<3>(r3);
     G1X r;
     r.zz = fp_quad_bcast<2>(r3);
     r.x = fp_neg(nX);
-    const Fp r4 = fp_mul(q == 0 ? fp_add_raw(Q, nX) : PPP, q == 0 ? R : (q == 1 ? S1 : ZZZab));
+    const Fp r4 = fp_mul(fp_select(q == 0, fp_add_raw(Q, nX), PPP), fp_select4(q, R, S1, ZZZab, ZZZab));
     r.y = fp_sub(fp_quad_bcast<0>(r4), fp_quad_bcast<1>(r4));
     r.zzz = fp_quad_bcast<2>(r4);
     return r;
@@ -406,12 +403,12 @@ VKZG_DEV G1X g1x_madd_acc_quad(const G1X &a, const G1A &b, bool neg, uint32_t q,
     const Fp r2 = fp_sqr(fp_select(odd, R, P));
     const Fp PP = fp_quad_bcast<0>(r2), RR = fp_quad_bcast<1>(r2);
     exc |= fp_is_zero(PP);
-    const Fp r3 = fp_mul_fold_v(q == 0 ? P : (q == 1 ? a.x : (q == 2 ? a.zz : V)), PP, RR, q == 3 ? -1 : 0);
+    const Fp r3 = fp_mul_fold_v(fp_select4(q, P, a.x, a.zz, V), PP, RR, q == 3 ? -1 : 0);
     const Fp PPP = fp_quad_bcast<0>(r3), Q = fp_quad_bcast<1>(r3), nX = fp_quad_bcast<3>(r3);
     G1X r;
     r.zz = fp_quad_bcast<2>(r3);
     r.x = fp_neg(nX);
-    const Fp r4 = fp_mul(q == 0 ? fp_add_raw(Q, nX) : PPP, q == 0 ? R : (q == 1 ? a.y : a.zzz));
+    const Fp r4 = fp_mul(fp_select(q == 0, fp_add_raw(Q, nX), PPP), fp_select4(q, R, a.y, a.zzz, a.zzz));
     r.y = fp_sub(fp_quad_bcast<0>(r4), fp_quad_bcast<1>(r4));  // R (Q - X3) - Y1 PPP
     r.zzz = fp_quad_bcast<2>(r4);
     return r;

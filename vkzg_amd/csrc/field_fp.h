@@ -265,6 +265,10 @@ VKZG_DEV Fp fp_select(bool c, const Fp &a, const Fp &b) {
     for (int i = 0; i < kFpLimbs; i++) r.v[i] = c ? a.v[i] : b.v[i];
     return r;
 }
+// The value of lane q of a quad: a, b, c or d.
+VKZG_DEV Fp fp_select4(uint32_t q, const Fp &a, const Fp &b, const Fp &c, const Fp &d) {
+    return fp_select((q & 2u) != 0, fp_select((q & 1u) != 0, d, c), fp_select((q & 1u) != 0, b, a));
+}
 
 // Zero mod p, for a value whose residue 0 has one form only: a product, a
 // constant, or a small multiple or negation of one (magnitude of the product

@@ -185,7 +185,7 @@ __global__ void __launch_bounds__(256) k_ladder_xyzz(G1X *pts, G1X *phi, const G
     const Fp z = fp_mul(p.z, fp_const(cfp::INV_SIGMA_M));
     const Fp r2 = fp_mul(fp_select(q == 1, p.x, z), z);
     const Fp zz = fp_quad_bcast<0>(r2), x = fp_quad_bcast<1>(r2);
-    const Fp r3 = fp_mul(q == 0 ? z : (q == 1 ? x : p.y), fp_select(q == 1, fp_const(cfp::BETA_M), zz));
+    const Fp r3 = fp_mul(fp_select4(q, z, x, p.y, p.y), fp_select(q == 1, fp_const(cfp::BETA_M), zz));
     if (q == 0) {
         pts[k].zz = zz;
         pts[k].zzz = r3;

@@ -15,13 +15,14 @@
 //   buckets  one lane per bucket sums its points          (XYZZ, checked);
 //            buckets of more than 24 points by a wave
 //   windows  blocks per (msm, window): sum_b (b+1) B_b by running sums over
-//            segments of at most 4 buckets, then trees in LDS
-//   combine  four lanes per MSM: Horner over windows (c doublings each),
-//            each doubling and addition shared by the quad, and the
-//            conversion to affine.
+//            segments of at most 4 buckets on quads, then trees in LDS
+//   combine  a wave per MSM: Horner over runs of windows (c doublings each) on
+//            its quads, a tree, and the conversion to affine.
 // The point order inside a bucket depends on atomics, but the sum is the same
 // group element, so results are deterministic after normalisation.
 #include "msm.h"
+
+#include "proj_quad.h"
 
 #include "glv.h"
 #include "proof_common.h"
@@ -30,9 +31,9 @@ namespace vkzg_amd {
 
 namespace {
 
-constexpr uint32_t kWinThreads = 128;
+constexpr uint32_t kWinQuads = 64;
 constexpr uint32_t kHotLen = 24;    // longer buckets are summed by a wave (k_msm_hot)
-constexpr uint32_t kWinSeg = 4;     // buckets per window thread: the sums are latency-bound
+constexpr uint32_t kWinSeg = 4;     // buckets per window quad: the sums are latency-bound
 constexpr uint32_t kHotBlocks = 2048;
 constexpr uint32_t kScanOneBlock = 16384;  // larger scans use k_msm_scan_tiles
 constexpr uint32_t kScanTile = 4096;       // buckets per block of k_msm_scan_tiles
@@ -255,100 +256,122 @@ __global__ void __launch_bounds__(64) k_msm_hot(G1X *buckets, const uint32_t *of
     }
 }
 
-// [k] p for 0 < k < 2^16 (double-and-add from the top set bit, checked operations)
-VKZG_DEV G1X g1x_mul_small(const G1X &p, uint32_t k) {
-    G1X acc = p;
+// [k] p, 0 < k < 2^16, by a quad
+VKZG_DEV G1PQ g1p_mul_small(const G1P &p, uint32_t k, uint32_t q) {
+    G1PQ acc = g1p_spread(p, q);
 #pragma unroll 1
     for (int b = 30 - __builtin_clz(k); b >= 0; b--) {
-        acc = g1x_dbl(acc);
-        if ((k >> b) & 1u) acc = g1x_add(acc, p);
+        acc = g1pq_dbl(acc, q);
+        if ((k >> b) & 1u) acc = g1p_add_quad(g1p_gather(acc), p, q);
     }
     return acc;
 }
 
+// The sum of the block's kWinQuads points, one per quad, in its quad 0.
+VKZG_DEV G1PQ g1pq_block_sum(G1PQ acc, Fp *sh, uint32_t t) {
+#pragma unroll 1
+    for (uint32_t stride = kWinQuads / 2; stride > 0; stride >>= 1) {
+        __syncthreads();
+        sh[t] = acc.r;
+        __syncthreads();
+        if (t / 4 < stride)
+            acc = g1p_add_quad(g1p_gather(acc), g1p_gather(G1PQ{sh[t + 4 * stride]}), t & 3u);
+    }
+    return acc;
+}
+VKZG_DEV void g1pq_store(G1P *out, const G1PQ &p, uint32_t q) {
+    const Fp y = g1pq_y(p);
+    if (q == 0) out->y = y;
+    else if (q == 2) out->x = p.r;
+    else if (q == 3) out->z = p.r;
+}
+
 // Block (msm, window, part): sum over the part's buckets b of (b + 1) B_b.
-// Thread t owns buckets [lo, lo + seg): running sums from the top give
-// R = sum B_b and T = sum (b - lo + 1) B_b, and its share is T + lo R; a
-// tree in LDS adds the shares.  A window's parts (enough of them for at most
-// kWinSeg buckets per thread) are added by k_msm_parts.
-__global__ void __launch_bounds__(kWinThreads) k_msm_windows(G1X *wpart, const G1X *buckets, uint32_t bk,
-                                                             uint32_t parts) {
-    __shared__ G1X sh[kWinThreads];
-    const uint32_t t = threadIdx.x;
+// Quad k owns buckets [lo, lo + seg): running sums from the top give R = sum B_b
+// and T = sum (b - lo + 1) B_b, and its share is T + lo R; a tree adds the
+// shares.  A window's parts (enough of them for at most kWinSeg buckets per
+// quad) are added by k_msm_parts.  The chain of additions and doublings is the
+// time here, so quads in homogeneous coordinates run it (proj_quad.h): with 38
+// windows of 64 buckets (the sums of a check of 128 cells) 285 -> 76 us against
+// a lane per bucket in XYZZ coordinates.
+__global__ void __launch_bounds__(4 * kWinQuads) k_msm_windows(G1P *wpart, const G1X *buckets, uint32_t bk,
+                                                               uint32_t parts) {
+    __shared__ Fp sh[4 * kWinQuads];
+    const uint32_t t = threadIdx.x, q = t & 3u, k = t >> 2;
     const uint32_t win = blockIdx.x / parts, part = blockIdx.x % parts;
     const G1X *B = buckets + (size_t)win * bk;
     const uint32_t per_part = bk / parts;
-    const uint32_t seg = per_part > kWinThreads ? per_part / kWinThreads : 1;
-    const uint32_t lo = part * per_part + t * seg;
-    G1X share = g1x_identity();
-    if (t * seg < per_part) {
-        G1X R = g1x_identity(), T = g1x_identity();
+    const uint32_t seg = per_part > kWinQuads ? per_part / kWinQuads : 1;
+    const uint32_t lo = part * per_part + k * seg;
+    G1PQ share = g1p_spread(g1p_identity(), q);
+    if (k * seg < per_part) {
+        G1P R = g1p_from_xyzz(B[lo + seg - 1], q);
+        if (seg == 1) {
+            share = g1p_mul_small(R, lo + 1, q);
+        } else {
+            G1P T = R;
 #pragma unroll 1
-        for (uint32_t b = lo + seg; b-- > lo;) {
-            R = g1x_add(R, B[b]);
-            T = g1x_add(T, R);
+            for (uint32_t b = lo + seg - 1; b-- > lo;) {
+                R = g1p_gather(g1p_add_quad(R, g1p_from_xyzz(B[b], q), q));
+                T = g1p_gather(g1p_add_quad(T, R, q));
+            }
+            share = lo ? g1p_add_quad(g1p_gather(g1p_mul_small(R, lo, q)), T, q) : g1p_spread(T, q);
         }
-        share = lo ? g1x_add(T, g1x_mul_small(R, lo)) : T;
     }
-    sh[t] = share;
-    __syncthreads();
-    for (uint32_t stride = kWinThreads / 2; stride > 0; stride >>= 1) {
-        if (t < stride) sh[t] = g1x_add(sh[t], sh[t + stride]);
-        __syncthreads();
-    }
-    if (t == 0) wpart[blockIdx.x] = sh[0];
+    share = g1pq_block_sum(share, sh, t);
+    if (k == 0) g1pq_store(&wpart[blockIdx.x], share, q);
 }
 
-// wsum[win] = sum of the window's parts (a tree over at most 64 parts).
-__global__ void __launch_bounds__(64) k_msm_parts(G1X *wsum, const G1X *wpart, uint32_t parts) {
-    __shared__ G1X sh[64];
-    const uint32_t t = threadIdx.x;
-    sh[t] = t < parts ? wpart[(size_t)blockIdx.x * parts + t] : g1x_identity();
-    __syncthreads();
-    for (uint32_t stride = 32; stride > 0; stride >>= 1) {
-        if (t < stride) sh[t] = g1x_add(sh[t], sh[t + stride]);
-        __syncthreads();
-    }
-    if (t == 0) wsum[blockIdx.x] = sh[0];
+// wsum[win] = sum of the window's parts (at most kWinQuads of them).
+__global__ void __launch_bounds__(4 * kWinQuads) k_msm_parts(G1P *wsum, const G1P *wpart, uint32_t parts) {
+    __shared__ Fp sh[4 * kWinQuads];
+    const uint32_t t = threadIdx.x, q = t & 3u, k = t >> 2;
+    const G1P p = k < parts ? wpart[(size_t)blockIdx.x * parts + k] : g1p_identity();
+    const G1PQ acc = g1pq_block_sum(g1p_spread(p, q), sh, t);
+    if (k == 0) g1pq_store(&wsum[blockIdx.x], acc, q);
 }
 
-// Horner over the windows with the checked addition (the rare path of k_msm_combine).
-VKZG_DEV_COLD void combine_checked(G1X *acc, const G1X *ws, uint32_t W, uint32_t c) {
-    G1X a = ws[W - 1];
-    for (uint32_t w = W - 1; w-- > 0;) {
-        for (uint32_t i = 0; i < c; i++) a = g1x_dbl(a);
-        a = g1x_add(a, ws[w]);
-    }
-    *acc = a;
-}
-
-// out[m] = sum_w 2^(c w) wsum[m W + w], affine ((0, 0) for the identity),
-// by the quad m = tid / 4.  The doubling chain is this launch's critical
-// path, so the loop uses the call-free addition; an equal or opposite pair
-// (flagged) redoes it checked.  Quads exit together.
-__global__ void __launch_bounds__(64) k_msm_combine(G1A *out, const G1X *wsum, uint32_t nmsm, uint32_t W,
-                                                    uint32_t c) {
-    const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t m = tid >> 2, q = tid & 3u;
-    if (m >= nmsm) return;
-    const G1X *ws = wsum + (size_t)m * W;
-    G1X acc = ws[W - 1];
-    bool exc = false;
+// out[m] = sum_w 2^(c w) wsum[m W + w], affine ((0, 0) for the identity), by
+// wave m.  The chain of c (W - 1) doublings is this launch's critical path, so
+// it runs on quads in homogeneous coordinates (two rounds of products per
+// doubling, complete additions: proj_quad.h).  The additions would lengthen it
+// by 3.5 rounds each, so the wave's 16 quads each take a run of L = ceil(W / 16)
+// windows, from the top down, by Horner, double their sum up to its place and
+// meet in a tree: L + 3 additions in the chain instead of W - 1.  With 19 windows
+// of 7 bits (the sums of a check of 128 cells), 730 us for a quad's three-round
+// XYZZ Horner -> 410 us.
+__global__ void __launch_bounds__(64) k_msm_combine(G1A *out, const G1P *wsum, uint32_t W, uint32_t c) {
+    const uint32_t m = blockIdx.x, g = threadIdx.x >> 2, q = threadIdx.x & 3u;
+    const G1P *ws = wsum + (size_t)m * W;
+    const uint32_t L = (W + 15) / 16;
+    const uint32_t hi = W > g * L ? W - g * L : 0, lo = hi > L ? hi - L : 0;
+    G1P acc = hi > 0 ? ws[hi - 1] : g1p_identity();
+    G1PQ a = g1p_spread(acc, q);
 #pragma unroll 1
-    for (uint32_t w = W - 1; w-- > 0;) {
+    for (uint32_t w = hi; w > lo + 1;) {
+        w--;
 #pragma unroll 1
-        for (uint32_t i = 0; i < c; i++) acc = g1x_dbl_quad(acc, q);
-        acc = g1x_add_quad(acc, ws[w], q, exc);
+        for (uint32_t i = 0; i < c; i++) a = g1pq_dbl(a, q);
+        a = g1p_add_quad(g1p_gather(a), ws[w - 1], q);
     }
-    if (exc) combine_checked(&acc, ws, W, c);
+    // the wave runs as long as its longest chain: quad 0's, c (W - 1) in all
+#pragma unroll 1
+    for (uint32_t i = 0; i < lo * c; i++) a = g1pq_dbl(a, q);
+#pragma unroll 1
+    for (uint32_t x = 4; x < 64; x <<= 1) {
+        G1PQ b;
+#pragma unroll
+        for (int i = 0; i < kFpLimbs; i++) b.r.v[i] = __shfl_xor(a.r.v[i], (int)x);
+        a = g1p_add_quad(g1p_gather(a), g1p_gather(b), q);
+    }
+    acc = g1p_gather(a);
     G1A r = g1a_identity();
-    if (!g1x_is_identity(acc)) {
-        // x = X / ZZ = X ZZZ / (ZZ ZZZ), y = Y / ZZZ = Y ZZ / (ZZ ZZZ): one inversion
-        const Fp inv = fp_inv(fp_mul(acc.zz, acc.zzz));
-        r.x = fp_mul(fp_mul(acc.x, acc.zzz), inv);
-        r.y = fp_mul(fp_mul(acc.y, acc.zz), inv);
+    if (!fp_is_zero(acc.z)) {
+        const Fp inv = fp_inv(acc.z);
+        r.x = fp_mul(fp_mul(acc.x, fp_const(cfp::SIGMA_OVER_NU_M)), inv);
+        r.y = fp_mul(fp_mul(acc.y, fp_const(cfp::SIGMA_M)), inv);
     }
-    if (q == 0) out[m] = r;
+    if (threadIdx.x == 0) out[m] = r;
 }
 
 }  // namespace
@@ -365,7 +388,7 @@ MsmShape msm_shape(uint32_t ne, uint32_t nmsm) {
     sh.W = (129 + c - 1) / c;
     sh.bk = 1u << (c - 1);
     sh.K = nmsm * sh.W * sh.bk;
-    sh.parts = sh.bk > kWinThreads * kWinSeg ? sh.bk / (kWinThreads * kWinSeg) : 1;
+    sh.parts = sh.bk > kWinQuads * kWinSeg ? sh.bk / (kWinQuads * kWinSeg) : 1;
     return sh;
 }
 
@@ -377,7 +400,7 @@ size_t msm_scratch_bytes(const MsmShape &sh) {
     b += 4ull * (sh.K / kScanTile + 1);  // scan tile totals
     b += 4 * nh * sh.W;                  // sorted references
     b += sizeof(G1X) * (size_t)sh.K;     // buckets
-    b += sizeof(G1X) * (size_t)sh.nmsm * sh.W * (sh.parts + 1);
+    b += sizeof(G1P) * (size_t)sh.nmsm * sh.W * (sh.parts + 1);
     return b + 16 * 256;  // each of the 10 regions is rounded up to 256 bytes
 }
 
@@ -400,8 +423,8 @@ hipError_t launch_msm(const MsmShape &sh, void *scratch, const G1A *pts, const u
     uint32_t *tot = reinterpret_cast<uint32_t *>(take(4ull * (sh.K / kScanTile + 1)));
     uint32_t *list = reinterpret_cast<uint32_t *>(take(4ull * nh * sh.W));
     G1X *buckets = reinterpret_cast<G1X *>(take(sizeof(G1X) * (size_t)sh.K));
-    G1X *wsum = reinterpret_cast<G1X *>(take(sizeof(G1X) * (size_t)sh.nmsm * sh.W));
-    G1X *wpart = reinterpret_cast<G1X *>(take(sizeof(G1X) * (size_t)sh.nmsm * sh.W * sh.parts));
+    G1P *wpart = reinterpret_cast<G1P *>(take(sizeof(G1P) * (size_t)sh.nmsm * sh.W * sh.parts));
+    G1P *wsum = sh.parts > 1 ? reinterpret_cast<G1P *>(take(sizeof(G1P) * (size_t)sh.nmsm * sh.W)) : wpart;
     if ((size_t)(p - static_cast<uint8_t *>(scratch)) > msm_scratch_bytes(sh)) return hipErrorInvalidValue;
     if (sh.K > kScanOneBlock && ntiles > 1024) return hipErrorInvalidValue;  // beyond 4M buckets
     hipLaunchKernelGGL(k_msm_split, dim3(blocks_for(sh.ne, 256)), dim3(256), 0, s, hs, sc, sh.ne);
@@ -420,11 +443,11 @@ hipError_t launch_msm(const MsmShape &sh, void *scratch, const G1A *pts, const u
                        sh.K, hot, cnt + sh.K);
     const dim3 hot_grid(sh.K < kHotBlocks ? sh.K : kHotBlocks);
     hipLaunchKernelGGL(k_msm_hot, hot_grid, dim3(64), 0, s, buckets, off, list, pts, hot, cnt + sh.K);
-    hipLaunchKernelGGL(k_msm_windows, dim3(sh.nmsm * sh.W * sh.parts), dim3(kWinThreads), 0, s, wpart, buckets,
+    hipLaunchKernelGGL(k_msm_windows, dim3(sh.nmsm * sh.W * sh.parts), dim3(4 * kWinQuads), 0, s, wpart, buckets,
                        sh.bk, sh.parts);
-    hipLaunchKernelGGL(k_msm_parts, dim3(sh.nmsm * sh.W), dim3(64), 0, s, wsum, wpart, sh.parts);
-    hipLaunchKernelGGL(k_msm_combine, dim3(blocks_for(sh.nmsm * 4ull, 64)), dim3(64), 0, s, out, wsum, sh.nmsm, sh.W,
-                       sh.c);
+    if (sh.parts > 1)
+        hipLaunchKernelGGL(k_msm_parts, dim3(sh.nmsm * sh.W), dim3(4 * kWinQuads), 0, s, wsum, wpart, sh.parts);
+    hipLaunchKernelGGL(k_msm_combine, dim3(sh.nmsm), dim3(64), 0, s, out, wsum, sh.W, sh.c);
     return hipGetLastError();
 }
 

@@ -5,11 +5,15 @@
 // Both G2 points of the check are setup constants, so their Miller-loop lines
 // are computed once, in affine coordinates, when the G2 setup is loaded
 // (k_g2_lines).  A call then needs only:
-//   k_pair_lines  one block per loop step: both lines evaluated at P1, P2
-//                 and multiplied together (68 steps);
-//   k_pair_final  one block: the Miller accumulation f <- f^2 L_s and the
+//   k_pair_lines  one block per four iterations of the loop: both points' lines
+//                 evaluated at P1, P2 and folded into one value;
+//   k_pair_final  one block: the Miller accumulation over the 16 groups and the
 //                 final exponentiation, with every Fp12 product spread over
-//                 144 lanes (tower.h).
+//                 144 lanes and every cyclotomic square over 96 (tower.h); the
+//                 other blocks are the subgroup checks of the batch's points.
+// The chain of Fp12 products is the time of both, ~75 Miller steps, 315
+// cyclotomic squares and 40 products: 1141 -> 935 us for k_pair_final, 8 -> 30 us
+// for k_pair_lines.
 //
 // Miller loop over |z| = 0xd201000000010000 from the top bit down: a
 // doubling line per bit, an addition line per set bit below the top (63 + 5
@@ -30,7 +34,9 @@
 // 1 exactly when its cube is (3 does not divide r).
 #include "pairing.h"
 
+#include "proj_quad.h"
 #include "proof_common.h"
+#include "verify.h"
 
 namespace vkzg_amd {
 
@@ -150,57 +156,109 @@ __global__ void __launch_bounds__(64) k_g2_lines(Fp2 *lines, const G2A *qs, uint
     if (bad) atomicOr(err, 2u);
 }
 
-// Block s: L[s] = l1_s(P1) * l2_s(P2), P2 negated when neg2.  A point at
-// infinity contributes the line 1.
+// Bit i of |z|: an addition line follows the doubling line of iteration i.
+VKZG_DEV bool z_bit(int i) { return ((kZAbs >> i) & 1u) != 0; }
+
+// Block g: the Miller accumulation over the kGroupIters iterations of group g
+// alone (from the top: iterations 62 - kGroupIters g down), L[g] = prod over them
+// of (l1_s(P1) l2_s(P2))^(2^(doublings left in the group)), P2 negated when
+// neg2.  A point at infinity contributes the line 1.  The accumulation's 63
+// squarings are a chain, its 68 products by lines are not: blocks fold them into
+// 16 values side by side (11 to 15 Fp12 products each), which leaves 75 products in
+// k_pair_final's chain instead of 131.
 __global__ void __launch_bounds__(kPairThreads) k_pair_lines(Fp *L, const Fp2 *lines1, const Fp2 *lines2,
                                                              const G1A *p1, const G1A *p2, uint32_t neg2) {
-    __shared__ Fp l1[12], l2[12], res[12];
-    const uint32_t t = threadIdx.x, s = blockIdx.x;
-    if (t < 12) {
-        l1[t] = fp_zero();
-        l2[t] = fp_zero();
-    }
-    __syncthreads();
-    if (t < 2) {
-        const Fp2 *ln = (t == 0 ? lines1 : lines2) + 2 * s;
-        G1A P = t == 0 ? *p1 : *p2;
-        Fp *l = t == 0 ? l1 : l2;
+    __shared__ Fp l[2 * kGroupLines][12], f[12], v[12];
+    const uint32_t t = threadIdx.x;
+    const int top = 62 - (int)(kGroupIters * blockIdx.x);
+    const int low = top >= (int)kGroupIters ? top - (int)kGroupIters + 1 : 0;
+    // the group's lines, and those before it
+    uint32_t s0 = 0, n = 0;
+    for (int i = 62; i >= low; i--) (i > top ? s0 : n) += z_bit(i) ? 2u : 1u;
+    if (t < 2 * n) {  // line s0 + t / 2 at P1 (t even) or P2
+        const bool second = (t & 1u) != 0;
+        const Fp2 *ln = (second ? lines2 : lines1) + 2 * (s0 + t / 2);
+        G1A P = second ? *p2 : *p1;
+        Fp *d = l[t];
+        for (int k = 0; k < 12; k++) d[k] = fp_zero();
         if (g1a_is_identity(P)) {
-            l[0] = fp_one();
+            d[0] = fp_one();
         } else {
-            if (t == 1 && neg2) P.y = fp_neg(P.y);
+            if (second && neg2) P.y = fp_neg(P.y);
             const Fp2 c0 = ln[0], c2 = ln[1];
-            l[0] = c0.c0;
-            l[1] = c0.c1;
-            l[4] = fp_mul(c2.c0, P.x);
-            l[5] = fp_mul(c2.c1, P.x);
-            l[6] = P.y;
+            d[0] = c0.c0;
+            d[1] = c0.c1;
+            d[4] = fp_mul(c2.c0, P.x);
+            d[5] = fp_mul(c2.c1, P.x);
+            d[6] = P.y;
         }
     }
     __syncthreads();
-    fp12_mul_lds(res, l1, l2);
-    if (t < 12) L[(size_t)s * 12 + t] = res[t];
+    uint32_t s = 0;
+#pragma unroll 1
+    for (int i = top; i >= low; i--) {
+        if (s > 0) fp12_mul_lds(f, f, f);
+#pragma unroll 1
+        for (uint32_t k = z_bit(i) ? 2 : 1; k > 0; k--, s++) {
+            fp12_mul_lds(s > 0 ? v : f, l[2 * s], l[2 * s + 1]);
+            if (s > 0) fp12_mul_lds(f, f, v);
+        }
+    }
+    if (t < 12) L[(size_t)blockIdx.x * 12 + t] = f[t];
 }
 
-__device__ void fp12_copy(Fp *dst, const Fp *src) {
+// The steps of the final exponentiation on Fp12 values R[0..] in LDS, d = op(a, b).
+// A table and a loop over it instead of a call per step: products and powers are
+// inlined, and this keeps one copy of each (the kernel is half as long).
+enum : uint8_t { kStepMul, kStepPow, kStepConj, kStepFrob1, kStepFrob2 };
+enum : uint8_t { rF, rG, rH, rA, rB, rC, rD, kPairRegs };
+struct PairStep {
+    uint8_t op, d, a, b;
+};
+static __constant__ PairStep kFinalSteps[] = {
+    // easy part: rG = conj(f), rH = 1/(f conj(f)) -> rF = f^((p^6 - 1)(p^2 + 1)), in the cyclotomic subgroup
+    {kStepMul, rH, rG, rH},       // 1/f = conj(f) / (f conj(f))
+    {kStepMul, rG, rG, rH},       // f^(p^6 - 1)
+    {kStepFrob2, rH, rG, 0},
+    {kStepMul, rF, rH, rG},
+    // hard part: rF^(3 (p^4 - p^2 + 1)/r); conj is the inverse here
+    {kStepPow, rA, rF, 0},
+    {kStepMul, rA, rA, rF},
+    {kStepConj, rA, rA, 0},       // A = F^(z - 1)
+    {kStepPow, rB, rA, 0},
+    {kStepMul, rB, rB, rA},
+    {kStepConj, rB, rB, 0},       // B = A^(z - 1)
+    {kStepPow, rC, rB, 0},
+    {kStepConj, rC, rC, 0},
+    {kStepFrob1, rG, rB, 0},
+    {kStepMul, rC, rC, rG},       // C = B^(z + p)
+    {kStepPow, rD, rC, 0},
+    {kStepPow, rA, rD, 0},        // C^(z^2)
+    {kStepFrob2, rG, rC, 0},
+    {kStepMul, rA, rA, rG},
+    {kStepConj, rG, rC, 0},
+    {kStepMul, rA, rA, rG},       // C^(z^2 + p^2 - 1)
+    {kStepMul, rG, rF, rF},
+    {kStepMul, rG, rG, rF},       // F^3
+    {kStepMul, rA, rA, rG},
+};
+
+// dst <- conj(src), dst may be src
+__device__ __forceinline__ void fp12_conj(Fp *dst, const Fp *src) {
+    if (threadIdx.x < 12) fp12_conj_to(dst, src, threadIdx.x);
+    __syncthreads();
+}
+// dst = src^|z| (dst != src) for src in the cyclotomic subgroup; unit: {one, zero} in LDS
+__device__ __forceinline__ void fp12_pow_zabs(Fp *dst, const Fp *src, const Fp *unit, const CycTerm &term) {
     if (threadIdx.x < 12) dst[threadIdx.x] = src[threadIdx.x];
     __syncthreads();
-}
-__device__ void fp12_conj_inplace(Fp *a) {
-    const uint32_t t = threadIdx.x;
-    if (t < 12 && ((t >> 1) & 1u)) a[t] = fp_neg(a[t]);
-    __syncthreads();
-}
-// dst = src^|z| (dst != src)
-__device__ void fp12_pow_zabs(Fp *dst, const Fp *src) {
-    fp12_copy(dst, src);
 #pragma unroll 1
     for (int i = 62; i >= 0; i--) {
-        fp12_mul_lds(dst, dst, dst);
-        if ((kZAbs >> i) & 1u) fp12_mul_lds(dst, dst, src);
+        fp12_cyc_sqr_lds(dst, unit, term);
+        if (z_bit(i)) fp12_mul_lds(dst, dst, src);
     }
 }
-__device__ void fp12_frob1(Fp *dst, const Fp *src) {
+__device__ __forceinline__ void fp12_frob1(Fp *dst, const Fp *src) {
     const uint32_t t = threadIdx.x;
     if (t < 6) {
         const Fp2 a = {src[2 * t], src[2 * t + 1]};
@@ -210,78 +268,92 @@ __device__ void fp12_frob1(Fp *dst, const Fp *src) {
     }
     __syncthreads();
 }
-__device__ void fp12_frob2(Fp *dst, const Fp *src) {
+__device__ __forceinline__ void fp12_frob2(Fp *dst, const Fp *src) {
     const uint32_t t = threadIdx.x;
     if (t < 12) dst[t] = fp_mul(src[t], frob2_const(t >> 1));
     __syncthreads();
 }
 
-// Miller accumulation over the 68 step products L, final exponentiation,
+// Block 0: Miller accumulation over the 16 group products L, final exponentiation,
 // status[0] = 1 when the result is 1 (else 0); out12 (may be null) receives
-// the result (12 Fp, Montgomery).
-__global__ void __launch_bounds__(kPairThreads) k_pair_final(uint32_t *status, Fp *out12, const Fp *L) {
-    __shared__ Fp f[12], g[12], h[12], A[12], B[12], C[12], D[12];
-    __shared__ Fp Ls[kPairSteps * 12];  // the step products, staged in LDS (42 KiB)
+// the result (12 Fp, Montgomery).  Its one chain of products leaves the rest of
+// the chip idle, so the other blocks check the membership in G1 of the npts
+// points pts (a quad each, 1/3 of the chain's time): err |= kVfyNotInGroup.
+__global__ void __launch_bounds__(kPairThreads) k_pair_final(uint32_t *status, Fp *out12, const Fp *L, const G1A *pts,
+                                                             uint32_t npts, uint32_t *err) {
+    __shared__ Fp R[kPairRegs][12], unit[2];
+    __shared__ Fp Ls[kPairGroups * 12];
     __shared__ uint32_t ok;
     const uint32_t t = threadIdx.x;
-    for (uint32_t i = t; i < kPairSteps * 12; i += blockDim.x) Ls[i] = L[i];
-    fp12_set_one(f, t);
-    __syncthreads();
-    uint32_t s = 0;
-#pragma unroll 1
-    for (int i = 62; i >= 0; i--) {
-        fp12_mul_lds(f, f, f);
-        fp12_mul_lds(f, f, Ls + 12 * s++);
-        if ((kZAbs >> i) & 1u) fp12_mul_lds(f, f, Ls + 12 * s++);
+    if (blockIdx.x > 0) {
+        const uint32_t k = (blockIdx.x - 1) * (kPairThreads / 4) + t / 4;
+        if (k < npts && !g1_in_subgroup(pts[k], t & 3u)) atomicOr(err, kVfyNotInGroup);
+        return;
     }
-    // ---- easy part: f^((p^6 - 1)(p^2 + 1))
-    fp12_copy(g, f);
-    fp12_conj_inplace(g);   // conj(f)
+    for (uint32_t i = t; i < kPairGroups * 12; i += blockDim.x) Ls[i] = L[i];
+    if (t < 2) unit[t] = t == 0 ? fp_one() : fp_zero();
+    __syncthreads();
+    Fp *const f = R[rF], *const g = R[rG], *const h = R[rH], *const A = R[rA];
+    if (t < 12) f[t] = Ls[t];
+    __syncthreads();
+#pragma unroll 1
+    for (int i = 62 - (int)kGroupIters; i >= 0; i--) {
+        const bool last = i == 0 || (62 - i) % (int)kGroupIters == (int)kGroupIters - 1;  // of its group
+#pragma unroll 1
+        for (int k = 0; k < (last ? 2 : 1); k++)
+            fp12_mul_lds(f, f, k == 0 ? f : Ls + 12 * ((62 - i) / (int)kGroupIters));
+    }
+    fp12_conj(g, f);
     fp12_mul_lds(h, f, g);  // f conj(f) = n0 + n1 w^2 + n2 w^4 (in Fp6)
     fp12_reduce(h);
-    if (t == 0) {
-        const Fp2 n0 = {h[0], h[1]}, n1 = {h[4], h[5]}, n2 = {h[8], h[9]};
-        // inverse in Fp2[v]/(v^3 - xi), v = w^2
-        const Fp2 c0 = fp2_sub(fp2_sqr(n0), fp2_mul_xi(fp2_mul(n1, n2)));
-        const Fp2 c1 = fp2_sub(fp2_mul_xi(fp2_sqr(n2)), fp2_mul(n0, n1));
-        const Fp2 c2 = fp2_sub(fp2_sqr(n1), fp2_mul(n0, n2));
-        const Fp2 den = fp2_add(fp2_mul(n0, c0), fp2_mul_xi(fp2_add(fp2_mul(n2, c1), fp2_mul(n1, c2))));
-        const Fp2 di = fp2_inv(den);
-        const Fp2 i0 = fp2_mul(c0, di), i1 = fp2_mul(c1, di), i2 = fp2_mul(c2, di);
-        for (int k = 0; k < 12; k++) h[k] = fp_zero();
-        h[0] = i0.c0;
-        h[1] = i0.c1;
-        h[4] = i1.c0;
-        h[5] = i1.c1;
-        h[8] = i2.c0;
-        h[9] = i2.c1;
+    // its inverse in Fp2[v]/(v^3 - xi), v = w^2, a lane per coefficient:
+    // c0 = n0^2 - xi n1 n2, c1 = xi n2^2 - n0 n1, c2 = n1^2 - n0 n2, over
+    // n0 c0 + xi (n2 c1 + n1 c2)
+    if (t < 3) {
+        const auto n = [&](uint32_t k) { return Fp2{h[4 * k], h[4 * k + 1]}; };
+        const auto xi_if = [](bool c, const Fp2 &v) {
+            const Fp2 x = fp2_mul_xi(v);
+            return Fp2{fp_select(c, x.c0, v.c0), fp_select(c, x.c1, v.c1)};
+        };
+        const uint32_t p = (3 - t) % 3;  // n0, n2, n1 beside c0, c1, c2
+        const Fp2 sq = xi_if(t == 1, fp2_sqr(n(p)));
+        const Fp2 pr = xi_if(t == 0, fp2_mul(n(t == 0 ? 1 : 0), n(t == 1 ? 1 : 2)));
+        const Fp2 c = fp2_sub(sq, pr);
+        const Fp2 term = xi_if(t > 0, fp2_mul(n(p), c));
+        Fp2 den = term;
+#pragma unroll
+        for (int i = 0; i < kFpLimbs; i++) {  // the three lanes' terms (sums of few, then reduced)
+            den.c0.v[i] = __shfl(term.c0.v[i], 0) + __shfl(term.c0.v[i], 1);
+            den.c1.v[i] = __shfl(term.c1.v[i], 0) + __shfl(term.c1.v[i], 1);
+        }
+        den = {fp_norm_wide(den.c0), fp_norm_wide(den.c1)};
+#pragma unroll
+        for (int i = 0; i < kFpLimbs; i++) {
+            den.c0.v[i] += __shfl(term.c0.v[i], 2);
+            den.c1.v[i] += __shfl(term.c1.v[i], 2);
+        }
+        den = {fp_norm_wide(den.c0), fp_norm_wide(den.c1)};
+        const Fp2 r = fp2_mul(c, fp2_inv(den));
+        h[4 * t] = r.c0;
+        h[4 * t + 1] = r.c1;
+        h[4 * t + 2] = fp_zero();
+        h[4 * t + 3] = fp_zero();
     }
     __syncthreads();
-    fp12_mul_lds(h, g, h);  // 1/f = conj(f) / (f conj(f))
-    fp12_mul_lds(g, g, h);  // f^(p^6 - 1)
-    fp12_frob2(h, g);
-    fp12_mul_lds(f, h, g);  // F = f^((p^6 - 1)(p^2 + 1)), in the cyclotomic subgroup
-    // ---- hard part: F^(3 (p^4 - p^2 + 1)/r); conj is the inverse here
-    fp12_pow_zabs(A, f);
-    fp12_mul_lds(A, A, f);
-    fp12_conj_inplace(A);  // A = F^(z - 1)
-    fp12_pow_zabs(B, A);
-    fp12_mul_lds(B, B, A);
-    fp12_conj_inplace(B);  // B = A^(z - 1)
-    fp12_pow_zabs(C, B);
-    fp12_conj_inplace(C);
-    fp12_frob1(g, B);
-    fp12_mul_lds(C, C, g);  // C = B^(z + p)
-    fp12_pow_zabs(D, C);
-    fp12_pow_zabs(A, D);    // C^(z^2)
-    fp12_frob2(g, C);
-    fp12_mul_lds(A, A, g);
-    fp12_copy(g, C);
-    fp12_conj_inplace(g);
-    fp12_mul_lds(A, A, g);  // C^(z^2 + p^2 - 1)
-    fp12_mul_lds(g, f, f);
-    fp12_mul_lds(g, g, f);  // F^3
-    fp12_mul_lds(A, A, g);
+    const CycTerm term = kCycTable.t[t < 96 ? t : 95];
+#pragma unroll 1
+    for (uint32_t k = 0; k < sizeof(kFinalSteps) / sizeof(PairStep); k++) {
+        const PairStep st = kFinalSteps[k];
+        Fp *d = R[st.d];
+        const Fp *a = R[st.a], *b = R[st.b];
+        switch (st.op) {
+            case kStepMul: fp12_mul_lds(d, a, b); break;
+            case kStepPow: fp12_pow_zabs(d, a, unit, term); break;
+            case kStepConj: fp12_conj(d, a); break;
+            case kStepFrob1: fp12_frob1(d, a); break;
+            default: fp12_frob2(d, a); break;
+        }
+    }
     if (t == 0) ok = 1;
     __syncthreads();
     if (t < 12) {
@@ -317,10 +389,12 @@ hipError_t launch_g2_lines(Fp2 *lines, const G2A *qs, uint32_t nq, uint32_t *err
 }
 
 hipError_t launch_pairing_check(uint32_t *status, Fp *out12, Fp *L, const Fp2 *lines1, const Fp2 *lines2,
-                                const G1A *p1, const G1A *p2, bool neg2, hipStream_t s) {
-    hipLaunchKernelGGL(k_pair_lines, dim3(kPairSteps), dim3(kPairThreads), 0, s, L, lines1, lines2, p1, p2,
+                                const G1A *p1, const G1A *p2, bool neg2, const G1A *pts, uint32_t npts,
+                                uint32_t *err, hipStream_t s) {
+    hipLaunchKernelGGL(k_pair_lines, dim3(kPairGroups), dim3(kPairThreads), 0, s, L, lines1, lines2, p1, p2,
                        neg2 ? 1u : 0u);
-    hipLaunchKernelGGL(k_pair_final, dim3(1), dim3(kPairThreads), 0, s, status, out12, L);
+    hipLaunchKernelGGL(k_pair_final, dim3(1 + (uint32_t)blocks_for(npts * 4ull, kPairThreads)), dim3(kPairThreads), 0, s,
+                       status, out12, L, pts, npts, err);
     return hipGetLastError();
 }
 

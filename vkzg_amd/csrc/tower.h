@@ -110,6 +110,17 @@ VKZG_DEV Fp fp_shfl_xor(const Fp &v, int mask) {
     return r;
 }
 
+// DPP within rows of 16 lanes: lane l takes the value of lane l + n (kRowShl + n,
+// lanes past the row's end 0) or l - n mod 16 (kRowRor + n).
+constexpr int kRowShl = 0x100, kRowRor = 0x120;
+template <int CTRL>
+VKZG_DEV Fp fp_row_dpp(const Fp &v) {
+    Fp r;
+#pragma unroll
+    for (int i = 0; i < kFpLimbs; i++) r.v[i] = __builtin_amdgcn_mov_dpp(v.v[i], CTRL, 0xf, 0xf, true);
+    return r;
+}
+
 constexpr uint32_t kFp12Threads = 192;  // lanes an Fp12 product uses (blockDim.x >= this)
 
 // dst = a * b for Fp12 values held in LDS (12 Fp each).  Every thread of the
@@ -119,12 +130,13 @@ constexpr uint32_t kFp12Threads = 192;  // lanes an Fp12 product uses (blockDim.
 // a_{m1} (times xi when m1 + m2 >= 6: (x + y u) xi = (x - y) + (x + y) u, an
 // N2 operand) and b_{m2}, m2 = M - m1 mod 6, component by component, DPP quad
 // broadcasts give every lane the four products, lane 0 of the quad forms the
-// real and lane 1 the imaginary part of the term, and an xor tree over the
-// group's eight quads adds the six terms.  A term's limbs are below 2^30 and
+// real and lane 1 the imaginary part of the term, and a tree over the group's
+// eight quads (rotations of a row of 16 lanes by DPP, then the other row) adds
+// the six terms.  A term's limbs are below 2^30 and
 // the sum of two just fits 32 bits, so the tree takes one carry pass after its
 // first level and one at its end.  The result is 12 products of magnitude
-// c p: operands of up to 9.3p give c <= 2 * 9.3 * 9.3 / 630 + 1/2 < 0.775 and so
-// a result below 9.3p again, a valid operand of the next product.
+// c p: operands of up to 12.3p give c <= 2 * 12.3 * 12.3 / 630 + 1/2 < 0.981 and
+// so a result below 11.8p, a valid operand of the next product or square.
 // Operands and result stay in LDS; the partial sums never leave registers.
 __device__ __forceinline__ void fp12_mul_lds(Fp *dst, const Fp *a, const Fp *b) {
     const uint32_t t = threadIdx.x;
@@ -147,10 +159,100 @@ __device__ __forceinline__ void fp12_mul_lds(Fp *dst, const Fp *a, const Fp *b) 
     const Fp p10 = fp_quad_bcast<2>(prod), p11 = fp_quad_bcast<3>(prod);
     Fp v = fp_select(q == 0, fp_sub_raw(p00, p11), fp_add_raw(p01, p10));
     if (!term || q > 1) v = fp_zero();
-    v = fp_norm_wide(fp_add_raw(v, fp_shfl_xor(v, 4)));
-    v = fp_add_raw(v, fp_shfl_xor(v, 8));
+    v = fp_norm_wide(fp_add_raw(v, fp_row_dpp<kRowRor + 4>(v)));
+    v = fp_add_raw(v, fp_row_dpp<kRowRor + 8>(v));
     v = fp_add_raw(v, fp_shfl_xor(v, 16));
     if (t < kFp12Threads && (t % 32) < 2) dst[2 * M + (t % 32)] = fp_norm_wide(v);
+    __syncthreads();
+}
+
+// Squares in the cyclotomic subgroup (Granger and Scott, "Faster squaring in the
+// cyclotomic subgroup of sixth degree extensions", 2010): with a = A + B w + C w^2
+// over Fp4 = Fp2[s]/(s^2 - xi), s = w^3, and bar: s -> -s,
+//   a^2 = (3 A^2 - 2 bar A) + (3 s C^2 + 2 bar B) w + (3 B^2 - 2 bar C) w^2.
+// Each of the 12 coefficients is then 3 times a sum of at most five products of
+// two coefficients of a (one of them doubled in some), plus or minus 2 z for one
+// coefficient z: eight lanes per coefficient, the sum of lanes 0 to 2 and 4 to 6
+// and, on lane 7, z times 1, which keeps z from growing -- 96 lanes, plain products
+// of values in LDS, and DPP within a row where the general product has 144 lanes,
+// operands to prepare and a tree over 32 lanes.  A square takes 1.6 us
+// where the general product takes 2.2.
+struct CycTerm {
+    uint8_t a, b;      // operands: 0..11 a coefficient, 12 one, 13 zero
+    uint8_t dbl, neg;  // +-(2a or a) b
+};
+struct CycTable {
+    CycTerm t[96];
+};
+constexpr CycTable cyc_table() {
+    CycTable r{};
+    for (int o = 0; o < 12; o++) {
+        const int m = o / 2, e = o % 2;
+        // x, y: the two coefficients squared or multiplied
+        const int x0 = 2 * (m == 0 || m == 3 ? 0 : (m == 1 || m == 4 ? 2 : 1)), x1 = x0 + 1;
+        const int y0 = x0 + 6, y1 = y0 + 1;
+        CycTerm *t = r.t + 8 * o;
+        for (int k = 0; k < 8; k++) t[k] = {13, 13, 0, 0};
+        t[7] = {(uint8_t)o, 12, 0, 0};
+        auto set = [&](int k, int a, int b, int dbl, int neg) {
+            t[k] = {(uint8_t)a, (uint8_t)b, (uint8_t)dbl, (uint8_t)neg};
+        };
+        if (m % 2 == 0) {  // x^2 + xi y^2 (xi y^2: (Re - Im, Re + Im) of y^2)
+            if (e == 0) set(0, x0, x0, 0, 0), set(1, x1, x1, 0, 1), set(5, y0, y1, 1, 1);
+            else set(0, x0, x1, 1, 0), set(5, y0, y1, 1, 0);
+            set(2, y0, y0, 0, 0), set(4, y1, y1, 0, 1);
+        } else if (m != 1) {  // 2 x y
+            if (e == 0) set(0, x0, y0, 1, 0), set(1, x1, y1, 1, 1);
+            else set(0, x0, y1, 1, 0), set(1, x1, y0, 1, 0);
+        } else {  // 2 xi x y
+            set(0, x0, y0, 1, 0), set(1, x1, y1, 1, 1);
+            set(4, x0, y1, 1, e ? 0 : 1), set(5, x1, y0, 1, e ? 0 : 1);
+        }
+    }
+    return r;
+}
+static __constant__ CycTable kCycTable = cyc_table();
+
+// a <- a^2 for a in the cyclotomic subgroup, in LDS; unit: {one, zero} there.
+// Every thread of the block calls it; t: this thread's term (unused from 96 up).
+// With coefficients of up to 12.3p a result is below 10.8p: at most 3 (3 or 4
+// times 12.3^2 / 630) for the exact values of the sums (|x0^2 - x1^2| <= z^2,
+// |y0^2 - y1^2 -+ 2 y0 y1| <= 2 z^2, twice |x y xi| <= 4 z^2), 3 (5/2 or 4/2) for the
+// products' roundings and 2 (12.3 / 630 + 1/2) for z.
+__device__ __forceinline__ void fp12_cyc_sqr_lds(Fp *a, const Fp *unit, const CycTerm &term) {
+    const uint32_t t = threadIdx.x, o = (t / 8) % 12, m = o / 2;
+    Fp x = *(term.a < 12 ? a + term.a : unit + (term.a - 12));
+    const Fp y = *(term.b < 12 ? a + term.b : unit + (term.b - 12));
+    __syncthreads();
+    if (t < 96) {
+#pragma unroll
+        for (int i = 0; i < kFpLimbs; i++) x.v[i] = (int32_t)((uint32_t)x.v[i] << term.dbl);
+        const Fp p = fp_mul(x, y);
+        const Fp s = fp_cond_neg(p, term.neg != 0);
+        // lanes 0 and 4: the sums of three; lane 0 then takes lane 4's and lane 7's product
+        const Fp s3 = fp_add_raw(fp_add_raw(s, fp_row_dpp<kRowShl + 1>(s)), fp_row_dpp<kRowShl + 2>(s));
+        const Fp s6 = fp_row_dpp<kRowShl + 4>(s3), z = fp_row_dpp<kRowShl + 7>(p);
+        const int32_t G = m % 2 ? 2 : -2;
+        if ((t & 7u) == 0) {
+            const int32_t three = fp_hidden(3);
+            int64_t acc = 0;
+            Fp r;
+#pragma unroll
+            for (int i = 0; i < kFpLimbs; i++) {
+                fp_mac(acc, s3.v[i], three);
+                fp_mac(acc, s6.v[i], three);
+                fp_mac(acc, z.v[i], G);
+                if (i + 1 < kFpLimbs) {
+                    r.v[i] = fp_digit((uint32_t)acc);
+                    acc = (acc + (1 << (kFpBits - 1))) >> kFpBits;
+                    fp_hide(acc);
+                } else {
+                    r.v[i] = (int32_t)acc;
+                }
+            }
+            a[o] = r;
+        }
+    }
     __syncthreads();
 }
 

@@ -8,11 +8,12 @@
 // A verification call:
 //   host    argument checks, commitment deduplication, grouping of cells by
 //           commitment and by cell index, pinned staging, one H2D copy;
-//   device  decompression of commitments and proofs and parsing of cells,
-//           with the G1 subgroup checks on a second stream;
+//   device  decompression of commitments and proofs and parsing of cells (and,
+//           for large batches, the G1 subgroup checks);
 //   host    the Fiat-Shamir challenge (SHA-256 over every input), computed
 //           while the device works;
-//   device  r^k, interpolation sums, the two MSMs and the pairing check;
+//   device  r^k, interpolation sums, the two MSMs and the pairing check (with
+//           the subgroup checks of smaller batches in the same launch);
 //   host    one 8-byte readback (verdict, error bits).
 #include <algorithm>
 #include <cstring>
@@ -46,8 +47,6 @@ struct VerifyState {
     size_t dev_bytes = 0;
     uint8_t *host = nullptr;
     size_t host_bytes = 0;
-    hipStream_t side = nullptr;
-    hipEvent_t fork = nullptr, join = nullptr;
 
     void ensure(size_t dbytes, size_t hbytes) {
         if (dbytes > dev_bytes) {
@@ -65,18 +64,9 @@ struct VerifyState {
             host_bytes = hbytes;
         }
     }
-    void streams() {
-        if (side) return;
-        ck(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
-        ck(hipEventCreateWithFlags(&fork, hipEventDisableTiming));
-        ck(hipEventCreateWithFlags(&join, hipEventDisableTiming));
-    }
     ~VerifyState() {
         if (dev) (void)hipFree(dev);
         if (host) (void)hipHostFree(host);
-        if (join) (void)hipEventDestroy(join);
-        if (fork) (void)hipEventDestroy(fork);
-        if (side) (void)hipStreamDestroy(side);
         setup.release();
     }
 };
@@ -233,9 +223,8 @@ vkzg_result verify_impl(vkzg_prover *p, int *ok, const uint8_t *commitments, con
     const size_t d_rp = dl.take(sizeof(Fr) * (size_t)n), d_part = dl.take(sizeof(Fr) * 64ull * nch);
     const size_t d_agg = dl.take(sizeof(Fr) * 64), d_sc = dl.take(sizeof(Fr) * (size_t)ne);
     const size_t d_pidx = dl.take(4ull * ne), d_mid = dl.take(ne), d_out = dl.take(sizeof(G1A) * 2);
-    const size_t d_L = dl.take(sizeof(Fp) * 12 * kPairSteps), d_msm = dl.take(msm_scratch_bytes(sh));
+    const size_t d_L = dl.take(sizeof(Fp) * 12 * kPairGroups), d_msm = dl.take(msm_scratch_bytes(sh));
     v.ensure(dl.size, hl.size);
-    v.streams();
     uint8_t *H = v.host;
     uint8_t *D = static_cast<uint8_t *>(v.dev);
     for (uint32_t j = 0; j < u; j++) std::memcpy(H + h_pts + 48ull * j, commitments + 48ull * uniq[j], 48);
@@ -258,11 +247,14 @@ vkzg_result verify_impl(vkzg_prover *p, int *ok, const uint8_t *commitments, con
     ck(hipMemsetAsync(res, 0, 16, s));
     ck(launch_vfy_points(pts, D + h_pts, u + n32, p->srs, 64, res + 1, s));
     ck(launch_vfy_cells(ev, D + h_cells, n32, res + 1, s));
-    // G1 membership of commitments and proofs, beside the rest of the pipeline
-    ck(hipEventRecord(v.fork, s));
-    ck(hipStreamWaitEvent(v.side, v.fork, 0));
-    ck(launch_vfy_subgroup(pts, u + n32, res + 1, v.side));
-    ck(hipEventRecord(v.join, v.side));
+    // G1 membership of commitments and proofs: with the pairing while a quad per
+    // point is at most one wave per SIMD (16,384 points), a third of its time;
+    // larger batches check it here, behind the host's hash of the cells, which
+    // takes 1 us per cell.  A stream of its own had no effect to count on: the
+    // runtime may put it on the hardware queue of this one.
+    const uint32_t npts = u + n32;
+    const bool with_pairing = npts * 4ull <= (uint64_t)p->cus * 4 * 64;
+    if (!with_pairing) ck(launch_vfy_subgroup(pts, npts, res + 1, s));
 
     uint32_t r[8];
     challenge(r, uniq, cidx, cell_indices, commitments, cells, proofs, n);
@@ -280,8 +272,7 @@ vkzg_result verify_impl(vkzg_prover *p, int *ok, const uint8_t *commitments, con
     }
     // e(sum r^k pi_k, [tau^64]G2) e(-RL, G2) == 1
     ck(launch_pairing_check(res, nullptr, reinterpret_cast<Fp *>(D + d_L), v.lines, v.lines + 2 * kPairSteps,
-                            out, out + 1, true, s));
-    ck(hipStreamWaitEvent(s, v.join, 0));
+                            out, out + 1, true, pts, with_pairing ? npts : 0, res + 1, s));
     ck(hipMemcpyAsync(H + h_res, res, 8, hipMemcpyDeviceToHost, s));
     ck(hipStreamSynchronize(s));
     uint32_t rr[2];
@@ -525,7 +516,7 @@ vkzg_result vkzg_amd_debug_pairing(vkzg_prover *p, uint8_t *out, const uint8_t *
             G1A *P = tmp.dalloc<G1A>(2);
             G2A *Q = tmp.dalloc<G2A>(1);
             Fp2 *lines = tmp.dalloc<Fp2>(2 * kPairSteps);
-            Fp *L = tmp.dalloc<Fp>(12 * kPairSteps);
+            Fp *L = tmp.dalloc<Fp>(12 * kPairGroups);
             Fp *f = tmp.dalloc<Fp>(12);
             uint32_t *w = tmp.dalloc<uint32_t>(4);
             Fp *hf = tmp.halloc<Fp>(12);
@@ -538,7 +529,7 @@ vkzg_result vkzg_amd_debug_pairing(vkzg_prover *p, uint8_t *out, const uint8_t *
                 ck(launch_vfy_points(P, d1, 1, nullptr, 0, w + 1, s));
                 ck(launch_g2_decompress(Q, w + 2, d2, 1, w + 1, s));
                 ck(launch_g2_lines(lines, Q, 1, w + 1, s));
-                ck(launch_pairing_check(w, f, L, lines, lines, P, P + 1, false, s));
+                ck(launch_pairing_check(w, f, L, lines, lines, P, P + 1, false, nullptr, 0, nullptr, s));
                 ck(launch_fp_canonical(f, 12, s));
                 ck(hipMemcpyAsync(hf, f, sizeof(Fp) * 12, hipMemcpyDeviceToHost, s));
                 ck(hipMemcpyAsync(hw, w, 16, hipMemcpyDeviceToHost, s));
