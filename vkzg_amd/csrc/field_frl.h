@@ -63,6 +63,11 @@ constexpr uint32_t R2[9] = {0x0a71b3c0u, 0x1d32207eu, 0x1663d999u, 0x1c5abc93u, 
 // 2^266 mod r: one product takes x 2^256 (the 8 x 32-bit Montgomery form) to x 2^261
 constexpr uint32_t FROM_R256[9] = {0x1ffff72bu, 0x000046a7u, 0x1f5f3540u, 0x0ce3021cu, 0x118f3661u,
                                    0x008176cbu, 0x054e487cu, 0x102e8190u, 0x001e092eu};
+// 2^256 mod r: one product takes x 2^261 to x 2^256
+constexpr uint32_t TO_R256[9] = {0x1ffffffeu, 0x0000000fu, 0x00d20080u, 0x096ff400u, 0x04ff5588u,
+                                 0x07f7f65eu, 0x15be6631u, 0x0b3598a0u, 0x001824b1u};
+// 2^261 / 4096: 1 / 4096 in Montgomery form
+constexpr uint32_t INV_4096_M[9] = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0x00020000u};
 // 2^261 mod r in 8 x 32-bit limbs: fr_mul(x 2^256, TO_R261) = x 2^261
 constexpr uint32_t TO_R261[8] = {0xffffffbau, 0x00000045u, 0x0072d846u, 0x1a25272eu,
                                  0x5dbeee8bu, 0xfe2eedcdu, 0x9eefbe41u, 0x4d043f42u};

@@ -104,9 +104,12 @@ hipError_t launch_phase_b_scalars(Fr *out, const Fr *roots, hipStream_t s);
 // With `splits` > 1 it writes `splits` scalar sets per blob,
 // scal[blob][m][j][i] = scal[blob][0][j][i] * 2^(8 start_m) mod r (each as
 // sign and magnitude).
-hipError_t launch_fk20_scalars(Fr *scal, const uint8_t *blobs, uint64_t blob_stride, uint32_t *err,
-                               const Fr *roots, const Fr *roots_inv, uint32_t *queue, Fr *coeffs,
-                               uint32_t splits, uint32_t nblobs, WindowPlan plan, hipStream_t s);
+// roots, roots_inv: FrL tables; scratch: kScalarScratch bytes per blob, for the
+// time of the launch.
+constexpr size_t kScalarScratch = 4096 * 32 + 16 * 4;
+hipError_t launch_fk20_scalars(Fr *scal, const uint8_t *blobs, uint64_t blob_stride, uint32_t *err, void *scratch,
+                               const uint4 *roots, const uint4 *roots_inv, uint32_t *queue, Fr *coeffs,
+                               uint32_t splits, uint32_t nblobs, uint32_t cus, WindowPlan plan, hipStream_t s);
 // nblobs * splits * nj MSMs of 64 terms (nj, a multiple of 64: bases of a blob).
 // Persistent: `grid` blocks drain the (64 MSMs, share) items from queue[0];
 // an MSM has parts * groups shares (parts divides 64): part[msm][share].

@@ -569,8 +569,11 @@ void proofs_range(vkzg_prover *p, WorkSet &ws, uint32_t off, uint32_t nb, uint8_
     Fp *prefix = ws.prefix + off * npos;
     G1X *buckets = ws.buckets + (size_t)off * 128 * kBuckets, *cvals = ws.cvals + (size_t)off * 128;
     if (steps != kAfterScalars) {
-        ck(launch_fk20_scalars(scal, d_blobs, blob_stride, err, p->roots, p->roots_inv, queue, coeffs,
-                               tn.ladder_splits, nb, tab.plan(), s));
+        // the buckets' memory, which phase B fills later, holds the transform's intermediates
+        static_assert(sizeof(G1X) * 128 * kBuckets >= kScalarScratch, "a blob's buckets must hold its intermediates");
+        const RecTables rt = rec_tables(p);
+        ck(launch_fk20_scalars(scal, d_blobs, blob_stride, err, buckets, rt.roots4, rt.roots_inv4, queue, coeffs,
+                               tn.ladder_splits, nb, p->cus, tab.plan(), s));
         clk.mark("fk20_scalars");
     }
     if (steps == kScalarsOnly) return;
