@@ -421,16 +421,15 @@ Tuning tuning_for(const vkzg_prover *p, uint32_t nb) {
 
 // Defaults before (or without) autotuning: small batches split the ladder into
 // segments, so that more lanes work on the few chains there are; phase A's
-// shares and the normalisation chunk are fitted to the batch and the chip
-// (groups 0, norm_chunk 0).
+// shares, the lanes of a bucket reduction and the normalisation chunk are fitted
+// to the batch and the chip (groups, reduce_lanes and norm_chunk 0).
 void default_tunings(vkzg_prover *p) {
     static const uint32_t ladder_splits[kTuneClasses] = {4, 2, 1, 1, 1};
-    static const uint32_t reduce_lanes[kTuneClasses] = {64, 64, 32, 16, 4};
     for (int c = 0; c < kTuneClasses; c++) {
         p->tune[c] = Tuning{};
         p->tune[c].groups = 0;
         p->tune[c].ladder_splits = ladder_splits[c];
-        p->tune[c].reduce_lanes = reduce_lanes[c];
+        p->tune[c].reduce_lanes = 0;
         p->tune[c].norm_chunk = 0;
     }
 }
@@ -449,6 +448,19 @@ uint32_t ladder_lanes(uint64_t chains, uint32_t cus) {
 constexpr uint64_t kPhaseBQuadWaves = 8;
 bool phase_b_quad(uint32_t nb, uint32_t cus) {
     return (uint64_t)nb * 128 * kBuckets * 4 <= (uint64_t)cus * 4 * 64 * kPhaseBQuadWaves;
+}
+
+// Lanes per output of the bucket reduction for reduce_lanes 0.  More lanes shorten
+// an output's chain and add work, so: as many as leave at most one wave per SIMD
+// while that is at least 8, then 8 on two waves per SIMD, then 4.  Measured (all
+// stages, ms): 6 blobs 1.20 on 32 lanes, 1.10 on 64; 16 blobs alike on 32 and 64;
+// 21 blobs 1.94 on 8, 1.77 on 16; 64 blobs 4.37 on 16, 4.35 on 8, 4.97 on 4; at 128
+// 8 is ahead of 4, at 256 4 of 8.
+uint32_t fit_reduce_lanes(uint32_t nb, uint32_t cus) {
+    const uint64_t outputs = (uint64_t)nb * 128, simd_lanes = (uint64_t)cus * 4 * 64;
+    for (uint32_t lanes = 64; lanes >= 8; lanes /= 2)
+        if (outputs * lanes <= simd_lanes) return lanes;
+    return outputs * 8 <= 2 * simd_lanes ? 8u : 4u;
 }
 
 // Points per lane of the normalisation for norm_chunk 0: the smallest chunk
@@ -498,7 +510,7 @@ bool tuning_valid(const Tuning &t) {
            t.norm_chunk <= 256 && t.splits >= 1 && t.splits <= (uint32_t)kMaxSplits &&
            (t.rec_waves == 1 || t.rec_waves == 2 || t.rec_waves == 4) && (t.rec_radix == 2 || t.rec_radix == 4 || t.rec_radix == 8) &&
            (t.ladder_splits == 1 || t.ladder_splits == 2 || t.ladder_splits == 4) &&
-           (t.reduce_lanes == 4 || t.reduce_lanes == 8 || t.reduce_lanes == 16 || t.reduce_lanes == 32 ||
+           (t.reduce_lanes == 0 || t.reduce_lanes == 4 || t.reduce_lanes == 8 || t.reduce_lanes == 16 || t.reduce_lanes == 32 ||
             t.reduce_lanes == 64) &&
            (t.window_bits == 0 || (t.window_bits >= kExtraWindowMin && t.window_bits <= kExtraWindowMax));
 }
@@ -612,7 +624,8 @@ void proofs_range(vkzg_prover *p, WorkSet &ws, uint32_t off, uint32_t nb, uint8_
                           tn.force_checked, s));
     }
     clk.mark("phase_b");
-    ck(launch_bucket_reduce(cvals, ws.cval_flags + off * 128, buckets, nb, tn.reduce_lanes, p->cus * 2,
+    const uint32_t reduce_lanes = tn.reduce_lanes ? tn.reduce_lanes : fit_reduce_lanes(nb, p->cus);
+    ck(launch_bucket_reduce(cvals, ws.cval_flags + off * 128, buckets, nb, reduce_lanes, p->cus * 2,
                             ws.queue_r + off, tn.force_checked, s));
     clk.mark("bucket_reduce");
     ck(launch_finalize(d_proofs, cvals, nb, (uint64_t)nb * 256 <= (uint64_t)p->cus * 4 * 64, tn.force_checked, s));
@@ -889,7 +902,7 @@ void autotune(vkzg_prover *p) {
         for (uint32_t g : {1u, 2u, 4u, 5u, 10u, 20u}) { Tuning t = best; t.groups = g; consider(t); }
         if (nb <= 64)
             for (uint32_t m : {2u, 4u}) { Tuning t = best; t.ladder_splits = m; consider(t); }
-        for (uint32_t r : {4u, 16u, 32u, 64u}) { Tuning t = best; t.reduce_lanes = r; consider(t); }
+        for (uint32_t r : {4u, 8u, 16u, 32u, 64u}) { Tuning t = best; t.reduce_lanes = r; consider(t); }
         for (uint32_t b : {1u, 2u}) { Tuning t = best; t.blocks_per_cu = b; consider(t); }
         for (uint32_t ch : {0u, 8u, 16u, 32u, 64u}) { Tuning t = best; t.norm_chunk = ch; consider(t); }
         if (nb >= 8) { Tuning t = best; t.splits = 2; consider(t); }
@@ -1315,8 +1328,10 @@ vkzg_result vkzg_amd_get_tuning(const vkzg_prover *p, size_t num_blobs, vkzg_amd
         std::lock_guard<std::mutex> lock(p->tune_mu);
         t = p->tune[tune_class((uint32_t)std::min<size_t>(num_blobs, 0xffffffffu))];
     }
-    if (!t.groups) {  // fitted: the groups a batch of this size takes
-        const uint32_t nb = (uint32_t)std::min<size_t>(num_blobs, p->max_batch);
+    // fitted: what a batch of this size takes
+    const uint32_t nb = (uint32_t)std::min<size_t>(num_blobs, p->max_batch);
+    if (!t.reduce_lanes) t.reduce_lanes = fit_reduce_lanes(nb, p->cus);
+    if (!t.groups) {
         t.groups = phase_a_shape((uint64_t)nb * 128 * t.ladder_splits, 0, phase_a_table(p, t.window_bits).W,
                                  (uint64_t)std::max(p->max_batch, kMinPartialBlobs) * kSlotsPerBlob, p->cus)
                        .groups;
@@ -1345,7 +1360,7 @@ vkzg_result vkzg_amd_set_tuning(vkzg_prover *p, size_t num_blobs, const vkzg_amd
     t.ladder_splits = in->ladder_splits;
     t.reduce_lanes = in->reduce_lanes;
     t.window_bits = in->phase_a_window_bits == p->c ? 0u : in->phase_a_window_bits;
-    if (t.groups == 0 || !tuning_valid(t)) return VKZG_ERR_BADARGS;
+    if (t.groups == 0 || t.reduce_lanes == 0 || !tuning_valid(t)) return VKZG_ERR_BADARGS;
     std::lock_guard<std::mutex> lock(p->mu);
     if (t.window_bits) {  // only a resident smaller table
         if (!p->extra_tables[t.window_bits - kExtraWindowMin].table) return VKZG_ERR_BADARGS;
