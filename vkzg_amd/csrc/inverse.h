@@ -1,7 +1,7 @@
 // Fp inversion by a binary GCD on 28-bit approximations (the "optimized
 // binary GCD" of T. Pornin, 2020, eprint 2020/972), for values in 14 x 28-bit
 // limbs.  Fermat's p - 2 power needs ~570 dependent multiplications; this
-// runs outer iterations of ~1,100 integer instructions each until every lane
+// runs outer iterations of ~1,300 integer instructions each until every lane
 // of the wave is done: 19 to 21 for almost every value, at most 30.  Within an
 // iteration there are no data-dependent branches.
 //
@@ -41,14 +41,28 @@ constexpr int kLimbs = 14;
 constexpr uint32_t kMask = (1u << 28) - 1u;
 constexpr int kOuter = 30;
 
+// acc += x * y as one v_mad_i64_i32.  A limb the compiler knows to be non-negative
+// it multiplies unsigned and corrects for the factor's sign in three more
+// instructions; hidden limbs (no instructions) stay signed.
+VKZG_HD void mac(int64_t &acc, int32_t x, int32_t y) { acc += (int64_t)x * y; }
+VKZG_HD int32_t hidden(int32_t x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("" : "+v"(x));
+#endif
+    return x;
+}
+
 // r = (x f + y g) / 2^28 for non-negative x, y < 2^382 (exact division);
 // returns true when the result is negative.
-VKZG_HD bool lin_shift(uint32_t (&r)[kLimbs], const uint32_t (&x)[kLimbs], const uint32_t (&y)[kLimbs],
+VKZG_HD bool lin_shift(uint32_t (&r)[kLimbs], const int32_t (&x)[kLimbs], const int32_t (&y)[kLimbs],
                        int32_t f, int32_t g) {
-    int64_t c = (int64_t)x[0] * f + (int64_t)y[0] * g;
+    int64_t c = 0;
+    mac(c, x[0], f);
+    mac(c, y[0], g);
     c >>= 28;  // the low 28 bits are zero
     for (int i = 1; i < kLimbs; i++) {
-        c += (int64_t)x[i] * f + (int64_t)y[i] * g;
+        mac(c, x[i], f);
+        mac(c, y[i], g);
         r[i - 1] = (uint32_t)c & kMask;
         c >>= 28;
     }
@@ -58,25 +72,29 @@ VKZG_HD bool lin_shift(uint32_t (&r)[kLimbs], const uint32_t (&x)[kLimbs], const
 
 // r = -r for a value with a signed top limb; the result is non-negative.
 VKZG_HD void negate(uint32_t (&r)[kLimbs]) {
-    int64_t c = 0;
+    int32_t c = 0;
     for (int i = 0; i < kLimbs - 1; i++) {
-        c -= (int64_t)r[i];
+        c -= (int32_t)r[i];
         r[i] = (uint32_t)c & kMask;
         c >>= 28;
     }
-    r[kLimbs - 1] = (uint32_t)(int32_t)(c - (int64_t)(int32_t)r[kLimbs - 1]);
+    r[kLimbs - 1] = (uint32_t)(c - (int32_t)r[kLimbs - 1]);
 }
 
 // r = (u f + v g + q p) / 2^28 with q = -(u f + v g) p^-1 mod 2^28, for signed
 // u, v (limbs 0..12 unsigned, limb 13 signed).
 VKZG_HD void lin_shift_mod(int32_t (&r)[kLimbs], const int32_t (&u)[kLimbs], const int32_t (&v)[kLimbs],
                            int32_t f, int32_t g) {
-    int64_t c = (int64_t)u[0] * f + (int64_t)v[0] * g;
-    const uint32_t q = ((uint32_t)c * cfp::GCD_N0) & kMask;
-    c += (int64_t)q * cfp::GCD_P[0];
+    int64_t c = 0;
+    mac(c, u[0], f);
+    mac(c, v[0], g);
+    const int32_t q = hidden((int32_t)(((uint32_t)c * cfp::GCD_N0) & kMask));
+    mac(c, q, (int32_t)cfp::GCD_P[0]);
     c >>= 28;
     for (int i = 1; i < kLimbs; i++) {
-        c += (int64_t)u[i] * f + (int64_t)v[i] * g + (int64_t)q * cfp::GCD_P[i];
+        mac(c, u[i], f);
+        mac(c, v[i], g);
+        mac(c, q, (int32_t)cfp::GCD_P[i]);
         r[i - 1] = (int32_t)((uint32_t)c & kMask);
         c >>= 28;
     }
@@ -127,39 +145,53 @@ VKZG_HD bool inverse(int32_t (&v)[kLimbs], const uint32_t (&y)[kLimbs]) {
         const int s = len - 30;
         const int li = s / 28, sh = s - 28 * li;
         uint64_t ah = approx(a, li, sh), bh = approx(b, li, sh);
+        // two runs of 14 steps, each with its rows as one word f + 2^16 g (every
+        // step is linear in them, and |f|, |g| <= 2^14 after 14 steps)
         int32_t f0 = 1, g0 = 0, f1 = 0, g1 = 1;
-        for (int j = 0; j < 28; j++) {
-            const bool odd = (ah & 1u) != 0;
-            const bool sw = odd && ah < bh;
-            const uint64_t ta = ah;
-            ah = sw ? bh : ah;
-            bh = sw ? ta : bh;
-            const int32_t tf = f0, tg = g0;
-            f0 = sw ? f1 : f0;
-            f1 = sw ? tf : f1;
-            g0 = sw ? g1 : g0;
-            g1 = sw ? tg : g1;
-            ah -= odd ? bh : 0u;
-            f0 -= odd ? f1 : 0;
-            g0 -= odd ? g1 : 0;
-            ah >>= 1;
-            f1 *= 2;
-            g1 *= 2;
+        for (int half = 0; half < 2; half++) {
+            int32_t r0 = 1, r1 = 1 << 16;
+            for (int j = 0; j < 14; j++) {
+                // a odd: a - b; negative: b takes a, and a the difference's
+                // magnitude (the swap).  Masks instead of selects: a comparison's
+                // lane mask would go through the scalar unit and back.
+                const int64_t odd = -(int64_t)(ah & 1u);
+                const int64_t d = (int64_t)(ah - (bh & (uint64_t)odd));
+                const int64_t neg = d >> 63;
+                bh += (uint64_t)(d & neg);
+                ah = (uint64_t)((d ^ neg) - neg) >> 1;
+                const int32_t rd = r0 - (r1 & (int32_t)odd);
+                r1 = (r1 + (rd & (int32_t)neg)) * 2;
+                r0 = (rd ^ (int32_t)neg) - (int32_t)neg;
+            }
+            const int32_t p0 = (int16_t)r0, p1 = (int16_t)r1;
+            const int32_t q0 = (r0 - p0) >> 16, q1 = (r1 - p1) >> 16;
+            const int32_t tf0 = f0, tg0 = g0;
+            f0 = p0 * tf0 + q0 * f1;
+            g0 = p0 * tg0 + q0 * g1;
+            f1 = p1 * tf0 + q1 * f1;
+            g1 = p1 * tg0 + q1 * g1;
         }
         uint32_t na[kLimbs], nb[kLimbs];
-        if (lin_shift(na, a, b, f0, g0)) {
+        int32_t xa[kLimbs], xb[kLimbs], xu[kLimbs], xv[kLimbs];
+        for (int i = 0; i < kLimbs; i++) {
+            xa[i] = hidden((int32_t)a[i]);
+            xb[i] = hidden((int32_t)b[i]);
+            xu[i] = hidden(u[i]);
+            xv[i] = hidden(v[i]);
+        }
+        if (lin_shift(na, xa, xb, f0, g0)) {
             negate(na);
             f0 = -f0;
             g0 = -g0;
         }
-        if (lin_shift(nb, a, b, f1, g1)) {
+        if (lin_shift(nb, xa, xb, f1, g1)) {
             negate(nb);
             f1 = -f1;
             g1 = -g1;
         }
         int32_t nu[kLimbs], nv[kLimbs];
-        lin_shift_mod(nu, u, v, f0, g0);
-        lin_shift_mod(nv, u, v, f1, g1);
+        lin_shift_mod(nu, xu, xv, f0, g0);
+        lin_shift_mod(nv, xu, xv, f1, g1);
         uint32_t left = 0;
         for (int i = 0; i < kLimbs; i++) {
             a[i] = na[i];
