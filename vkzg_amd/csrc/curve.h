@@ -422,6 +422,15 @@ VKZG_DEV G1X g1x_neg(const G1X &p) {
 
 // --------------------------------------------------------------- encoding
 
+// The words of a point that is not the identity: canonical x, y > (p-1)/2.
+VKZG_DEV void g1a_compressed_words(uint32_t *w, const FpU &x, bool y_large) {
+    uint32_t xw[12];
+    fp_to_words(xw, x);
+    xw[11] |= y_large ? 0xa0000000u : 0x80000000u;
+#pragma unroll
+    for (int i = 0; i < 12; i++) w[i] = __builtin_bswap32(xw[11 - i]);
+}
+
 // Affine (Montgomery) -> 48-byte ZCash compressed encoding as 12 big-endian
 // words: x big-endian, 0x80 compressed flag, 0x20 when y > (p-1)/2, identity
 // = 0xc0 followed by zeros (k_compress_proofs.comp:21-46).
@@ -432,17 +441,7 @@ VKZG_DEV_CALL void g1a_compress_words(uint32_t *w, const G1A &p) {
         for (int i = 1; i < 12; i++) w[i] = 0;
         return;
     }
-    const FpU x = fp_to_canonical(p.x);
-    const FpU y = fp_to_canonical(p.y);
-    uint32_t xw[12];
-    fp_to_words(xw, x);
-#pragma unroll
-    for (int i = 0; i < 12; i++) w[11 - i] = xw[i];
-    uint32_t flags = 0x80000000u;
-    if (fp_is_lex_largest(y)) flags |= 0x20000000u;
-    w[0] |= flags;
-#pragma unroll
-    for (int i = 0; i < 12; i++) w[i] = __builtin_bswap32(w[i]);
+    g1a_compressed_words(w, fp_to_canonical(p.x), fp_is_lex_largest(fp_to_canonical(p.y)));
 }
 
 // 48-byte ZCash compressed encoding (src: its 12 words as stored, 4-byte
