@@ -96,6 +96,22 @@ hipError_t launch_table_multiples(G1AT *table, const G1A *pw, uint32_t n, Window
                                   Fp *prefix, hipStream_t s);
 hipError_t launch_phase_b_scalars(Fr *out, const Fr *roots, hipStream_t s);
 
+// ----------------------------------------------------------------- copies
+// Up to two copies between pinned host memory (hipHostMalloc) and device memory
+// in one kernel; addresses and sizes are multiples of 4 bytes.  For transfers
+// below kKernelCopyMax, where the host side is a single memcpy too (larger ones go
+// out in slices beside the copy threads): a copy engine's hand-over costs about 10
+// us on either side of a transfer that takes 5 to 10, and two pieces are two
+// transfers.  Recovery of one blob, 256 KiB each way and its map: 139 us with copy
+// engines, 116 with two of these kernels.
+struct CopyPart {
+    void *dst = nullptr;
+    const void *src = nullptr;
+    size_t bytes = 0;
+};
+constexpr size_t kKernelCopyMax = (size_t)1 << 20;
+hipError_t launch_copy(const CopyPart &a, const CopyPart &b, hipStream_t s);
+
 // ----------------------------------------------------------------- proofs
 // Blob b is read at blobs + b * blob_stride.  Also clears queue[0], the tile
 // counter of the phase-A launch that follows, and, when coeffs is non-null,

@@ -760,13 +760,26 @@ size_t copy_slice(size_t bytes) {
     return std::max(kMinSlice, std::min(kMaxSlice, s));
 }
 
-// host (pageable) -> pinned staging -> dev, enqueued on s.
-void stage_upload(vkzg_prover *p, uint8_t *dev, uint8_t *pinned, const uint8_t *host, size_t bytes, hipStream_t s) {
-    if (bytes < kPooledCopyMin) {
-        std::memcpy(pinned, host, bytes);
-        ck(hipMemcpyAsync(dev, pinned, bytes, hipMemcpyHostToDevice, s));
+// Up to two pinned <-> device copies enqueued on s: small ones by one kernel.
+void enqueue_copies(const CopyPart &a, const CopyPart &b, hipMemcpyKind kind, hipStream_t s) {
+    if (a.bytes < kKernelCopyMax && b.bytes < kKernelCopyMax) {
+        ck(launch_copy(a, b, s));
         return;
     }
+    for (const CopyPart *c : {&a, &b})
+        if (c->bytes) ck(hipMemcpyAsync(c->dst, c->src, c->bytes, kind, s));
+}
+
+// host (pageable) -> pinned staging -> dev, enqueued on s; `more`: a pinned ->
+// device copy that goes along.
+void stage_upload(vkzg_prover *p, uint8_t *dev, uint8_t *pinned, const uint8_t *host, size_t bytes, hipStream_t s,
+                  const CopyPart &more) {
+    if (bytes < kPooledCopyMin) {
+        std::memcpy(pinned, host, bytes);
+        enqueue_copies(CopyPart{dev, pinned, bytes}, more, hipMemcpyHostToDevice, s);
+        return;
+    }
+    enqueue_copies(more, CopyPart{}, hipMemcpyHostToDevice, s);
     const size_t slice = copy_slice(bytes);
     std::atomic<bool> failed{false};
     p->copiers.run((bytes + slice - 1) / slice, [&](size_t k) {
@@ -778,9 +791,12 @@ void stage_upload(vkzg_prover *p, uint8_t *dev, uint8_t *pinned, const uint8_t *
 }
 
 // dev -> pinned staging, enqueued on s in slices with an event behind each
-// (small ones whole, with one event).
-void start_download(vkzg_prover *p, uint8_t *pinned, const uint8_t *dev, size_t bytes, hipStream_t s) {
+// (small ones whole, with one event); `more`: a device -> pinned copy that goes
+// along, ahead of the first event.
+void start_download(vkzg_prover *p, uint8_t *pinned, const uint8_t *dev, size_t bytes, hipStream_t s,
+                    const CopyPart &more = CopyPart{}) {
     const size_t slice = bytes < kPooledCopyMin ? bytes : copy_slice(bytes);
+    if (bytes >= kPooledCopyMin) enqueue_copies(more, CopyPart{}, hipMemcpyDeviceToHost, s);
     size_t k = 0;
     for (size_t off = 0; off < bytes; off += slice, k++) {
         if (k == p->download_ev.size()) {
@@ -788,7 +804,10 @@ void start_download(vkzg_prover *p, uint8_t *pinned, const uint8_t *dev, size_t 
             ck(hipEventCreateWithFlags(&e, hipEventDisableTiming));
             p->download_ev.push_back(e);
         }
-        ck(hipMemcpyAsync(pinned + off, dev + off, std::min(slice, bytes - off), hipMemcpyDeviceToHost, s));
+        if (bytes < kPooledCopyMin)
+            enqueue_copies(CopyPart{pinned, dev, bytes}, more, hipMemcpyDeviceToHost, s);
+        else
+            ck(hipMemcpyAsync(pinned + off, dev + off, std::min(slice, bytes - off), hipMemcpyDeviceToHost, s));
         ck(hipEventRecord(p->download_ev[k], s));
     }
 }
@@ -1122,8 +1141,8 @@ vkzg_result vkzg_compute_proofs_batch(vkzg_prover *p, uint8_t *proofs, const uin
             p->last_splits = tn.splits;
             enqueue_proofs(p, p->ws, p->streams, p->ws.proofs, p->ws.blobs, nb, s, clk, tn,
                            &p->graphs);
-            ck(hipMemcpyAsync(p->h_err, p->ws.err, nb * 4, hipMemcpyDeviceToHost, s));
-            ck(hipMemcpyAsync(p->h_out, p->ws.proofs, nb * kProofBytes, hipMemcpyDeviceToHost, s));
+            enqueue_copies(CopyPart{p->h_err, p->ws.err, nb * 4}, CopyPart{p->h_out, p->ws.proofs, nb * kProofBytes},
+                           hipMemcpyDeviceToHost, s);
             ck(hipStreamSynchronize(s));
             clk.finish();
             for (uint32_t b = 0; b < nb; b++)
@@ -1150,9 +1169,9 @@ vkzg_result vkzg_recover_cells_batch(vkzg_prover *p, uint8_t *cells_out, const u
             const uint8_t *pm = cell_present + done * 128;
             if (!chunk_missing_ok(pm, nb)) return VKZG_ERR_BADARGS;
             hipStream_t s = p->stream;
-            stage_upload(p, p->ws.cells, p->h_in, cells + done * kCellsBytes, nb * kCellsBytes, s);
             std::memcpy(p->h_present, pm, nb * 128);
-            ck(hipMemcpyAsync(p->ws.present, p->h_present, nb * 128, hipMemcpyHostToDevice, s));
+            stage_upload(p, p->ws.cells, p->h_in, cells + done * kCellsBytes, nb * kCellsBytes, s,
+                         CopyPart{p->ws.present, p->h_present, nb * 128});
             StageClock clk(p, s, true);
             const Tuning tn = tuning_for(p, nb);
             p->last_splits = tn.splits;
@@ -1192,14 +1211,15 @@ vkzg_result vkzg_amd_compute_cells_and_proofs(vkzg_prover *p, uint8_t *cells, ui
                 // while the proofs are computed.
                 hipStream_t c = p->copy_stream;
                 ck(hipStreamWaitEvent(c, p->results_ready, 0));
-                ck(hipMemcpyAsync(p->h_err, p->ws.err, nb * 4, hipMemcpyDeviceToHost, c));
-                start_download(p, p->h_out, p->ws.cells_out, nb * kCellsBytes, c);
+                start_download(p, p->h_out, p->ws.cells_out, nb * kCellsBytes, c,
+                               CopyPart{p->h_err, p->ws.err, nb * 4});
                 // behind the flags: the first slice
                 if (hipEventSynchronize(p->download_ev[0]) != hipSuccess) throw HipFail{};
             } else {
-                ck(hipMemcpyAsync(p->h_err, p->ws.err, nb * 4, hipMemcpyDeviceToHost, s));
+                enqueue_copies(CopyPart{p->h_err, p->ws.err, nb * 4}, CopyPart{}, hipMemcpyDeviceToHost, s);
             }
-            if (proofs) ck(hipMemcpyAsync(p->h_proofs, p->ws.proofs, nb * kProofBytes, hipMemcpyDeviceToHost, s));
+            if (proofs)
+                enqueue_copies(CopyPart{p->h_proofs, p->ws.proofs, nb * kProofBytes}, CopyPart{}, hipMemcpyDeviceToHost, s);
             if (!cells) ck(hipStreamSynchronize(s));
             bool bad = false;
             for (uint32_t b = 0; b < nb; b++) bad |= p->h_err[b] != 0;
@@ -1230,9 +1250,9 @@ vkzg_result vkzg_amd_recover_cells_and_proofs(vkzg_prover *p, uint8_t *cells_out
             const uint8_t *pm = cell_present + done * 128;
             if (!chunk_missing_ok(pm, nb)) return VKZG_ERR_BADARGS;
             hipStream_t s = p->stream;
-            stage_upload(p, p->ws.cells, p->h_in, cells + done * kCellsBytes, nb * kCellsBytes, s);
             std::memcpy(p->h_present, pm, nb * 128);
-            ck(hipMemcpyAsync(p->ws.present, p->h_present, nb * 128, hipMemcpyHostToDevice, s));
+            stage_upload(p, p->ws.cells, p->h_in, cells + done * kCellsBytes, nb * kCellsBytes, s,
+                         CopyPart{p->ws.present, p->h_present, nb * 128});
             const Tuning tn = tuning_for(p, nb);
             Tuning one = tn;
             one.splits = 1;
@@ -1248,7 +1268,8 @@ vkzg_result vkzg_amd_recover_cells_and_proofs(vkzg_prover *p, uint8_t *cells_out
             // holds p(w^brev13(64c+t)) and brev13(i) = 2 brev12(i) for i < 4096).
             enqueue_cells_and_proofs(p, p->ws, nullptr, nullptr, p->ws.proofs, p->ws.cells_out, kCellsBytes, nb,
                                      s, one, &p->graphs);
-            ck(hipMemcpyAsync(p->h_proofs, p->ws.proofs, nb * kProofBytes, hipMemcpyDeviceToHost, s));
+            enqueue_copies(CopyPart{p->h_proofs, p->ws.proofs, nb * kProofBytes}, CopyPart{},
+                           hipMemcpyDeviceToHost, s);
             finish_download(p, cells_out + done * kCellsBytes, p->h_out, nb * kCellsBytes);
             ck(hipStreamSynchronize(p->copy_stream));
             ck(hipStreamSynchronize(s));

@@ -431,7 +431,9 @@ struct PhaseAShape {
 PhaseAShape phase_a_shape(uint64_t nmsm, uint32_t groups, uint32_t windows, uint64_t slots, uint32_t cus);
 
 // host (pageable) -> pinned staging -> dev, enqueued on s.
-void stage_upload(vkzg_prover *p, uint8_t *dev, uint8_t *pinned, const uint8_t *host, size_t bytes, hipStream_t s);
+void enqueue_copies(const CopyPart &a, const CopyPart &b, hipMemcpyKind kind, hipStream_t s);
+void stage_upload(vkzg_prover *p, uint8_t *dev, uint8_t *pinned, const uint8_t *host, size_t bytes, hipStream_t s,
+                  const CopyPart &more = CopyPart{});
 
 // Enqueue a pipeline through `cache` when graphs are on and stage timing is
 // off (timing records events between stages), else launch it directly.

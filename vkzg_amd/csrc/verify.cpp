@@ -243,8 +243,8 @@ vkzg_result verify_impl(vkzg_prover *p, int *ok, const uint8_t *commitments, con
     Fr *ev = reinterpret_cast<Fr *>(D + d_ev), *rp = reinterpret_cast<Fr *>(D + d_rp);
     Fr *agg = reinterpret_cast<Fr *>(D + d_agg), *sc = reinterpret_cast<Fr *>(D + d_sc);
     G1A *out = reinterpret_cast<G1A *>(D + d_out);
-    ck(hipMemcpyAsync(D, H, in_bytes, hipMemcpyHostToDevice, s));
-    ck(hipMemsetAsync(res, 0, 16, s));
+    std::memset(H + h_res, 0, 16);
+    enqueue_copies(CopyPart{D, H, in_bytes}, CopyPart{res, H + h_res, 16}, hipMemcpyHostToDevice, s);
     ck(launch_vfy_points(pts, D + h_pts, u + n32, p->srs, 64, res + 1, s));
     ck(launch_vfy_cells(ev, D + h_cells, n32, res + 1, s));
     // G1 membership of commitments and proofs: with the pairing while a quad per
@@ -259,7 +259,7 @@ vkzg_result verify_impl(vkzg_prover *p, int *ok, const uint8_t *commitments, con
     uint32_t r[8];
     challenge(r, uniq, cidx, cell_indices, commitments, cells, proofs, n);
     std::memcpy(H + h_r, r, 32);
-    ck(hipMemcpyAsync(D + d_r, H + h_r, 32, hipMemcpyHostToDevice, s));
+    enqueue_copies(CopyPart{D + d_r, H + h_r, 32}, CopyPart{}, hipMemcpyHostToDevice, s);
     ck(launch_vfy_weights(rp, reinterpret_cast<const Fr *>(D + d_r), n32, s));
     ck(launch_vfy_interp(reinterpret_cast<Fr *>(D + d_part), agg, U32(h_chunks), nch, U32(h_iord), ev, rp,
                          p->roots_inv, s));
@@ -273,7 +273,7 @@ vkzg_result verify_impl(vkzg_prover *p, int *ok, const uint8_t *commitments, con
     // e(sum r^k pi_k, [tau^64]G2) e(-RL, G2) == 1
     ck(launch_pairing_check(res, nullptr, reinterpret_cast<Fp *>(D + d_L), v.lines, v.lines + 2 * kPairSteps,
                             out, out + 1, true, pts, with_pairing ? npts : 0, res + 1, s));
-    ck(hipMemcpyAsync(H + h_res, res, 8, hipMemcpyDeviceToHost, s));
+    enqueue_copies(CopyPart{H + h_res, res, 8}, CopyPart{}, hipMemcpyDeviceToHost, s);
     ck(hipStreamSynchronize(s));
     uint32_t rr[2];
     std::memcpy(rr, H + h_res, 8);
@@ -458,8 +458,8 @@ vkzg_result vkzg_amd_blob_to_commitments(vkzg_prover *p, uint8_t *commitments, c
             if (shares > 1) ck(launch_sum_groups(sum, part, shares, nmsm, p->cus, 0, s));
             ck(launch_sum_groups(out, sum, 64, nb, p->cus, 0, s));
             ck(launch_compress_points(D + o_cm, out, nb, s));
-            ck(hipMemcpyAsync(H + o_err, D + o_err, 4ull * nb + 0, hipMemcpyDeviceToHost, s));
-            ck(hipMemcpyAsync(H + o_cm, D + o_cm, 48ull * nb, hipMemcpyDeviceToHost, s));
+            enqueue_copies(CopyPart{H + o_err, D + o_err, 4 * nb}, CopyPart{H + o_cm, D + o_cm, 48 * nb},
+                           hipMemcpyDeviceToHost, s);
             ck(hipStreamSynchronize(s));
             for (uint32_t b = 0; b < nb; b++) {
                 uint32_t e;
