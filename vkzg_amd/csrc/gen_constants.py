@@ -106,6 +106,7 @@ def main():
     out.append(arr30("INV_SIGMA_M", pow(SIGMA, -1, P) * RP % P))
     out.append(arr30("NU_M", NU * RP % P))
     out.append(arr30("SIGMA_OVER_NU_M", SIGMA * pow(NU, -1, P) * RP % P))
+    out.append(arr30("NU_BETA_M", NU * BETA * RP % P))
     out.append(arr30("NU_BETA2_M", NU * BETA * BETA * RP % P))
     out.append(arr30("R3_M", RP ** 3 % P))  # Montgomery form of R^2: turns a plain inverse of xR into x^-1 R
     # 2^384 mod p as a plain value: a Montgomery product of x R by it gives

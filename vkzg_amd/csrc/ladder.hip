@@ -77,7 +77,7 @@ __global__ __launch_bounds__(256) void k_ladder(G1J *lad, const G1X *u, uint32_t
         G1X f = ladder_fold(ub, j, [&](const G1X &a, const G1X &b) { return g1x_add_quad(a, b, q, exc); });
         // uniform in the quad
         if (exc) f = ladder_fold(ub, j, [](const G1X &a, const G1X &b) { return g1x_add(a, b); });
-        G1PQ p = g1pq_from_xyzz<false>(f, q);
+        G1PQ p = g1pq_from_xyzz(f, q);
 #pragma unroll 1
         for (uint32_t d = d0; d < d1; d++) {
             const Fp y = g1pq_y(p);

@@ -14,7 +14,7 @@ struct MsmShape {
     uint32_t W = 0;     // windows of a 128-bit half scalar, ceil(129 / c)
     uint32_t bk = 0;    // buckets per window, 2^(c-1)
     uint32_t K = 0;     // buckets in all, nmsm * W * bk
-    uint32_t parts = 1; // window-sum blocks per window (bk / (128 * buckets per thread))
+    uint32_t parts = 1; // window-sum blocks per window (bk / (64 quads * 4 buckets))
 };
 
 MsmShape msm_shape(uint32_t ne, uint32_t nmsm);
@@ -24,6 +24,6 @@ size_t msm_scratch_bytes(const MsmShape &sh);
 // ((0, 0) for the identity).  sc: canonical scalars below r; pidx < 2^30;
 // scratch: msm_scratch_bytes(sh) bytes of device memory.
 hipError_t launch_msm(const MsmShape &sh, void *scratch, const G1A *pts, const uint32_t *pidx, const Fr *sc,
-                      const uint8_t *mid, G1A *out, hipStream_t s);
+                      const uint8_t *mid, G1A *out, uint32_t cus, hipStream_t s);
 
 }  // namespace vkzg_amd

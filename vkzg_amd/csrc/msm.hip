@@ -12,8 +12,8 @@
 //   count    histogram of (msm, window, |digit|) keys     (atomics)
 //   scan     bucket offsets (one block; three passes above 16k buckets)
 //   scatter  point references sorted by key               (atomics)
-//   buckets  one lane per bucket sums its points          (XYZZ, checked);
-//            buckets of more than 24 points by a wave
+//   buckets  one lane (XYZZ, checked) or four quads (homogeneous) per bucket
+//            sum its points; buckets of more than 24 points by a wave
 //   windows  blocks per (msm, window): sum_b (b+1) B_b by running sums over
 //            segments of at most 4 buckets on quads, then trees in LDS
 //   combine  a wave per MSM: Horner over runs of windows (c doublings each) on
@@ -211,10 +211,10 @@ VKZG_DEV_COLD void bucket_checked(G1X *acc, const G1A *pts, const uint32_t *list
     *acc = a;
 }
 
-// One lane per bucket.  A bucket with more than kHotLen points (the few
-// digits of a narrow top window collect most points of every scalar) goes to
-// the hot list instead, for k_msm_hot.
-__global__ void __launch_bounds__(64) k_msm_buckets(G1X *buckets, const uint32_t *off, const uint32_t *list, const G1A *pts,
+// One lane per bucket (launches that fill the chip so).  A bucket with more than
+// kHotLen points (the few digits of a narrow top window collect most points of
+// every scalar) goes to the hot list instead, for k_msm_hot.
+__global__ void __launch_bounds__(64) k_msm_buckets(G1P *buckets, const uint32_t *off, const uint32_t *list, const G1A *pts,
                               uint32_t K, uint32_t *hot, uint32_t *hot_n) {
     const uint32_t key = blockIdx.x * blockDim.x + threadIdx.x;
     if (key >= K) return;
@@ -228,31 +228,71 @@ __global__ void __launch_bounds__(64) k_msm_buckets(G1X *buckets, const uint32_t
 #pragma unroll 1
     for (uint32_t q = lo; q < hi; q++) acc = g1x_madd_fast(acc, msm_point(pts, list[q]), exc);
     if (exc) bucket_checked(&acc, pts, list, lo, hi);
-    buckets[key] = acc;
+    buckets[key] = g1p_from_xyzz_lane(acc);
 }
 
-// Hot buckets, one wave each (blocks stride over the list): the lanes sum
-// interleaved shares of the bucket's points, then a tree in LDS.
-__global__ void __launch_bounds__(64) k_msm_hot(G1X *buckets, const uint32_t *off, const uint32_t *list,
+// msm_point in homogeneous coordinates
+VKZG_DEV G1P msm_point_homog(const G1A *pts, uint32_t ref) {
+    const G1A p = pts[ref & kPtMask];
+    const Fp nu = fp_select((ref & (1u << 30)) != 0, fp_const(cfp::NU_BETA_M), fp_const(cfp::NU_M));
+    const bool inf = g1a_is_identity(p);
+    return G1P{fp_mul(p.x, nu), fp_select(inf, fp_one(), fp_cond_neg(p.y, (ref >> 31) != 0)),
+               fp_select(inf, fp_zero(), fp_const(cfp::SIGMA_M))};
+}
+
+// The points list[lo..hi) summed by QUADS consecutive quads of one wave (quad k of
+// them: every QUADS-th point, then a tree): complete additions in homogeneous
+// coordinates (proj_quad.h), 3.5 rounds of products and one for a point's x.
+template <uint32_t QUADS>
+VKZG_DEV G1PQ quads_sum(const G1A *pts, const uint32_t *list, uint32_t lo, uint32_t hi, uint32_t k, uint32_t q) {
+    G1PQ acc = g1p_spread(g1p_identity(), q);
+#pragma unroll 1
+    for (uint32_t i = lo + k; i < hi; i += QUADS) {
+        const G1P p = msm_point_homog(pts, list[i]);
+        acc = i == lo + k ? g1p_spread(p, q) : g1p_add_quad(g1p_gather(acc), p, q);
+    }
+#pragma unroll 1
+    for (uint32_t m = 1; m < QUADS; m <<= 1) {
+        const G1PQ other = g1pq_shfl_xor(acc, (int)(4 * m));
+        acc = g1p_add_quad(g1p_gather(acc), g1p_gather(other), q);
+    }
+    return acc;
+}
+VKZG_DEV void g1pq_store(G1P *out, const G1PQ &p, uint32_t q) {
+    const Fp y = g1pq_y(p);
+    if (q == 0) out->y = y;
+    else if (q == 2) out->x = p.r;
+    else if (q == 3) out->z = p.r;
+}
+
+// Four quads per bucket, for launches that leave SIMDs idle with a lane each: there
+// a bucket's chain of up to kHotLen additions is the time (a check of 128 cells:
+// 170 -> 37 us).
+__global__ void __launch_bounds__(64) k_msm_buckets_quads(G1P *buckets, const uint32_t *off, const uint32_t *list,
+                                                          const G1A *pts, uint32_t K, uint32_t *hot, uint32_t *hot_n) {
+    const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t key = tid / 16, k = (tid >> 2) & 3u, q = tid & 3u;
+    if (key >= K) return;
+    const uint32_t lo = off[key], hi = off[key + 1];
+    if (hi - lo > kHotLen) {
+        if ((tid & 15u) == 0) hot[atomicAdd(hot_n, 1u)] = key;
+        return;
+    }
+    const G1PQ acc = quads_sum<4>(pts, list, lo, hi, k, q);
+    if (k == 0) g1pq_store(&buckets[key], acc, q);
+}
+
+// Hot buckets, one wave (16 quads) each; blocks stride over the list.  A check of
+// 128 cells: 135 -> 74 us against a lane per share and a tree of lanes.
+__global__ void __launch_bounds__(64) k_msm_hot(G1P *buckets, const uint32_t *off, const uint32_t *list,
                                                 const G1A *pts, const uint32_t *hot, const uint32_t *hot_n) {
-    __shared__ G1X sh[64];
-    const uint32_t t = threadIdx.x;
+    const uint32_t k = threadIdx.x >> 2, q = threadIdx.x & 3u;
     const uint32_t n = *hot_n;
 #pragma unroll 1
-    for (uint32_t q = blockIdx.x; q < n; q += gridDim.x) {
-        const uint32_t key = hot[q];
-        const uint32_t lo = off[key], hi = off[key + 1];
-        G1X acc = g1x_identity();
-#pragma unroll 1
-        for (uint32_t i = lo + t; i < hi; i += 64) acc = g1x_madd(acc, msm_point(pts, list[i]));
-        sh[t] = acc;
-        __syncthreads();
-        for (uint32_t stride = 32; stride > 0; stride >>= 1) {
-            if (t < stride) sh[t] = g1x_add(sh[t], sh[t + stride]);
-            __syncthreads();
-        }
-        if (t == 0) buckets[key] = sh[0];
-        __syncthreads();
+    for (uint32_t h = blockIdx.x; h < n; h += gridDim.x) {
+        const uint32_t key = hot[h];
+        const G1PQ acc = quads_sum<16>(pts, list, off[key], off[key + 1], k, q);
+        if (k == 0) g1pq_store(&buckets[key], acc, q);
     }
 }
 
@@ -279,13 +319,6 @@ VKZG_DEV G1PQ g1pq_block_sum(G1PQ acc, Fp *sh, uint32_t t) {
     }
     return acc;
 }
-VKZG_DEV void g1pq_store(G1P *out, const G1PQ &p, uint32_t q) {
-    const Fp y = g1pq_y(p);
-    if (q == 0) out->y = y;
-    else if (q == 2) out->x = p.r;
-    else if (q == 3) out->z = p.r;
-}
-
 // Block (msm, window, part): sum over the part's buckets b of (b + 1) B_b.
 // Quad k owns buckets [lo, lo + seg): running sums from the top give R = sum B_b
 // and T = sum (b - lo + 1) B_b, and its share is T + lo R; a tree adds the
@@ -294,25 +327,25 @@ VKZG_DEV void g1pq_store(G1P *out, const G1PQ &p, uint32_t q) {
 // time here, so quads in homogeneous coordinates run it (proj_quad.h): with 38
 // windows of 64 buckets (the sums of a check of 128 cells) 285 -> 76 us against
 // a lane per bucket in XYZZ coordinates.
-__global__ void __launch_bounds__(4 * kWinQuads) k_msm_windows(G1P *wpart, const G1X *buckets, uint32_t bk,
+__global__ void __launch_bounds__(4 * kWinQuads) k_msm_windows(G1P *wpart, const G1P *buckets, uint32_t bk,
                                                                uint32_t parts) {
     __shared__ Fp sh[4 * kWinQuads];
     const uint32_t t = threadIdx.x, q = t & 3u, k = t >> 2;
     const uint32_t win = blockIdx.x / parts, part = blockIdx.x % parts;
-    const G1X *B = buckets + (size_t)win * bk;
+    const G1P *B = buckets + (size_t)win * bk;
     const uint32_t per_part = bk / parts;
     const uint32_t seg = per_part > kWinQuads ? per_part / kWinQuads : 1;
     const uint32_t lo = part * per_part + k * seg;
     G1PQ share = g1p_spread(g1p_identity(), q);
     if (k * seg < per_part) {
-        G1P R = g1p_from_xyzz(B[lo + seg - 1], q);
+        G1P R = B[lo + seg - 1];
         if (seg == 1) {
             share = g1p_mul_small(R, lo + 1, q);
         } else {
             G1P T = R;
 #pragma unroll 1
             for (uint32_t b = lo + seg - 1; b-- > lo;) {
-                R = g1p_gather(g1p_add_quad(R, g1p_from_xyzz(B[b], q), q));
+                R = g1p_gather(g1p_add_quad(R, B[b], q));
                 T = g1p_gather(g1p_add_quad(T, R, q));
             }
             share = lo ? g1p_add_quad(g1p_gather(g1p_mul_small(R, lo, q)), T, q) : g1p_spread(T, q);
@@ -399,13 +432,13 @@ size_t msm_scratch_bytes(const MsmShape &sh) {
     b += 4ull * (4 * (size_t)sh.K + 3);  // cnt (+ hot count), cur, off, hot list
     b += 4ull * (sh.K / kScanTile + 1);  // scan tile totals
     b += 4 * nh * sh.W;                  // sorted references
-    b += sizeof(G1X) * (size_t)sh.K;     // buckets
+    b += sizeof(G1P) * (size_t)sh.K;     // buckets
     b += sizeof(G1P) * (size_t)sh.nmsm * sh.W * (sh.parts + 1);
     return b + 16 * 256;  // each of the 10 regions is rounded up to 256 bytes
 }
 
 hipError_t launch_msm(const MsmShape &sh, void *scratch, const G1A *pts, const uint32_t *pidx, const Fr *sc,
-                      const uint8_t *mid, G1A *out, hipStream_t s) {
+                      const uint8_t *mid, G1A *out, uint32_t cus, hipStream_t s) {
     if (sh.ne == 0 || sh.nmsm == 0) return hipErrorInvalidValue;
     const uint32_t nh = 2 * sh.ne;
     uint8_t *p = static_cast<uint8_t *>(scratch);
@@ -422,7 +455,7 @@ hipError_t launch_msm(const MsmShape &sh, void *scratch, const G1A *pts, const u
     const uint32_t ntiles = (sh.K + kScanTile - 1) / kScanTile;
     uint32_t *tot = reinterpret_cast<uint32_t *>(take(4ull * (sh.K / kScanTile + 1)));
     uint32_t *list = reinterpret_cast<uint32_t *>(take(4ull * nh * sh.W));
-    G1X *buckets = reinterpret_cast<G1X *>(take(sizeof(G1X) * (size_t)sh.K));
+    G1P *buckets = reinterpret_cast<G1P *>(take(sizeof(G1P) * (size_t)sh.K));
     G1P *wpart = reinterpret_cast<G1P *>(take(sizeof(G1P) * (size_t)sh.nmsm * sh.W * sh.parts));
     G1P *wsum = sh.parts > 1 ? reinterpret_cast<G1P *>(take(sizeof(G1P) * (size_t)sh.nmsm * sh.W)) : wpart;
     if ((size_t)(p - static_cast<uint8_t *>(scratch)) > msm_scratch_bytes(sh)) return hipErrorInvalidValue;
@@ -439,8 +472,13 @@ hipError_t launch_msm(const MsmShape &sh, void *scratch, const G1A *pts, const u
     }
     hipLaunchKernelGGL(k_msm_scatter, dim3(blocks_for(nh, 256)), dim3(256), 0, s, list, cur, hs, mid, pidx, nh,
                        sh.c, sh.W);
-    hipLaunchKernelGGL(k_msm_buckets, dim3(blocks_for(sh.K, 64)), dim3(64), 0, s, buckets, off, list, pts,
-                       sh.K, hot, cnt + sh.K);
+    // four quads per bucket while they are at most one wave per SIMD
+    if (sh.K * 16ull <= (uint64_t)cus * 4 * 64)
+        hipLaunchKernelGGL(k_msm_buckets_quads, dim3(blocks_for(sh.K * 16ull, 64)), dim3(64), 0, s, buckets, off, list,
+                           pts, sh.K, hot, cnt + sh.K);
+    else
+        hipLaunchKernelGGL(k_msm_buckets, dim3(blocks_for(sh.K, 64)), dim3(64), 0, s, buckets, off, list, pts, sh.K,
+                           hot, cnt + sh.K);
     const dim3 hot_grid(sh.K < kHotBlocks ? sh.K : kHotBlocks);
     hipLaunchKernelGGL(k_msm_hot, hot_grid, dim3(64), 0, s, buckets, off, list, pts, hot, cnt + sh.K);
     hipLaunchKernelGGL(k_msm_windows, dim3(sh.nmsm * sh.W * sh.parts), dim3(4 * kWinQuads), 0, s, wpart, buckets,

@@ -104,21 +104,26 @@ VKZG_DEV G1PQ g1p_add_quad(const G1P &a, const G1P &b, uint32_t q) {
     return G1PQ{fp_mul_sum(f0, f1, g0, g1)};
 }
 
-// Conversions.  XYZZ: (nu X ZZZ : Y ZZ : sigma ZZ ZZZ), two rounds; NU = false
-// leaves nu out (chains that only double).
-template <bool NU>
+// Conversions.  XYZZ to (X ZZZ : Y ZZ : sigma ZZ ZZZ), two rounds, without nu: for
+// chains that only double.
 VKZG_DEV G1PQ g1pq_from_xyzz(const G1X &p, uint32_t q) {
     const Fp r = fp_mul(fp_select4(q, p.y, p.zz, p.x, p.zz), fp_select(q == 0, p.zz, p.zzz));
-    const Fp t = fp_mul(r, fp_select(q == 2 && NU, fp_const(cfp::NU_M), fp_const(cfp::SIGMA_M)));
-    return G1PQ{fp_select4(q, r, fp_zero(), NU ? t : r, t)};
-}
-// The same in every lane, ready for g1p_add_quad: the identity is (0 : 1 : 0).
-VKZG_DEV G1P g1p_from_xyzz(const G1X &p, uint32_t q) {
-    G1P r = g1p_gather(g1pq_from_xyzz<true>(p, q));
-    r.y = fp_select(fp_is_zero(p.zz), fp_one(), r.y);
-    return r;
+    const Fp z = fp_mul(r, fp_const(cfp::SIGMA_M));
+    return G1PQ{fp_select4(q, r, fp_zero(), r, z)};
 }
 VKZG_DEV G1P g1p_identity() { return G1P{fp_zero(), fp_one(), fp_zero()}; }
+// XYZZ by one lane, ready for g1p_add_quad: (nu X ZZZ : Y ZZ : sigma ZZ ZZZ).
+VKZG_DEV G1P g1p_from_xyzz_lane(const G1X &p) {
+    if (fp_is_zero(p.zz)) return g1p_identity();
+    return G1P{fp_mul(fp_mul(p.x, p.zzz), fp_const(cfp::NU_M)), fp_mul(p.y, p.zz),
+               fp_mul(fp_mul(p.zz, p.zzz), fp_const(cfp::SIGMA_M))};
+}
+VKZG_DEV G1PQ g1pq_shfl_xor(const G1PQ &p, int m) {
+    G1PQ r;
+#pragma unroll
+    for (int i = 0; i < kFpLimbs; i++) r.r.v[i] = __shfl_xor(p.r.v[i], m);
+    return r;
+}
 // An affine point that is not the identity.
 VKZG_DEV G1P g1p_from_affine(const G1A &p) {
     return G1P{fp_mul(p.x, fp_const(cfp::NU_M)), p.y, fp_const(cfp::SIGMA_M)};

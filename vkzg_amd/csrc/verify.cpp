@@ -265,7 +265,7 @@ vkzg_result verify_impl(vkzg_prover *p, int *ok, const uint8_t *commitments, con
                          p->roots_inv, s));
     ck(launch_vfy_entries(sc, U32(d_pidx), D + d_mid, rp, U32(h_coff), U32(h_cgrp), U32(h_cidx), p->roots, agg,
                           n32, u, s));
-    ck(launch_msm(sh, D + d_msm, pts, U32(d_pidx), sc, D + d_mid, out, s));
+    ck(launch_msm(sh, D + d_msm, pts, U32(d_pidx), sc, D + d_mid, out, p->cus, s));
     if (terms) {
         ck(launch_compress_affine(D + d_terms, out, 2, s));
         ck(hipMemcpyAsync(H + h_terms, D + d_terms, 96, hipMemcpyDeviceToHost, s));
@@ -587,7 +587,7 @@ vkzg_result vkzg_amd_debug_g1_msm(vkzg_prover *p, uint8_t out[48], const uint8_t
             ck(hipMemsetAsync(mid, 0, n, s));
             ck(hipMemsetAsync(err, 0, 4, s));
             ck(launch_vfy_points(pts, dp, n32, nullptr, 0, err, s));
-            ck(launch_msm(sh, scratch, pts, pidx, dsc, mid, res, s));
+            ck(launch_msm(sh, scratch, pts, pidx, dsc, mid, res, p->cus, s));
             ck(launch_compress_affine(dout, res, 1, s));
             ck(hipMemcpyAsync(out, dout, 48, hipMemcpyDeviceToHost, s));
             ck(hipMemcpyAsync(herr, err, 4, hipMemcpyDeviceToHost, s));
