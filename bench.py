@@ -3,8 +3,8 @@
 
 Headline: computeProofsBatch (FK20, 128 cell proofs per blob) on a 256-blob
 batch with the blobs already resident in HBM; one step = one 256-blob call
-through vkzg_amd_compute_proofs_device, which replays the call's captured HIP
-graph (the library's default path).  Prints ONE JSON line.
+through vkzg_amd_compute_proofs_device (the library's default path: kernels
+launched one by one).  Prints ONE JSON line.
 
 Also measured (in "secondary"): recoverCellsBatch on 64 blobs with exactly 64
 of 128 cells present, the plain one-call-per-blob proof form, the per-stage
@@ -48,7 +48,8 @@ def stage_work(info, nb, items_per_output):
     madd, add, dbl_j = 10, 14, 7  # Fp multiplications per operation
     return {
         "fk20_scalars": nb * (12 * 2048 + 4096 + 64 * 448 + 8192 + 4096) * FR_M,
-        # 8 lanes per MSM, 8 terms each, then a 3-level lane tree (7 adds)
+        # 64 W mixed additions per MSM, and 7 for the sum of its shares (their
+        # number varies with the batch)
         "phase_a": nb * 128 * (64 * W * madd + 7 * add) * FP_M,
         # 128 chains of 8 (LAD_POS - 1) doublings, after the split-circulant
         # folds of u (3 additions for each of 64 chains, 1 for the other 64)
@@ -351,8 +352,8 @@ def main():
                   "classes": {str(n): prover.get_tuning(n) for n in (1, 4, 16, 64, 256)}}
     for _ in range(a.warmup):
         prover.compute_proofs_device(d_proofs.ptr, d_blobs.ptr, nb, stream.handle)
-    # The timed steps: the library's default path, one captured HIP graph
-    # replayed per call (the synchronous entry points do the same).
+    # The timed steps: the library's default path, every kernel of a call
+    # launched on the stream.
     stream.synchronize()
     t0 = time.perf_counter()
     for _ in range(a.steps):
@@ -486,7 +487,7 @@ def main():
         d_ucells = hip.DeviceBuffer.from_bytes(ucells)
         d_uout = hip.DeviceBuffer(len(ucells))
         d_umask = hip.DeviceBuffer.from_bytes(umask)
-        for n in calls:  # first use of each size captures its graph
+        for n in calls:  # warm-up, every size once
             prover.recover_cells_device(d_uout.ptr, d_ucells.ptr, d_umask.ptr, umask[:128 * n], n,
                                         stream.handle)
         t0 = time.perf_counter()

@@ -124,7 +124,7 @@ typedef struct {
     double setup_ms;           /* wall time of prover creation */
     uint32_t last_splits;      /* sub-streams the last call's batches were spread over */
     uint32_t graphs_enabled;   /* 1 unless VKZG_AMD_GRAPHS=0 */
-    uint64_t graph_captures;   /* pipelines captured into HIP graphs by the synchronous calls */
+    uint64_t graph_captures;   /* pipelines captured into HIP graphs by the host-buffer calls */
     uint64_t graph_replays;    /* calls served by replaying a captured graph */
     uint32_t autotuned;        /* 1 after vkzg_amd_autotune */
     double autotune_ms;        /* its wall time */
@@ -170,8 +170,9 @@ vkzg_result vkzg_amd_load_window_table(vkzg_prover *p, uint32_t window_bits);
 vkzg_result vkzg_amd_get_tuning(const vkzg_prover *p, size_t num_blobs, vkzg_amd_tuning *out);
 /* Sets the tuning of the size class of `num_blobs`; BADARGS when a field is out of range. */
 vkzg_result vkzg_amd_set_tuning(vkzg_prover *p, size_t num_blobs, const vkzg_amd_tuning *t);
-/* Replays of captured HIP graphs on (enable != 0, the default unless
- * VKZG_AMD_GRAPHS=0) or off (every call launches its kernels directly). */
+/* Replays of captured HIP graphs by the host-buffer calls on (enable != 0, the
+ * default unless VKZG_AMD_GRAPHS=0) or off (every call launches its kernels
+ * directly, as the device-pointer calls always do). */
 vkzg_result vkzg_amd_set_graphs(vkzg_prover *p, int enable);
 
 /* Times candidate tunings on synthetic blobs for every size class up to the

@@ -169,7 +169,8 @@ struct StreamSet {
 // Instantiated HIP graphs of whole pipelines, keyed by what the captured
 // launches depend on (kind, blob count, split count, buffer addresses).  A
 // pipeline is captured the first time its key is seen and replayed after
-// that, which turns 10-20 kernel launches into one graph launch.  The
+// that, which turns 10-20 kernel launches into one graph launch (entry points
+// with buffers of the prover's own, and the server's slots).  The
 // captured pipelines hold kernels and event dependencies only: no memset or
 // memcpy nodes.
 struct GraphKey {
