@@ -101,7 +101,7 @@ hipError_t launch_phase_b_scalars(Fr *out, const Fr *roots, hipStream_t s);
 // in one kernel; addresses and sizes are multiples of 4 bytes.  For transfers
 // below kKernelCopyMax, where the host side is a single memcpy too (larger ones go
 // out in slices beside the copy threads): a copy engine's hand-over costs about 10
-// us on either side of a transfer that takes 5 to 10, and two pieces are two
+// us on either side of a transfer that takes 5 to 60, and two pieces are two
 // transfers.  Recovery of one blob, 256 KiB each way and its map: 139 us with copy
 // engines, 116 with two of these kernels.
 struct CopyPart {
@@ -109,7 +109,7 @@ struct CopyPart {
     const void *src = nullptr;
     size_t bytes = 0;
 };
-constexpr size_t kKernelCopyMax = (size_t)1 << 20;
+constexpr size_t kKernelCopyMax = (size_t)3 << 20;
 hipError_t launch_copy(const CopyPart &a, const CopyPart &b, hipStream_t s);
 
 // ----------------------------------------------------------------- proofs

@@ -8,6 +8,7 @@
 #include <condition_variable>
 #include <cstdint>
 #include <functional>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <system_error>
@@ -251,21 +252,23 @@ class CopyThreads {
         wake_.notify_all();
         for (std::thread &t : threads_) t.join();
     }
+    // f(0), ..., f(n - 1), on this thread and on those that wake up in time: it
+    // returns when every call has returned, not when every thread has been awake
+    // (a wake-up takes about as long as a small copy).
     void run(size_t n, const std::function<void(size_t)> &f) {
         if (!started_) start();
+        const auto job = std::make_shared<Job>(f, n);
         {
             std::lock_guard<std::mutex> lock(mu_);
-            job_ = &f;
-            count_ = n;
-            next_ = 0;
-            busy_ = threads_.size();
+            job_ = job;
             generation_++;
         }
-        wake_.notify_all();
-        take(f, n);
+        // a thread per two items: each wake-up costs this thread a system call
+        for (size_t k = 0; k < (n + 1) / 2 && k < threads_.size(); k++) wake_.notify_one();
+        take(*job);
         std::unique_lock<std::mutex> lock(mu_);
-        done_.wait(lock, [this] { return busy_ == 0; });
-        job_ = nullptr;
+        done_.wait(lock, [&] { return job->done == n; });
+        job_.reset();
     }
     void set_device(int device) { device_ = device; }
 
@@ -281,34 +284,42 @@ class CopyThreads {
             }
         }
     }
-    void take(const std::function<void(size_t)> &f, size_t n) {
-        for (size_t k; (k = next_.fetch_add(1)) < n;) f(k);
+    // f is the caller's and lives until done == n; a thread that comes later takes
+    // no item and so never calls it.
+    struct Job {
+        Job(const std::function<void(size_t)> &fn, size_t items) : f(fn), n(items) {}
+        const std::function<void(size_t)> &f;
+        const size_t n;
+        std::atomic<size_t> next{0};
+        size_t done = 0;  // under mu_
+    };
+    void take(Job &job) {
+        size_t did = 0;
+        for (size_t k; (k = job.next.fetch_add(1)) < job.n; did++) job.f(k);
+        if (!did) return;
+        std::lock_guard<std::mutex> lock(mu_);
+        job.done += did;
+        if (job.done == job.n) done_.notify_all();
     }
     void loop() {
         (void)hipSetDevice(device_);
         uint64_t seen = 0;
         for (;;) {
-            const std::function<void(size_t)> *f;
-            size_t n;
+            std::shared_ptr<Job> job;
             {
                 std::unique_lock<std::mutex> lock(mu_);
                 wake_.wait(lock, [&] { return stop_ || generation_ != seen; });
                 if (stop_) return;
                 seen = generation_;
-                f = job_;
-                n = count_;
+                job = job_;
             }
-            take(*f, n);
-            std::lock_guard<std::mutex> lock(mu_);
-            if (--busy_ == 0) done_.notify_one();
+            if (job) take(*job);
         }
     }
     std::mutex mu_;
     std::condition_variable wake_, done_;
     std::vector<std::thread> threads_;
-    const std::function<void(size_t)> *job_ = nullptr;
-    size_t count_ = 0, busy_ = 0;
-    std::atomic<size_t> next_{0};
+    std::shared_ptr<Job> job_;
     uint64_t generation_ = 0;
     bool started_ = false, stop_ = false;
     int device_ = 0;
