@@ -11,10 +11,10 @@
 // Fp2 operations run on one lane.  Fp12 products run on a whole workgroup:
 // the 144 Fp products a_i * b_j go to 144 lanes at once (one Montgomery
 // multiplication of latency instead of 54-144 in sequence), then cross-lane
-// exchanges inside each wave (DPP quad broadcasts and an xor tree) combine
-// them into the 12 result coefficients.  That keeps the pairing's long
-// dependent chain (about 480 Fp12 products) near a millisecond on one CU,
-// where a one-lane tower would take over ten.
+// exchanges inside each wave (DPP quad broadcasts and a tree) combine them into
+// the 12 result coefficients.  That keeps the pairing's long dependent chain
+// (about 115 Fp12 products and 315 cyclotomic squares) below a millisecond on
+// one CU, where a one-lane tower would take over ten.
 #pragma once
 
 #include "curve.h"
