@@ -181,15 +181,6 @@ VKZG_DEV G1X g1x_from_affine(const G1A &a) {
     r.zzz = fp_one();
     return r;
 }
-VKZG_DEV G1X g1x_from_jacobian(const G1J &p) {
-    if (fp_is_zero(p.z)) return g1x_identity();
-    G1X r;
-    r.x = p.x;
-    r.y = p.y;
-    r.zz = fp_sqr(p.z);
-    r.zzz = fp_mul(r.zz, p.z);
-    return r;
-}
 // (X, Y, ZZ, ZZZ) with ZZ^3 == ZZZ^2 -> Jacobian with Z = ZZ*ZZZ:
 // X_J = X*ZZ^4, Y_J = Y*ZZZ^4 (no inversion).
 VKZG_DEV_CALL G1J g1j_from_xyzz(const G1X &p) {

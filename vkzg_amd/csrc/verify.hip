@@ -157,7 +157,7 @@ __global__ void k_vfy_entries(Fr *sc, uint32_t *pidx, uint8_t *mid, const Fr *rp
 // Commitment scalars of nb blobs: sc[b * 4096 + i] = coefficient i of blob b's
 // polynomial in phase A's form (sign and biased magnitude), MSM j of a blob
 // taking coefficients [64 j, 64 j + 64); err[b] = 1 for a blob with a
-// non-canonical element (as k_fk20_scalars, k_blob_to_fr.comp:23-37).  Clears
+// non-canonical element (as k_blob_dft, k_blob_to_fr.comp:23-37).  Clears
 // the work counter of the phase-A launch that follows.
 // One block per blob holds the whole transform in LDS; with 16 waves (four per
 // SIMD) instead of 4 it takes 0.09 instead of 0.14 ms.
