@@ -6,6 +6,8 @@ import random
 
 import pytest
 
+import vkzg_amd
+
 pytestmark = pytest.mark.gpu
 
 R = 0x73EDA753299D7D483339D80809A1D80553BDA402FFFE5BFEFFFFFFFF00000001
@@ -49,3 +51,34 @@ def test_batch_sizes(gpu_seeded_prover, n):
     single = {b: gpu_seeded_prover.blob_to_kzg_commitments(b, 1) for b in one}
     got = gpu_seeded_prover.blob_to_kzg_commitments(b"".join(pick), n)
     assert got == b"".join(single[b] for b in pick)
+
+
+@pytest.mark.parametrize("windows", [28, 31, 36, 42, 51, 63, 85, 127, 0])
+def test_smaller_plans(seeded_setup_bytes, oracle_mod, monkeypatch, windows):
+    """The tables of a prover with less free memory, and the bucket method of one
+    with none to spare (0): digits at the ends of the plan's windows, several
+    blobs a call, and calls on both sides of the 64-blob launch sequence."""
+    monkeypatch.setenv("VKZG_AMD_COMMIT_WINDOWS", str(windows))
+    monkeypatch.setenv("VKZG_AMD_WINDOW", "6")
+    n = windows or 24
+    c, k = divmod(255, n)
+    bits = [w * c + max(0, w - (n - k)) for w in range(n)]
+    bits = [b for b in bits if b + c < 250]
+    half = 1 << (c - 1)
+    point = lambda k: seeded_setup_bytes[48 * k:48 * (k + 1)]
+    cases = [(0, 1), (64, R - 1), (4095, (R - 1) // 2), (63, (R + 1) // 2), (1000, 1 << 253)]
+    cases += [(65 + i, sum((half + i) << b for b in bits) % R) for i in (-1, 0, 1)]
+    with vkzg_amd.Prover(max_batch_size=1, setup_g1_monomial=seeded_setup_bytes) as p:
+        one = [monomials([x]) for x in cases]
+        got = p.blob_to_kzg_commitments(b"".join(one), len(one))
+        want = [oracle_mod.g1_mul(point(k), c % R) for k, c in cases]
+        assert [got[48 * n:48 * (n + 1)] for n in range(len(cases))] == want
+        assert p.blob_to_kzg_commitments(bytes(131072), 1) == bytes([0xC0]) + bytes(47)
+        pick = [(i * i + i // 3) % len(one) for i in range(67)]
+        got = p.blob_to_kzg_commitments(b"".join(one[i] for i in pick), 67)
+        assert got == b"".join(want[i] for i in pick)
+        bad = bytearray(one[0])
+        bad[:32] = b"\xff" * 32
+        with pytest.raises(vkzg_amd.VkzgError) as e:
+            p.blob_to_kzg_commitments(one[1] + bytes(bad), 2)
+        assert e.value.code == vkzg_amd.ERR_INVALID_BLOB

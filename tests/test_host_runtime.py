@@ -1,0 +1,103 @@
+"""CPU tests of the library's host code: libvkzg.so in a process of its own
+against tests/c/hip_host.cpp, a HIP runtime whose device memory is host memory
+and whose kernels are only counted.  What is checked is what the host decides:
+what a call does after one that failed, which plan it takes, what it counts."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+REPO = os.path.dirname(HERE)
+
+PREAMBLE = """
+import ctypes, os, sys
+H = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+for f in ("host_live", "host_launches", "host_copies"):
+    getattr(H, f).restype = ctypes.c_uint64
+H.host_fail_alloc.argtypes = [ctypes.c_int64]
+H.host_fail_left.restype = ctypes.c_int64
+H.host_limit.argtypes = [ctypes.c_uint64]
+sys.path.insert(0, sys.argv[2])
+import vkzg_amd
+BLOB, CELLS, GIB = 131072, 262144, 1 << 30
+
+def launches(name):
+    return H.host_launches(name.encode())
+"""
+
+
+@pytest.fixture(scope="module")
+def run(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("hip") / "hip_host.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-o", so, os.path.join(HERE, "c", "hip_host.cpp")], check=True)
+
+    def script(body, **env):
+        r = subprocess.run([sys.executable, "-c", PREAMBLE + body, so, REPO], capture_output=True, text=True,
+                           timeout=100, env=dict(os.environ, VKZG_AMD_WINDOW="6", **env))
+        assert r.returncode == 0, r.stdout + r.stderr
+
+    return script
+
+
+def test_commitments_after_an_allocation_that_failed(run):
+    """Whichever allocation of a prover's first commitment call fails, the call
+    either reports it or takes the bucket method, and the next one is summed from
+    a table that was built whole: never from one that a failure cut short."""
+    run("""
+def table_build(p):
+    before = launches("k_table_multiples"), launches("k_phase_a"), launches("k_msm_buckets")
+    try:
+        p.blob_to_kzg_commitments(bytes(BLOB), 1)
+        ok = True
+    except vkzg_amd.VkzgError:
+        ok = False
+    after = launches("k_table_multiples"), launches("k_phase_a"), launches("k_msm_buckets")
+    return (ok,) + tuple(b - a for a, b in zip(before, after))
+
+with vkzg_amd.Prover(max_batch_size=1) as p:
+    first = table_build(p)
+    whole, live = first[1], H.host_live()
+    assert first[0] and whole > 1 and first[2] == 1 and table_build(p) == (True, 0, 1, 0)
+k = 0
+while True:
+    k += 1
+    with vkzg_amd.Prover(max_batch_size=1) as p:
+        H.host_fail_alloc(k)
+        one = table_build(p)
+        if H.host_fail_left() > 0:
+            break  # the call makes fewer allocations than that
+        H.host_fail_alloc(0)
+        if one[0] and one[1] < whole:
+            assert one[2] == 0 and one[3] == 1, (k, one)  # no table: buckets
+        two, three = table_build(p), table_build(p)
+        assert two[0] and two[2] == 1 and sorted((one[1], two[1])) == [0, whole], (k, one, two)
+        assert three == (True, 0, 1, 0), (k, three)
+        assert abs(H.host_live() - live) < 8 << 20, (k, H.host_live() - live)  # nothing of the failed build is kept
+H.host_fail_alloc(0)
+assert k > 6 and H.host_live() == 0
+""")
+
+
+@pytest.mark.parametrize("free_gib,windows", [(200, 25), (32, 28), (20, 31), (10, 36), (3, 63), (1.2, 127), (0.5, 0), (0.01, 0)])
+def test_commitment_plan_fits_the_free_memory(run, free_gib, windows):
+    """The first commitment call within the free memory there is, temporaries
+    included: fewer windows' larger tables while there is plenty, the bucket
+    method where no table fits."""
+    run("""
+free, windows = %r, %d
+with vkzg_amd.Prover(max_batch_size=1) as p:
+    H.host_limit(int(H.host_live() + free * GIB))
+    before = H.host_live()
+    p.blob_to_kzg_commitments(bytes(2 * BLOB), 2)
+    held = H.host_live() - before
+    if windows == 0:
+        assert launches("k_msm_buckets") > 0 and launches("k_phase_a") == 0 and held < free * GIB / 2
+    else:
+        c, k = 255 // windows, 255 %% windows
+        table = 4096 * (windows + k) * 2 ** (c - 1) * 128
+        assert launches("k_msm_buckets") == 0 and table <= held < table + (16 << 20) and table <= free * GIB / 8
+    p.blob_to_kzg_commitments(bytes(65 * BLOB), 65)
+""" % (free_gib, windows))

@@ -30,9 +30,7 @@ namespace vkzg_amd {
 constexpr size_t kSetupBytes = 4096 * 48;
 constexpr uint32_t kDefaultBatch = 256;
 
-uint64_t table_bytes_for(uint32_t c, uint32_t k = 0) {
-    return 8192ull * window_plan(c, k).entries() * sizeof(G1AT);
-}
+uint64_t table_bytes_for(uint32_t c, uint32_t k = 0) { return vkzg_amd::table_bytes_for(window_plan(c, k), 8192); }
 
 // Window plan of the resident phase-A table: $VKZG_AMD_WINDOW = c if set
 // (6..14, all windows c bits); else the fewest windows W whose cheapest plan
@@ -238,39 +236,61 @@ void build_phase_b_items(const Fr *kpm, std::vector<uint32_t> &items, std::vecto
     offsets.push_back(n2);
 }
 
-// Fills t with a freshly built table of the window plan over n bases: the W
-// chains 2^bit(w) base (affine), then every multiple d * 2^bit(w) base,
+// Threads of one k_table_multiples launch at most, each with a run of up to 64
+// multiples: what the launches of a build share as scratch.
+constexpr uint32_t kTableSlice = 1u << 18;
+uint32_t table_run(WindowPlan plan) { return std::min(plan.H(), 64u); }
+uint64_t table_threads(WindowPlan plan, uint32_t n) {
+    return (uint64_t)n * (plan.W + plan.k) * (plan.H() / table_run(plan));
+}
+
+uint64_t table_bytes_for(WindowPlan plan, uint32_t n) { return (uint64_t)n * plan.entries() * sizeof(G1AT); }
+
+uint64_t table_scratch_for(WindowPlan plan, uint32_t n) {
+    const uint64_t chains = (uint64_t)plan.W * n;
+    const uint64_t runs = table_run(plan) * std::min<uint64_t>(table_threads(plan, n), kTableSlice);
+    return chains * sizeof(G1A) + std::max(chains, runs) * (sizeof(G1J) + sizeof(Fp));
+}
+
+// The W chains 2^bit(w) base (affine), then every multiple d * 2^bit(w) base,
 // d <= 2^(width(w)-1).
-void build_phase_a_table(vkzg_prover *p, PhaseATable &t, WindowPlan plan, const G1A *bases, uint32_t nbases) {
+PhaseATable build_phase_a_table(vkzg_prover *p, WindowPlan plan, const G1A *bases, uint32_t nbases) {
     hipStream_t s = p->stream;
-    const uint32_t c = plan.c;
-    t.c = c;
+    PhaseATable t;
+    t.c = plan.c;
     t.W = plan.W;
     t.H = plan.H();
     t.k = plan.k;
-    t.bytes = (uint64_t)nbases * plan.entries() * sizeof(G1AT);
-    t.table = p->arena.dalloc<G1AT>(t.bytes / sizeof(G1AT));
-    G1J *pwj = p->arena.dalloc<G1J>((size_t)t.W * nbases);
-    Fp *pw_prefix = p->arena.dalloc<Fp>((size_t)t.W * nbases);
-    G1A *pw = p->arena.dalloc<G1A>((size_t)t.W * nbases);
-    ck(launch_table_chains(pwj, bases, nbases, plan, s));
-    ck(launch_jac_to_affine(pw, pwj, pw_prefix, (uint64_t)t.W * nbases, 16, s));
-    ck(hipStreamSynchronize(s));
-    p->arena.dfree(pwj);
-    p->arena.dfree(pw_prefix);
-    const uint32_t S = t.H < 64 ? t.H : 64;
-    const uint64_t total_threads = (uint64_t)nbases * (t.W + t.k) * (t.H / S);  // S entries each
-    const uint32_t slice = 1u << 18;
-    G1J *scratch = p->arena.dalloc<G1J>((size_t)S * slice);
-    Fp *pref = p->arena.dalloc<Fp>((size_t)S * slice);
-    for (uint64_t t0 = 0; t0 < total_threads; t0 += slice) {
-        const uint32_t n = (uint32_t)std::min<uint64_t>(slice, total_threads - t0);
-        ck(launch_table_multiples(t.table, pw, nbases, plan, t0, n, scratch, pref, s));
+    t.bytes = table_bytes_for(plan, nbases);
+    DeviceArena tmp;
+    try {
+        t.table = p->arena.dalloc<G1AT>(t.bytes / sizeof(G1AT));
+        const uint64_t chains = (uint64_t)t.W * nbases;
+        G1A *pw = tmp.dalloc<G1A>(chains);
+        G1J *pwj = tmp.dalloc<G1J>(chains);
+        Fp *pw_prefix = tmp.dalloc<Fp>(chains);
+        ck(launch_table_chains(pwj, bases, nbases, plan, s));
+        ck(launch_jac_to_affine(pw, pwj, pw_prefix, chains, 16, s));
+        ck(hipStreamSynchronize(s));
+        tmp.dfree(pwj);
+        tmp.dfree(pw_prefix);
+        const uint64_t total_threads = table_threads(plan, nbases);
+        const uint64_t runs = table_run(plan) * std::min<uint64_t>(total_threads, kTableSlice);
+        G1J *scratch = tmp.dalloc<G1J>(runs);
+        Fp *pref = tmp.dalloc<Fp>(runs);
+        for (uint64_t t0 = 0; t0 < total_threads; t0 += kTableSlice) {
+            const uint32_t n = (uint32_t)std::min<uint64_t>(kTableSlice, total_threads - t0);
+            ck(launch_table_multiples(t.table, pw, nbases, plan, t0, n, scratch, pref, s));
+        }
+        ck(hipStreamSynchronize(s));
+    } catch (HipFail &) {
+        (void)hipStreamSynchronize(s);
+        tmp.release();
+        if (t.table) p->arena.dfree(t.table);
+        throw;
     }
-    ck(hipStreamSynchronize(s));
-    p->arena.dfree(scratch);
-    p->arena.dfree(pref);
-    p->arena.dfree(pw);
+    tmp.release();
+    return t;
 }
 
 PhaseATable phase_a_table(const vkzg_prover *p, uint32_t window_bits) {
@@ -344,8 +364,7 @@ void build_tables(vkzg_prover *p, const uint8_t *setup) {
     // Phase-A multiples table.
     size_t free_b = 0, total_b = 0;
     ck(hipMemGetInfo(&free_b, &total_b));
-    PhaseATable main_table;
-    build_phase_a_table(p, main_table, choose_window(free_b), p->xext, 8192);
+    const PhaseATable main_table = build_phase_a_table(p, choose_window(free_b), p->xext, 8192);
     p->c = main_table.c;
     p->W = main_table.W;
     p->H = main_table.H;
@@ -890,7 +909,7 @@ void autotune(vkzg_prover *p) {
             size_t free_b = 0, total_b = 0;
             ck(hipMemGetInfo(&free_b, &total_b));
             if (table_bytes_for(w) > free_b / 2) continue;
-            build_phase_a_table(p, slot, window_plan(w, 0), p->xext, 8192);
+            slot = build_phase_a_table(p, window_plan(w, 0), p->xext, 8192);
         }
         windows.push_back(w);
     }
@@ -1412,10 +1431,8 @@ vkzg_result vkzg_amd_load_window_table(vkzg_prover *p, uint32_t window_bits) {
         size_t free_b = 0, total_b = 0;
         ck(hipMemGetInfo(&free_b, &total_b));
         if (table_bytes_for(window_bits) > free_b) return VKZG_ERR_MALLOC;
-        build_phase_a_table(p, slot, window_plan(window_bits, 0), p->xext, 8192);
+        slot = build_phase_a_table(p, window_plan(window_bits, 0), p->xext, 8192);
     } catch (HipFail &) {
-        if (slot.table) p->arena.dfree(slot.table);
-        slot = PhaseATable{};
         return VKZG_ERR_GPU;
     }
     p->extra_named[window_bits - kExtraWindowMin] = true;

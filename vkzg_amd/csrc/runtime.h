@@ -76,6 +76,13 @@ struct HipFail {};
 inline void ck(hipError_t e) {
     if (e != hipSuccess) throw HipFail{};
 }
+// An allocation's result.  The error of one that failed is taken back: the
+// launches of a later call read hipGetLastError.
+inline void ck_alloc(hipError_t e) {
+    if (e == hipSuccess) return;
+    (void)hipGetLastError();
+    throw HipFail{};
+}
 
 struct DeviceGuard {
     int prev = 0;
@@ -92,14 +99,14 @@ struct DeviceArena {
     template <typename T>
     T *dalloc(size_t count) {
         void *ptr = nullptr;
-        ck(hipMalloc(&ptr, count * sizeof(T) ? count * sizeof(T) : 16));
+        ck_alloc(hipMalloc(&ptr, count * sizeof(T) ? count * sizeof(T) : 16));
         dev.push_back(ptr);
         return static_cast<T *>(ptr);
     }
     template <typename T>
     T *halloc(size_t count) {
         void *ptr = nullptr;
-        ck(hipHostMalloc(&ptr, count * sizeof(T) ? count * sizeof(T) : 16, hipHostMallocDefault));
+        ck_alloc(hipHostMalloc(&ptr, count * sizeof(T) ? count * sizeof(T) : 16, hipHostMallocDefault));
         host.push_back(ptr);
         return static_cast<T *>(ptr);
     }
@@ -431,9 +438,12 @@ Tuning tuning_for(const vkzg_prover *p, uint32_t nb);
 // The phase-A table a tuning names (window_bits 0: the main one).
 PhaseATable phase_a_table(const vkzg_prover *p, uint32_t window_bits);
 
-// Fills t with a multiples table of `plan` over n affine bases (device memory of
-// the prover's arena).
-void build_phase_a_table(vkzg_prover *p, PhaseATable &t, WindowPlan plan, const G1A *bases, uint32_t n);
+// A multiples table of `plan` over n affine bases (device memory of the prover's
+// arena); where a step of it fails, nothing is left of it.
+PhaseATable build_phase_a_table(vkzg_prover *p, WindowPlan plan, const G1A *bases, uint32_t n);
+// The device memory that takes: the table, and its temporaries beside it.
+uint64_t table_bytes_for(WindowPlan plan, uint32_t n);
+uint64_t table_scratch_for(WindowPlan plan, uint32_t n);
 
 // The shares phase A cuts each of nmsm MSMs into (groups != 0: that many window
 // groups), with room for `slots` partials and sums.

@@ -16,6 +16,7 @@
 //           the subgroup checks of smaller batches in the same launch);
 //   host    one 8-byte readback (verdict, error bits).
 #include <algorithm>
+#include <cstdlib>
 #include <cstring>
 #include <new>
 #include <string>
@@ -53,14 +54,14 @@ struct VerifyState {
             if (dev) (void)hipFree(dev);
             dev = nullptr;
             dev_bytes = 0;
-            ck(hipMalloc(&dev, dbytes));
+            ck_alloc(hipMalloc(&dev, dbytes));
             dev_bytes = dbytes;
         }
         if (hbytes > host_bytes) {
             if (host) (void)hipHostFree(host);
             host = nullptr;
             host_bytes = 0;
-            ck(hipHostMalloc(reinterpret_cast<void **>(&host), hbytes, hipHostMallocDefault));
+            ck_alloc(hipHostMalloc(reinterpret_cast<void **>(&host), hbytes, hipHostMallocDefault));
             host_bytes = hbytes;
         }
     }
@@ -303,18 +304,46 @@ vkzg_result locked(vkzg_prover *p, Body body) {
 // commitment call: a commitment is 4096 fixed bases against 4096 scalars, so
 // with W windows it takes 4096 W mixed additions and no buckets, sorting or
 // doublings (64 blobs: 1.25 ms on the device, 0.9 of them the additions, where
-// the bucket method they replace took 4.9).  W is the smallest of 25 and up
-// whose table fits an eighth of the free memory: 7.5 GiB at 25 (the first call
-// takes 30 ms), half as much with each step of a few windows more.
+// the bucket method took 4.9).  W is the smallest of 25 and up whose table fits
+// an eighth of the free memory, and half of it with the build's temporaries: 7.5
+// GiB and 3.5 for their time at 25 (the first call takes 30 ms), half as much with
+// each step of a few windows more, down to 128 MiB at 127.  Where none fits, or
+// its build fails, 0: commitments take the bucket method (launch_msm), whose
+// memory goes with the batch.  $VKZG_AMD_COMMIT_WINDOWS = 25..127 fixes W, 0 the
+// bucket method.
+uint32_t commit_windows(uint64_t free_bytes) {
+    if (const char *env = std::getenv("VKZG_AMD_COMMIT_WINDOWS")) {
+        const int W = std::atoi(env);
+        if (W == 0 || (W >= 25 && W <= 127)) return (uint32_t)W;
+    }
+    for (const uint32_t W : {25u, 28u, 31u, 36u, 42u, 51u, 63u, 85u, 127u}) {
+        const WindowPlan plan = window_plan(255 / W, 255 % W);
+        const uint64_t table = table_bytes_for(plan, 4096);
+        if (table <= free_bytes / 8 && table + table_scratch_for(plan, 4096) <= free_bytes / 2) return W;
+    }
+    return 0;
+}
 void build_commit_table(vkzg_prover *p, PhaseATable &t) {
     size_t free_b = 0, total = 0;
     ck(hipMemGetInfo(&free_b, &total));
-    for (const uint32_t W : {25u, 28u, 31u, 36u, 42u, 51u, 63u, 85u, 127u}) {
-        const WindowPlan plan = window_plan(255 / W, 255 % W);
-        if (W < 127 && 4096ull * plan.entries() * sizeof(G1AT) > free_b / 8) continue;
-        build_phase_a_table(p, t, plan, p->srs, 4096);
-        return;
+    const uint32_t W = commit_windows(free_b);
+    if (W == 0) return;
+    try {
+        t = build_phase_a_table(p, window_plan(255 / W, 255 % W), p->srs, 4096);
+    } catch (HipFail &) {
     }
+}
+
+// Blobs per launch sequence of the bucket method: 64, fewer where what it takes
+// (2.6 MiB per blob) is more than half of the free memory.
+uint32_t bucket_chunk(size_t held_bytes) {
+    size_t free_b = 0, total = 0;
+    ck(hipMemGetInfo(&free_b, &total));
+    uint32_t chunk = 64;
+    while (chunk > 1 && (uint64_t)chunk * (kBlobBytes + 4096 * (sizeof(Fr) + 5)) + msm_scratch_bytes(msm_shape(chunk * 4096, chunk)) >
+                            (free_b + held_bytes) / 2)
+        chunk /= 2;
+    return chunk;
 }
 constexpr uint64_t kCommitSlots = 1ull << 19;  // partials of one launch sequence (two waves on every SIMD are 2^17)
 
@@ -429,35 +458,57 @@ vkzg_result vkzg_amd_blob_to_commitments(vkzg_prover *p, uint8_t *commitments, c
         VerifyState &v = *p->vfy;
         hipStream_t s = p->stream;
         if (!v.commit.table) build_commit_table(p, v.commit);
-        const PhaseATable &tab = v.commit;
-        const uint32_t chunk = 64;  // blobs per launch sequence
+        const PhaseATable tab = v.commit;
+        const bool fixed = tab.table != nullptr;
+        const uint32_t chunk = fixed ? 64 : bucket_chunk(v.dev_bytes);  // blobs per launch sequence
         for (size_t done = 0; done < num_blobs;) {
             const uint32_t nb = (uint32_t)std::min<size_t>(chunk, num_blobs - done);
-            // 64 MSMs of 64 terms per blob, each in shares; then the sums over
-            // the shares and over a blob's 64 MSMs
-            const uint32_t nmsm = nb * 64;
-            const PhaseAShape shape = phase_a_shape(nmsm, 0, tab.W, kCommitSlots, p->cus);
-            const uint32_t shares = shape.parts * shape.groups;
             Layout l;
             const size_t o_blobs = l.take(kBlobBytes * nb), o_err = l.take(4ull * nb), o_cm = l.take(48ull * nb);
             const size_t host_bytes = l.size;
-            const size_t o_sc = l.take(sizeof(Fr) * 4096ull * nb), o_queue = l.take(4);
-            const size_t o_part = l.take(sizeof(G1X) * (size_t)nmsm * shares), o_sum = l.take(sizeof(G1X) * nmsm);
-            const size_t o_out = l.take(sizeof(G1X) * nb);
-            v.ensure(l.size, host_bytes);
+            const size_t o_sc = l.take(sizeof(Fr) * 4096ull * nb);
+            const auto upload = [&](uint8_t *D) {
+                stage_upload(p, D + o_blobs, v.host + o_blobs, blobs + done * kBlobBytes, kBlobBytes * nb, s);
+            };
+            if (fixed) {
+                // 64 MSMs of 64 terms per blob, each in shares; then the sums over
+                // the shares and over a blob's 64 MSMs
+                const uint32_t nmsm = nb * 64;
+                const PhaseAShape shape = phase_a_shape(nmsm, 0, tab.W, kCommitSlots, p->cus);
+                const uint32_t shares = shape.parts * shape.groups;
+                const size_t o_queue = l.take(4), o_part = l.take(sizeof(G1X) * (size_t)nmsm * shares);
+                const size_t o_sum = l.take(sizeof(G1X) * nmsm), o_out = l.take(sizeof(G1X) * nb);
+                v.ensure(l.size, host_bytes);
+                uint8_t *D = static_cast<uint8_t *>(v.dev);
+                upload(D);
+                Fr *sc = reinterpret_cast<Fr *>(D + o_sc);
+                uint32_t *queue = reinterpret_cast<uint32_t *>(D + o_queue);
+                G1X *part = reinterpret_cast<G1X *>(D + o_part), *out = reinterpret_cast<G1X *>(D + o_out);
+                G1X *sum = shares > 1 ? reinterpret_cast<G1X *>(D + o_sum) : part;
+                ck(launch_commit_scalars(sc, queue, nullptr, nullptr, reinterpret_cast<uint32_t *>(D + o_err),
+                                         D + o_blobs, nb, p->roots_inv, tab.plan(), s));
+                ck(launch_phase_a(part, sc, tab.table, tab.plan(), 64, nb, 1, shape.parts, shape.groups, p->cus * 2,
+                                  queue, 0, s));
+                if (shares > 1) ck(launch_sum_groups(sum, part, shares, nmsm, p->cus, 0, s));
+                ck(launch_sum_groups(out, sum, 64, nb, p->cus, 0, s));
+                ck(launch_compress_points(D + o_cm, out, nb, s));
+            } else {
+                const uint32_t ne = nb * 4096;
+                const MsmShape sh = msm_shape(ne, nb);
+                const size_t o_pidx = l.take(4ull * ne), o_mid = l.take(ne), o_out = l.take(sizeof(G1A) * nb);
+                const size_t o_msm = l.take(msm_scratch_bytes(sh));
+                v.ensure(l.size, host_bytes);
+                uint8_t *D = static_cast<uint8_t *>(v.dev);
+                upload(D);
+                Fr *sc = reinterpret_cast<Fr *>(D + o_sc);
+                uint32_t *pidx = reinterpret_cast<uint32_t *>(D + o_pidx);
+                G1A *out = reinterpret_cast<G1A *>(D + o_out);
+                ck(launch_commit_scalars(sc, nullptr, pidx, D + o_mid, reinterpret_cast<uint32_t *>(D + o_err),
+                                         D + o_blobs, nb, p->roots_inv, WindowPlan{}, s));
+                ck(launch_msm(sh, D + o_msm, p->srs, pidx, sc, D + o_mid, out, p->cus, s));
+                ck(launch_compress_affine(D + o_cm, out, nb, s));
+            }
             uint8_t *H = v.host, *D = static_cast<uint8_t *>(v.dev);
-            stage_upload(p, D + o_blobs, H + o_blobs, blobs + done * kBlobBytes, kBlobBytes * nb, s);
-            Fr *sc = reinterpret_cast<Fr *>(D + o_sc);
-            uint32_t *queue = reinterpret_cast<uint32_t *>(D + o_queue);
-            G1X *part = reinterpret_cast<G1X *>(D + o_part), *out = reinterpret_cast<G1X *>(D + o_out);
-            G1X *sum = shares > 1 ? reinterpret_cast<G1X *>(D + o_sum) : part;
-            ck(launch_commit_scalars(sc, queue, reinterpret_cast<uint32_t *>(D + o_err), D + o_blobs, nb, p->roots_inv,
-                                     tab.plan(), s));
-            ck(launch_phase_a(part, sc, tab.table, tab.plan(), 64, nb, 1, shape.parts, shape.groups, p->cus * 2, queue,
-                              0, s));
-            if (shares > 1) ck(launch_sum_groups(sum, part, shares, nmsm, p->cus, 0, s));
-            ck(launch_sum_groups(out, sum, 64, nb, p->cus, 0, s));
-            ck(launch_compress_points(D + o_cm, out, nb, s));
             enqueue_copies(CopyPart{H + o_err, D + o_err, 4 * nb}, CopyPart{H + o_cm, D + o_cm, 48 * nb},
                            hipMemcpyDeviceToHost, s);
             ck(hipStreamSynchronize(s));

@@ -23,8 +23,9 @@ hipError_t launch_vfy_interp(Fr *part, Fr *agg, const uint32_t *chunks, uint32_t
 hipError_t launch_vfy_entries(Fr *sc, uint32_t *pidx, uint8_t *mid, const Fr *rp, const uint32_t *cgrp_off,
                               const uint32_t *cgrp, const uint32_t *cell_idx, const Fr *roots, const Fr *agg,
                               uint32_t n, uint32_t u, hipStream_t s);
-hipError_t launch_commit_scalars(Fr *sc, uint32_t *queue, uint32_t *err, const uint8_t *blobs, uint32_t nb,
-                                 const Fr *roots_inv, WindowPlan plan, hipStream_t s);
+hipError_t launch_commit_scalars(Fr *sc, uint32_t *queue, uint32_t *pidx, uint8_t *mid, uint32_t *err,
+                                 const uint8_t *blobs, uint32_t nb, const Fr *roots_inv, WindowPlan plan,
+                                 hipStream_t s);
 hipError_t launch_compress_points(uint8_t *out, const G1X *pts, uint32_t n, hipStream_t s);
 hipError_t launch_compress_affine(uint8_t *out, const G1A *pts, uint32_t n, hipStream_t s);
 
