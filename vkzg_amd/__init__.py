@@ -66,6 +66,16 @@ class _Out:
         self.at = _bytes_at(self.value)
 
 
+def _in(data):
+    """len(data) bytes for the library, without a copy where data is bytes.  Wider
+    elements (an array of 16-bit numbers) hold more: refused; a shorter bytes() is
+    filled up with zeros."""
+    raw = bytes(data)
+    if len(raw) > len(data):
+        raise ValueError("byte string too long")
+    return raw if len(raw) == len(data) else raw.ljust(len(data), b"\0")
+
+
 class Prover:
     """One vkzg_prover on the current HIP device."""
 
@@ -119,7 +129,7 @@ class Prover:
             raise ValueError("blobs.length must be blobCount * %d" % BYTES_PER_BLOB)
         nbytes = blob_count * CELL_PROOFS_PER_BLOB * BYTES_PER_PROOF
         out = _Out(nbytes)
-        _check(load().vkzg_compute_proofs_batch(self._h, out.at, bytes(blobs), blob_count))
+        _check(load().vkzg_compute_proofs_batch(self._h, out.at, _in(blobs), blob_count))
         return out.value
 
     def recover_cells_batch(self, cells, cell_present, blob_count):
@@ -129,7 +139,7 @@ class Prover:
         if len(cell_present) != blob_count * CELL_PROOFS_PER_BLOB:
             raise ValueError("cellPresent.length must be blobCount * %d" % CELL_PROOFS_PER_BLOB)
         out = _Out(len(cells))
-        _check(load().vkzg_recover_cells_batch(self._h, out.at, bytes(cells), bytes(cell_present), blob_count))
+        _check(load().vkzg_recover_cells_batch(self._h, out.at, _in(cells), _in(cell_present), blob_count))
         return out.value
 
     def compute_cells_and_kzg_proofs_batch(self, blobs, blob_count):
@@ -139,7 +149,7 @@ class Prover:
         ncells = blob_count * CELL_PROOFS_PER_BLOB * BYTES_PER_CELL
         nproofs = blob_count * CELL_PROOFS_PER_BLOB * BYTES_PER_PROOF
         cells, proofs = _Out(ncells), _Out(nproofs)
-        _check(load().vkzg_amd_compute_cells_and_proofs(self._h, cells.at, proofs.at, bytes(blobs), blob_count))
+        _check(load().vkzg_amd_compute_cells_and_proofs(self._h, cells.at, proofs.at, _in(blobs), blob_count))
         return cells.value, proofs.value
 
     def recover_cells_and_kzg_proofs_batch(self, cells, cell_present, blob_count):
@@ -151,7 +161,7 @@ class Prover:
             raise ValueError("cellPresent.length must be blobCount * %d" % CELL_PROOFS_PER_BLOB)
         nproofs = blob_count * CELL_PROOFS_PER_BLOB * BYTES_PER_PROOF
         out, proofs = _Out(len(cells)), _Out(nproofs)
-        _check(load().vkzg_amd_recover_cells_and_proofs(self._h, out.at, proofs.at, bytes(cells), bytes(cell_present),
+        _check(load().vkzg_amd_recover_cells_and_proofs(self._h, out.at, proofs.at, _in(cells), _in(cell_present),
                                                         blob_count))
         return out.value, proofs.value
 
@@ -198,7 +208,7 @@ class Prover:
         if len(blobs) != blob_count * BYTES_PER_BLOB:
             raise ValueError("blobs.length must be blobCount * %d" % BYTES_PER_BLOB)
         out = _Out(48 * blob_count)
-        _check(load().vkzg_amd_blob_to_commitments(self._h, out.at, bytes(blobs), blob_count))
+        _check(load().vkzg_amd_blob_to_commitments(self._h, out.at, _in(blobs), blob_count))
         return out.value
 
     def debug_pairing(self, g1_points, g2_points):
@@ -273,7 +283,7 @@ class Prover:
                                                      stream))
 
     def recover_cells_device(self, d_out, d_cells, d_present, h_present, blob_count, stream=None):
-        _check(load().vkzg_amd_recover_cells_device(self._h, d_out, d_cells, d_present, bytes(h_present),
+        _check(load().vkzg_amd_recover_cells_device(self._h, d_out, d_cells, d_present, _in(h_present),
                                                     blob_count, stream))
 
 
