@@ -18,6 +18,7 @@
 #pragma once
 
 #include "curve.h"
+#include "fp12_tree.h"
 
 namespace vkzg_amd {
 
@@ -103,50 +104,29 @@ VKZG_DEV bool fp2_is_lex_largest(const Fp2 &y) {
 
 // ------------------------------------------------------------ Fp12 in LDS
 
-VKZG_DEV Fp fp_shfl_xor(const Fp &v, int mask) {
-    Fp r;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) r.v[i] = __shfl_xor(v.v[i], mask);
-    return r;
-}
-
-// DPP within rows of 16 lanes: lane l takes the value of lane l + n (kRowShl + n,
-// lanes past the row's end 0) or l - n mod 16 (kRowRor + n).
-constexpr int kRowShl = 0x100, kRowRor = 0x120;
-template <int CTRL>
-VKZG_DEV Fp fp_row_dpp(const Fp &v) {
-    Fp r;
-#pragma unroll
-    for (int i = 0; i < kFpLimbs; i++) r.v[i] = __builtin_amdgcn_mov_dpp(v.v[i], CTRL, 0xf, 0xf, true);
-    return r;
-}
-
 constexpr uint32_t kFp12Threads = 192;  // lanes an Fp12 product uses (blockDim.x >= this)
 
 // dst = a * b for Fp12 values held in LDS (12 Fp each).  Every thread of the
 // block calls it (it contains barriers); blockDim.x >= 192.  dst may alias a
-// or b.  Lane t works on output power M = t / 32 and on term m1 = (t % 32) / 4
-// (terms 6 and 7 of a group are empty): the quad's four lanes multiply
+// or b.  Lane t works on output power M = t / 32 and on term m1 of it, four lanes
+// to a term (fp12_term): the quad's lanes multiply
 // a_{m1} (times xi when m1 + m2 >= 6: (x + y u) xi = (x - y) + (x + y) u, an
 // N2 operand) and b_{m2}, m2 = M - m1 mod 6, component by component, DPP quad
 // broadcasts give every lane the four products, lane 0 of the quad forms the
 // real and lane 1 the imaginary part of the term, and a tree over the group's
-// eight quads (rotations of a row of 16 lanes by DPP, then the other row) adds
-// the six terms.  A term's limbs are below 2^30 and
-// the sum of two just fits 32 bits, so the tree takes one carry pass after its
-// first level and one at its end.  The result is 12 products of magnitude
+// quads (fp12_tree) adds the six terms.  The result is 12 products of magnitude
 // c p: operands of up to 12.3p give c <= 2 * 12.3 * 12.3 / 630 + 1/2 < 0.981 and
 // so a result below 11.8p, a valid operand of the next product or square.
 // Operands and result stay in LDS; the partial sums never leave registers.
 __device__ __forceinline__ void fp12_mul_lds(Fp *dst, const Fp *a, const Fp *b) {
     const uint32_t t = threadIdx.x;
-    const uint32_t M = (t / 32) % 6, m1 = (t % 32) / 4, q = t & 3u;
-    const bool term = t < kFp12Threads && m1 < 6;
-    const uint32_t m1c = term ? m1 : 0;
-    const uint32_t m2 = (M + 6 - m1c) % 6;
-    const bool wrap = m1c > M;
+    const uint32_t M = (t / 32) % 6, q = t & 3u;
+    const bool term = t < kFp12Threads && fp12_has_term(t);
+    const uint32_t m1 = term ? fp12_term(t) : 0;
+    const uint32_t m2 = (M + 6 - m1) % 6;
+    const bool wrap = m1 > M;
     const uint32_t e = q >> 1;
-    const Fp x_in = a[2 * m1c + e], x_other = a[2 * m1c + (e ^ 1u)];
+    const Fp x_in = a[2 * m1 + e], x_other = a[2 * m1 + (e ^ 1u)];
     const Fp y_in = b[2 * m2 + (q & 1u)];
     __syncthreads();  // dst may alias a or b
     // wrapped: real part a0 - a1, imaginary part a1 + a0
@@ -159,10 +139,8 @@ __device__ __forceinline__ void fp12_mul_lds(Fp *dst, const Fp *a, const Fp *b) 
     const Fp p10 = fp_quad_bcast<2>(prod), p11 = fp_quad_bcast<3>(prod);
     Fp v = fp_select(q == 0, fp_sub_raw(p00, p11), fp_add_raw(p01, p10));
     if (!term || q > 1) v = fp_zero();
-    v = fp_norm_wide(fp_add_raw(v, fp_row_dpp<kRowRor + 4>(v)));
-    v = fp_add_raw(v, fp_row_dpp<kRowRor + 8>(v));
-    v = fp_add_raw(v, fp_shfl_xor(v, 16));
-    if (t < kFp12Threads && (t % 32) < 2) dst[2 * M + (t % 32)] = fp_norm_wide(v);
+    v = fp12_tree(v);
+    if (t < kFp12Threads && (t % 32) < 2) dst[2 * M + (t % 32)] = v;
     __syncthreads();
 }
 
