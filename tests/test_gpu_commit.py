@@ -82,3 +82,17 @@ def test_smaller_plans(seeded_setup_bytes, oracle_mod, monkeypatch, windows):
         with pytest.raises(vkzg_amd.VkzgError) as e:
             p.blob_to_kzg_commitments(one[1] + bytes(bad), 2)
         assert e.value.code == vkzg_amd.ERR_INVALID_BLOB
+
+
+@pytest.mark.parametrize("windows", [25, 85])
+def test_points_of_order_three(monkeypatch, windows):
+    """A setup whose points are all (0, 2), of order 3 on the curve: every run of
+    multiples in the tables meets a cancellation and is made again with checked
+    additions."""
+    monkeypatch.setenv("VKZG_AMD_COMMIT_WINDOWS", str(windows))
+    monkeypatch.setenv("VKZG_AMD_WINDOW", "6")
+    point = {0: bytes([0xC0]) + bytes(47), 1: bytes([0x80]) + bytes(47), 2: bytes([0xA0]) + bytes(47)}
+    cases = [(0, 1), (65, 2), (4095, 3), (7, 511), (8, 512), (9, 513), (10, 1 << 200), (11, 3 << 100), (12, (1 << 253) + 1)]
+    with vkzg_amd.Prover(max_batch_size=1, setup_g1_monomial=point[1] * 4096) as p:
+        got = p.blob_to_kzg_commitments(b"".join(monomials([x]) for x in cases), len(cases))
+    assert [got[48 * n:48 * (n + 1)] for n in range(len(cases))] == [point[c % 3] for _, c in cases]

@@ -7,6 +7,7 @@ in through embed_setup.S.  Run:  python3 vkzg_amd/build.py [-j N]
 import argparse
 import concurrent.futures as cf
 import os
+import struct
 import subprocess
 import sys
 
@@ -57,6 +58,57 @@ def compile_one(src):
     return obj
 
 
+# A branch of the device's instruction set reaches +-32767 words.  In a function
+# past that the compiler goes through a register pair for a far branch, and may
+# take the one that holds the return address of a function that saves none: the
+# function then returns into itself.  Kernels do not return and may be longer.
+BRANCH_REACH = 32767 * 4
+
+
+def device_functions(lib):
+    """{name: bytes} of the functions in the library's device code that are not kernels."""
+    data = open(lib, "rb").read()
+    out = {}
+    at = data.find(b"__CLANG_OFFLOAD_BUNDLE__")
+    while at >= 0:
+        n, = struct.unpack_from("<Q", data, at + 24)
+        entry = at + 32
+        for _ in range(n):
+            off, size, name = struct.unpack_from("<QQQ", data, entry)
+            triple = data[entry + 24:entry + 24 + name]
+            entry += 24 + name
+            if triple.startswith(b"hip") and size:
+                out.update(_functions(data[at + off:at + off + size]))
+        at = data.find(b"__CLANG_OFFLOAD_BUNDLE__", at + 24)
+    return out
+
+
+def _functions(elf):
+    """{name: bytes} of an ELF64 code object's functions without a kernel descriptor (name.kd)."""
+    shoff, = struct.unpack_from("<Q", elf, 40)
+    shentsize, shnum = struct.unpack_from("<HH", elf, 58)
+    sections = [struct.unpack_from("<IIQQQQIIQQ", elf, shoff + k * shentsize) for k in range(shnum)]
+    functions, kernels = {}, set()
+    for kind, offset, size, link in [(s[1], s[4], s[5], s[6]) for s in sections]:
+        if kind != 2:  # SHT_SYMTAB
+            continue
+        names = sections[link][4]
+        for at in range(offset, offset + size, 24):
+            name, info, _, shndx, _, bytes_ = struct.unpack_from("<IBBHQQ", elf, at)
+            text = elf[names + name:elf.index(b"\0", names + name)].decode()
+            if text.endswith(".kd"):
+                kernels.add(text[:-3])
+            elif info & 15 == 2 and shndx:  # STT_FUNC, defined
+                functions[text] = bytes_
+    return {f: b for f, b in functions.items() if f not in kernels}
+
+
+def check_device_functions(lib, limit=BRANCH_REACH):
+    far = sorted("%s (%d bytes)" % (f, b) for f, b in device_functions(lib).items() if b > limit)
+    if far:
+        raise RuntimeError("device functions longer than a branch reaches: " + ", ".join(far))
+
+
 def build(jobs=8, verbose=True):
     os.makedirs(OUT_DIR, exist_ok=True)
     setup_file = os.path.join(HERE, "data", "g1_monomial_mainnet.bin")
@@ -70,6 +122,7 @@ def build(jobs=8, verbose=True):
     # extern "C" functions keep default visibility in the objects.
     run([HIPCC, "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", tmp] + objs + [embed_obj] +
         ["-Wl,--version-script=" + os.path.join(CSRC, "exports.map")])
+    check_device_functions(tmp)
     os.replace(tmp, LIB)
     if verbose:
         print("built", LIB)

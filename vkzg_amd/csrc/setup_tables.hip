@@ -64,21 +64,30 @@ __global__ void k_table_chains(G1J *out, const G1A *bases, uint32_t n, WindowPla
 }
 
 // The running sum d0*P, (d0+1)*P, ... with checked additions (rare fallback).
+// d0 P's additions and the run's go through one copy of the addition: with two,
+// the function is longer than a branch reaches.
 __device__ __attribute__((noinline)) void table_run_slow(G1J *scratch, Fp *prefix, Fp *acc_out,
                                                          G1A P, uint32_t d0, uint32_t S,
                                                          uint32_t thread_count, uint32_t lt) {
     G1J q = g1j_identity();
-    for (int bit = 31 - __builtin_clz(d0); bit >= 0; bit--) {
-        q = g1j_dbl(q);
-        if ((d0 >> bit) & 1u) q = g1j_madd(q, P);
-    }
     Fp acc = fp_one();
-    for (uint32_t m = 0; m < S; m++) {
-        const size_t slot = (size_t)m * thread_count + lt;
-        scratch[slot] = q;
-        prefix[slot] = acc;
-        if (!fp_is_zero(q.z)) acc = fp_mul(acc, q.z);
-        q = g1j_madd(q, P);
+    int bit = 31 - __builtin_clz(d0);
+    uint32_t m = 0;
+#pragma unroll 1
+    while (bit >= 0 || m < S) {
+        bool add = true;
+        if (bit >= 0) {
+            q = g1j_dbl(q);
+            add = ((d0 >> bit) & 1u) != 0;
+            bit--;
+        } else {
+            const size_t slot = (size_t)m * thread_count + lt;
+            scratch[slot] = q;
+            prefix[slot] = acc;
+            if (!fp_is_zero(q.z)) acc = fp_mul(acc, q.z);
+            m++;
+        }
+        if (add) q = g1j_madd(q, P);
     }
     *acc_out = acc;
 }
