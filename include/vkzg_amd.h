@@ -168,7 +168,10 @@ vkzg_result vkzg_amd_load_window_table(vkzg_prover *p, uint32_t window_bits);
 
 /* The tuning used for a batch of `num_blobs` blobs. */
 vkzg_result vkzg_amd_get_tuning(const vkzg_prover *p, size_t num_blobs, vkzg_amd_tuning *out);
-/* Sets the tuning of the size class of `num_blobs`; BADARGS when a field is out of range. */
+/* Sets the tuning of the size class of `num_blobs`; BADARGS when a field is out of range.
+ * What get_tuning reported for `num_blobs` puts the class back to what it was: a phase_a_groups
+ * or reduce_lanes equal to the fit for num_blobs (beside the other fields given) leaves that
+ * field fitted to every batch of the class, unless the autotuner has chosen it. */
 vkzg_result vkzg_amd_set_tuning(vkzg_prover *p, size_t num_blobs, const vkzg_amd_tuning *t);
 /* Replays of captured HIP graphs by the host-buffer calls on (enable != 0, the
  * default unless VKZG_AMD_GRAPHS=0) or off (every call launches its kernels

@@ -210,7 +210,9 @@ hipError_t hipEventDestroy(hipEvent_t e) {
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {
-    *ms = 1.0f;
+    static uint32_t x = 1;  // different times, so that a tuner chooses
+    x = x * 1664525u + 1013904223u;
+    *ms = 1.0f + (float)(x >> 8) / (1 << 24);
     return hipSuccess;
 }
 

@@ -101,3 +101,43 @@ with vkzg_amd.Prover(max_batch_size=1) as p:
         assert launches("k_msm_buckets") == 0 and table <= held < table + (16 << 20) and table <= free * GIB / 8
     p.blob_to_kzg_commitments(bytes(65 * BLOB), 65)
 """ % (free_gib, windows))
+
+
+def test_a_tuning_can_be_put_back(run):
+    """Fields that are fitted to each batch are fitted again, at every size of the
+    class, after a tuning that get_tuning reported is set: straight away, after a
+    change in between, and after one that touched another field only.  What is set
+    is what get_tuning reports for that size."""
+    run("""
+classes = [(1,), range(2, 5), range(5, 17), range(17, 65), (65, 100, 200, 256)]
+with vkzg_amd.Prover(max_batch_size=256) as p:
+    want = {n: p.get_tuning(n) for c in classes for n in c}
+    assert len({(t["phase_a_groups"], t["reduce_lanes"]) for t in want.values()}) > 4  # the fits do vary
+    for c in classes:
+        for n in c:
+            saved = p.get_tuning(n)
+            p.set_tuning(n, **saved)
+            assert all(p.get_tuning(m) == want[m] for m in c), n
+            for change in (dict(phase_a_groups=3), dict(reduce_lanes=8, phase_a_groups=20, ladder_splits=4),
+                           dict(ladder_splits=2), dict(splits=2), dict(phase_a_groups=7, splits=3)):
+                p.set_tuning(n, **change)
+                assert p.get_tuning(n) == dict(saved, **change), (n, change)
+                p.set_tuning(n, **saved)
+                assert all(p.get_tuning(m) == want[m] for m in c), (n, change)
+    p.set_tuning(11, splits=2)
+    assert all(p.get_tuning(m) == dict(want[m], splits=2) for m in classes[2])
+    for bad in (dict(phase_a_groups=0), dict(reduce_lanes=0), dict(phase_a_groups=21)):
+        try:
+            p.set_tuning(3, **bad)
+            assert False, bad
+        except vkzg_amd.VkzgError as e:
+            assert e.code == vkzg_amd.ERR_BADARGS
+    p.autotune()  # its choices are pinned, and stay so
+    tuned = {n: p.get_tuning(n) for c in classes for n in c}
+    assert sum(len({tuned[n]["phase_a_groups"] for n in c}) == 1 for c in classes[1:]) > 0
+    assert sum(len({tuned[n]["reduce_lanes"] for n in c}) == 1 for c in classes[1:]) > 0
+    for n in (1, 3, 11, 40, 200):
+        p.set_tuning(n, phase_a_groups=9)
+        p.set_tuning(n, **tuned[n])
+    assert all(p.get_tuning(n) == t for n, t in tuned.items())
+""")

@@ -450,6 +450,7 @@ void default_tunings(vkzg_prover *p) {
         p->tune[c].ladder_splits = ladder_splits[c];
         p->tune[c].reduce_lanes = 0;
         p->tune[c].norm_chunk = 0;
+        p->tune_base[c] = p->tune[c];
     }
 }
 
@@ -1016,6 +1017,10 @@ void autotune(vkzg_prover *p) {
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
+    {
+        std::lock_guard<std::mutex> lock(p->tune_mu);
+        std::copy(std::begin(p->tune), std::end(p->tune), std::begin(p->tune_base));
+    }
     p->autotuned = true;
     p->autotune_ms =
         std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
@@ -1367,14 +1372,9 @@ vkzg_result vkzg_amd_recover_cells_device(vkzg_prover *p, void *d_cells_out, con
     return VKZG_OK;
 }
 
-vkzg_result vkzg_amd_get_tuning(const vkzg_prover *p, size_t num_blobs, vkzg_amd_tuning *out) {
-    if (!p || !out || num_blobs == 0) return VKZG_ERR_BADARGS;
-    Tuning t;
-    {
-        std::lock_guard<std::mutex> lock(p->tune_mu);
-        t = p->tune[tune_class((uint32_t)std::min<size_t>(num_blobs, 0xffffffffu))];
-    }
-    // fitted: what a batch of this size takes
+// t with the groups and reduce_lanes that a batch of num_blobs takes in the place
+// of fitted ones.
+static Tuning with_fits(const vkzg_prover *p, Tuning t, size_t num_blobs) {
     const uint32_t nb = (uint32_t)std::min<size_t>(num_blobs, p->max_batch);
     if (!t.reduce_lanes) t.reduce_lanes = fit_reduce_lanes(nb, p->cus);
     if (!t.groups) {
@@ -1382,6 +1382,17 @@ vkzg_result vkzg_amd_get_tuning(const vkzg_prover *p, size_t num_blobs, vkzg_amd
                                  (uint64_t)std::max(p->max_batch, kMinPartialBlobs) * kSlotsPerBlob, p->cus)
                        .groups;
     }
+    return t;
+}
+
+vkzg_result vkzg_amd_get_tuning(const vkzg_prover *p, size_t num_blobs, vkzg_amd_tuning *out) {
+    if (!p || !out || num_blobs == 0) return VKZG_ERR_BADARGS;
+    Tuning t;
+    {
+        std::lock_guard<std::mutex> lock(p->tune_mu);
+        t = p->tune[tune_class((uint32_t)std::min<size_t>(num_blobs, 0xffffffffu))];
+    }
+    t = with_fits(p, t, num_blobs);
     out->phase_a_groups = t.groups;
     out->phase_a_blocks_per_cu = t.blocks_per_cu;
     out->normalize_chunk = t.norm_chunk;
@@ -1413,7 +1424,15 @@ vkzg_result vkzg_amd_set_tuning(vkzg_prover *p, size_t num_blobs, const vkzg_amd
         p->extra_named[t.window_bits - kExtraWindowMin] = true;
     }
     std::lock_guard<std::mutex> tlock(p->tune_mu);
-    p->tune[tune_class((uint32_t)std::min<size_t>(num_blobs, 0xffffffffu))] = t;
+    const int c = tune_class((uint32_t)std::min<size_t>(num_blobs, 0xffffffffu));
+    // What get_tuning reports for a fitted field puts it back to fitted, where the
+    // class had it so before any call of this function.
+    Tuning fit = t;
+    fit.groups = fit.reduce_lanes = 0;
+    fit = with_fits(p, fit, num_blobs);
+    if (p->tune_base[c].groups == 0 && t.groups == fit.groups) t.groups = 0;
+    if (p->tune_base[c].reduce_lanes == 0 && t.reduce_lanes == fit.reduce_lanes) t.reduce_lanes = 0;
+    p->tune[c] = t;
     return VKZG_OK;
 }
 

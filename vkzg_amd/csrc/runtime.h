@@ -355,6 +355,7 @@ struct vkzg_prover {
     // without holding mu.
     mutable std::mutex tune_mu;
     vkzg_amd::Tuning tune[vkzg_amd::kTuneClasses];
+    vkzg_amd::Tuning tune_base[vkzg_amd::kTuneClasses];  // before any set_tuning: the defaults, or the autotuner's choice
     std::atomic<uint32_t> force_checked{0};  // vkzg_amd_debug_force_checked
     bool autotuned = false;
     double autotune_ms = 0;
