@@ -129,7 +129,8 @@ typedef struct {
     uint32_t autotuned;        /* 1 after vkzg_amd_autotune */
     double autotune_ms;        /* its wall time */
     uint32_t phase_b_items;    /* bucket items (point additions) one blob's 128 phase-B outputs add up */
-    uint64_t resident_table_bytes; /* the main phase-A table plus any smaller ones the autotuner kept */
+    uint64_t resident_table_bytes; /* the main phase-A table, any smaller ones kept beside it, and the
+                                      commitments' table once a commitment call has built it */
     uint32_t extra_table_windows;  /* bit c set: a smaller phase-A table of window c is resident */
 } vkzg_amd_info;
 
@@ -190,9 +191,9 @@ vkzg_result vkzg_amd_autotune(vkzg_prover *p, double *ms_out);
  * device batches of up to `batch_blobs` blobs and runs up to `slots` batches
  * at once, each with its own device working set; requests arriving while
  * batches run join the next free slot.  `hbm_budget_bytes` caps the device
- * memory of the prover's resident phase-A tables plus the slots' working
- * sets (fewer slots, then smaller batches); a budget the tables alone fill
- * is VKZG_ERR_MALLOC.  Request buffers belong to the
+ * memory of the prover's resident tables (vkzg_amd_info.resident_table_bytes)
+ * plus the slots' working sets (fewer slots, then smaller batches); a budget
+ * the tables alone fill is VKZG_ERR_MALLOC.  Request buffers belong to the
  * caller and must stay valid until vkzg_amd_server_wait returns.  A request
  * with an invalid blob fails alone (VKZG_ERR_INVALID_BLOB, its outputs
  * unspecified); more than 64 missing cells is rejected at submission.
@@ -213,7 +214,8 @@ typedef struct {
 typedef struct {
     uint64_t requests, blobs, batches;
     uint32_t slots, batch_blobs;
-    uint64_t slot_bytes;
+    uint64_t slot_bytes;      /* working set of a slot; one of under 8 blobs takes up to 16 MB beside it, for speed,
+                                 where hbm_budget_bytes leaves room for that */
 } vkzg_amd_server_counters;
 
 void vkzg_amd_server_options_default(vkzg_amd_server_options *opts);

@@ -40,3 +40,19 @@ def test_smallest_prover(vectors, monkeypatch):
     with vkzg_amd.Prover(max_batch_size=1) as p:
         blobs, want = batch(vectors, 2)
         assert p.compute_cell_kzg_proofs_batch(blobs, 2) == want
+
+
+@pytest.mark.parametrize("cap", [1, 3])
+def test_slots_without_room_to_spare(gpu_prover, vectors, cap):
+    """A server whose budget leaves its slots no room beside their working sets:
+    phase A's partials reach into the memory of the buckets."""
+    info = gpu_prover.info()
+    with vkzg_amd.Server(gpu_prover, batch_blobs=1, slots=1) as one:
+        per_blob = one.stats()["slot_bytes"]
+    with vkzg_amd.Server(gpu_prover, batch_blobs=cap, slots=1,
+                         hbm_budget_bytes=info["resident_table_bytes"] + cap * per_blob) as srv:
+        assert srv.stats()["batch_blobs"] == cap
+        for n in (1, 2, cap, 7):
+            blobs, want = batch(vectors, n)
+            for _ in range(3):  # captured, then replayed
+                assert srv.wait(srv.submit_proofs(blobs, n))[0] == want

@@ -141,3 +141,50 @@ with vkzg_amd.Prover(max_batch_size=256) as p:
         p.set_tuning(n, **tuned[n])
     assert all(p.get_tuning(n) == t for n, t in tuned.items())
 """)
+
+
+def test_resident_tables_count_the_commitments_table(run):
+    run("""
+with vkzg_amd.Prover(max_batch_size=1) as p:
+    one = p.info()["resident_table_bytes"]
+    vkzg_amd.Server(p, batch_blobs=1, slots=1, hbm_budget_bytes=one + (64 << 20)).close()
+    before = H.host_live()
+    p.blob_to_kzg_commitments(bytes(BLOB), 1)
+    two = p.info()["resident_table_bytes"]
+    table = 4096 * 30 * 512 * 128  # 25 windows, 5 of them a bit wider
+    assert two - one == table and table <= H.host_live() - before < table + (32 << 20)
+    for budget in (one + (64 << 20), two):
+        try:
+            vkzg_amd.Server(p, batch_blobs=1, slots=1, hbm_budget_bytes=budget)
+            assert False, budget
+        except vkzg_amd.VkzgError as e:
+            assert e.code == vkzg_amd.ERR_MALLOC
+    vkzg_amd.Server(p, batch_blobs=1, slots=1, hbm_budget_bytes=two + (64 << 20)).close()
+""")
+
+
+def test_a_servers_slots_stay_within_its_budget(run):
+    """What a server allocates is what its budget leaves beside the tables, with
+    slots of one blob and of many; the prover reports its own working set whole."""
+    run("""
+for n in (1, 2, 7, 8, 20):
+    before = H.host_live()
+    with vkzg_amd.Prover(max_batch_size=n) as p:
+        info = p.info()
+        took = H.host_live() - before - info["resident_table_bytes"]
+        assert 0 <= took - info["working_bytes"] < 4 << 20, (n, took, info)  # the setup's points, roots and items
+with vkzg_amd.Prover(max_batch_size=20) as p:
+    tables = p.info()["resident_table_bytes"]
+    with vkzg_amd.Server(p, batch_blobs=1, slots=1) as s:
+        per_blob = s.stats()["slot_bytes"]
+    for blobs, slots in ((1, 1), (1, 4), (3, 2), (7, 1), (8, 2), (64, 3)):
+        for room in (1.0, 1.5, 2.0, 4.2, 9.9, 30.0):
+            budget = tables + int(per_blob * room)
+            before = H.host_live()
+            with vkzg_amd.Server(p, batch_blobs=blobs, slots=slots, hbm_budget_bytes=budget) as s:
+                st = s.stats()
+                took = H.host_live() - before
+                assert took <= budget - tables, (blobs, slots, room, took)
+                assert st["slots"] * st["slot_bytes"] <= took <= st["slots"] * (st["slot_bytes"] + (16 << 20))
+                assert st["batch_blobs"] == min(blobs, int(room))
+""")

@@ -387,7 +387,11 @@ uint64_t WorkSet::bytes_per_blob() {
            2 * 8192 * sizeof(Fr);
 }
 
-void WorkSet::allocate(uint32_t B) {
+uint64_t WorkSet::spread_bytes(uint32_t B) {
+    return B < kMinPartialBlobs ? (kMinPartialBlobs - B) * kSlotsPerBlob * sizeof(G1X) : 0;
+}
+
+void WorkSet::allocate(uint32_t B, bool spread) {
     cap = B;
     blobs = arena.dalloc<uint8_t>((size_t)B * kBlobBytes);
     proofs = arena.dalloc<uint8_t>((size_t)B * kProofBytes);
@@ -399,14 +403,14 @@ void WorkSet::allocate(uint32_t B) {
     queue_r = arena.dalloc<uint32_t>(B);
     ck(hipMemset(queue_r, 0, (size_t)B * sizeof(uint32_t)));
     scal = arena.dalloc<Fr>((size_t)B * 128 * 64 * kMaxLadSplits);
-    // room for a few blobs' partials at least, so that one blob can be spread too
-    u_slots = (uint64_t)std::max(B, kMinPartialBlobs) * kSlotsPerBlob;
+    const size_t partials = (spread ? std::max(B, kMinPartialBlobs) : B) * kSlotsPerBlob;
+    u_slots = partials + (uint64_t)B * 128 * kBuckets;
     u = arena.dalloc<G1X>((size_t)u_slots);
+    buckets = u + partials;
     lad = arena.dalloc<G1J>((size_t)B * 128 * kLadPos);
     lad_aff = arena.dalloc<G1A>((size_t)B * 128 * kLadPos);
     lad_phi = arena.dalloc<G1A>((size_t)B * 128 * kLadPos);
     prefix = arena.dalloc<Fp>((size_t)B * 128 * kLadPos);
-    buckets = arena.dalloc<G1X>((size_t)B * 128 * kBuckets);
     bucket_flags = arena.dalloc<uint8_t>((size_t)B * 128 * kBuckets);
     cval_flags = arena.dalloc<uint8_t>((size_t)B * 128);
     cvals = arena.dalloc<G1X>((size_t)B * 128);
@@ -586,7 +590,7 @@ void proofs_range(vkzg_prover *p, WorkSet &ws, uint32_t off, uint32_t nb, uint8_
     uint32_t *queue = ws.queue + off;
     Fr *scal = ws.scal + (size_t)off * 8192 * kMaxLadSplits;
     // phase-A partials [nb][splits][128][shares], then their sums
-    // [nb][splits][128].  A batch in one stream may use the whole buffer, a
+    // [nb][splits][128].  A batch in one stream may use all the room there is, a
     // sub-batch the slots of its own blobs.
     const uint64_t nmsm = (uint64_t)nb * 128 * tn.ladder_splits;
     const uint64_t slots = tn.splits == 1 && off == 0 ? ws.u_slots : (uint64_t)nb * kSlotsPerBlob;
@@ -1379,7 +1383,7 @@ static Tuning with_fits(const vkzg_prover *p, Tuning t, size_t num_blobs) {
     if (!t.reduce_lanes) t.reduce_lanes = fit_reduce_lanes(nb, p->cus);
     if (!t.groups) {
         t.groups = phase_a_shape((uint64_t)nb * 128 * t.ladder_splits, 0, phase_a_table(p, t.window_bits).W,
-                                 (uint64_t)std::max(p->max_batch, kMinPartialBlobs) * kSlotsPerBlob, p->cus)
+                                 p->ws.u_slots, p->cus)
                        .groups;
     }
     return t;
@@ -1489,14 +1493,14 @@ vkzg_result vkzg_amd_prover_info(const vkzg_prover *p, vkzg_amd_info *out) {
     out->window_bits = p->c;
     out->windows = p->W;
     out->table_bytes = p->table_bytes;
-    out->resident_table_bytes = p->table_bytes;
+    out->resident_table_bytes = p->table_bytes + p->commit_table_bytes;
     out->extra_table_windows = 0;
     for (uint32_t i = 0; i <= kExtraWindowMax - kExtraWindowMin; i++)
         if (p->extra_tables[i].table) {
             out->resident_table_bytes += p->extra_tables[i].bytes;
             out->extra_table_windows |= 1u << (kExtraWindowMin + i);
         }
-    out->working_bytes = WorkSet::bytes_per_blob() * p->max_batch;
+    out->working_bytes = WorkSet::bytes_per_blob() * p->max_batch + WorkSet::spread_bytes(p->max_batch);
     out->last_splits = p->last_splits;
     out->graphs_enabled = p->use_graphs ? 1u : 0u;
     out->graph_captures = p->graphs.captures;

@@ -140,7 +140,10 @@ struct WorkSet {
     uint32_t *queue_r = nullptr;  // bucket-reduction work counter, likewise
     Fr *scal = nullptr;
     G1X *u = nullptr, *buckets = nullptr, *cvals = nullptr;
-    uint64_t u_slots = 0;  // G1X entries of u
+    // G1X entries from u on that a batch in one stream may use for phase A's
+    // partials and sums: u's own, and the buckets behind them, which phase B
+    // fills once the ladder has read the sums.
+    uint64_t u_slots = 0;
     uint8_t *bucket_flags = nullptr;  // phase-B buckets to recompute with checked operations
     uint8_t *cval_flags = nullptr;    // reduced outputs to recompute likewise
     G1J *lad = nullptr;
@@ -150,9 +153,14 @@ struct WorkSet {
     uint8_t *cells = nullptr, *present = nullptr, *cells_out = nullptr;
     Fr *bufA = nullptr, *bufB = nullptr;
 
-    void allocate(uint32_t blobs_cap);
+    // spread: with room for the partials of kMinPartialBlobs blobs at least, so that
+    // one blob's MSMs can be cut into enough shares to fill the chip.  A set of
+    // fewer blobs without it is slower, not different.
+    void allocate(uint32_t blobs_cap, bool spread = true);
     ~WorkSet() { arena.release(); }
     static uint64_t bytes_per_blob();
+    // What `spread` takes beside blobs_cap * bytes_per_blob().
+    static uint64_t spread_bytes(uint32_t blobs_cap);
 };
 
 // Sub-streams a batch is spread over, with the events that fork them from
@@ -392,6 +400,7 @@ struct vkzg_prover {
 
     // Batch verification and commitments (created on first use).
     vkzg_amd::VerifyState *vfy = nullptr;
+    std::atomic<uint64_t> commit_table_bytes{0};  // its table of multiples of the setup's points
 
     // Per-stage timing of the last call (events on the stream of the first
     // sub-batch), accumulated over its chunks.

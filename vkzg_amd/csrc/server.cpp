@@ -306,14 +306,15 @@ vkzg_result vkzg_amd_server_new(vkzg_amd_server **out, vkzg_prover *p,
     uint32_t nslots = opts && opts->slots ? opts->slots : 2;
     const uint64_t budget = opts ? opts->hbm_budget_bytes : 0;
     const uint64_t per_blob = WorkSet::bytes_per_blob();
+    bool spread = true;
     if (budget) {
-        // Admission by HBM budget: the prover's resident phase-A tables count
-        // against it; then as many slots as fit, and smaller batches when
-        // even one full slot would not.
+        // Admission by HBM budget: the prover's resident tables count against
+        // it; then as many slots as fit, and smaller batches when even one
+        // full slot would not.
         uint64_t tables = 0;
         {
             std::lock_guard<std::mutex> lock(p->mu);
-            tables = p->table_bytes;
+            tables = p->table_bytes + p->commit_table_bytes;
             for (const auto &t : p->extra_tables) tables += t.bytes;
         }
         if (budget <= tables) return VKZG_ERR_MALLOC;
@@ -321,13 +322,17 @@ vkzg_result vkzg_amd_server_new(vkzg_amd_server **out, vkzg_prover *p,
         if (fit_blobs == 0) return VKZG_ERR_MALLOC;
         if (fit_blobs < sv->cap) sv->cap = (uint32_t)fit_blobs;
         nslots = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(nslots, fit_blobs / sv->cap));
+        // The room for a few blobs' partials that a smaller slot takes beside its
+        // working set only where the budget leaves it.
+        const uint64_t left = budget - tables - nslots * sv->cap * per_blob;
+        spread = nslots * WorkSet::spread_bytes(sv->cap) <= left;
     }
     sv->slot_bytes = per_blob * sv->cap;
     try {
         DeviceGuard guard(p->device);
         for (uint32_t i = 0; i < nslots; i++) {
             auto s = std::make_unique<Slot>();
-            s->ws.allocate(sv->cap);
+            s->ws.allocate(sv->cap, spread);
             s->ss.create();
             ck(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking));
             ck(hipEventCreateWithFlags(&s->done_ev, hipEventBlockingSync | hipEventDisableTiming));

@@ -330,6 +330,7 @@ void build_commit_table(vkzg_prover *p, PhaseATable &t) {
     if (W == 0) return;
     try {
         t = build_phase_a_table(p, window_plan(255 / W, 255 % W), p->srs, 4096);
+        p->commit_table_bytes = t.bytes;
     } catch (HipFail &) {
     }
 }
