@@ -188,3 +188,18 @@ with vkzg_amd.Prover(max_batch_size=20) as p:
                 assert st["slots"] * st["slot_bytes"] <= took <= st["slots"] * (st["slot_bytes"] + (16 << 20))
                 assert st["batch_blobs"] == min(blobs, int(room))
 """)
+
+
+def test_every_size_of_a_call_keeps_its_graphs(run):
+    """Cells with proofs at every batch size up to 160, again and again: captured
+    the first time only, though each call is two graphs."""
+    run("""
+L = vkzg_amd._lib.load()
+n = 160
+blobs, cells, proofs = (ctypes.create_string_buffer(n * k) for k in (BLOB, CELLS, 128 * 48))
+with vkzg_amd.Prover(max_batch_size=n) as p:
+    for rep in range(2):
+        for k in range(1, n + 1):
+            assert L.vkzg_amd_compute_cells_and_proofs(p.handle, cells, proofs, blobs, k) == 0
+    assert p.info()["graph_captures"] == 2 * n and p.info()["graph_replays"] == 2 * n
+""")

@@ -207,7 +207,8 @@ struct GraphCache {
     std::vector<Entry> entries;
     uint64_t tick = 0;
     uint64_t captures = 0, replays = 0;
-    static constexpr size_t kCapacity = 256;  // every batch size of both kinds up to 128
+    // Every batch size up to 256 of a call that takes two graphs (cells with proofs).
+    static constexpr size_t kCapacity = 512;
 
     // Enqueue `body(s)` on s through a cached graph.
     template <typename Body>
