@@ -203,3 +203,20 @@ with vkzg_amd.Prover(max_batch_size=n) as p:
             assert L.vkzg_amd_compute_cells_and_proofs(p.handle, cells, proofs, blobs, k) == 0
     assert p.info()["graph_captures"] == 2 * n and p.info()["graph_replays"] == 2 * n
 """)
+
+
+def test_large_copies_are_few(run):
+    """A copy of up to 12 MiB takes at most three DMAs each way: with more, calls on
+    buffers in use are slower than with one."""
+    run("""
+L = vkzg_amd._lib.load()
+n = 97
+cells, out = ctypes.create_string_buffer(n * CELLS), ctypes.create_string_buffer(n * CELLS)
+mask = ctypes.create_string_buffer(bytes([1] * 64 + [0] * 64) * n, n * 128)
+with vkzg_amd.Prover(max_batch_size=n) as p:
+    for k in list(range(1, 50)) + [96, 97]:
+        before = H.host_copies()
+        assert L.vkzg_recover_cells_batch(p.handle, out, cells, mask, k) == 0
+        dmas = H.host_copies() - before
+        assert dmas == 0 if k < 12 else dmas <= 6 if k <= 48 else dmas <= 2 * -(-k * CELLS // (4 << 20)), (k, dmas)
+""")

@@ -776,12 +776,17 @@ void enqueue_cells_and_proofs(vkzg_prover *p, WorkSet &ws, uint8_t *d_cells, hip
 constexpr size_t kPooledCopyMin = kKernelCopyMax;
 constexpr size_t kMinSlice = (size_t)1 << 20, kMaxSlice = (size_t)4 << 20;
 
-// About six slices: each costs its DMA about 10 us and a thread's wake-up as much.
-// With sixteen of 256 KiB up, recovery of 16 blobs between buffers in use took 679
-// us where a DMA per direction took 410; with these 440, and 64 blobs 1095 against
-// 1130.
+// Three slices (more only past 12 MiB), since each costs its DMA about 10 us; on the
+// way out each is copied in three parts, since a copy is what takes long, above
+// all into new pages.  Recovery, us, between buffers in use and into new ones: with
+// six slices copied whole 453 and 856 (16 blobs), 584 and 1056 (24), 679 and 1324
+// (32), 1122 and 2379 (64); with three 434 and 814, 560 and 1098, 668 and 1380, 1152
+// and 2870; with three in three parts 405 and 656, 511 and 872, 611 and 1064, 1065 and
+// 1881; one DMA per direction with the copies before and after it 418 and 1450, 541
+// and 2130, 659 and 2830, 1145 and 5650.
+constexpr size_t kSlices = 3, kSliceParts = 3;
 size_t copy_slice(size_t bytes) {
-    const size_t s = (bytes / 6 + 4095) & ~(size_t)4095;
+    const size_t s = (bytes / kSlices + 4095) & ~(size_t)4095;
     return std::max(kMinSlice, std::min(kMaxSlice, s));
 }
 
@@ -815,13 +820,17 @@ void stage_upload(vkzg_prover *p, uint8_t *dev, uint8_t *pinned, const uint8_t *
     if (failed) throw HipFail{};
 }
 
-// dev -> pinned staging, enqueued on s in slices with an event behind each
-// (small ones whole, with one event); `more`: a device -> pinned copy that goes
-// along, ahead of the first event.
+// dev -> pinned staging, enqueued on s: small ones whole, others in slices with an
+// event behind each; `more`: a device -> pinned copy that goes along, ahead of the
+// first event.
 void start_download(vkzg_prover *p, uint8_t *pinned, const uint8_t *dev, size_t bytes, hipStream_t s,
                     const CopyPart &more = CopyPart{}) {
-    const size_t slice = bytes < kPooledCopyMin ? bytes : copy_slice(bytes);
-    if (bytes >= kPooledCopyMin) enqueue_copies(more, CopyPart{}, hipMemcpyDeviceToHost, s);
+    if (bytes < kPooledCopyMin) {
+        enqueue_copies(CopyPart{pinned, dev, bytes}, more, hipMemcpyDeviceToHost, s);
+        return;
+    }
+    enqueue_copies(more, CopyPart{}, hipMemcpyDeviceToHost, s);
+    const size_t slice = copy_slice(bytes);
     size_t k = 0;
     for (size_t off = 0; off < bytes; off += slice, k++) {
         if (k == p->download_ev.size()) {
@@ -829,30 +838,34 @@ void start_download(vkzg_prover *p, uint8_t *pinned, const uint8_t *dev, size_t 
             ck(hipEventCreateWithFlags(&e, hipEventDisableTiming));
             p->download_ev.push_back(e);
         }
-        if (bytes < kPooledCopyMin)
-            enqueue_copies(CopyPart{pinned, dev, bytes}, more, hipMemcpyDeviceToHost, s);
-        else
-            ck(hipMemcpyAsync(pinned + off, dev + off, std::min(slice, bytes - off), hipMemcpyDeviceToHost, s));
+        ck(hipMemcpyAsync(pinned + off, dev + off, std::min(slice, bytes - off), hipMemcpyDeviceToHost, s));
         ck(hipEventRecord(p->download_ev[k], s));
     }
 }
 
-// The slices of start_download -> host, each once its DMA is done.
-void finish_download(vkzg_prover *p, uint8_t *host, const uint8_t *pinned, size_t bytes) {
-    const size_t slice = bytes < kPooledCopyMin ? bytes : copy_slice(bytes);
-    std::atomic<bool> failed{false};
-    const auto part = [&](size_t k) {
-        const size_t off = k * slice;
-        if (hipEventSynchronize(p->download_ev[k]) != hipSuccess) failed = true;
-        else std::memcpy(host + off, pinned + off, std::min(slice, bytes - off));
-    };
+// Until the first slice of start_download on s, and what went along, is there: of
+// a small one all of s.
+void wait_download(vkzg_prover *p, size_t bytes, hipStream_t s) {
+    ck(bytes < kPooledCopyMin ? hipStreamSynchronize(s) : hipEventSynchronize(p->download_ev[0]));
+}
+
+// The slices of start_download on s -> host, each once its DMA is done.
+void finish_download(vkzg_prover *p, uint8_t *host, const uint8_t *pinned, size_t bytes, hipStream_t s) {
+    wait_download(p, bytes, s);
     if (bytes < kPooledCopyMin) {
-        part(0);
-    } else {
-        // the copy threads are woken when there is something to copy
-        if (hipEventSynchronize(p->download_ev[0]) != hipSuccess) throw HipFail{};
-        p->copiers.run((bytes + slice - 1) / slice, part);
+        std::memcpy(host, pinned, bytes);
+        return;
     }
+    // the copy threads are woken when there is something to copy
+    const size_t slice = copy_slice(bytes), part = (slice / kSliceParts + 4095) & ~(size_t)4095;
+    std::atomic<bool> failed{false};
+    p->copiers.run((bytes + slice - 1) / slice * kSliceParts, [&](size_t i) {
+        const size_t k = i / kSliceParts, end = std::min(bytes, (k + 1) * slice);
+        const size_t off = k * slice + i % kSliceParts * part;
+        if (off >= end) return;  // of a short last slice
+        if (hipEventSynchronize(p->download_ev[k]) != hipSuccess) failed = true;
+        else std::memcpy(host + off, pinned + off, std::min(part, end - off));
+    });
     if (failed) throw HipFail{};
 }
 
@@ -1207,7 +1220,7 @@ vkzg_result vkzg_recover_cells_batch(vkzg_prover *p, uint8_t *cells_out, const u
             enqueue_recovery(p, p->ws, p->streams, p->ws.cells_out, p->ws.cells, p->ws.present, nb,
                              s, clk, tn, &p->graphs);
             start_download(p, p->h_out, p->ws.cells_out, nb * kCellsBytes, s);
-            finish_download(p, cells_out + done * kCellsBytes, p->h_out, nb * kCellsBytes);
+            finish_download(p, cells_out + done * kCellsBytes, p->h_out, nb * kCellsBytes, s);
             ck(hipStreamSynchronize(s));
             clk.finish();
             done += nb;
@@ -1242,8 +1255,7 @@ vkzg_result vkzg_amd_compute_cells_and_proofs(vkzg_prover *p, uint8_t *cells, ui
                 ck(hipStreamWaitEvent(c, p->results_ready, 0));
                 start_download(p, p->h_out, p->ws.cells_out, nb * kCellsBytes, c,
                                CopyPart{p->h_err, p->ws.err, nb * 4});
-                // behind the flags: the first slice
-                if (hipEventSynchronize(p->download_ev[0]) != hipSuccess) throw HipFail{};
+                wait_download(p, nb * kCellsBytes, c);
             } else {
                 enqueue_copies(CopyPart{p->h_err, p->ws.err, nb * 4}, CopyPart{}, hipMemcpyDeviceToHost, s);
             }
@@ -1252,7 +1264,8 @@ vkzg_result vkzg_amd_compute_cells_and_proofs(vkzg_prover *p, uint8_t *cells, ui
             if (!cells) ck(hipStreamSynchronize(s));
             bool bad = false;
             for (uint32_t b = 0; b < nb; b++) bad |= p->h_err[b] != 0;
-            if (cells && !bad) finish_download(p, cells + done * kCellsBytes, p->h_out, nb * kCellsBytes);
+            if (cells && !bad)
+                finish_download(p, cells + done * kCellsBytes, p->h_out, nb * kCellsBytes, p->copy_stream);
             if (cells) ck(hipStreamSynchronize(p->copy_stream));
             ck(hipStreamSynchronize(s));
             if (bad) return VKZG_ERR_INVALID_BLOB;
@@ -1299,7 +1312,7 @@ vkzg_result vkzg_amd_recover_cells_and_proofs(vkzg_prover *p, uint8_t *cells_out
                                      s, one, &p->graphs);
             enqueue_copies(CopyPart{p->h_proofs, p->ws.proofs, nb * kProofBytes}, CopyPart{},
                            hipMemcpyDeviceToHost, s);
-            finish_download(p, cells_out + done * kCellsBytes, p->h_out, nb * kCellsBytes);
+            finish_download(p, cells_out + done * kCellsBytes, p->h_out, nb * kCellsBytes, p->copy_stream);
             ck(hipStreamSynchronize(p->copy_stream));
             ck(hipStreamSynchronize(s));
             std::memcpy(proofs_out + done * kProofBytes, p->h_proofs, nb * kProofBytes);
