@@ -469,9 +469,10 @@ def main():
         rec_stages = prover.last_stage_times()
         secondary["recovery_stage_ms"] = rec_stages
         prover.set_stage_timing(False)
-        # Each of the five recovery kernels reads 256 KiB and writes 256 KiB
-        # per blob (8192 values of 32 bytes, or the 2048-byte cells of the
-        # first and last), plus the 128-byte mask of the first and third.
+        # Each of the recovery kernels (three by default) reads 256 KiB and
+        # writes 256 KiB per blob (8192 values of 32 bytes, or the 2048-byte
+        # cells of the first and last); the 128-byte mask and 4 KiB of
+        # vanishing values between the first two are not counted.
         pass_bytes = nr * 2 * 8192 * 32
         gbps = {k: pass_bytes / (v * 1e-3) / 1e9 for k, v in rec_stages.items() if v > 0}
         secondary["recovery_pass_hbm"] = {

@@ -62,7 +62,6 @@ VKZG_DEV G1J g1j_identity() {
     r.z = fp_zero();
     return r;
 }
-VKZG_DEV bool g1j_is_identity(const G1J &p) { return fp_is_zero(p.z); }
 VKZG_DEV G1J g1j_from_affine(const G1A &a) {
     if (g1a_is_identity(a)) return g1j_identity();
     G1J r;

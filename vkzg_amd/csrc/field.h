@@ -43,40 +43,6 @@ VKZG_DEV void reduce_once(uint32_t *r, const uint32_t *t, const uint32_t (&m)[N]
     for (int i = 0; i < N; i++) r[i] = br ? t[i] : d[i];
 }
 
-template <int N>
-VKZG_DEV void add_mod(uint32_t *r, const uint32_t *a, const uint32_t *b, const uint32_t (&m)[N]) {
-    uint32_t t[N];
-    uint32_t c = 0;
-#pragma unroll
-    for (int i = 0; i < N; i++) {
-        const uint64_t s = (uint64_t)a[i] + b[i] + c;
-        t[i] = (uint32_t)s;
-        c = (uint32_t)(s >> 32);
-    }
-    // a + b < 2m < 2^(32N): no carry out of the top limb.
-    reduce_once<N>(r, t, m);
-}
-
-template <int N>
-VKZG_DEV void sub_mod(uint32_t *r, const uint32_t *a, const uint32_t *b, const uint32_t (&m)[N]) {
-    uint32_t t[N];
-    uint32_t br = 0;
-#pragma unroll
-    for (int i = 0; i < N; i++) {
-        const uint64_t s = (uint64_t)a[i] - b[i] - br;
-        t[i] = (uint32_t)s;
-        br = (uint32_t)(s >> 32) & 1u;
-    }
-    const uint32_t mask = 0u - br;
-    uint32_t c = 0;
-#pragma unroll
-    for (int i = 0; i < N; i++) {
-        const uint64_t s = (uint64_t)t[i] + (m[i] & mask) + c;
-        r[i] = (uint32_t)s;
-        c = (uint32_t)(s >> 32);
-    }
-}
-
 // acc (64-bit) += x * y and hi += carry-out: v_mad_u64_u32 leaves its carry
 // in VCC and v_addc folds it into the third accumulator word, two VALU
 // instructions per limb product (the compiler's own lowering of the same
@@ -280,14 +246,6 @@ VKZG_DEV void mont_mul_cios(uint32_t *r, const uint32_t *a, const uint32_t *b,
 }
 
 template <int N>
-VKZG_DEV bool limbs_zero(const uint32_t *a) {
-    uint32_t acc = 0;
-#pragma unroll
-    for (int i = 0; i < N; i++) acc |= a[i];
-    return acc == 0;
-}
-
-template <int N>
 VKZG_DEV bool limbs_eq(const uint32_t *a, const uint32_t *b) {
     uint32_t acc = 0;
 #pragma unroll
@@ -344,7 +302,6 @@ VKZG_DEV Fr fr_sub(const Fr &a, const Fr &b) {
     return r;
 }
 VKZG_DEV Fr fr_neg(const Fr &a) { return fr_sub(fr_zero(), a); }
-VKZG_DEV bool fr_is_zero(const Fr &a) { return limbs_zero<8>(a.v); }
 
 // Montgomery -> canonical (multiply by plain 1).
 VKZG_DEV Fr fr_to_canonical(const Fr &a) {

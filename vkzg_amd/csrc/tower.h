@@ -49,7 +49,6 @@ VKZG_DEV Fp2 fp2_mul(const Fp2 &a, const Fp2 &b) {
 VKZG_DEV Fp2 fp2_sqr(const Fp2 &a) {
     return {fp_mul(fp_add_raw(a.c0, a.c1), fp_sub(a.c0, a.c1)), fp_mul(fp_dbl_raw(a.c0), a.c1)};
 }
-VKZG_DEV Fp2 fp2_mul_fp(const Fp2 &a, const Fp &s) { return {fp_mul(a.c0, s), fp_mul(a.c1, s)}; }
 // a * xi = (a0 - a1) + (a0 + a1) u
 VKZG_DEV Fp2 fp2_mul_xi(const Fp2 &a) { return {fp_sub(a.c0, a.c1), fp_add(a.c0, a.c1)}; }
 // 1/a = conj(a) / (a0^2 + a1^2); 0 -> 0
@@ -240,9 +239,6 @@ __device__ __forceinline__ void fp12_reduce(Fp *a) {
     __syncthreads();
 }
 
-VKZG_DEV void fp12_set_one(Fp *a, uint32_t t) {
-    if (t < 12) a[t] = t == 0 ? fp_one() : fp_zero();
-}
 // w -> -w: odd powers negated (the p^6-power Frobenius)
 VKZG_DEV void fp12_conj_to(Fp *dst, const Fp *a, uint32_t t) {
     if (t < 12) dst[t] = ((t >> 1) & 1u) ? fp_neg(a[t]) : a[t];
