@@ -12,7 +12,7 @@
 //                 144 lanes and every cyclotomic square over 96 (tower.h); the
 //                 other blocks are the subgroup checks of the batch's points.
 // The chain of Fp12 products is the time of both, ~75 Miller steps, 315
-// cyclotomic squares and 40 products: 1141 -> 935 us for k_pair_final, 8 -> 30 us
+// cyclotomic squares and 40 products: 1141 -> 842 us for k_pair_final, 8 -> 30 us
 // for k_pair_lines.
 //
 // Miller loop over |z| = 0xd201000000010000 from the top bit down: a

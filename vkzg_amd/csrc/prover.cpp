@@ -1325,10 +1325,12 @@ vkzg_result vkzg_amd_recover_cells_and_proofs(vkzg_prover *p, uint8_t *cells_out
 }
 
 // The device-pointer entry points launch kernel by kernel.  A graph of such a call
-// is good for its buffers only, and saves nothing when it is replayed: recovery of
-// 64 blobs 143 us launched, 155 replayed, 230 to 260 with the capture that every
-// new buffer takes; proofs of 1 to 256 blobs alike within 1% launched and replayed,
-// 110 to 450 us more with a capture.
+// is good for its buffers' addresses only, and saves nothing when it is replayed:
+// recovery of 64 blobs 143 us launched, 155 replayed; proofs of 1 to 256 blobs alike
+// within 1%.  Its capture, at addresses not seen before, took 80 to 110 us in
+// recovery and 110 to 410 us in proofs; a caller whose allocator hands out the same
+// addresses again replayed it, and gains nothing here on the first pass over new
+// inputs.
 vkzg_result vkzg_amd_compute_proofs_device(vkzg_prover *p, void *d_proofs, const void *d_blobs,
                                            size_t num_blobs, void *hip_stream) {
     if (!p || !d_proofs || !d_blobs) return VKZG_ERR_BADARGS;
